@@ -71,6 +71,7 @@ SYMBOLS = {
 
 # what include/fbgemm_amd_bench.h declares: the switches inside libfbgemm_amd.so ...
 BENCH_SWITCHES = {
+    "fbgemm_amd_set_burst": (C.c_int, [_I32]),
     "fbgemm_amd_set_lean": (C.c_int, [_I32]),
     "fbgemm_amd_set_narrow_below_waves": (C.c_int, [_I32]),
     "fbgemm_amd_set_wide4": (C.c_int, [_I32]),

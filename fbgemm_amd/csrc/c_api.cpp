@@ -222,6 +222,46 @@ int wide4_mode() {
   return m < 0 ? 0 : (m > 2 ? 2 : m);
 }
 
+// Which launches the burst kernel (lookup_burst.h) takes, and in which form. `bags`: of all tables;
+// us of the single-table kernel over 1 M uniform rows, other kernels -> burst kernel:
+//                       10 bags x 100   1024 x 20      4096 x 20      8192 x 20      8192 x 10
+//   4-bit, 128 wide     47.7 -> 10.8    17.3 -> 9.4    19.0 -> 12.1   20.6 -> 19.5   14.6 -> 16.3
+//   8-bit, 100 wide     47.7 -> 11.2    17.4 -> 9.5    19.9 -> 12.0   32.0 -> 19.2   23.7 -> 15.7
+//   fp16, 256 wide      57.1 -> 14.3    20.0 -> 10.0   25.4 -> 17.3   28.0 -> 25.9   18.7 -> 19.7
+//   8-bit, 512 wide     52.0 -> 13.6    18.4 -> 10.9   20.4 -> 24.0   30.8 -> 37.7   19.9 -> 27.2
+// It is bound by how many workgroups the device holds at a time, so the line lies at workgroups:
+// 4096 (16 per compute unit: all resident at once), and 8192 where bags are long enough to need
+// several rounds in the other kernels and a workgroup covers the whole row.
+// Four waves per bag pay while all such workgroups are resident together (four per compute unit:
+// 1024; 1024 bags x 100: 22.0 -> 13.9) and, for long bags, in two rounds of them (2048 x 100: 24.9 -> 21.9).
+struct Burst {
+  int waves = 0; // 0: another kernel takes the launch
+  int lds_bytes = 0;
+};
+// 1 / 4: every launch it can take goes to the burst kernel with that many waves per bag, 0: none does,
+// -1: by the rule (tests: fbgemm_amd_set_burst).
+int g_burst_override = -1;
+constexpr int BURST_COLS = 256;
+Burst plan_burst(int64_t bags, int32_t T, int32_t max_D, int64_t lookups) {
+  Burst b;
+  const int64_t windows = ((int64_t)max_D + BURST_COLS - 1) / BURST_COLS;
+  if (g_burst_override == 0 || narrow_below_waves() == 0 || bags <= 0 || T > 65535 || windows > 65535 ||
+      (g_burst_override < 0 && lookups >= SORT_MIN_LOOKUPS)) // those launches order their bags
+    return b;
+  const int64_t groups = bags * windows, avg_len = lookups / bags;
+  if (g_burst_override > 0) {
+    b.waves = g_burst_override;
+  } else if (groups <= 4096 || (groups <= 8192 && windows == 1 && avg_len >= 16)) {
+    b.waves = (groups <= 1024 && avg_len >= 16) || (groups <= 2048 && avg_len >= 64) ? 4 : 1;
+  }
+  b.lds_bytes = b.waves == 4 ? 32768 : (groups <= 2048 ? 16384 : 8192);
+  return b;
+}
+// Where the burst kernel would take the launch, bags shorter than this are not cut into segments
+// (tolerance-grade mode): 1000 bags x 100 of a 4-bit table 23.4 us in segments, 13.7 us whole; x 400
+// 46 and 38 us, 10 x 2000 42 and 111 us.
+constexpr int64_t SPLIT_MIN_LEN_OVER_BURST = 256;
+
 struct DeviceScratch {
   Status* status = nullptr;
   int64_t* offsets = nullptr; // lengths -> offsets
@@ -514,10 +554,12 @@ int spmdm_launch_impl(
   // 4- and 8-bit rows only: every other row type is summed the reference's way in either mode,
   // in one piece.
   int K = 1;
+  const Burst burst = plan_burst(output_size, 1, d.D, index_size);
   if (!noalloc && cfg->accumulate == FBGEMM_AMD_ACC_FAST && !cfg->is_weight_positional && output_size * 32 <= 0x7fffffffLL &&
       (ty == ST_INT4 || ty == ST_INT8)) {
     const int G16 = bags_per_wave(d.lanes, d.packed);
     K = split_factor((output_size + G16 - 1) / G16, index_size / output_size);
+    if (burst.waves && index_size / output_size < SPLIT_MIN_LEN_OVER_BURST) K = 1;
   }
   const int64_t pooled_bags = output_size * K;       // what the lookup kernel sees as bags
   const int64_t pooled_stride = K > 1 ? D : out_stride; // segments' sums are rows of D floats
@@ -558,7 +600,7 @@ int spmdm_launch_impl(
 
   // Ordering the bags pays once several waves' worth of bags and enough lookups exist
   // (the scheduler launch costs 6-8 us and buys ~5 % of the lookup: it pays from a few million lookups on)
-  const bool sort = K == 1 && sort_bags_default() && output_size > 2 * G && index_size >= (int64_t)SORT_MIN_LOOKUPS;
+  const bool sort = K == 1 && !burst.waves && sort_bags_default() && output_size > 2 * G && index_size >= (int64_t)SORT_MIN_LOOKUPS;
   if (cfg->use_offsets) {
     a.offsets = d_offsets_or_lengths;
     a.off64 = cfg->offset_bits == 64;
@@ -622,7 +664,9 @@ int spmdm_launch_impl(
                                     cfg->normalize_by_lengths != 0, d_out, cfg->output_ty, out_stride, stream));
     return 0;
   }
-  if (lean_enabled() && !cfg->is_weight_positional && lean_shape(d))
+  if (burst.waves)
+    HIP_TRY(launch_lookup_burst(a, cfg->index_bits == 64, d.D, burst.waves, burst.lds_bytes, stream));
+  else if (lean_enabled() && !cfg->is_weight_positional && lean_shape(d))
     HIP_TRY(launch_lookup_lean(a, cfg->index_bits == 64, cfg->accumulate != FBGEMM_AMD_ACC_FAST, false, stream));
   else
     HIP_TRY(launch_lookup(a, cfg->index_bits == 64, stream));
@@ -635,6 +679,11 @@ extern "C" {
 
 int fbgemm_amd_set_narrow_below_waves(int32_t waves) {
   g_narrow_override = waves < 0 ? -1 : waves;
+  return 0;
+}
+
+int fbgemm_amd_set_burst(int32_t waves) {
+  g_burst_override = waves == 0 || waves == 1 || waves == 4 ? waves : -1;
   return 0;
 }
 
@@ -1187,12 +1236,14 @@ int tbe_forward_impl(
   // (Only when every table has rows the tolerance-grade arithmetic applies to: fp16 / fp32 / 2-bit
   // / odd-shaped tables are summed the reference's way in either mode, and a bag cut into
   // segments is not.)
+  const Burst burst = plan_burst((int64_t)plan->T * B, plan->T, plan->max_D, indices_numel);
   bool all_fast_rows = true;
   for (const TableDesc& d : plan->tables) all_fast_rows = all_fast_rows && (d.ty == ST_INT4 || d.ty == ST_INT8);
   if (allow_split && plan->accumulate == FBGEMM_AMD_ACC_FAST && all_fast_rows && (int64_t)B * 32 <= 0x7fffffffLL) {
     int64_t wide_waves = 0;
     for (const TableDesc& d : plan->tables) wide_waves += (B + d.bags - 1) / d.bags;
-    const int K = split_factor(wide_waves, indices_numel / ((int64_t)plan->T * B));
+    int K = split_factor(wide_waves, indices_numel / ((int64_t)plan->T * B));
+    if (burst.waves && indices_numel / ((int64_t)plan->T * B) < SPLIT_MIN_LEN_OVER_BURST) K = 1;
     if (K > 1) {
       if (int rc = shared.begin(plan, stream)) return rc;
       hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
@@ -1251,7 +1302,9 @@ int tbe_forward_impl(
     // the lane shapes depend on B and (through the average bag length) on the number of indices:
     // remember the choice of the last forward with the same B and about the same indices
     const int64_t bucket = indices_numel >> 16;
-    if (plan->shape_B == B && plan->shape_bucket == bucket && plan->shape_narrow == narrow_below_waves()) {
+    if (burst.waves && !d_q8_out) {
+      variant = 3; // the burst kernel: no lane shapes, work lists or bag order
+    } else if (plan->shape_B == B && plan->shape_bucket == bucket && plan->shape_narrow == narrow_below_waves()) {
       variant = plan->shape_variant;
     } else {
       int64_t wide_waves = 0;
@@ -1279,7 +1332,7 @@ int tbe_forward_impl(
         return fail(FBGEMM_AMD_E_ARG, "the first forward of a plan with a new batch size allocates its work lists: "
                     "run it once outside the stream capture");
       std::vector<int> lean_members, general_members;
-      for (int t = 0; t < plan->T; ++t) (lean && lean_shape(tables[t]) ? lean_members : general_members).push_back(t);
+      for (int t = 0; t < plan->T && variant != 3; ++t) (lean && lean_shape(tables[t]) ? lean_members : general_members).push_back(t);
       fbgemm_amd_tbe_plan::Work nw;
       // what is allocated below goes back when a later step fails
       struct Undo {
@@ -1299,7 +1352,7 @@ int tbe_forward_impl(
         nw.n_general_tables = (int32_t)ids.size();
       }
       // the bag order: one buffer for this stream, one ahead for the next stream
-      for (int k = 0; k < 2; ++k)
+      for (int k = 0; k < 2 && variant != 3; ++k)
         if (int rc = make_order_slot(nw, k, plan->T, B)) return rc;
       nw.order_stream[0] = stream;
       nw.order_claimed[0] = true;
@@ -1328,7 +1381,7 @@ int tbe_forward_impl(
     // of this plan on the streams that share it must not overlap
     fbgemm_amd_tbe_plan::Work& W = it->second;
     constexpr int NS = fbgemm_amd_tbe_plan::ORDER_SLOTS;
-    order_slot = -1;
+    order_slot = variant == 3 ? 0 : -1;
     for (int k = 0; k < NS && order_slot < 0; ++k)
       if (W.order_claimed[k] && W.order_stream[k] == stream) order_slot = k;
     for (int k = 0; k < NS && order_slot < 0; ++k)
@@ -1339,7 +1392,7 @@ int tbe_forward_impl(
         order_slot = k;
       }
     if (order_slot < 0) order_slot = 0;
-    if (!W.order_claimed[order_slot]) {
+    if (variant != 3 && !W.order_claimed[order_slot]) {
       W.order_claimed[order_slot] = true;
       W.order_stream[order_slot] = stream;
       // keep one buffer ahead for the next stream, when that is possible now
@@ -1450,6 +1503,10 @@ int tbe_forward_impl(
   a.status = (Status*)d_status;
   a.fp8_shift = plan->fp8_shift;
   a.fp8_mult = plan->fp8_mult;
+  if (variant == 3) {
+    HIP_TRY(launch_lookup_burst(a, index_bits == 64, plan->max_D, burst.waves, burst.lds_bytes, stream));
+    return 0;
+  }
   if (sort_bags_default() && indices_numel >= (int64_t)SORT_MIN_LOOKUPS) {
     if (!reuse_order) HIP_TRY(launch_bag_order(d_offsets, offset_bits == 64, B, plan->T, w.d_order[order_slot], stream));
     a.order = w.d_order[order_slot];

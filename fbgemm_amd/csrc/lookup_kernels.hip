@@ -191,6 +191,20 @@ hipError_t launch_lookup(const LookupArgs& a, bool idx64, hipStream_t stream) {
   return idx64 ? launch_lookup_i64(a, (unsigned)blocks, stream) : launch_lookup_i32(a, (unsigned)blocks, stream);
 }
 
+hipError_t launch_lookup_burst_i64(const LookupArgs& a, dim3 grid, bool four_waves, int lds_bytes, hipStream_t stream);
+hipError_t launch_lookup_burst_i32(const LookupArgs& a, dim3 grid, bool four_waves, int lds_bytes, hipStream_t stream);
+
+// The burst kernel (lookup_burst.h): a workgroup per bag and window of 256 columns. max_D: the widest
+// table of the launch; waves: 1 or 4 per workgroup; lds_bytes: what a workgroup's staged rows may take.
+hipError_t launch_lookup_burst(const LookupArgs& a, bool idx64, int32_t max_D, int waves, int lds_bytes, hipStream_t stream) {
+  if (a.B <= 0 || a.T <= 0) return hipSuccess;
+  const int windows = (max_D + 255) / 256;
+  // 8 rows of the widest window (256 columns of fp32) have to fit
+  if (a.T > 65535 || windows > 65535 || lds_bytes < 8192 || (waves != 1 && waves != 4)) return hipErrorInvalidValue;
+  const dim3 grid((unsigned)a.B, (unsigned)a.T, (unsigned)windows);
+  return idx64 ? launch_lookup_burst_i64(a, grid, waves == 4, lds_bytes, stream) : launch_lookup_burst_i32(a, grid, waves == 4, lds_bytes, stream);
+}
+
 hipError_t launch_bag_order(const void* offsets, bool off64, int32_t B, int32_t T, BagEntry* order, hipStream_t stream) {
   if (T <= 0 || B <= 0) return hipSuccess;
   // Tables of up to SORT_WHOLE_TABLE bags are ordered as a whole: their launches are a few rounds of

@@ -158,6 +158,10 @@ hipError_t launch_lookup_lean(const LookupArgs& a, bool idx64, bool, bool wide4,
   g_last_lean_wide4 = wide4 ? 1 : 0;
   return launch_lookup(a, idx64, s);
 }
+hipError_t launch_lookup_burst(const LookupArgs& a, bool idx64, int32_t, int, int lds_bytes, hipStream_t s) {
+  if (lds_bytes < 8192) return hipErrorInvalidValue; // eight rows of the widest window
+  return launch_lookup(a, idx64, s);
+}
 hipError_t launch_lengths_to_offsets(const void*, bool, int64_t n, int64_t* offsets, hipStream_t) {
   for (int64_t i = 0; i <= n; ++i) offsets[i] = 0; // the whole buffer must be there
   return LAUNCHED();
