@@ -263,7 +263,9 @@ Burst plan_burst(int64_t bags, int32_t T, int32_t max_D, int64_t lookups) {
 constexpr int64_t SPLIT_MIN_LEN_OVER_BURST = 256;
 
 struct DeviceScratch {
-  Status* status = nullptr;
+  FlaggedStatus* status = nullptr; // clear between the calls that use it
+  int32_t* flag = nullptr;         // pinned: what a report sets besides the block
+  bool status_dirty = true;        // a call is using the block, or ended without reading it
   int64_t* offsets = nullptr; // lengths -> offsets
   int64_t offsets_cap = 0;
   BagEntry* order = nullptr;  // bag order of single-table calls
@@ -328,7 +330,16 @@ int get_scratch(DeviceScratch** out) {
       s = idle.back();
       idle.pop_back();
     } else {
-      HIP_TRY(hipMalloc((void**)&s.status, sizeof(Status)));
+      int32_t* flag = nullptr;
+      HIP_TRY(hipHostMalloc((void**)&flag, 64, hipHostMallocCoherent));
+      const hipError_t e = hipMalloc((void**)&s.status, sizeof(FlaggedStatus));
+      if (e != hipSuccess) {
+        (void)hipHostFree(flag);
+        s.status = nullptr;
+        return fail(FBGEMM_AMD_E_HIP, "hipMalloc of a status block: %s", hipGetErrorString(e));
+      }
+      s.flag = flag;
+      s.status_dirty = true;
     }
   }
   *out = &s;
@@ -393,6 +404,41 @@ int fbgemm_amd_status_read(const void* d_status, void* stream, int32_t* bits, in
   HIP_TRY(hipStreamSynchronize((hipStream_t)stream));
   if (bits) *bits = h.bits;
   if (first_bad_pos) *first_bad_pos = h.first_bad_pos == ~0ull ? -1 : (int64_t)h.first_bad_pos;
+  return 0;
+}
+
+int fbgemm_amd_status_begin(void** d_status) {
+  if (!d_status) return fail(FBGEMM_AMD_E_ARG, "d_status is null");
+  std::lock_guard<std::mutex> lk(g_mu);
+  DeviceScratch* s;
+  if (int rc = get_scratch(&s)) return rc;
+  if (s->status_dirty) { // new, or left behind by a call that failed on its way: nothing may write it any more
+    HIP_TRY(hipDeviceSynchronize());
+    const FlaggedStatus clear{Status{0, STATUS_FLAGGED, ~0ull}, s->flag};
+    HIP_TRY(hipMemcpy(s->status, &clear, sizeof(clear), hipMemcpyHostToDevice));
+    *s->flag = 0;
+  }
+  s->status_dirty = true; // until fbgemm_amd_status_end has looked
+  *d_status = s->status;
+  return 0;
+}
+
+int fbgemm_amd_status_end(void* stream, int32_t* bits, int64_t* first_bad_pos) {
+  DeviceScratch* s;
+  {
+    std::lock_guard<std::mutex> lk(g_mu);
+    if (int rc = get_scratch(&s)) return rc;
+  }
+  HIP_TRY(hipStreamSynchronize((hipStream_t)stream));
+  int32_t b = 0;
+  int64_t pos = -1;
+  if (__atomic_load_n(s->flag, __ATOMIC_ACQUIRE)) { // the block stays dirty: the next call clears it
+    if (int rc = fbgemm_amd_status_read(s->status, stream, &b, &pos)) return rc;
+  } else {
+    s->status_dirty = false;
+  }
+  if (bits) *bits = b;
+  if (first_bad_pos) *first_bad_pos = pos;
   return 0;
 }
 
@@ -722,19 +768,18 @@ int fbgemm_amd_spmdm_run(
     int64_t data_size, const void* d_input, const void* d_indices,
     const void* d_offsets_or_lengths, const float* d_weights, void* d_out,
     const int32_t* d_remap, void* stream) {
-  Status* st;
-  {
-    std::lock_guard<std::mutex> lk(g_mu);
-    DeviceScratch* s;
-    if (int rc = get_scratch(&s)) return rc;
-    st = s->status;
+  if (output_size == 0 && index_size > 0 && data_size >= 0) { // known without a launch (see spmdm_launch_impl)
+    if (int rc = check_cfg(cfg)) return rc;
+    HIP_TRY(hipStreamSynchronize((hipStream_t)stream));
+    return cfg->no_bag ? 1 : 0;
   }
-  if (int rc = fbgemm_amd_status_clear(st, stream)) return rc;
+  void* st;
+  if (int rc = fbgemm_amd_status_begin(&st)) return rc;
   if (int rc = fbgemm_amd_spmdm_launch(cfg, output_size, index_size, data_size, d_input, d_indices,
                                       d_offsets_or_lengths, d_weights, d_out, d_remap, st, stream))
     return rc;
   int32_t bits = 0;
-  if (int rc = fbgemm_amd_status_read(st, stream, &bits, nullptr)) return rc;
+  if (int rc = fbgemm_amd_status_end(stream, &bits, nullptr)) return rc;
   return bits == 0 ? 1 : 0;
 }
 
@@ -1875,13 +1920,14 @@ int fbgemm_amd_compressed_indices_remap(
   std::lock_guard<std::mutex> lk(g_mu);
   DeviceScratch* s;
   if (int rc = get_scratch(&s)) return rc;
+  if (!d_status) s->status_dirty = true; // what is recorded there is nobody's
   // one scratch buffer: n + 1 running counts (int64), then the n mapped rows (int32)
   if (int rc = grow(&s->fixed, &s->fixed_cap, (n + 1) + (n + 1) / 2 + 1, stream)) return rc;
   if (int rc = grow(&s->partial, &s->partial_cap, prune_partials(n + 1), stream)) return rc;
   HIP_TRY(launch_compressed_indices_remap(d_indices, index_bits == 64, d_mapping, mapping_numel, d_offsets, offsets_numel,
                                           d_weights, first, n, d_out_indices, d_out_offsets, d_out_weights, s->fixed,
                                           s->partial, reinterpret_cast<int32_t*>(s->fixed + n + 1),
-                                          d_status ? (Status*)d_status : s->status, stream));
+                                          d_status ? (Status*)d_status : &s->status->st, stream));
   return 0;
 }
 

@@ -158,7 +158,7 @@ __global__ __launch_bounds__(SCAN_THREADS) void bounds_fix_offsets_kernel(
     }
   }
   if (mode == 1 && bad) atomicAdd(&bad_count, bad);
-  if (mode == 0 && err) atomicOr(&status->bits, err);
+  if (mode == 0 && err) status_or(status, err);
   __syncthreads();
   if (mode == 1 && threadIdx.x == 0 && bad_count) atomicAdd(reinterpret_cast<unsigned long long*>(warning), (unsigned long long)bad_count);
 }
@@ -195,8 +195,7 @@ __global__ __launch_bounds__(256) void bounds_check_bags_kernel(
       if (idx == -1) continue; // pruned row
       if (idx < 0 || idx >= num_rows) {
         if (mode == 0) {
-          atomicOr(&status->bits, ERR_INDEX_OUT_OF_RANGE);
-          atomicMin(&status->first_bad_pos, (unsigned long long)i);
+          status_index(status, i);
         } else {
           ++bad;
           write_index(indices, is64, i, 0);

@@ -34,6 +34,28 @@ struct Status {
   unsigned long long first_bad_pos;
 };
 
+// The block behind calls that wait for their result (StatusScope in c_api.cpp): `pad` of the block
+// says that a pinned host word follows, which every report sets besides. The host then reads that
+// word after its wait, and neither clears the block before the call nor copies it back after it
+// unless something was reported: two operations on the stream less per call.
+constexpr int32_t STATUS_FLAGGED = 0x464c4147;
+struct FlaggedStatus {
+  Status st;
+  int32_t* flag;
+};
+
+#if defined(__HIPCC__)
+__device__ __forceinline__ void status_or(Status* st, int32_t bits) {
+  atomicOr(&st->bits, bits);
+  if (st->pad == STATUS_FLAGGED)
+    __hip_atomic_store(reinterpret_cast<FlaggedStatus*>(st)->flag, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+__device__ __forceinline__ void status_index(Status* st, int64_t pos) {
+  atomicMin(&st->first_bad_pos, (unsigned long long)pos);
+  status_or(st, ERR_INDEX_OUT_OF_RANGE);
+}
+#endif
+
 // How a wave walks one table. Filled on the host from the table's element
 // type, dimension, stride and alignment.
 struct TableDesc {

@@ -34,11 +34,10 @@ __device__ __forceinline__ constexpr int type_bits(int ty) {
 }
 
 __device__ __forceinline__ void report(Status* st, int32_t bit) {
-  atomicOr(&st->bits, bit);
+  status_or(st, bit);
 }
 __device__ __forceinline__ void report_index(Status* st, int64_t pos) {
-  atomicOr(&st->bits, ERR_INDEX_OUT_OF_RANGE);
-  atomicMin(&st->first_bad_pos, (unsigned long long)pos);
+  status_index(st, pos);
 }
 
 // ---- per-row accumulate ---------------------------------------------------

@@ -42,8 +42,7 @@ __device__ __forceinline__ int32_t mapped_row(const index_t* indices, const int3
                                               Status* status) {
   const int64_t idx = (int64_t)indices[k];
   if (idx < 0 || idx >= mapping_numel) {
-    atomicOr(&status->bits, ERR_INDEX_OUT_OF_RANGE);
-    atomicMin(&status->first_bad_pos, (unsigned long long)k);
+    status_index(status, k);
     return -1;
   }
   return mapping[idx];

@@ -369,8 +369,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 8))) voi
       ok = false; // pruned row: zeros
     } else if (idx < 0 || idx >= d.num_rows) {
       if (sub == 0) {
-        atomicOr(&status->bits, ERR_INDEX_OUT_OF_RANGE);
-        atomicMin(&status->first_bad_pos, (unsigned long long)pos);
+        status_index(status, pos);
       }
       ok = false;
     }
@@ -487,8 +486,7 @@ __global__ __launch_bounds__(256) void row_lookup_kernel(
     if (live) {
       const bool ok = idx >= 0 && idx < d.num_rows;
       if (!ok && sub == 0) {
-        atomicOr(&status->bits, ERR_INDEX_OUT_OF_RANGE);
-        atomicMin(&status->first_bad_pos, (unsigned long long)pos);
+        status_index(status, pos);
       }
       const uint8_t* row = table + (ok ? idx : 0) * d.row_stride;
       uint8_t* orow = reinterpret_cast<uint8_t*>(out) + pos * out_stride_bytes;

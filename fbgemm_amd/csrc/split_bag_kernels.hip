@@ -40,7 +40,7 @@ __global__ __launch_bounds__(256) void split_offsets_kernel(const void* offsets,
   }
   if (v == bags - 1) {
     voff[bags * K] = o1;
-    if (relative && o1 != index_size) atomicOr(&status->bits, ERR_LENGTH_MISMATCH);
+    if (relative && o1 != index_size) status_or(status, ERR_LENGTH_MISMATCH);
   }
 }
 

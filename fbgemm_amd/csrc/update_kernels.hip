@@ -51,11 +51,10 @@ __global__ __launch_bounds__(256) void inplace_update_kernel(
       }
       if (bad) {
         if (sub == 0 && status) {
-          atomicOr(&status->bits, ERR_INDEX_OUT_OF_RANGE);
-          atomicMin(&status->first_bad_pos, (unsigned long long)u);
+          status_index(status, u);
         }
       } else if (uoff < 0 || uoff + bytes > update_bytes) {
-        if (sub == 0 && status) atomicOr(&status->bits, ERR_BAG_OVERRUN);
+        if (sub == 0 && status) status_or(status, ERR_BAG_OVERRUN);
       } else {
         const uint8_t* src = update + uoff;
         uint8_t* dst = (placement ? w1 : w0) + woff + r * bytes;

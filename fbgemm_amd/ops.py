@@ -56,6 +56,7 @@ class Status:
 
     def __init__(self, device=None):
         self.buf = torch.zeros(4, dtype=torch.int32, device=device or "cuda")
+        self.ptr = _ptr(self.buf)
         self.clear()
 
     def clear(self):
@@ -68,9 +69,39 @@ class Status:
         return bits.value, pos.value
 
 
+class _OwnStatus:
+    """The calling thread's own status block, for one call that waits for its result."""
+
+    def __init__(self):
+        self.ptr = C.c_void_p()
+        check(_lib.lib().fbgemm_amd_status_begin(C.byref(self.ptr)))
+
+    def read(self):
+        """Synchronizes the current stream. Returns (bits, first_bad_pos)."""
+        bits, pos = C.c_int32(0), C.c_int64(-1)
+        check(_lib.lib().fbgemm_amd_status_end(_stream(), C.byref(bits), C.byref(pos)))
+        return bits.value, pos.value
+
+
 def _make_kernel(weight_ty, block_size, normalize_by_lengths, is_weight_positional, use_offsets,
                  output_stride, input_stride, scale_bias_last, output_ty, has_weight, sparse, no_bag=False,
                  fp8=(0, 0)):
+    # the descriptor of a call, per index and offset width and arithmetic; the library only reads it
+    configs = {}
+
+    def config(index_bits, offset_bits, accumulate):
+        key = (index_bits, offset_bits, accumulate)
+        cfg = configs.get(key)
+        if cfg is None:
+            cfg = configs[key] = SpmdmConfig(
+                weight_ty=weight_ty, output_ty=output_ty, index_bits=index_bits, offset_bits=offset_bits, block_size=block_size,
+                output_stride=output_stride, input_stride=input_stride,
+                normalize_by_lengths=int(normalize_by_lengths),
+                is_weight_positional=int(is_weight_positional), use_offsets=int(use_offsets),
+                scale_bias_last=int(scale_bias_last), no_bag=int(no_bag), fp8_exponent_bits=fp8[0],
+                fp8_exponent_bias=fp8[1], accumulate=accumulate)
+        return cfg
+
     def kernel(output_size, index_size, data_size, input, indices, offsets_or_lengths, weights, out,
                compressed_indices_table=None, status=None, accumulate=ACC_EXACT):
         _require_cuda(input, indices, offsets_or_lengths, weights, out, compressed_indices_table)
@@ -83,14 +114,7 @@ def _make_kernel(weight_ty, block_size, normalize_by_lengths, is_weight_position
             raise TypeError("weights must be float32")
         if compressed_indices_table is not None and compressed_indices_table.dtype != torch.int32:
             raise TypeError("compressed_indices_table must be int32")
-        cfg = SpmdmConfig(
-            weight_ty=weight_ty, output_ty=output_ty, index_bits=_bits(indices),
-            offset_bits=32 if offsets_or_lengths is None else _bits(offsets_or_lengths), block_size=block_size,
-            output_stride=output_stride, input_stride=input_stride,
-            normalize_by_lengths=int(normalize_by_lengths),
-            is_weight_positional=int(is_weight_positional), use_offsets=int(use_offsets),
-            scale_bias_last=int(scale_bias_last), no_bag=int(no_bag), fp8_exponent_bits=fp8[0],
-            fp8_exponent_bias=fp8[1], accumulate=int(accumulate))
+        cfg = config(_bits(indices), 32 if offsets_or_lengths is None else _bits(offsets_or_lengths), int(accumulate))
         lib = _lib.lib()
         if status is not None:
             check(lib.fbgemm_amd_spmdm_launch(
@@ -341,10 +365,10 @@ def int_nbit_split_embedding_codegen_lookup_function(
         if total_L == 0 or (offsets.numel() - 1) // plan.T == 0:
             return out.zero_()
         own = status is None
-        st = Status(dev_weights.device) if own else status
+        st = _OwnStatus() if own else status
         check(_lib.lib().fbgemm_amd_tbe_forward_nobag(
             plan.handle, _ptr(dev_weights), _ptr(uvm_weights), _ptr(indices.contiguous()), _ptr(offsets.contiguous()),
-            _bits(indices), indices.numel(), offsets.numel(), D, output_dtype, _ptr(out), _ptr(st.buf), _stream()))
+            _bits(indices), indices.numel(), offsets.numel(), D, output_dtype, _ptr(out), st.ptr, _stream()))
         if own:
             bits, pos = st.read()
             if bits:
@@ -376,7 +400,7 @@ def int_nbit_split_embedding_codegen_lookup_function(
     if B == 0:
         return out
     own = status is None
-    st = Status(dev_weights.device) if own else status
+    st = _OwnStatus() if own else status
     ro = None
     if index_remappings is not None:
         _require_cuda(index_remappings, index_remappings_offsets)
@@ -400,7 +424,7 @@ def int_nbit_split_embedding_codegen_lookup_function(
         _ptr(offsets.contiguous()), _bits(indices), indices.numel(), offsets.numel(), pooling_mode,
         _ptr(indice_weights), output_dtype, _ptr(out), _ptr(index_remappings),
         32 if index_remappings is None else _bits(index_remappings), _ptr(ro), 0 if ro is None else ro.numel(),
-        _ptr(st.buf), _stream()))
+        st.ptr, _stream()))
     if own:
         bits, pos = st.read()
         if bits:
@@ -481,12 +505,12 @@ def emb_inplace_update(dev_weights, uvm_weights, weights_placements, weights_off
         plan = _plan_for(dev_weights, uvm_weights, weights_placements, weights_offsets, weights_tys, D_offsets,
                          row_alignment)
     own = status is None
-    st = Status(dev_weights.device) if own else status
+    st = _OwnStatus() if own else status
     update_weights = update_weights.contiguous()
     check(_lib.lib().fbgemm_amd_tbe_inplace_update(
         plan.handle, _ptr(dev_weights), _ptr(uvm_weights), _ptr(update_weights), update_weights.numel(),
         _ptr(update_table_indices.contiguous()), _ptr(update_row_indices.contiguous()), _bits(update_row_indices),
-        _ptr(update_offsets.contiguous()), n, _ptr(st.buf), _stream()))
+        _ptr(update_offsets.contiguous()), n, st.ptr, _stream()))
     if own:
         bits, pos = st.read()
         if bits & ERR_INDEX_OUT_OF_RANGE:
@@ -527,10 +551,10 @@ def bounds_check_indices(rows_per_table, indices, offsets, bounds_check_mode, wa
         raise RuntimeError("max_B must not be negative with B_offsets")
     rpt = rows_per_table.to(torch.int64).contiguous()
     bo = None if B_offsets is None else B_offsets.to(torch.int32).contiguous()
-    status = Status(indices.device) if bounds_check_mode == BOUNDS_FATAL else None
+    status = _OwnStatus() if bounds_check_mode == BOUNDS_FATAL else None
     check(_lib.lib().fbgemm_amd_bounds_check_indices(
         _ptr(rpt), rpt.numel(), _ptr(indices), _ptr(offsets), _bits(indices), indices.numel(), offsets.numel(),
-        int(bounds_check_mode), _ptr(warning), _ptr(bo), None if status is None else _ptr(status.buf), _stream()))
+        int(bounds_check_mode), _ptr(warning), _ptr(bo), None if status is None else status.ptr, _stream()))
     if status is not None:
         bits, pos = status.read()
         if bits & ERR_LENGTH_MISMATCH:
@@ -649,11 +673,11 @@ def compressed_indices_remap(indices, compressed_indices_mapping, offsets, weigh
     out_indices = torch.empty_like(indices)
     out_offsets = torch.empty_like(offsets)
     out_weights = None if weights is None else torch.empty_like(weights)
-    st = Status(indices.device)
+    st = _OwnStatus()
     check(_lib.lib().fbgemm_amd_compressed_indices_remap(
         offsets.numel(), _ptr(indices), _bits(indices), _ptr(mapping), mapping.numel(), _ptr(offsets),
         _ptr(None if weights is None else weights.contiguous()), _ptr(out_indices), _ptr(out_offsets), _ptr(out_weights),
-        _ptr(st.buf), _stream()))
+        st.ptr, _stream()))
     bits, pos = st.read()
     if bits:
         raise IndexError(f"compressed_indices_remap: index at position {pos} is outside the mapping")

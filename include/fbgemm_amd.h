@@ -71,6 +71,14 @@ int fbgemm_amd_status_clear(void* d_status, void* stream);
  * out-of-range index, or -1. Either out pointer may be NULL. */
 int fbgemm_amd_status_read(const void* d_status, void* stream, int32_t* bits, int64_t* first_bad_pos);
 
+/* The calling thread's own block, for calls that wait for their result: begin hands
+ * out the block (cleared), the launches of this thread that follow take it as their
+ * d_status, end waits for `stream` and returns what they recorded (bits, and the
+ * first offending position or -1). One pair at a time per thread, on one device.
+ * Costs no operation on the stream unless something was recorded. */
+int fbgemm_amd_status_begin(void** d_status);
+int fbgemm_amd_status_end(void* stream, int32_t* bits, int64_t* first_bad_pos);
+
 /* ---- single-table pooled lookup ----------------------------------------- *
  *
  * Replaces the kernels returned by fbgemm::GenerateEmbeddingSpMDMWithStrides,

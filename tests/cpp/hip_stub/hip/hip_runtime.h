@@ -25,6 +25,9 @@ enum : unsigned { hipStreamNonBlocking = 1, hipEventDisableTiming = 2, hipEventD
 
 hipError_t hipMalloc(void** p, size_t bytes);
 hipError_t hipFree(void* p);
+enum : unsigned { hipHostMallocCoherent = 0x40000000 };
+hipError_t hipHostMalloc(void** p, size_t bytes, unsigned flags);
+hipError_t hipHostFree(void* p);
 hipError_t hipMemcpy(void* dst, const void* src, size_t bytes, hipMemcpyKind kind);
 hipError_t hipMemcpyAsync(void* dst, const void* src, size_t bytes, hipMemcpyKind kind, hipStream_t stream);
 hipError_t hipMemsetAsync(void* dst, int value, size_t bytes, hipStream_t stream);

@@ -50,6 +50,14 @@ hipError_t hipFree(void* p) {
   free(p);
   return hipSuccess;
 }
+hipError_t hipHostMalloc(void** p, size_t bytes, unsigned) {
+  *p = malloc(bytes);
+  return *p ? hipSuccess : hipErrorOutOfMemory;
+}
+hipError_t hipHostFree(void* p) {
+  free(p);
+  return hipSuccess;
+}
 hipError_t hipMemcpy(void* dst, const void* src, size_t bytes, hipMemcpyKind) {
   if (bytes) memcpy(dst, src, bytes);
   return hipSuccess;
