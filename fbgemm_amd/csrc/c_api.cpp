@@ -274,6 +274,7 @@ struct DeviceScratch {
   int64_t fixed_cap = 0;
   int64_t* partial = nullptr; // bounds check: per-block maxima of the offset scan
   int64_t partial_cap = 0;
+  unsigned long long* counter = nullptr; // zero between calls (check_remap_kernel)
   int64_t* seg_offsets = nullptr; // split bags: where every segment starts
   int64_t seg_offsets_cap = 0;
   float* seg_partial = nullptr;   // split bags: the segments' fp32 sums
@@ -1956,6 +1957,60 @@ int fbgemm_amd_bounds_check_indices(
   HIP_TRY(launch_bounds_check(d_rows_per_table, T, d_indices, d_offsets, index_bits == 64, indices_numel, total_B,
                               d_B_offsets ? 0 : total_B / T, d_B_offsets, bounds_check_mode, d_warning, s->fixed,
                               s->partial, (Status*)d_status, stream));
+  return 0;
+}
+
+extern "C" int fbgemm_amd_check_remap_indices(
+    const int64_t* d_rows_per_table, int32_t T, const void* d_indices, const void* d_offsets, int32_t index_bits,
+    int64_t indices_numel, int64_t offsets_numel, int32_t bounds_check_mode, int64_t* d_warning,
+    const int64_t* d_logical_rows_per_table, const void* d_index_remappings, int32_t remap_bits,
+    const int64_t* d_index_remappings_offsets, void* d_out_indices, void* d_out_offsets, void* stream_) {
+  if (T <= 0 || !d_rows_per_table) return fail(FBGEMM_AMD_E_ARG, "rows_per_table must hold T >= 1 entries");
+  if (index_bits != 32 && index_bits != 64) return fail(FBGEMM_AMD_E_ARG, "index_bits must be 32 or 64");
+  if (bounds_check_mode != 1 && bounds_check_mode != 2) return fail(FBGEMM_AMD_E_ARG, "bounds_check_mode must be 1 (WARNING) or 2 (IGNORE)");
+  if (offsets_numel < 1 || !d_offsets || !d_out_offsets) return fail(FBGEMM_AMD_E_ARG, "offsets must hold at least one entry");
+  const int64_t total_B = offsets_numel - 1;
+  if (total_B % T != 0)
+    return fail(FBGEMM_AMD_E_ARG, "offsets size %lld is not equal to B (%lld) * T (%d) + 1", (long long)offsets_numel,
+                (long long)(total_B / T), T);
+  if (total_B == 0) return fail(FBGEMM_AMD_E_ARG, "B must not be zero");
+  if (indices_numel < 0 || (indices_numel > 0 && (!d_indices || !d_out_indices))) return fail(FBGEMM_AMD_E_ARG, "null data pointer");
+  if (bounds_check_mode == 1 && !d_warning) return fail(FBGEMM_AMD_E_ARG, "WARNING mode needs the warning counter");
+  if (d_index_remappings_offsets && (!d_index_remappings || !d_logical_rows_per_table || (remap_bits != 32 && remap_bits != 64)))
+    return fail(FBGEMM_AMD_E_ARG, "a mapping needs its 32- or 64-bit entries and the rows before pruning");
+  hipStream_t stream = (hipStream_t)stream_;
+  std::lock_guard<std::mutex> lk(g_mu);
+  DeviceScratch* s;
+  if (int rc = get_scratch(&s)) return rc;
+  if (int rc = grow(&s->partial, &s->partial_cap, check_remap_partials(total_B), stream)) return rc;
+  if (!s->counter) {
+    unsigned long long* counter = nullptr;
+    const unsigned long long zero = 0;
+    HIP_TRY(hipMalloc((void**)&counter, sizeof(zero)));
+    const hipError_t e = hipMemcpy(counter, &zero, sizeof(zero), hipMemcpyHostToDevice);
+    if (e != hipSuccess) {
+      (void)hipFree(counter);
+      return fail(FBGEMM_AMD_E_HIP, "hipMemcpy of a counter: %s", hipGetErrorString(e));
+    }
+    s->counter = counter;
+  }
+  CheckRemapArgs a;
+  memset(&a, 0, sizeof(a));
+  a.rows = d_rows_per_table;
+  a.logical_rows = d_logical_rows_per_table;
+  a.indices = d_indices;
+  a.offsets = d_offsets;
+  a.out_indices = d_out_indices;
+  a.out_offsets = d_out_offsets;
+  a.N = indices_numel;
+  a.total_B = total_B;
+  a.B = total_B / T;
+  a.remap = d_index_remappings;
+  a.remap_offsets = d_index_remappings_offsets;
+  a.warning = d_warning;
+  a.counter = s->counter;
+  a.mode = bounds_check_mode;
+  HIP_TRY(launch_check_remap(a, index_bits == 64, remap_bits == 64, s->partial, stream));
   return 0;
 }
 

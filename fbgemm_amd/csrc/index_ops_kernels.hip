@@ -214,6 +214,195 @@ __global__ __launch_bounds__(256) void bounds_check_bags_kernel(
   }
 }
 
+// ---- bounds check and pruned-row mapping in one pass, out of place --------------------
+//
+// What a serving forward does to its indices before the lookup (WARNING and IGNORE mode): with
+// plain tables one bounds check; with array-pruned tables a check against the logical rows, the
+// mapping, and a check against the physical rows. Done by the operators one after the other that
+// is two copies (the caller's tensors stay as they are), up to six launches and five passes over
+// the indices. Here the inputs are read once and the checked (and mapped) indices and the repaired
+// offsets written once. A workgroup owns 256 bags (gridDim.y workgroups share their indices): it
+// makes the running maximum of their offsets, which decides what the bags are, and then walks
+// their indices as one range, 8 loads in flight per thread: the mapping is a random gather, bound
+// by round trips unless many of them overlap.
+//   64 tables x 32 bags x 30 entries: 16 us of copies and check -> 8.8 us (its chain of five round
+//   trips). 32 pruned tables x 4096 bags x 27: 121 us of copies, check, mapping (64.6) and check ->
+//   78 us: the random 4-byte reads of 256 MB of mappings, a line each, 6 TB/s of lines.
+// The warning counter is what the last of the separate checks leaves there: with a mapping the
+// second check's, which starts from zero and whose offsets are already in order.
+constexpr int CR_BAGS = 256; // bags of a workgroup, one per thread
+constexpr int CR_LOADS = 8;
+constexpr int CR_ONE_LAUNCH_BLOCKS = 16; // up to here every workgroup reads the offsets before its own itself
+
+__device__ __forceinline__ int64_t cr_block_max(int64_t v, int64_t* lds) {
+  for (int m = 32; m > 0; m >>= 1) {
+    const int64_t o = __shfl_xor(v, m, 64);
+    v = v > o ? v : o;
+  }
+  if ((threadIdx.x & 63) == 0) lds[threadIdx.x >> 6] = v;
+  __syncthreads();
+  int64_t r = lds[0];
+  for (int w = 1; w < CR_BAGS / 64; ++w) r = r > lds[w] ? r : lds[w];
+  __syncthreads();
+  return r;
+}
+
+__global__ __launch_bounds__(CR_BAGS) void check_remap_partial_kernel(const void* offsets, int is64, int64_t total_B, int64_t N,
+                                                                      int64_t* partial, int64_t* warning, int mode) {
+  __shared__ int64_t lds[CR_BAGS / 64];
+  if (mode == 1 && blockIdx.x == 0 && threadIdx.x == 0) warning[0] = 0;
+  const int64_t k = (int64_t)blockIdx.x * CR_BAGS + threadIdx.x;
+  const int64_t m = cr_block_max(k < total_B ? clamped_offset(offsets, is64, k, total_B, N) : 0, lds);
+  if (threadIdx.x == 0) partial[blockIdx.x] = m;
+}
+
+template <typename index_t, typename remap_t>
+__global__ __launch_bounds__(CR_BAGS) void check_remap_kernel(CheckRemapArgs a) {
+  constexpr bool IS64 = sizeof(index_t) == 8;
+  __shared__ int64_t fixed[CR_BAGS + 1];
+  __shared__ int64_t t_rows[CR_BAGS], t_logical[CR_BAGS], t_remap[CR_BAGS], t_cap[CR_BAGS];
+  __shared__ int64_t lds[CR_BAGS / 64];
+  __shared__ int bad_count;
+  const int tid = threadIdx.x;
+  const int64_t k0 = (int64_t)blockIdx.x * CR_BAGS;
+  const int nb = (int)(a.total_B - k0 < CR_BAGS ? a.total_B - k0 : CR_BAGS);
+  // every load the walk over the offsets needs, before anything waits: this bag's offset, the one
+  // behind the last bag, and what the bags before these leave
+  const int64_t mine = tid < nb ? clamped_offset(a.offsets, IS64, k0 + tid, a.total_B, a.N) : 0;
+  const int64_t behind = clamped_offset(a.offsets, IS64, k0 + nb, a.total_B, a.N);
+  int64_t carry = 0;
+  if (a.prefix) {
+    carry = a.partial[blockIdx.x];
+  } else if (a.partial) {
+    for (int64_t b = tid; b < (int64_t)blockIdx.x; b += CR_BAGS) carry = carry > a.partial[b] ? carry : a.partial[b];
+  } else {
+#pragma unroll
+    for (int u = 0; u < CR_ONE_LAUNCH_BLOCKS - 1; ++u) {
+      const int64_t k = tid + u * CR_BAGS;
+      const int64_t v = k < k0 ? clamped_offset(a.offsets, IS64, k, a.total_B, a.N) : 0;
+      carry = carry > v ? carry : v;
+    }
+  }
+  // the tables of these bags, at most one per bag
+  const bool small = a.total_B <= 0xffffffffll;
+  auto table_of = [&](int64_t k) { return small ? (int64_t)((uint32_t)k / (uint32_t)a.B) : k / a.B; };
+  const int64_t t0 = table_of(k0);
+  const int nt = (int)(table_of(k0 + nb - 1) - t0) + 1;
+  if (tid == 0) bad_count = 0;
+  if (tid < nt) {
+    t_rows[tid] = a.rows[t0 + tid];
+    if (a.remap_offsets) {
+      t_logical[tid] = a.logical_rows[t0 + tid];
+      t_remap[tid] = a.remap_offsets[t0 + tid];
+      t_cap[tid] = a.remap_offsets[t0 + tid + 1] - t_remap[tid];
+    }
+  }
+  carry = cr_block_max(carry, lds);
+  // running maximum: the repaired offsets
+  int64_t run = mine;
+  for (int step = 1; step < 64; step <<= 1) {
+    const int64_t o = __shfl_up(run, step, 64);
+    if ((tid & 63) >= step) run = run > o ? run : o;
+  }
+  if ((tid & 63) == 63) lds[tid >> 6] = run;
+  __syncthreads();
+  for (int w = 0; w < (tid >> 6); ++w) run = run > lds[w] ? run : lds[w];
+  run = run > carry ? run : carry;
+  if (tid < nb) fixed[tid] = run;
+  if (tid == nb - 1) fixed[nb] = run > behind ? run : behind;
+  __syncthreads();
+  int bad = 0;
+  if (blockIdx.y == 0) {
+    if (tid < nb) {
+      const int64_t k = k0 + tid;
+      write_index(a.out_offsets, IS64, k, run);
+      // see bounds_fix_offsets_kernel
+      const int64_t end = k + 1 == a.total_B ? a.N : read_index(a.offsets, IS64, k + 1);
+      const int64_t first = k == 0 ? read_index(a.offsets, IS64, 0) : 0;
+      if (first < 0 || first > a.N || run > end || end > a.N) ++bad;
+      if (k + 1 == a.total_B) {
+        write_index(a.out_offsets, IS64, a.total_B, fixed[nb]);
+        if (read_index(a.offsets, IS64, a.total_B) != a.N) ++bad;
+      }
+    }
+    if (a.remap_offsets) bad = 0; // the second check starts from zero, and from offsets that are in order
+  }
+  // the indices of these bags; what lies before the first bag is nobody's and passes through
+  const int64_t lo0 = blockIdx.x == 0 ? 0 : fixed[0], hi0 = fixed[nb], own = fixed[0];
+  const int64_t share = (hi0 - lo0 + gridDim.y - 1) / gridDim.y;
+  const int64_t lo = lo0 + share * blockIdx.y;
+  const int64_t hi = lo + share < hi0 ? lo + share : hi0;
+  const index_t* in = reinterpret_cast<const index_t*>(a.indices);
+  const remap_t* remap = reinterpret_cast<const remap_t*>(a.remap);
+  index_t* out = reinterpret_cast<index_t*>(a.out_indices);
+  for (int64_t i0 = lo + tid; i0 < hi; i0 += CR_LOADS * CR_BAGS) {
+    index_t v[CR_LOADS];
+    int t[CR_LOADS];
+    bool gather[CR_LOADS];
+#pragma unroll
+    for (int u = 0; u < CR_LOADS; ++u) {
+      const int64_t i = i0 + u * CR_BAGS;
+      v[u] = i < hi ? in[i] : 0;
+    }
+#pragma unroll
+    for (int u = 0; u < CR_LOADS; ++u) {
+      const int64_t i = i0 + u * CR_BAGS;
+      // the last of the tables that starts at or before i
+      int l = 0, h = nt;
+      while (h - l > 1) {
+        const int mid = (l + h) >> 1;
+        if (fixed[(t0 + mid) * a.B - k0] <= i) l = mid;
+        else h = mid;
+      }
+      t[u] = l;
+      gather[u] = false;
+      if (a.remap_offsets && i < hi && i >= own) {
+        if (v[u] != (index_t)-1 && (v[u] < 0 || (int64_t)v[u] >= t_logical[l])) v[u] = 0;
+        if (t_cap[l] > 0) {
+          gather[u] = v[u] >= 0 && (int64_t)v[u] < t_cap[l];
+          if (!gather[u]) v[u] = (index_t)-1;
+        }
+      }
+    }
+    if (a.remap_offsets) {
+      remap_t m[CR_LOADS];
+#pragma unroll
+      for (int u = 0; u < CR_LOADS; ++u)
+        if (gather[u]) m[u] = remap[t_remap[t[u]] + (int64_t)v[u]];
+#pragma unroll
+      for (int u = 0; u < CR_LOADS; ++u)
+        if (gather[u]) v[u] = (index_t)m[u];
+    }
+#pragma unroll
+    for (int u = 0; u < CR_LOADS; ++u) {
+      const int64_t i = i0 + u * CR_BAGS;
+      if (i < hi) {
+        if (i >= own && v[u] != (index_t)-1 && (v[u] < 0 || (int64_t)v[u] >= t_rows[t[u]])) {
+          v[u] = 0;
+          ++bad;
+        }
+        out[i] = v[u];
+      }
+    }
+  }
+  if (a.mode != 1) return;
+  if (bad) atomicAdd(&bad_count, bad);
+  __syncthreads();
+  if (tid != 0) return;
+  unsigned long long* warning = reinterpret_cast<unsigned long long*>(a.warning);
+  if (a.partial) { // the kernel before this one has set the counter to zero
+    if (bad_count) atomicAdd(warning, (unsigned long long)bad_count);
+    return;
+  }
+  // one launch: the workgroups add up in the library's counter (zero between calls): their number in
+  // the low 16 bits, what they found above; the last one hands the sum over. One atomic and no fence.
+  const unsigned long long had = atomicAdd(a.counter, ((unsigned long long)bad_count << 16) + 1ull);
+  if ((had & 0xffffull) + 1 == (unsigned long long)gridDim.x * gridDim.y) {
+    *warning = (had >> 16) + (unsigned long long)bad_count;
+    atomicExch(a.counter, 0ull);
+  }
+}
+
 // MurmurHash3 finalizers, as the reference hashes sparse ids
 // (embedding_forward_quantized_cpu_template.cpp:102-120)
 __device__ __forceinline__ uint32_t pruned_hash(uint32_t h) {
@@ -295,6 +484,34 @@ hipError_t launch_bounds_check(const int64_t* rows_per_table, int32_t T, void* i
 }
 
 int64_t bounds_check_partials(int64_t total_B) { return (total_B + 1 + SCAN_BLOCK - 1) / SCAN_BLOCK; }
+
+int64_t check_remap_partials(int64_t total_B) { return (total_B + CR_BAGS - 1) / CR_BAGS; }
+
+hipError_t launch_check_remap(CheckRemapArgs a, bool is64, bool remap64, int64_t* partial, hipStream_t stream) {
+  const int64_t blocks = check_remap_partials(a.total_B);
+  if (a.total_B <= 0 || a.B <= 0 || blocks > 0x7fffffffLL) return hipErrorInvalidValue;
+  a.partial = nullptr;
+  a.prefix = 0;
+  if (blocks > CR_ONE_LAUNCH_BLOCKS) {
+    a.partial = partial;
+    hipLaunchKernelGGL(check_remap_partial_kernel, dim3((unsigned)blocks), dim3(CR_BAGS), 0, stream, a.offsets, is64 ? 1 : 0, a.total_B,
+                       a.N, partial, a.warning, a.mode);
+    if (blocks > 4096) { // more maxima than a workgroup should read for itself
+      a.prefix = 1;
+      hipLaunchKernelGGL(bounds_carry_kernel, dim3(1), dim3(SCAN_THREADS), 0, stream, partial, blocks);
+    }
+  }
+  // a workgroup per 2048 indices (one turn of 8 loads per thread), per 512 where that leaves the device half empty
+  const int64_t per = a.N < (int64_t)256 * CR_LOADS * CR_BAGS ? 2 * CR_BAGS : CR_LOADS * CR_BAGS;
+  int64_t shares = (a.N / blocks + per - 1) / per;
+  shares = shares < 1 ? 1 : (shares > 1024 ? 1024 : shares);
+  const dim3 grid((unsigned)blocks, (unsigned)shares), block(CR_BAGS);
+  if (is64 && remap64) hipLaunchKernelGGL((check_remap_kernel<int64_t, int64_t>), grid, block, 0, stream, a);
+  else if (is64) hipLaunchKernelGGL((check_remap_kernel<int64_t, int32_t>), grid, block, 0, stream, a);
+  else if (remap64) hipLaunchKernelGGL((check_remap_kernel<int32_t, int64_t>), grid, block, 0, stream, a);
+  else hipLaunchKernelGGL((check_remap_kernel<int32_t, int32_t>), grid, block, 0, stream, a);
+  return hipGetLastError();
+}
 
 hipError_t launch_pruned_hashmap_lookup(const void* indices, const void* offsets, bool idx64, const void* hash_table,
                                         bool hash64, const int64_t* hash_table_offsets, int32_t B, int32_t T,

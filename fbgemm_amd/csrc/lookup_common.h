@@ -186,4 +186,22 @@ struct LookupArgs {
   Status* status;
 };
 
+// The bounds check with the pruned-row mapping (check_remap_kernel).
+struct CheckRemapArgs {
+  const int64_t* rows;         // T physical row counts
+  const int64_t* logical_rows; // T row counts before pruning; with remap_offsets only
+  const void* indices;         // N
+  const void* offsets;         // total_B + 1
+  void* out_indices;
+  void* out_offsets;
+  int64_t N, total_B, B;       // total_B = T * B
+  const void* remap;
+  const int64_t* remap_offsets; // T + 1, or nullptr: no mapping
+  int64_t* warning;
+  unsigned long long* counter;  // zero between calls
+  const int64_t* partial;       // set by the launcher
+  int32_t prefix;               // likewise
+  int32_t mode;                 // 1 WARNING, 2 IGNORE
+};
+
 } // namespace fbgemm_amd

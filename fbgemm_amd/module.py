@@ -341,6 +341,29 @@ class IntNBitTableBatchedEmbeddingBagsCodegen(torch.nn.Module):
         hashed = self.index_remapping_hash_table.numel() > 0
         arrayed = self.index_remappings_array.numel() > 0
         fuse_remap = arrayed and not check and self.pooling_mode != PoolingMode.NONE
+        T = self.rows_per_table.numel()
+        one_pass = (check and not hashed and self.bounds_check_mode_int != BoundsCheckMode.FATAL.value
+                    and offsets.numel() > T  # B > 0
+                    and (not arrayed or (self.original_rows_per_table.numel() == T and self._feature_remap_offsets.numel() == T + 1)))
+        if one_pass:
+            # the check, or check, mapping and check, on copies: the caller's tensors stay as they are
+            indices, offsets = ops.check_remap_indices(
+                self.rows_per_table, indices, offsets, self.bounds_check_mode_int, self.bounds_check_warning, per_sample_weights,
+                self.original_rows_per_table if arrayed else None, self._feature_remap_array if arrayed else None,
+                self._feature_remap_offsets if arrayed else None)
+        else:
+            indices, offsets = self._check_and_remap(indices, offsets, per_sample_weights, check, hashed, arrayed, fuse_remap)
+        return ops.int_nbit_split_embedding_codegen_lookup_function(
+            self.weights_dev, self.weights_uvm, self.weights_placements, self.weights_offsets, self.weights_tys,
+            self.D_offsets, self.total_D, self.max_int2_D, self.max_int4_D, self.max_int8_D, self.max_float16_D,
+            self.max_float32_D, indices, offsets, int(self.pooling_mode), per_sample_weights, self.output_dtype,
+            row_alignment=self.row_alignment, max_float8_D=self.max_float8_D,
+            fp8_exponent_bits=self.fp8_exponent_bits, fp8_exponent_bias=self.fp8_exponent_bias,
+            index_remappings=self._feature_remap_array if fuse_remap else None,
+            index_remappings_offsets=self._feature_remap_offsets if fuse_remap else None)
+
+    def _check_and_remap(self, indices, offsets, per_sample_weights, check, hashed, arrayed, fuse_remap):
+        """The operators one after the other: FATAL mode, hash-based pruning, no check."""
         if check and (hashed or arrayed or self.bounds_check_mode_int != BoundsCheckMode.FATAL.value):
             # in-place repairs must not reach the caller's tensors
             indices, offsets = indices.clone(), offsets.clone()
@@ -355,11 +378,4 @@ class IntNBitTableBatchedEmbeddingBagsCodegen(torch.nn.Module):
         if check:
             ops.bounds_check_indices(self.rows_per_table, indices, offsets, self.bounds_check_mode_int,
                                      self.bounds_check_warning, per_sample_weights)
-        return ops.int_nbit_split_embedding_codegen_lookup_function(
-            self.weights_dev, self.weights_uvm, self.weights_placements, self.weights_offsets, self.weights_tys,
-            self.D_offsets, self.total_D, self.max_int2_D, self.max_int4_D, self.max_int8_D, self.max_float16_D,
-            self.max_float32_D, indices, offsets, int(self.pooling_mode), per_sample_weights, self.output_dtype,
-            row_alignment=self.row_alignment, max_float8_D=self.max_float8_D,
-            fp8_exponent_bits=self.fp8_exponent_bits, fp8_exponent_bias=self.fp8_exponent_bias,
-            index_remappings=self._feature_remap_array if fuse_remap else None,
-            index_remappings_offsets=self._feature_remap_offsets if fuse_remap else None)
+        return indices, offsets

@@ -565,6 +565,39 @@ def bounds_check_indices(rows_per_table, indices, offsets, bounds_check_mode, wa
             raise RuntimeError(f"Index {pos} is out of bounds: {int(indices[pos])}")
 
 
+def check_remap_indices(rows_per_table, indices, offsets, bounds_check_mode, warning, weights=None,
+                        logical_rows_per_table=None, index_remappings=None, index_remappings_offsets=None):
+    """``bounds_check_indices`` (WARNING or IGNORE) on copies of ``indices`` and ``offsets``, which are returned;
+    with ``index_remappings`` the check against the logical rows, ``pruned_array_lookup`` and the check against
+    ``rows_per_table`` in one pass. ``warning`` ends as the last of those checks would leave it."""
+    _require_cuda(rows_per_table, indices, offsets, warning, weights, logical_rows_per_table, index_remappings,
+                  index_remappings_offsets)
+    if indices.dtype != offsets.dtype:
+        raise TypeError("indices and offsets must have the same dtype")
+    # a strided vector is copied; what a copy leaves in another order is refused, as by bounds_check_indices
+    indices = indices if indices.is_contiguous() else indices.clone()
+    offsets = offsets if offsets.is_contiguous() else offsets.clone()
+    if not (indices.is_contiguous() and offsets.is_contiguous()):
+        raise ValueError("indices and offsets are modified in place and must be contiguous")
+    if weights is not None and weights.numel() != 0 and weights.size(0) != indices.numel():
+        raise RuntimeError(f"weights size {weights.size(0)} is not equal to indices size {indices.numel()}")
+    rows = rows_per_table.to(torch.int64).contiguous()
+    logical = offs = None
+    if index_remappings is not None:
+        logical = logical_rows_per_table.to(torch.int64).contiguous()
+        offs = index_remappings_offsets.to(torch.int64).contiguous()
+        index_remappings = index_remappings.contiguous()
+        if logical.numel() != rows.numel() or offs.numel() != rows.numel() + 1:
+            raise ValueError("the mappings do not belong to these tables")
+    out_indices, out_offsets = torch.empty_like(indices), torch.empty_like(offsets)
+    check(_lib.lib().fbgemm_amd_check_remap_indices(
+        _ptr(rows), rows.numel(), _ptr(indices), _ptr(offsets), _bits(indices), indices.numel(), offsets.numel(),
+        int(bounds_check_mode), _ptr(warning), _ptr(logical), _ptr(index_remappings),
+        32 if index_remappings is None else _bits(index_remappings), _ptr(offs), _ptr(out_indices), _ptr(out_offsets),
+        _stream()))
+    return out_indices, out_offsets
+
+
 def pruned_hashmap_lookup(indices, offsets, hash_table, hash_table_offsets):
     """pruned_hashmap_lookup (embedding_forward_quantized_host_cpu.cpp:338-341;
     embedding_forward_quantized_cpu_template.cpp:524-603)."""

@@ -400,6 +400,19 @@ int fbgemm_amd_bounds_check_indices(
     int64_t indices_numel, int64_t offsets_numel, int32_t bounds_check_mode, int64_t* d_warning,
     const int32_t* d_B_offsets, void* d_status, void* stream);
 
+/* bounds_check_indices in WARNING or IGNORE mode on copies of the inputs, with the
+ * array-based pruned-row mapping in the same pass when there is one: the check
+ * against d_logical_rows_per_table, pruned_array_lookup, and the check against
+ * d_rows_per_table, each index read and written once. d_index_remappings_offsets
+ * (T + 1 entries) may be NULL: then only the check. d_out_indices and d_out_offsets
+ * have the inputs' sizes and must not overlap them; d_warning ends as the last check
+ * of the separate calls would leave it. B must not be zero. */
+int fbgemm_amd_check_remap_indices(
+    const int64_t* d_rows_per_table, int32_t T, const void* d_indices, const void* d_offsets, int32_t index_bits,
+    int64_t indices_numel, int64_t offsets_numel, int32_t bounds_check_mode, int64_t* d_warning,
+    const int64_t* d_logical_rows_per_table, const void* d_index_remappings, int32_t remap_bits,
+    const int64_t* d_index_remappings_offsets, void* d_out_indices, void* d_out_offsets, void* stream);
+
 /* pruned_hashmap_lookup (embedding_forward_quantized_cpu_template.cpp:524-603; GPU
  * embedding_forward_quantized_split_lookup.cu:19-118): d_hash_table holds
  * [slots][2] (sparse id, dense id) pairs of hash_bits each, -1 = empty, built by

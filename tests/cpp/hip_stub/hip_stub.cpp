@@ -230,6 +230,12 @@ hipError_t launch_quantize_segments(const float* input, int64_t lines, int32_t, 
 }
 hipError_t launch_bounds_check(const int64_t*, int32_t, void*, void*, bool, int64_t, int64_t, int64_t, const int32_t*, int, int64_t*,
                                int64_t*, int64_t*, Status*, hipStream_t) { return LAUNCHED(); }
+int64_t check_remap_partials(int64_t total_B) { return total_B / 256 + 1; }
+hipError_t launch_check_remap(CheckRemapArgs a, bool, bool, int64_t* partial, hipStream_t) {
+  (void)*(volatile const int64_t*)&partial[(a.total_B + 255) / 256 - 1];
+  (void)*(volatile const unsigned long long*)a.counter;
+  return LAUNCHED();
+}
 int64_t bounds_check_partials(int64_t total_B) { return total_B / 1024 + 2; }
 hipError_t launch_quantize_rowwise(const void*, bool, int64_t, int32_t, int32_t, int32_t, int32_t, int64_t, void*, const void*,
                                    hipStream_t) { return LAUNCHED(); }
