@@ -76,27 +76,58 @@ int sort_bags_default() {
 // round trips inside a wave, and spreading its bags over more waves shortens nothing per wave but
 // lets every compute unit work (measured: the 1 024-bag 8-bit table 13.0 -> 9.7 us, the 4 096-bag
 // 4-bit table 22.8 -> 15.8 us; rounds of 16 rows on top of that changed nothing).
-void plan_lanes(TableDesc& d, uintptr_t base_addr, int64_t out_stride, bool has_sb, bool allow_packed, bool narrow = false) {
+//
+// Rows that are no whole number of 16-byte chunks take them all the same: the last chunk either reads
+// past the data into bytes the row owns (`room`: bytes of a row from data_off on that may be read), or
+// starts early and overlaps its neighbour, whose columns its lane then computes and writes a second
+// time. Lanes of 4 bytes, or of single bytes, would need 4 to 16 times the load instructions and leave
+// the wave with a quarter of the bags (10 000 bags x 25 of a 100-wide 8-bit table 36.5 -> 30.8 us; 40
+// tables of every type and 4 .. 300 wide, 1000 bags x 12: 69.5 -> 44.7 us).
+void plan_lanes(TableDesc& d, uintptr_t base_addr, int64_t out_stride, bool has_sb, int64_t room, bool allow_packed, bool narrow = false) {
   const int bits = type_bits(d.ty);
   d.data_bytes = (int32_t)(((int64_t)d.D * bits + 7) / 8);
   const bool a4 = base_addr % 4 == 0 && d.weights_offset % 4 == 0 && d.row_stride % 4 == 0 &&
       d.data_off % 4 == 0 && (!has_sb || d.sb_off % 4 == 0);
   const int min_vb = bits >= 16 ? bits / 8 : 1;
+  const int64_t data16 = ((int64_t)d.data_bytes + 15) / 16 * 16, data8 = ((int64_t)d.data_bytes + 7) / 8 * 8,
+                data4 = ((int64_t)d.data_bytes + 3) / 4 * 4;
   int vb = min_vb;
-  if (a4 && d.data_bytes % 16 == 0 && d.ty != ST_INT2) vb = 16;
-  else if (a4 && d.data_bytes % 4 == 0) vb = 4;
+  if (d.ty == ST_INT2) { // 64 columns per lane would be too many accumulators
+    if (a4 && !narrow && d.data_bytes > 8 && (data8 <= room || d.data_bytes % 4 == 0)) vb = 8;
+    else if (a4 && (data4 <= room || d.data_bytes % 4 == 0)) vb = 4;
+  } else if (a4 && (data16 <= room || (d.data_bytes % 4 == 0 && d.data_bytes >= 16))) {
+    vb = 16;
+  } else if (a4 && (data4 <= room || d.data_bytes % 4 == 0)) {
+    vb = 4;
+  }
   if (narrow && vb == 16) vb = 4;
   d.vb = vb;
   const int chunks = (d.data_bytes + vb - 1) / vb;
+  // the last chunk: at its place when it ends inside the row's own bytes, early otherwise
+  d.last_chunk = (int64_t)chunks * vb <= std::max<int64_t>(room, d.data_bytes) ? (chunks - 1) * vb : d.data_bytes - vb;
   // Wide rows: give a lane several 16-byte chunks (up to 32 accumulators), so
-  // that the per-row bookkeeping is shared by more elements.
+  // that the per-row bookkeeping is shared by more elements: as many as divide the row, else as
+  // many as leave the fewest lanes of the wave without a chunk.
   const int type_c = bits >= 16 ? 4 : (bits == 8 ? 2 : 1);
   int C = 1;
-  if (vb == 16)
+  if (vb == 16) {
     for (int c = type_c; c > 1; c >>= 1)
       if (chunks % c == 0 && chunks / c >= 2) { C = c; break; }
+    if (C == 1) {
+      double best = 0;
+      for (int c = type_c; c >= 1; c >>= 1) {
+        const int lanes = std::max(2, (chunks + c - 1) / c);
+        const int turns = (lanes + 63) / 64; // column passes
+        const double used = (lanes <= 64 ? (double)bags_per_wave(lanes, 0) : 1.0 / turns) * chunks / (64.0 * c);
+        if (used > 1.05 * best) {
+          best = used;
+          C = c;
+        }
+      }
+    }
+  }
   d.chunks = C;
-  d.lanes = std::max(2, std::min(64, chunks / C)); // >= 2: a wave stages at most 32 bags
+  d.lanes = std::max(2, std::min(64, (chunks + C - 1) / C)); // >= 2: a wave stages at most 32 bags
   d.passes = (chunks + d.lanes * C - 1) / (d.lanes * C);
   // Whole-row chunks for 4- and 8-bit rows with the fp16 header first and a
   // stride that is a multiple of 16: the header rides in chunk 0 and costs no
@@ -125,25 +156,27 @@ void plan_lanes(TableDesc& d, uintptr_t base_addr, int64_t out_stride, bool has_
       for (int k = 0; k < 2; ++k) {
         const int esz = k == 0 ? 4 : 2;
         const int al = std::min(16, GE * esz);
-        if ((out_stride * esz) % al == 0 && ((int64_t)d.out_col * esz) % al == 0) d.vec_store |= 1 << k;
+        if ((out_stride * esz) % al == 0 && ((int64_t)d.out_col * esz) % al == 0) d.vec_store |= 5 << k;
       }
       return;
     }
   }
-  // whole-run vector stores: each lane writes E = vb*8/bits consecutive
-  // elements; allowed when every run starts on a multiple of min(16, run bytes)
-  // and no run is cut by the end of the row.
+  // whole-run vector stores: each lane writes E = vb*8/bits consecutive elements. Bits 0 and 1 (the
+  // lean kernel): every run starts on a multiple of min(16, run bytes) and no run is cut by the end
+  // of the row. Bits 2 and 3 (the general kernel, which writes a cut run element by element): runs
+  // are whole dwords on dword boundaries, all that the wide stores need.
   const int E = vb * 8 / bits;
   d.vec_store = 0;
-  if (d.D % E == 0) {
-    for (int k = 0; k < 2; ++k) {
-      const int esz = k == 0 ? 4 : 2;
-      const int run = E * esz;
-      const int al = std::min(16, run);
-      if ((run == 2 || run == 4 || run == 8 || run % 16 == 0) && (out_stride * esz) % al == 0 &&
-          ((int64_t)d.out_col * esz) % al == 0)
-        d.vec_store |= 1 << k;
-    }
+  for (int k = 0; k < 2; ++k) {
+    const int esz = k == 0 ? 4 : 2;
+    const int run = E * esz;
+    const int al = std::min(16, run);
+    if (d.D % E == 0 && (run == 2 || run == 4 || run == 8 || run % 16 == 0) && (out_stride * esz) % al == 0 &&
+        ((int64_t)d.out_col * esz) % al == 0)
+      d.vec_store |= 1 << k;
+    if ((run == 4 || run == 8 || run % 16 == 0) && (out_stride * esz) % 4 == 0 && ((int64_t)d.out_col * esz) % 4 == 0 &&
+        ((int64_t)d.last_chunk * 8 / bits * esz) % 4 == 0)
+      d.vec_store |= 4 << k;
   }
 }
 
@@ -596,7 +629,10 @@ int spmdm_launch_impl(
                               (Status*)d_status, stream));
     return 0;
   }
-  plan_lanes(d, (uintptr_t)d_input, out_stride, has_sb, false);
+  // bytes of a row that are known to be there (the last row may end with them), from data_off on
+  const int64_t packed_bytes = (D * bits + 7) / 8;
+  const int64_t room = has_sb && cfg->scale_bias_last ? packed_bytes + (d.sb_fp32 ? 8 : 4) : packed_bytes;
+  plan_lanes(d, (uintptr_t)d_input, out_stride, has_sb, room, false);
   // few, long bags, and the caller accepts sums in another order: cut every bag into K segments.
   // 4- and 8-bit rows only: every other row type is summed the reference's way in either mode,
   // in one piece.
@@ -610,11 +646,11 @@ int spmdm_launch_impl(
   }
   const int64_t pooled_bags = output_size * K;       // what the lookup kernel sees as bags
   const int64_t pooled_stride = K > 1 ? D : out_stride; // segments' sums are rows of D floats
-  if (K > 1) plan_lanes(d, (uintptr_t)d_input, pooled_stride, has_sb, false);
+  if (K > 1) plan_lanes(d, (uintptr_t)d_input, pooled_stride, has_sb, room, false);
   {
     // a launch of fewer than four waves per compute unit: prefer narrow lanes
     const int G16 = bags_per_wave(d.lanes, d.packed);
-    if (d.vb == 16 && (pooled_bags + G16 - 1) / G16 < narrow_below_waves()) plan_lanes(d, (uintptr_t)d_input, pooled_stride, has_sb, false, true);
+    if (d.vb == 16 && (pooled_bags + G16 - 1) / G16 < narrow_below_waves()) plan_lanes(d, (uintptr_t)d_input, pooled_stride, has_sb, room, false, true);
   }
   d.lanes_recip = (65536 + d.lanes - 1) / d.lanes;
   d.bags = bags_per_wave(d.lanes, d.packed);
@@ -1071,7 +1107,7 @@ int fbgemm_amd_tbe_plan_create(
     d.sb_off = 0;
     d.data_off = q ? 4 : 0;
     // weights buffers come from hipMalloc / torch: at least 256-byte aligned
-    plan_lanes(d, 0, plan->total_D, q, false);
+    plan_lanes(d, 0, plan->total_D, q, d.row_stride - d.data_off, false); // a row owns its whole stride
     d.lanes_recip = (65536 + d.lanes - 1) / d.lanes;
     d.bags = bags_per_wave(d.lanes, d.packed);
   }
@@ -1084,7 +1120,7 @@ int fbgemm_amd_tbe_plan_create(
   bool any_packed = false;
   for (int t = 0; t < T; ++t) {
     TableDesc& d = plan->tables_packed[t];
-    plan_lanes(d, 0, plan->total_D, quantised(d.ty), true);
+    plan_lanes(d, 0, plan->total_D, quantised(d.ty), d.row_stride - d.data_off, true);
     d.lanes_recip = (65536 + d.lanes - 1) / d.lanes;
     d.bags = bags_per_wave(d.lanes, d.packed);
     any_packed = any_packed || d.packed;
@@ -1098,7 +1134,7 @@ int fbgemm_amd_tbe_plan_create(
   plan->tables_narrow = plan->tables;
   for (int t = 0; t < T; ++t) {
     TableDesc& d = plan->tables_narrow[t];
-    plan_lanes(d, 0, plan->total_D, quantised(d.ty), false, true);
+    plan_lanes(d, 0, plan->total_D, quantised(d.ty), d.row_stride - d.data_off, false, true);
     d.lanes_recip = (65536 + d.lanes - 1) / d.lanes;
     d.bags = bags_per_wave(d.lanes, d.packed);
   }

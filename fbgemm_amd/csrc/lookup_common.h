@@ -65,7 +65,7 @@ struct TableDesc {
   int32_t D;              // elements per row
   int32_t out_col;        // first output column of this table's block
   int32_t ty;             // ST_*
-  int32_t vb;             // bytes each lane loads per row and pass: 1, 2, 4 or 16
+  int32_t vb;             // bytes each lane loads per row and pass: 1, 2, 4, 8 or 16
   int32_t sb_off;         // byte offset of (scale, bias) inside a row
   int32_t data_off;       // byte offset of the element data inside a row
   int32_t sb_fp32;        // 1: scale/bias are two floats, 0: two halfs
@@ -75,7 +75,8 @@ struct TableDesc {
   int32_t data_bytes;     // bytes of element data per row (unpadded)
   int32_t skip_minus_one; // 1: an index of -1 is a pruned row and is skipped
   int32_t vec_store;      // bit 0 / bit 1: every lane's output run is aligned for whole-run
-                          // vector stores with 4-byte / 2-byte output elements
+                          // vector stores with 4-byte / 2-byte output elements; bits 2 / 3: the
+                          // runs of the general kernel are dwords on dword boundaries
   int32_t chunks;         // 16-byte chunks per lane and pass (1, 2 or 4)
   int32_t inline_hdr;     // 1: lanes own 16-byte chunks of the WHOLE row (fp16 scale/bias
                           // header first, then data), so the header arrives with the data
@@ -83,6 +84,8 @@ struct TableDesc {
   int32_t packed;         // 1: bags lie end to end in the wave (see bags_per_wave)
   int32_t lanes_recip;    // ceil(65536 / lanes): j / lanes == (j * lanes_recip) >> 16 for 0 <= j <= 64
   int32_t bags;           // bags_per_wave(lanes, packed), so that no kernel divides
+  int32_t last_chunk;     // byte of the row's data where its last chunk starts: chunk k starts at
+                          // min(k * vb, last_chunk) (general kernel, without inline_hdr)
 };
 
 #if defined(__HIPCC__)

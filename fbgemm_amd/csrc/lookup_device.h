@@ -260,16 +260,18 @@ __device__ __forceinline__ uint32_t pack_bf16x2(float lo, float hi) {
 }
 __device__ __forceinline__ uint32_t pack_half2(float lo, float hi) { return to_half_bits(lo) | (to_half_bits(hi) << 16); }
 
+// `p` on a dword boundary (2-byte stores: on their own)
 template <int NBYTES>
 __device__ __forceinline__ void store_words(void* p, const uint32_t* w) {
   if constexpr (NBYTES >= 16) {
 #pragma unroll
     for (int i = 0; i < NBYTES / 16; ++i) {
-      uint4 v = make_uint4(w[4 * i], w[4 * i + 1], w[4 * i + 2], w[4 * i + 3]);
-      reinterpret_cast<uint4*>(p)[i] = v;
+      const Dwordx4 v = {{w[4 * i], w[4 * i + 1], w[4 * i + 2], w[4 * i + 3]}};
+      reinterpret_cast<Dwordx4*>(p)[i] = v;
     }
   } else if constexpr (NBYTES == 8) {
-    *reinterpret_cast<uint2*>(p) = make_uint2(w[0], w[1]);
+    const Dwordx2 v = {{w[0], w[1]}};
+    *reinterpret_cast<Dwordx2*>(p) = v;
   } else if constexpr (NBYTES == 4) {
     *reinterpret_cast<uint32_t*>(p) = w[0];
   } else {
@@ -281,7 +283,7 @@ template <int E>
 __device__ __forceinline__ void write_out(const LookupArgs& a, const float (&acc)[E], int64_t elem_pos, int col0, int D, bool vec_ok) {
   if (a.out_ty == ST_FP32) {
     float* o = reinterpret_cast<float*>(a.out) + elem_pos;
-    if (vec_ok) {
+    if (vec_ok && col0 + E <= D) {
       uint32_t w[E];
 #pragma unroll
       for (int e = 0; e < E; ++e) w[e] = float_to_bits(acc[e]);
@@ -294,7 +296,7 @@ __device__ __forceinline__ void write_out(const LookupArgs& a, const float (&acc
   } else {
     uint16_t* o = reinterpret_cast<uint16_t*>(a.out) + elem_pos;
     const bool bf = a.out_ty == ST_BF16;
-    if (vec_ok && E >= 2) {
+    if (vec_ok && E >= 2 && col0 + E <= D) {
       uint32_t w[(E + 1) / 2];
       if (bf) {
 #pragma unroll

@@ -14,7 +14,8 @@ namespace fbgemm_amd {
 // One wave pools bags_per_wave(lanes) bags of one table, `RN` entries of every bag per
 // round. Each lane owns C chunks of VB bytes of every row: chunk c of lane
 // `sub` starts at byte (c * lanes + sub) * VB of the row data, so every load
-// instruction of the wave reads contiguous bytes of each row.
+// instruction of the wave reads contiguous bytes of each row (the row's last
+// chunk may start earlier, TableDesc::last_chunk).
 //
 // Per-entry work (index load, per-sample weight, -1 / bounds / remap handling,
 // row offset, the scale/bias fetch and its two products with the weight) is
@@ -147,30 +148,22 @@ __device__ __forceinline__ bool pool_bags(const LookupArgs& a, const TableDesc& 
   StageMul* my_mul = stage_mul + lgrp * RN;
   // the reference keeps the bag length in an int when it forms 1/len
   const float inv_len = (a.normalize && n > 0) ? 1.0f / (float)n : 1.0f;
-  const int chunk_stride = S * VB; // bytes between a lane's consecutive chunks
 
   for (int pass = 0; pass < d.passes; ++pass) {
     const int chunk0 = pass * S * C + sub;
+    // the lane's chunks: whether they are its to write, and their bytes inside the row (INHDR) or its
+    // data. A slot past the row shadows the last chunk: same bytes, nothing written.
+    const int nchunks = ((INHDR ? d.data_bytes + 4 : d.data_bytes) + VB - 1) / VB;
+    const int last = INHDR ? (nchunks - 1) * VB : d.last_chunk;
     bool on[C];
-    bool all_on = bag_ok;
-    int rowb[C]; // INHDR: byte offset of the lane's chunks inside the row
-    if constexpr (INHDR) {
-      const int nchunks = (d.data_bytes + 4 + VB - 1) / VB;
+    int rowb[C];
 #pragma unroll
-      for (int c = 0; c < C; ++c) {
-        const int k = chunk0 + c * S;
-        on[c] = bag_ok && k < nchunks;
-        rowb[c] = (k < nchunks ? k : nchunks - 1) * VB; // a slot past the row shadows the last chunk
-      }
-    } else {
-#pragma unroll
-      for (int c = 0; c < C; ++c) {
-        on[c] = bag_ok && (chunk0 + c * S) * VB < d.data_bytes;
-        all_on = all_on && on[c];
-        rowb[c] = 0;
-      }
+    for (int c = 0; c < C; ++c) {
+      const int k = chunk0 + c * S;
+      on[c] = bag_ok && k < nchunks;
+      rowb[c] = min(k * VB, last);
     }
-    const uint8_t* pdata = INHDR ? wbase : wbase + d.data_off + chunk0 * VB;
+    const uint8_t* pdata = INHDR ? wbase : wbase + d.data_off;
 
     float acc[C][E];
 #pragma unroll
@@ -254,14 +247,12 @@ __device__ __forceinline__ bool pool_bags(const LookupArgs& a, const TableDesc& 
       return hole;
     };
 
-    // wave-uniform: every lane of the wave pools a bag and owns C live chunks
-    // (whole-row chunks: slots past the row are clamped, lanes without a bag never enter the loop)
-    const bool wave_on = INHDR || (__builtin_amdgcn_ballot_w64(!all_on) == 0ull && __builtin_amdgcn_ballot_w64(true) == ~0ull);
     load_idx(0);
-    // wave-uniform: the staged round has RN rows to add for every bag of the wave
+    // wave-uniform: the staged round has RN rows to add for every bag of the wave that is in the loop
+    // (lanes without a bag never enter it)
     // (the staging call comes first on its own line: it must run on every wave)
     const bool hole0 = stage_rows(0);
-    bool fast = wave_on && __builtin_amdgcn_ballot_w64(hole0) == 0ull;
+    bool fast = __builtin_amdgcn_ballot_w64(hole0) == 0ull;
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
 
@@ -303,7 +294,7 @@ __device__ __forceinline__ bool pool_bags(const LookupArgs& a, const TableDesc& 
           if (e < RN) {
             const uint8_t* p = pdata + my_row[e].off;
 #pragma unroll
-            for (int c = 0; c < C; ++c) load_raw<VB>(raw[e][c], INHDR ? p + rowb[c] : p + c * chunk_stride);
+            for (int c = 0; c < C; ++c) load_raw<VB>(raw[e][c], p + rowb[c]);
           }
         }
       } else {
@@ -320,10 +311,7 @@ __device__ __forceinline__ bool pool_bags(const LookupArgs& a, const TableDesc& 
               const int64_t off = my_row[e].off;
               if (off >= 0) {
 #pragma unroll
-                for (int c = 0; c < C; ++c) {
-                  if constexpr (INHDR) load_raw<VB>(raw[e][c], pdata + off + rowb[c]);
-                  else if (on[c]) load_raw<VB>(raw[e][c], pdata + off + c * chunk_stride);
-                }
+                for (int c = 0; c < C; ++c) load_raw<VB>(raw[e][c], pdata + off + rowb[c]);
               }
             }
           }
@@ -387,14 +375,14 @@ __device__ __forceinline__ bool pool_bags(const LookupArgs& a, const TableDesc& 
       // offsets (and plain weights) of the next round; the column lanes have
       // read this round's entries by now
       const bool hole = stage_rows(r + 1);
-      fast = wave_on && __builtin_amdgcn_ballot_w64(hole) == 0ull;
+      fast = __builtin_amdgcn_ballot_w64(hole) == 0ull;
       __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
       __builtin_amdgcn_wave_barrier();
     }
 
     if (__builtin_amdgcn_ballot_w64(give_up) != 0ull) return false; // every lane of the wave is back here
 
-    const bool vec_ok = a.out_aligned && ((d.vec_store >> (a.out_ty == ST_FP32 ? 0 : 1)) & 1);
+    const bool vec_ok = a.out_aligned && ((d.vec_store >> (a.out_ty == ST_FP32 ? 2 : 3)) & 1);
 #pragma unroll
     for (int c = 0; c < C; ++c) {
       if (on[c]) {
@@ -406,7 +394,7 @@ __device__ __forceinline__ bool pool_bags(const LookupArgs& a, const TableDesc& 
           const int col0 = (chunk0 + c * S) * E - E / 4;
           write_out_runs<E>(a, acc[c], (int64_t)bag * a.out_stride + d.out_col, col0, d.D, vec_ok);
         } else {
-          const int col0 = (chunk0 + c * S) * E;
+          const int col0 = rowb[c] * 8 / BITS;
           const int64_t elem_pos = (int64_t)bag * a.out_stride + d.out_col + col0;
           write_out<E>(a, acc[c], elem_pos, col0, d.D, vec_ok);
         }
@@ -430,7 +418,7 @@ __device__ __forceinline__ void run_bags(const LookupArgs& a, const TableDesc& d
 // Row types and the lane shapes the host may pick for them (TableDesc::vb,
 // TableDesc::chunks): 16-byte chunks with up to 4 (fp16 / bf16 / fp32), 2
 // (int8) or 1 (int4) chunks per lane so that a lane holds at most 32
-// accumulators; 4-byte and element-sized chunks for everything else.
+// accumulators; 8-byte ones for 2-bit rows; 4-byte and element-sized chunks for everything else.
 template <typename index_t, bool GENERAL, int TY>
 __device__ __forceinline__ void pool_dispatch_vb(const LookupArgs& a, const TableDesc& d, int table, int first_slot,
                                                  int lane, StageRow* stage_row, StageMul* stage_mul) {
@@ -447,12 +435,14 @@ __device__ __forceinline__ void pool_dispatch_vb(const LookupArgs& a, const Tabl
   }
   if (d.vb == 16) {
     if constexpr (TY == ST_INT2) {
-      run_bags<index_t, GENERAL, TY, 4, 1, 8>(a, d, table, first_slot, lane, stage_row, stage_mul); // not selected by the host
+      // not selected by the host
     } else {
       if (d.chunks == 4 && MAXC >= 4) run_bags<index_t, GENERAL, TY, 16, (MAXC >= 4 ? 4 : 1), 2>(a, d, table, first_slot, lane, stage_row, stage_mul);
       else if (d.chunks == 2 && MAXC >= 2) run_bags<index_t, GENERAL, TY, 16, (MAXC >= 2 ? 2 : 1), 4>(a, d, table, first_slot, lane, stage_row, stage_mul);
       else run_bags<index_t, GENERAL, TY, 16, 1, 8>(a, d, table, first_slot, lane, stage_row, stage_mul);
     }
+  } else if (TY == ST_INT2 && d.vb == 8) {
+    if constexpr (TY == ST_INT2) run_bags<index_t, GENERAL, TY, 8, 1, 8>(a, d, table, first_slot, lane, stage_row, stage_mul);
   } else if (d.vb == 4) {
     run_bags<index_t, GENERAL, TY, 4, 1, 8>(a, d, table, first_slot, lane, stage_row, stage_mul);
   } else {
