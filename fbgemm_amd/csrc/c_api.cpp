@@ -256,17 +256,22 @@ int wide4_mode() {
 }
 
 // Which launches the burst kernel (lookup_burst.h) takes, and in which form. `bags`: of all tables;
-// us of the single-table kernel over 1 M uniform rows, other kernels -> burst kernel:
-//                       10 bags x 100   1024 x 20      4096 x 20      8192 x 20      8192 x 10
-//   4-bit, 128 wide     47.7 -> 10.8    17.3 -> 9.4    19.0 -> 12.1   20.6 -> 19.5   14.6 -> 16.3
-//   8-bit, 100 wide     47.7 -> 11.2    17.4 -> 9.5    19.9 -> 12.0   32.0 -> 19.2   23.7 -> 15.7
-//   fp16, 256 wide      57.1 -> 14.3    20.0 -> 10.0   25.4 -> 17.3   28.0 -> 25.9   18.7 -> 19.7
-//   8-bit, 512 wide     52.0 -> 13.6    18.4 -> 10.9   20.4 -> 24.0   30.8 -> 37.7   19.9 -> 27.2
+// us of the single-table kernel over 1 M uniform rows, the better of the other kernels -> burst kernel:
+//                       10 bags x 100   1024 x 20      8192 x 10      8192 x 25      16384 x 10     16384 x 25
+//   4-bit, 128 wide     47.7 -> 10.8    17.3 -> 9.4    15.1 -> 14.6   21.8 -> 19.0   18.0 -> 22.2   27.4 -> 28.3
+//   8-bit, 100 wide     47.7 -> 11.2    17.4 -> 9.5    20.5 -> 14.6   29.1 -> 20.5   23.3 -> 22.1   37.5 -> 30.2
+//   8-bit, 36 wide                                     14.6 -> 13.8   20.8 -> 17.7   22.0 -> 21.4   31.9 -> 26.4
+//   fp16, 64 wide                                      18.3 -> 12.8   25.8 -> 16.8   21.2 -> 19.6   30.8 -> 24.5
+//   fp16, 200 wide                                     21.8 -> 19.3   33.7 -> 29.3   27.1 -> 28.8   48.8 -> 47.5
+//   8-bit, 512 wide     52.0 -> 13.6    18.4 -> 10.9   14.8 -> 17.1 and 20.4 -> 24.0 (4096 x 10 and x 20)
 // It is bound by how many workgroups the device holds at a time, so the line lies at workgroups:
-// 4096 (16 per compute unit: all resident at once), and 8192 where bags are long enough to need
-// several rounds in the other kernels and a workgroup covers the whole row.
+// 4096 (16 per compute unit: all resident at once), 8192 where a workgroup covers the whole row, and
+// 16384 for bags of three rounds and more in the other kernels.
 // Four waves per bag pay while all such workgroups are resident together (four per compute unit:
 // 1024; 1024 bags x 100: 22.0 -> 13.9) and, for long bags, in two rounds of them (2048 x 100: 24.9 -> 21.9).
+// LDS: large launches want many workgroups resident, so they stage in 4 KB what takes at most two
+// stagings there (8-bit, 100 wide, 8192 x 60: 35.6 -> 31.2), in 8 KB otherwise (fp16, 200 wide, 16384 x 25:
+// 47.5 against 49.2); small ones stage as much as they can.
 struct Burst {
   int waves = 0; // 0: another kernel takes the launch
   int lds_bytes = 0;
@@ -274,20 +279,23 @@ struct Burst {
 // 1 / 4: every launch it can take goes to the burst kernel with that many waves per bag, 0: none does,
 // -1: by the rule (tests: fbgemm_amd_set_burst).
 int g_burst_override = -1;
-constexpr int BURST_COLS = 256;
-Burst plan_burst(int64_t bags, int32_t T, int32_t max_D, int64_t lookups) {
+constexpr int32_t BURST_COLS = 256;
+Burst plan_burst(int64_t bags, int32_t T, int32_t max_D, int32_t max_bits, int64_t lookups) {
   Burst b;
   const int64_t windows = ((int64_t)max_D + BURST_COLS - 1) / BURST_COLS;
   if (g_burst_override == 0 || narrow_below_waves() == 0 || bags <= 0 || T > 65535 || windows > 65535 ||
       (g_burst_override < 0 && lookups >= SORT_MIN_LOOKUPS)) // those launches order their bags
     return b;
   const int64_t groups = bags * windows, avg_len = lookups / bags;
-  if (g_burst_override > 0) {
+  if (g_burst_override > 0)
     b.waves = g_burst_override;
-  } else if (groups <= 4096 || (groups <= 8192 && windows == 1 && avg_len >= 16)) {
+  else if (groups <= 4096 || (windows == 1 && (groups <= 8192 ? avg_len >= 8 : groups <= 16384 && avg_len >= 24)))
     b.waves = (groups <= 1024 && avg_len >= 16) || (groups <= 2048 && avg_len >= 64) ? 4 : 1;
-  }
-  b.lds_bytes = b.waves == 4 ? 32768 : (groups <= 2048 ? 16384 : 8192);
+  // bytes of a staged row, of the widest type and table of the launch
+  const int64_t pitch = ((int64_t)std::min(max_D, BURST_COLS) * max_bits / 8 + 15) / 16 * 16;
+  b.lds_bytes = b.waves == 4 ? 32768
+      : groups <= 2048       ? 16384
+      : groups > 4096 && 8 * pitch <= 4096 && std::min<int64_t>(avg_len, 64) * pitch <= 8192 ? 4096 : 8192;
   return b;
 }
 // Where the burst kernel would take the launch, bags shorter than this are not cut into segments
@@ -637,7 +645,7 @@ int spmdm_launch_impl(
   // 4- and 8-bit rows only: every other row type is summed the reference's way in either mode,
   // in one piece.
   int K = 1;
-  const Burst burst = plan_burst(output_size, 1, d.D, index_size);
+  const Burst burst = plan_burst(output_size, 1, d.D, bits, index_size);
   if (!noalloc && cfg->accumulate == FBGEMM_AMD_ACC_FAST && !cfg->is_weight_positional && output_size * 32 <= 0x7fffffffLL &&
       (ty == ST_INT4 || ty == ST_INT8)) {
     const int G16 = bags_per_wave(d.lanes, d.packed);
@@ -832,6 +840,7 @@ struct fbgemm_amd_tbe_plan {
   TableDesc* d_tables = nullptr;
   int32_t* d_D_offsets = nullptr; // the T + 1 output column offsets, for the 8-bit pooled output
   int32_t max_D = 0;
+  int32_t max_bits = 0;           // of the row types
   float* pooled_tmp = nullptr;    // fp32 [B, total_D] the 8-bit pooled output is quantized from
   int64_t pooled_tmp_cap = 0;
   int64_t* seg_offsets = nullptr; // split bags: where every segment starts (T*B*K + 1)
@@ -1102,6 +1111,7 @@ int fbgemm_amd_tbe_plan_create(
     d.num_rows = std::max<int64_t>(0, (next - d.weights_offset) / d.row_stride);
     d.skip_minus_one = 1;
     plan->has_fp8 = plan->has_fp8 || d.ty == ST_FP8;
+    plan->max_bits = std::max(plan->max_bits, type_bits(d.ty));
     const bool q = quantised(d.ty);
     d.sb_fp32 = 0;
     d.sb_off = 0;
@@ -1318,7 +1328,7 @@ int tbe_forward_impl(
   // (Only when every table has rows the tolerance-grade arithmetic applies to: fp16 / fp32 / 2-bit
   // / odd-shaped tables are summed the reference's way in either mode, and a bag cut into
   // segments is not.)
-  const Burst burst = plan_burst((int64_t)plan->T * B, plan->T, plan->max_D, indices_numel);
+  const Burst burst = plan_burst((int64_t)plan->T * B, plan->T, plan->max_D, plan->max_bits, indices_numel);
   bool all_fast_rows = true;
   for (const TableDesc& d : plan->tables) all_fast_rows = all_fast_rows && (d.ty == ST_INT4 || d.ty == ST_INT8);
   if (allow_split && plan->accumulate == FBGEMM_AMD_ACC_FAST && all_fast_rows && (int64_t)B * 32 <= 0x7fffffffLL) {

@@ -5,12 +5,15 @@
 // are nowhere near the caches or the TLBs; bytes and arithmetic do not show. So one workgroup owns
 // one bag (and up to 256 of its columns) and asks for ALL of it at once: a thread per entry reads
 // the index, the weight and the row's scale and bias, then every thread copies 16-byte pieces of
-// different rows into LDS with up to 8 loads in flight, and only then are the rows added up, each
+// different rows into LDS with 4 or 8 loads in flight, and only then are the rows added up, each
 // column by one lane, in index order: the sequence of roundings is the reference's, bit for bit.
 // A bag needs three round trips instead of two and one per 8 rows.
 //
 // WAVES = 1: a wave per bag, a lane owns 4 columns (64 lanes * 4 = the 256 columns), up to 64 rows
-// at a time in 8 KB of LDS (16 KB where the launch leaves it). WAVES = 4: four waves per bag, a lane
+// at a time in 4, 8 or 16 KB of LDS. Large launches are bound by how many workgroups are resident, so
+// this form keeps 4 loads per thread and adds 4 rows per turn, which fits 5 waves per SIMD without
+// spills (8 and 8 need 128 registers, 4 waves: 5000 bags x 25 of a 4-bit table 16.0 us, so 14.6; 6 and
+// 8 waves per SIMD spill: 16.8 and 16.0). WAVES = 4: four waves per bag, a lane
 // owns one column, up to 256 rows at a time in 32 KB: for fewer bags than compute units have room
 // for, whose rows one wave would need many loads each for, and whose summing loop (a dependent add
 // and fma per row and column) is the longest part left. Which of them, and from where on the other
@@ -21,7 +24,6 @@
 namespace fbgemm_amd {
 
 constexpr int BURST_COLS = 256; // columns of a workgroup
-constexpr int BURST_MIN_WAVES = 4; // waves per SIMD: at 5 the compiler spills
 
 // What a row's window of columns looks like in memory and in LDS: np pieces of `size` bytes, piece
 // k at byte k * size of the window, the last one at `last` (which is less where a whole piece there
@@ -98,19 +100,19 @@ __device__ __forceinline__ void burst_add(float (&acc)[K], const uint8_t* p, int
 
 // `rows` staged rows (a multiple of 8: holes carry the multiplier (-0, -0) and zeros, which leave an
 // accumulator as it is) added up in order.
-template <int TY, int K>
+template <int TY, int K, int R>
 __device__ __forceinline__ void burst_sum(float (&acc)[K], const uint8_t* col, int pitch, int shift, const StageMul* mul, int rows,
                                           int fp8_shift, float fp8_mult) {
 #pragma unroll 1
-  for (int r = 0; r < rows; r += 8) {
+  for (int r = 0; r < rows; r += R) {
 #pragma unroll
-    for (int u = 0; u < 8; ++u) burst_add<TY, K>(acc, col + (r + u) * pitch, shift, mul[r + u], fp8_shift, fp8_mult);
+    for (int u = 0; u < R; ++u) burst_add<TY, K>(acc, col + (r + u) * pitch, shift, mul[r + u], fp8_shift, fp8_mult);
   }
 }
 
 // The pieces of `rows` rows into LDS: S lanes (a power of two) take the pieces of a row, the
-// workgroup as many rows per load instruction as it has such groups, 8 loads per thread in flight.
-template <int SIZE, int THREADS>
+// workgroup as many rows per load instruction as it has such groups, U loads per thread in flight.
+template <int SIZE, int THREADS, int U>
 __device__ __forceinline__ void burst_copy(const uint8_t* base, const StageRow* off, int rows, const BurstWindow& w, uint8_t* lds) {
   constexpr int NW = SIZE == 16 ? 4 : 1;
   int log = 0;
@@ -121,10 +123,10 @@ __device__ __forceinline__ void burst_copy(const uint8_t* base, const StageRow* 
   for (int k = sub; k < w.np; k += S) { // one turn, but for single bytes
     const int from = k * SIZE < w.last ? k * SIZE : w.last;
 #pragma unroll 1
-    for (int r0 = group; r0 < rows; r0 += 8 * groups) {
-      uint32_t v[8][NW];
+    for (int r0 = group; r0 < rows; r0 += U * groups) {
+      uint32_t v[U][NW];
 #pragma unroll
-      for (int u = 0; u < 8; ++u) {
+      for (int u = 0; u < U; ++u) {
         const int r = r0 + u * groups;
 #pragma unroll
         for (int i = 0; i < NW; ++i) v[u][i] = 0;
@@ -134,7 +136,7 @@ __device__ __forceinline__ void burst_copy(const uint8_t* base, const StageRow* 
         }
       }
 #pragma unroll
-      for (int u = 0; u < 8; ++u) {
+      for (int u = 0; u < U; ++u) {
         const int r = r0 + u * groups;
         if (r < rows) {
           uint8_t* p = lds + r * w.pitch + k * SIZE;
@@ -179,9 +181,11 @@ __device__ __forceinline__ void burst_store(const LookupArgs& a, const float (&a
 
 // blockIdx: (bag, table, window of columns)
 template <typename index_t, int WAVES>
-__global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(BURST_MIN_WAVES, 8))) void lookup_burst_kernel(const LookupArgs a, int lds_bytes) {
+__global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(WAVES == 1 ? 5 : 4, 8))) void lookup_burst_kernel(const LookupArgs a, int lds_bytes) {
   constexpr int THREADS = 64 * WAVES;
   constexpr int K = BURST_COLS / THREADS; // columns per lane
+  constexpr int LOADS = WAVES == 1 ? 4 : 8;   // in flight per thread
+  constexpr int UNROLL = WAVES == 1 ? 4 : 8;  // rows added up per turn
   extern __shared__ __align__(16) uint8_t burst_lds[];
   StageRow* st_row = reinterpret_cast<StageRow*>(burst_lds);
   StageMul* st_mul = reinterpret_cast<StageMul*>(burst_lds + THREADS * sizeof(StageRow));
@@ -309,13 +313,13 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(BURS
     }
     load_entry(r0 + cap + tid);
     __syncthreads();
-    if (w.size == 16) burst_copy<16, THREADS>(first, st_row, rows, w, lds);
-    else if (w.size == 4) burst_copy<4, THREADS>(first, st_row, rows, w, lds);
-    else burst_copy<1, THREADS>(first, st_row, rows, w, lds);
+    if (w.size == 16) burst_copy<16, THREADS, LOADS>(first, st_row, rows, w, lds);
+    else if (w.size == 4) burst_copy<4, THREADS, LOADS>(first, st_row, rows, w, lds);
+    else burst_copy<1, THREADS, LOADS>(first, st_row, rows, w, lds);
     __syncthreads();
     if (mine) {
 #define FBGEMM_AMD_BURST_SUM(TY) \
-  case TY: burst_sum<TY, K>(acc, lds + at, w.pitch, shift, st_mul, rows, a.fp8_shift, a.fp8_mult); break;
+  case TY: burst_sum<TY, K, UNROLL>(acc, lds + at, w.pitch, shift, st_mul, rows, a.fp8_shift, a.fp8_mult); break;
       switch (d.ty) {
         FBGEMM_AMD_BURST_SUM(ST_INT4)
         FBGEMM_AMD_BURST_SUM(ST_INT8)

@@ -91,31 +91,56 @@ __global__ __launch_bounds__(1024) void bag_order_kernel(const void* offsets, in
 
 // ---- helpers ----------------------------------------------------------------
 
-// lengths -> offsets (exclusive prefix sum), one workgroup. Used when the
-// caller passes Caffe2-style lengths instead of offsets.
-template <typename T>
-__global__ __launch_bounds__(1024) void lengths_to_offsets_kernel(const T* lengths, int64_t n, int64_t* offsets) {
-  __shared__ int64_t part[1024];
-  const int tid = threadIdx.x;
-  const int64_t per = (n + 1023) / 1024;
-  const int64_t lo = (int64_t)tid * per;
-  const int64_t hi = lo + per < n ? lo + per : n;
-  int64_t sum = 0;
-  for (int64_t i = lo; i < hi; ++i) sum += (int64_t)(int)lengths[i];
-  part[tid] = sum;
+// lengths -> offsets (exclusive prefix sum). Used when the caller passes Caffe2-style lengths instead
+// of offsets. One launch without scratch: a workgroup owns a run of lengths, adds up everything before
+// it itself (from the caches, 8 loads in flight per thread) and scans its own run 1024 at a time. One
+// workgroup walking the whole array took 12.2 us for 10 000 lengths, this 6.3. At most
+// LENGTHS_MAX_BLOCKS runs, which bounds what is read twice (512 bytes per length).
+constexpr int LENGTHS_BLOCK = 1024;
+constexpr int LENGTHS_MAX_BLOCKS = 256;
+__device__ __forceinline__ int64_t lengths_block_scan(int64_t v, int64_t* lds, int64_t* total) { // inclusive
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  for (int step = 1; step < 64; step <<= 1) {
+    const int64_t o = __shfl_up(v, step, 64);
+    if (lane >= step) v += o;
+  }
+  __syncthreads(); // what an earlier call left in lds has been read
+  if (lane == 63) lds[wave] = v;
   __syncthreads();
-  for (int step = 1; step < 1024; step <<= 1) {
-    int64_t v = tid >= step ? part[tid - step] : 0;
-    __syncthreads();
-    part[tid] += v;
-    __syncthreads();
+  int64_t before = 0, all = 0;
+#pragma unroll
+  for (int w = 0; w < LENGTHS_BLOCK / 64; ++w) {
+    if (w < wave) before += lds[w];
+    all += lds[w];
   }
-  int64_t run = part[tid] - sum;
-  for (int64_t i = lo; i < hi; ++i) {
-    offsets[i] = run;
-    run += (int64_t)(int)lengths[i];
+  *total = all;
+  return v + before;
+}
+
+template <typename T>
+__global__ __launch_bounds__(LENGTHS_BLOCK) void lengths_to_offsets_kernel(const T* lengths, int64_t n, int64_t run, int64_t* offsets) {
+  __shared__ int64_t lds[LENGTHS_BLOCK / 64];
+  const int tid = threadIdx.x;
+  const int64_t first = (int64_t)blockIdx.x * run, end = first + run < n ? first + run : n;
+  int64_t sum = 0;
+  for (int64_t i0 = tid; i0 < first; i0 += 8 * LENGTHS_BLOCK) {
+    int v[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) v[u] = i0 + u * LENGTHS_BLOCK < first ? (int)lengths[i0 + u * LENGTHS_BLOCK] : 0;
+#pragma unroll
+    for (int u = 0; u < 8; ++u) sum += v[u];
   }
-  if (tid == 1023) offsets[n] = part[1023];
+  int64_t carry;
+  int64_t mine = first + tid < end ? (int64_t)(int)lengths[first + tid] : 0; // in flight beside the sums
+  lengths_block_scan(sum, lds, &carry);
+  for (int64_t i = first + tid; i - tid < end; i += LENGTHS_BLOCK) {
+    int64_t total;
+    const int64_t upto = lengths_block_scan(mine, lds, &total);
+    if (i < end) offsets[i] = carry + upto - mine;
+    carry += total;
+    mine = i + LENGTHS_BLOCK < end ? (int64_t)(int)lengths[i + LENGTHS_BLOCK] : 0;
+  }
+  if (end == n && tid == 0) offsets[n] = carry;
 }
 
 __global__ void status_clear_kernel(Status* st) {
@@ -195,12 +220,12 @@ hipError_t launch_lookup_burst_i64(const LookupArgs& a, dim3 grid, bool four_wav
 hipError_t launch_lookup_burst_i32(const LookupArgs& a, dim3 grid, bool four_waves, int lds_bytes, hipStream_t stream);
 
 // The burst kernel (lookup_burst.h): a workgroup per bag and window of 256 columns. max_D: the widest
-// table of the launch; waves: 1 or 4 per workgroup; lds_bytes: what a workgroup's staged rows may take.
+// table of the launch; waves: 1 or 4 per workgroup; lds_bytes: what a workgroup's
+// staged rows may take, at least 8 rows of the widest window.
 hipError_t launch_lookup_burst(const LookupArgs& a, bool idx64, int32_t max_D, int waves, int lds_bytes, hipStream_t stream) {
   if (a.B <= 0 || a.T <= 0) return hipSuccess;
   const int windows = (max_D + 255) / 256;
-  // 8 rows of the widest window (256 columns of fp32) have to fit
-  if (a.T > 65535 || windows > 65535 || lds_bytes < 8192 || (waves != 1 && waves != 4)) return hipErrorInvalidValue;
+  if (a.T > 65535 || windows > 65535 || lds_bytes < 1024 || (waves != 1 && waves != 4)) return hipErrorInvalidValue;
   const dim3 grid((unsigned)a.B, (unsigned)a.T, (unsigned)windows);
   return idx64 ? launch_lookup_burst_i64(a, grid, waves == 4, lds_bytes, stream) : launch_lookup_burst_i32(a, grid, waves == 4, lds_bytes, stream);
 }
@@ -218,8 +243,11 @@ hipError_t launch_bag_order(const void* offsets, bool off64, int32_t B, int32_t 
 }
 
 hipError_t launch_lengths_to_offsets(const void* lengths, bool is64, int64_t n, int64_t* offsets, hipStream_t stream) {
-  if (is64) hipLaunchKernelGGL(lengths_to_offsets_kernel<int64_t>, dim3(1), dim3(1024), 0, stream, (const int64_t*)lengths, n, offsets);
-  else hipLaunchKernelGGL(lengths_to_offsets_kernel<int32_t>, dim3(1), dim3(1024), 0, stream, (const int32_t*)lengths, n, offsets);
+  const int64_t tiles = n > 0 ? (n + LENGTHS_BLOCK - 1) / LENGTHS_BLOCK : 1;
+  const int64_t run = (tiles + LENGTHS_MAX_BLOCKS - 1) / LENGTHS_MAX_BLOCKS * LENGTHS_BLOCK;
+  const unsigned blocks = (unsigned)(n > 0 ? (n + run - 1) / run : 1);
+  if (is64) hipLaunchKernelGGL(lengths_to_offsets_kernel<int64_t>, dim3(blocks), dim3(LENGTHS_BLOCK), 0, stream, (const int64_t*)lengths, n, run, offsets);
+  else hipLaunchKernelGGL(lengths_to_offsets_kernel<int32_t>, dim3(blocks), dim3(LENGTHS_BLOCK), 0, stream, (const int32_t*)lengths, n, run, offsets);
   return hipGetLastError();
 }
 

@@ -167,7 +167,7 @@ hipError_t launch_lookup_lean(const LookupArgs& a, bool idx64, bool, bool wide4,
   return launch_lookup(a, idx64, s);
 }
 hipError_t launch_lookup_burst(const LookupArgs& a, bool idx64, int32_t, int, int lds_bytes, hipStream_t s) {
-  if (lds_bytes < 8192) return hipErrorInvalidValue; // eight rows of the widest window
+  if (lds_bytes < 4096) return hipErrorInvalidValue;
   return launch_lookup(a, idx64, s);
 }
 hipError_t launch_lengths_to_offsets(const void*, bool, int64_t n, int64_t* offsets, hipStream_t) {

@@ -109,13 +109,13 @@ def test_rejected_inputs(ops, oracle, burst, waves):
     assert bits(good, off, len(good) + 1)[0] == ops.ERR_LENGTH_MISMATCH
 
 
-@pytest.mark.parametrize("bags", [4095, 4096, 4097, 8192, 8193])
+@pytest.mark.parametrize("bags", [4095, 4097, 8192, 8193, 16384, 16385])
 def test_both_sides_of_the_line(ops, oracle, bags):
     """The rule's own choice just below, at and above the numbers of bags where it changes."""
     rng = np.random.default_rng(bags)
     D, rows = 20, 500
     table, _ = H.make_table(rng, INT4, rows, D, True)
-    lens = rng.integers(14, 21, size=bags)
+    lens = rng.integers(20, 33, size=bags)
     off = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
     idx = rng.integers(0, rows, size=int(off[-1])).astype(np.int32)
     S.check_case(ops, oracle, ty=INT4, D=D, table=table, idx=idx, off_or_len=off, w=None, normalize=False, out_ty=FP32,
