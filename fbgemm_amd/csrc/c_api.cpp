@@ -1394,9 +1394,7 @@ int tbe_forward_impl(
     // the lane shapes depend on B and (through the average bag length) on the number of indices:
     // remember the choice of the last forward with the same B and about the same indices
     const int64_t bucket = indices_numel >> 16;
-    if (burst.waves && !d_q8_out) {
-      variant = 3; // the burst kernel: no lane shapes, work lists or bag order
-    } else if (plan->shape_B == B && plan->shape_bucket == bucket && plan->shape_narrow == narrow_below_waves()) {
+    if (plan->shape_B == B && plan->shape_bucket == bucket && plan->shape_narrow == narrow_below_waves()) {
       variant = plan->shape_variant;
     } else {
       int64_t wide_waves = 0;
@@ -1424,7 +1422,7 @@ int tbe_forward_impl(
         return fail(FBGEMM_AMD_E_ARG, "the first forward of a plan with a new batch size allocates its work lists: "
                     "run it once outside the stream capture");
       std::vector<int> lean_members, general_members;
-      for (int t = 0; t < plan->T && variant != 3; ++t) (lean && lean_shape(tables[t]) ? lean_members : general_members).push_back(t);
+      for (int t = 0; t < plan->T; ++t) (lean && lean_shape(tables[t]) ? lean_members : general_members).push_back(t);
       fbgemm_amd_tbe_plan::Work nw;
       // what is allocated below goes back when a later step fails
       struct Undo {
@@ -1444,7 +1442,7 @@ int tbe_forward_impl(
         nw.n_general_tables = (int32_t)ids.size();
       }
       // the bag order: one buffer for this stream, one ahead for the next stream
-      for (int k = 0; k < 2 && variant != 3; ++k)
+      for (int k = 0; k < 2; ++k)
         if (int rc = make_order_slot(nw, k, plan->T, B)) return rc;
       nw.order_stream[0] = stream;
       nw.order_claimed[0] = true;
@@ -1473,7 +1471,7 @@ int tbe_forward_impl(
     // of this plan on the streams that share it must not overlap
     fbgemm_amd_tbe_plan::Work& W = it->second;
     constexpr int NS = fbgemm_amd_tbe_plan::ORDER_SLOTS;
-    order_slot = variant == 3 ? 0 : -1;
+    order_slot = -1;
     for (int k = 0; k < NS && order_slot < 0; ++k)
       if (W.order_claimed[k] && W.order_stream[k] == stream) order_slot = k;
     for (int k = 0; k < NS && order_slot < 0; ++k)
@@ -1484,7 +1482,7 @@ int tbe_forward_impl(
         order_slot = k;
       }
     if (order_slot < 0) order_slot = 0;
-    if (variant != 3 && !W.order_claimed[order_slot]) {
+    if (!W.order_claimed[order_slot]) {
       W.order_claimed[order_slot] = true;
       W.order_stream[order_slot] = stream;
       // keep one buffer ahead for the next stream, when that is possible now
@@ -1513,7 +1511,7 @@ int tbe_forward_impl(
       }
     }
     // the lean kernel of this forward, where there is a choice
-    if (W.lean_wide4 && !d_q8_out && W.d_redo[order_slot] && W.d_redo_count[order_slot] && sort_bags_default() &&
+    if (W.lean_wide4 && !d_q8_out && !burst.waves && W.d_redo[order_slot] && W.d_redo_count[order_slot] && sort_bags_default() &&
         indices_numel >= (int64_t)SORT_MIN_LOOKUPS) {
       const int mode = wide4_mode();
       if (mode == 2) {
@@ -1595,7 +1593,11 @@ int tbe_forward_impl(
   a.status = (Status*)d_status;
   a.fp8_shift = plan->fp8_shift;
   a.fp8_mult = plan->fp8_mult;
-  if (variant == 3) {
+  // The burst kernel needs none of the work set. The set is there all the same: whether a forward may
+  // be captured must depend on its batch size alone, and a later one of the same size may have shorter
+  // or longer bags, or the 8-bit output, and take the other kernels.
+  if (burst.waves && !d_q8_out) {
+    a.tables = plan->d_tables;
     HIP_TRY(launch_lookup_burst(a, index_bits == 64, plan->max_D, burst.waves, burst.lds_bytes, stream));
     return 0;
   }

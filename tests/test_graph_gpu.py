@@ -356,3 +356,39 @@ def test_mappings_changed_before_a_capture_are_refused(oracle):
     torch.cuda.synchronize()
     H.assert_same_bits(captured.cpu().view(torch.int16).numpy().view(np.uint16), expect(m2), "replay")
     assert st.read() == (0, -1)
+
+
+@pytest.mark.parametrize("seen,captured", [(25, 2), (2, 25)])
+def test_capture_with_other_bag_lengths_than_seen(oracle, seen, captured):
+    """Which kernel a forward takes depends on its bags' average length as well; whether it may be captured
+    depends on the batch size alone."""
+    assert torch.cuda.is_available()
+    from fbgemm_amd import ops
+    from test_tbe_gpu import build_weights
+    rng = np.random.default_rng(seen)
+    D, rows, B = 64, 500, 5000
+    weights, wo, _ = build_weights(rng, [(rows, D, INT4)], 16)
+    tys, D_offsets = np.array([INT4], np.uint8), np.array([0, D], np.int32)
+    meta = (cu(weights), torch.zeros(0, dtype=torch.uint8, device="cuda"), cu(np.zeros(1, np.int32)), cu(wo), cu(tys), cu(D_offsets))
+    st = ops.Status()
+    call = lambda i, o: ops.int_nbit_split_embedding_codegen_lookup_function(
+        *meta, D, 0, D, 0, 0, 0, i, o, 0, None, FP32, row_alignment=16, status=st)
+    draw = lambda L: (rng.integers(0, rows, size=B * L).astype(np.int32), (np.arange(B + 1) * L).astype(np.int32))
+    call(*map(cu, draw(seen)))
+    idx, off = draw(captured)
+    d_idx, d_off = cu(idx), cu(off)
+    torch.cuda.synchronize()
+    side = torch.cuda.Stream()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=side):
+        out = call(d_idx, d_off)
+    for replay in range(3):
+        idx, _ = draw(captured)
+        d_idx.copy_(cu(idx))
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        rc, want = oracle.tbe_forward(weights, wo, tys, D_offsets, D, idx, off, 0, None, FP32, 16)
+        assert rc == 0
+        H.assert_same_bits(out.cpu().numpy(), want, f"replay {replay}")
+    assert st.read() == (0, -1)
