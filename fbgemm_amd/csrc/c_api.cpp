@@ -316,6 +316,8 @@ struct DeviceScratch {
   int64_t* partial = nullptr; // bounds check: per-block maxima of the offset scan
   int64_t partial_cap = 0;
   unsigned long long* counter = nullptr; // zero between calls (check_remap_kernel)
+  bool counter_owned = false;            // ... of one stream: its calls follow one another
+  hipStream_t counter_stream = nullptr;
   int64_t* seg_offsets = nullptr; // split bags: where every segment starts
   int64_t seg_offsets_cap = 0;
   float* seg_partial = nullptr;   // split bags: the segments' fp32 sums
@@ -370,6 +372,7 @@ int get_scratch(DeviceScratch** out) {
     if (!idle.empty()) {
       HIP_TRY(hipDeviceSynchronize()); // what its last owner enqueued has finished
       s = idle.back();
+      s.counter_owned = false;
       idle.pop_back();
     } else {
       int32_t* flag = nullptr;
@@ -2056,7 +2059,18 @@ extern "C" int fbgemm_amd_check_remap_indices(
   a.remap = d_index_remappings;
   a.remap_offsets = d_index_remappings_offsets;
   a.warning = d_warning;
-  a.counter = s->counter;
+  // The counter outlives the call, so two calls at a time would leave it wrong for good: it serves the
+  // first stream this thread comes with, and no captured call (a graph may be replayed on any stream).
+  // The others take the form of two launches, which keeps nothing.
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  (void)hipStreamIsCapturing(stream, &cap);
+  if (cap == hipStreamCaptureStatusNone) {
+    if (!s->counter_owned) {
+      s->counter_owned = true;
+      s->counter_stream = stream;
+    }
+    if (s->counter_stream == stream) a.counter = s->counter;
+  }
   a.mode = bounds_check_mode;
   HIP_TRY(launch_check_remap(a, index_bits == 64, remap_bits == 64, s->partial, stream));
   return 0;

@@ -492,7 +492,7 @@ hipError_t launch_check_remap(CheckRemapArgs a, bool is64, bool remap64, int64_t
   if (a.total_B <= 0 || a.B <= 0 || blocks > 0x7fffffffLL) return hipErrorInvalidValue;
   a.partial = nullptr;
   a.prefix = 0;
-  if (blocks > CR_ONE_LAUNCH_BLOCKS) {
+  if (blocks > CR_ONE_LAUNCH_BLOCKS || (a.mode == 1 && !a.counter)) {
     a.partial = partial;
     hipLaunchKernelGGL(check_remap_partial_kernel, dim3((unsigned)blocks), dim3(CR_BAGS), 0, stream, a.offsets, is64 ? 1 : 0, a.total_B,
                        a.N, partial, a.warning, a.mode);

@@ -233,7 +233,7 @@ hipError_t launch_bounds_check(const int64_t*, int32_t, void*, void*, bool, int6
 int64_t check_remap_partials(int64_t total_B) { return total_B / 256 + 1; }
 hipError_t launch_check_remap(CheckRemapArgs a, bool, bool, int64_t* partial, hipStream_t) {
   (void)*(volatile const int64_t*)&partial[(a.total_B + 255) / 256 - 1];
-  (void)*(volatile const unsigned long long*)a.counter;
+  if (a.counter) (void)*(volatile const unsigned long long*)a.counter;
   return LAUNCHED();
 }
 int64_t bounds_check_partials(int64_t total_B) { return total_B / 1024 + 2; }

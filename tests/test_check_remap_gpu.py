@@ -79,3 +79,40 @@ def test_same_as_the_operators(ops, mode, mapped, dtype):
                 assert torch.equal(gi[start:], wi[start:]), tag
                 assert torch.equal(w0, w1), (tag, int(w0), int(w1))
                 assert all(torch.equal(a, b) for a, b in zip(before, args[1:3])), tag
+
+
+def test_streams_and_captured_calls(ops):
+    """Calls of one thread on several streams and from graphs that are replayed beside them leave the
+    right warning count, and nothing behind for a later call."""
+    rng = np.random.default_rng(8)
+    T, B, L = 8, 64, 30
+    rows = torch.full((T,), 100, dtype=torch.int64, device="cuda")
+    offsets = torch.arange(T * B + 1, device="cuda") * L
+    idx = rng.integers(0, 100, size=T * B * L)
+    where = rng.choice(len(idx), 37, replace=False)
+    idx[where] = 100
+    indices = torch.from_numpy(idx).cuda()
+    want = indices.clone()
+    want[torch.from_numpy(where).cuda()] = 0
+    streams = [torch.cuda.Stream() for _ in range(3)]
+    warnings = [torch.zeros(1, dtype=torch.int64, device="cuda") for _ in streams]
+    call = lambda k: ops.check_remap_indices(rows, indices, offsets, 1, warnings[k])
+    torch.cuda.synchronize()
+    call(0)  # scratch is made outside a capture
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=streams[2]):
+        captured = call(2)
+    for _ in range(20):
+        outs = []
+        for k, s in enumerate(streams[:2]):
+            with torch.cuda.stream(s):
+                outs.append(call(k))
+        graph.replay()
+        torch.cuda.synchronize()
+        for o in outs + [captured]:
+            assert torch.equal(o[0], want) and torch.equal(o[1], offsets)
+        assert [int(w) for w in warnings] == [37, 37, 37]
+        for w in warnings:
+            w.fill_(-1)
+        torch.cuda.synchronize()
