@@ -477,11 +477,16 @@ int fbgemm_amd_status_end(void* stream, int32_t* bits, int64_t* first_bad_pos) {
   HIP_TRY(hipStreamSynchronize((hipStream_t)stream));
   int32_t b = 0;
   int64_t pos = -1;
-  if (__atomic_load_n(s->flag, __ATOMIC_ACQUIRE)) { // the block stays dirty: the next call clears it
+  if (__atomic_load_n(s->flag, __ATOMIC_ACQUIRE)) {
+    // cleared here, on the call's own stream, which is quiet: clearing it at the next call would have to
+    // wait for the whole device, and may not while another thread captures
     if (int rc = fbgemm_amd_status_read(s->status, stream, &b, &pos)) return rc;
-  } else {
-    s->status_dirty = false;
+    const FlaggedStatus clear{Status{0, STATUS_FLAGGED, ~0ull}, s->flag};
+    HIP_TRY(hipMemcpyAsync(s->status, &clear, sizeof(clear), hipMemcpyHostToDevice, (hipStream_t)stream));
+    HIP_TRY(hipStreamSynchronize((hipStream_t)stream));
+    __atomic_store_n(s->flag, 0, __ATOMIC_RELEASE);
   }
+  s->status_dirty = false;
   if (bits) *bits = b;
   if (first_bad_pos) *first_bad_pos = pos;
   return 0;

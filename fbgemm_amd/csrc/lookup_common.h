@@ -34,7 +34,7 @@ struct Status {
   unsigned long long first_bad_pos;
 };
 
-// The block behind calls that wait for their result (StatusScope in c_api.cpp): `pad` of the block
+// The block behind calls that wait for their result (fbgemm_amd_status_begin): `pad` of the block
 // says that a pinned host word follows, which every report sets besides. The host then reads that
 // word after its wait, and neither clears the block before the call nor copies it back after it
 // unless something was reported: two operations on the stream less per call.
