@@ -604,10 +604,10 @@ def side_op(a):
         row_bytes = cols * 4 + cols // 2 + 4
         if a.op == "quantize":
             launch = lambda: ops.quantize_rowwise(x, 4, False, ops.QLAYOUT_TBE, out=q)
-            kernel, workload = "quantize_rowwise_kernel", f"fp32 [{rows}, {cols}] -> 4-bit rows, fp16 scale/bias first"
+            kernel, workload = "quantize_rows_kernel", f"fp32 [{rows}, {cols}] -> 4-bit rows, fp16 scale/bias first"
         else:
             launch = lambda: ops.dequantize_rowwise(q, cols, 4, False, ops.QLAYOUT_TBE, torch.float32)
-            kernel, workload = "dequantize_rowwise_kernel", f"4-bit rows, fp16 scale/bias first [{rows}, {cols}] -> fp32"
+            kernel, workload = "dequantize_rows_kernel", f"4-bit rows, fp16 scale/bias first [{rows}, {cols}] -> fp32"
         alg_bytes, units = rows * row_bytes, rows
 
         def cpu():  # the oracle's scalar restatement on a sample, one core
@@ -984,7 +984,7 @@ def main():
         ms_per_step = wall * 1e3 / a.steps
         forward_ms = ev0.elapsed_time(ev1) / a.steps
         kernel_ms = forward_ms
-        kernel_name = "lookup_kernel (+ bag_order_kernel), per " + ("graph replay" if a.graph else "forward")
+        kernel_name = "lookup_burst_kernel (lookup_kernel + bag_order_kernel for large launches), per " + ("graph replay" if a.graph else "forward")
     calibration_copy(a, torch)
 
     gbps = useful / (ms_per_step * 1e-3) / 1e9
