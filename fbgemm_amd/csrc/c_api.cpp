@@ -2038,7 +2038,6 @@ extern "C" int fbgemm_amd_check_remap_indices(
   std::lock_guard<std::mutex> lk(g_mu);
   DeviceScratch* s;
   if (int rc = get_scratch(&s)) return rc;
-  if (int rc = grow(&s->partial, &s->partial_cap, check_remap_partials(total_B), stream)) return rc;
   if (!s->counter) {
     unsigned long long* counter = nullptr;
     const unsigned long long zero = 0;
@@ -2066,7 +2065,7 @@ extern "C" int fbgemm_amd_check_remap_indices(
   a.warning = d_warning;
   // The counter outlives the call, so two calls at a time would leave it wrong for good: it serves the
   // first stream this thread comes with, and no captured call (a graph may be replayed on any stream).
-  // The others take the form of two launches, which keeps nothing.
+  // The others take the form of two launches, which uses no memory but the call's own outputs.
   hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
   (void)hipStreamIsCapturing(stream, &cap);
   if (cap == hipStreamCaptureStatusNone) {
@@ -2077,7 +2076,7 @@ extern "C" int fbgemm_amd_check_remap_indices(
     if (s->counter_stream == stream) a.counter = s->counter;
   }
   a.mode = bounds_check_mode;
-  HIP_TRY(launch_check_remap(a, index_bits == 64, remap_bits == 64, s->partial, stream));
+  HIP_TRY(launch_check_remap(a, index_bits == 64, remap_bits == 64, stream));
   return 0;
 }
 

@@ -230,9 +230,23 @@ __global__ __launch_bounds__(256) void bounds_check_bags_kernel(
 //   78 us: the random 4-byte reads of 256 MB of mappings, a line each, 6 TB/s of lines.
 // The warning counter is what the last of the separate checks leaves there: with a mapping the
 // second check's, which starts from zero and whose offsets are already in order.
+//
+// What a workgroup needs of the bags before its own is the maximum of their offsets. Up to 16
+// workgroups read those offsets themselves. With more, a kernel before this one leaves the maximum of
+// every 512 offsets in out_offsets, at the place of the last of them, and at every sixteenth such place
+// that of all 8192 up to there, so that the call needs no memory but its own outputs. A workgroup
+// combines the 8192s and the 512s before its own bags, a line each but few, with the rest of the
+// offsets. The workgroup that owns a place overwrites it with the running maximum up to there while
+// others may still read it, which comes to the same: a later workgroup's maximum is over everything
+// before its own bags whichever of the two values it finds. Unmapped checks of 32 x 4096, 64 x 8192,
+// 64 x 16384 and 128 x 16640 bags take 18.7, 28.1, 49.3 and 109 us (with every workgroup's maximum in
+// an array of the library's, which two calls at a time would share: 17.4, 26.5, 49.3 and 111).
 constexpr int CR_BAGS = 256; // bags of a workgroup, one per thread
 constexpr int CR_LOADS = 8;
 constexpr int CR_ONE_LAUNCH_BLOCKS = 16; // up to here every workgroup reads the offsets before its own itself
+constexpr int CR_GROUP = 2 * CR_BAGS;         // offsets to a maximum that the kernel before leaves
+constexpr int CR_SUPER = 16;                  // groups to a maximum of the second level
+constexpr int64_t CR_OWN_CARRY_SUPERS = 1024; // up to here every workgroup goes over those before its own itself
 
 __device__ __forceinline__ int64_t cr_block_max(int64_t v, int64_t* lds) {
   for (int m = 32; m > 0; m >>= 1) {
@@ -247,13 +261,55 @@ __device__ __forceinline__ int64_t cr_block_max(int64_t v, int64_t* lds) {
   return r;
 }
 
-__global__ __launch_bounds__(CR_BAGS) void check_remap_partial_kernel(const void* offsets, int is64, int64_t total_B, int64_t N,
-                                                                      int64_t* partial, int64_t* warning, int mode) {
+// where the maximum of the offsets of group g is left
+__device__ __forceinline__ int64_t cr_place(int64_t g) { return (g + 1) * CR_GROUP - 1; }
+
+template <typename index_t>
+__global__ __launch_bounds__(CR_BAGS) void check_remap_partial_kernel(const index_t* offsets, int64_t total_B, int64_t N, index_t* out_offsets,
+                                                                      int64_t* warning, int mode) {
+  constexpr int PER = CR_GROUP / CR_BAGS; // offsets per thread and group
   __shared__ int64_t lds[CR_BAGS / 64];
   if (mode == 1 && blockIdx.x == 0 && threadIdx.x == 0) warning[0] = 0;
-  const int64_t k = (int64_t)blockIdx.x * CR_BAGS + threadIdx.x;
-  const int64_t m = cr_block_max(k < total_B ? clamped_offset(offsets, is64, k, total_B, N) : 0, lds);
-  if (threadIdx.x == 0) partial[blockIdx.x] = m;
+  const int64_t place = cr_place(blockIdx.x);
+  if (place >= total_B) return; // nobody comes after it
+  int64_t m = 0;
+  auto take = [&](auto n) { // the last n offsets per thread up to the place, all in flight together
+    constexpr int COUNT = decltype(n)::value;
+    index_t v[COUNT];
+#pragma unroll
+    for (int u = 0; u < COUNT; ++u) v[u] = offsets[place + 1 - (u + 1) * CR_BAGS + threadIdx.x];
+#pragma unroll
+    for (int u = 0; u < COUNT; ++u) m = m > (int64_t)v[u] ? m : (int64_t)v[u];
+  };
+  if ((blockIdx.x + 1) % CR_SUPER == 0) take(std::integral_constant<int, PER * CR_SUPER>{});
+  else take(std::integral_constant<int, PER>{});
+  m = cr_block_max(m < N ? m : N, lds); // of offsets clamped to 0 .. N
+  if (threadIdx.x == 0) out_offsets[place] = (index_t)m;
+}
+
+// One workgroup: the first `n` maxima of the second level become running maxima.
+__global__ __launch_bounds__(SCAN_THREADS) void check_remap_carry_kernel(void* out_offsets, int is64, int64_t n) {
+  __shared__ int64_t lds[SCAN_THREADS / 64];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  int64_t carry = 0;
+  for (int64_t b0 = 0; b0 < n; b0 += SCAN_THREADS) {
+    const int64_t b = b0 + threadIdx.x;
+    int64_t run = b < n ? read_index(out_offsets, is64, cr_place(b * CR_SUPER + CR_SUPER - 1)) : 0;
+    for (int step = 1; step < 64; step <<= 1) {
+      const int64_t o = __shfl_up(run, step, 64);
+      if (lane >= step) run = run > o ? run : o;
+    }
+    if (lane == 63) lds[wave] = run;
+    __syncthreads();
+    int64_t before = carry;
+    for (int w = 0; w < SCAN_THREADS / 64; ++w) {
+      if (w < wave) before = before > lds[w] ? before : lds[w];
+      carry = carry > lds[w] ? carry : lds[w];
+    }
+    run = run > before ? run : before;
+    if (b < n) write_index(out_offsets, is64, cr_place(b * CR_SUPER + CR_SUPER - 1), run);
+    __syncthreads(); // lds is free again
+  }
 }
 
 template <typename index_t, typename remap_t>
@@ -271,10 +327,17 @@ __global__ __launch_bounds__(CR_BAGS) void check_remap_kernel(CheckRemapArgs a) 
   const int64_t mine = tid < nb ? clamped_offset(a.offsets, IS64, k0 + tid, a.total_B, a.N) : 0;
   const int64_t behind = clamped_offset(a.offsets, IS64, k0 + nb, a.total_B, a.N);
   int64_t carry = 0;
-  if (a.prefix) {
-    carry = a.partial[blockIdx.x];
-  } else if (a.partial) {
-    for (int64_t b = tid; b < (int64_t)blockIdx.x; b += CR_BAGS) carry = carry > a.partial[b] ? carry : a.partial[b];
+  if (a.carry) {
+    const index_t* place = reinterpret_cast<const index_t*>(a.out_offsets);
+    const int64_t groups = k0 / CR_GROUP, supers = groups / CR_SUPER;
+    const int64_t rest = groups * CR_GROUP + tid;
+    if (rest < k0) carry = clamped_offset(a.offsets, IS64, rest, a.total_B, a.N);
+    const int64_t first = a.carry == 2 && supers > 0 ? supers - 1 : 0; // running maxima: the last says it all
+    for (int64_t j = first + tid; j < supers + groups % CR_SUPER; j += CR_BAGS) {
+      const int64_t g = j < supers ? j * CR_SUPER + CR_SUPER - 1 : supers * CR_SUPER + (j - supers);
+      const int64_t v = (int64_t)__hip_atomic_load(place + cr_place(g), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
+      carry = carry > v ? carry : v;
+    }
   } else {
 #pragma unroll
     for (int u = 0; u < CR_ONE_LAUNCH_BLOCKS - 1; ++u) {
@@ -298,6 +361,7 @@ __global__ __launch_bounds__(CR_BAGS) void check_remap_kernel(CheckRemapArgs a) 
     }
   }
   carry = cr_block_max(carry, lds);
+  carry = carry < a.N ? carry : a.N; // it is; whatever else may have been there leads to no index that is not
   // running maximum: the repaired offsets
   int64_t run = mine;
   for (int step = 1; step < 64; step <<= 1) {
@@ -390,7 +454,7 @@ __global__ __launch_bounds__(CR_BAGS) void check_remap_kernel(CheckRemapArgs a) 
   __syncthreads();
   if (tid != 0) return;
   unsigned long long* warning = reinterpret_cast<unsigned long long*>(a.warning);
-  if (a.partial) { // the kernel before this one has set the counter to zero
+  if (a.carry) { // the kernel before this one has set the counter to zero
     if (bad_count) atomicAdd(warning, (unsigned long long)bad_count);
     return;
   }
@@ -485,20 +549,22 @@ hipError_t launch_bounds_check(const int64_t* rows_per_table, int32_t T, void* i
 
 int64_t bounds_check_partials(int64_t total_B) { return (total_B + 1 + SCAN_BLOCK - 1) / SCAN_BLOCK; }
 
-int64_t check_remap_partials(int64_t total_B) { return (total_B + CR_BAGS - 1) / CR_BAGS; }
-
-hipError_t launch_check_remap(CheckRemapArgs a, bool is64, bool remap64, int64_t* partial, hipStream_t stream) {
-  const int64_t blocks = check_remap_partials(a.total_B);
+hipError_t launch_check_remap(CheckRemapArgs a, bool is64, bool remap64, hipStream_t stream) {
+  const int64_t blocks = (a.total_B + CR_BAGS - 1) / CR_BAGS;
   if (a.total_B <= 0 || a.B <= 0 || blocks > 0x7fffffffLL) return hipErrorInvalidValue;
-  a.partial = nullptr;
-  a.prefix = 0;
+  a.carry = 0;
   if (blocks > CR_ONE_LAUNCH_BLOCKS || (a.mode == 1 && !a.counter)) {
-    a.partial = partial;
-    hipLaunchKernelGGL(check_remap_partial_kernel, dim3((unsigned)blocks), dim3(CR_BAGS), 0, stream, a.offsets, is64 ? 1 : 0, a.total_B,
-                       a.N, partial, a.warning, a.mode);
-    if (blocks > 4096) { // more maxima than a workgroup should read for itself
-      a.prefix = 1;
-      hipLaunchKernelGGL(bounds_carry_kernel, dim3(1), dim3(SCAN_THREADS), 0, stream, partial, blocks);
+    a.carry = 1;
+    const int64_t groups = (a.total_B + CR_GROUP - 1) / CR_GROUP, supers = a.total_B / (CR_GROUP * CR_SUPER);
+    if (is64)
+      hipLaunchKernelGGL(check_remap_partial_kernel<int64_t>, dim3((unsigned)groups), dim3(CR_BAGS), 0, stream, (const int64_t*)a.offsets,
+                         a.total_B, a.N, (int64_t*)a.out_offsets, a.warning, a.mode);
+    else
+      hipLaunchKernelGGL(check_remap_partial_kernel<int32_t>, dim3((unsigned)groups), dim3(CR_BAGS), 0, stream, (const int32_t*)a.offsets,
+                         a.total_B, a.N, (int32_t*)a.out_offsets, a.warning, a.mode);
+    if (supers > CR_OWN_CARRY_SUPERS) {
+      a.carry = 2;
+      hipLaunchKernelGGL(check_remap_carry_kernel, dim3(1), dim3(SCAN_THREADS), 0, stream, a.out_offsets, is64 ? 1 : 0, supers);
     }
   }
   // a workgroup per 2048 indices (one turn of 8 loads per thread), per 512 where that leaves the device half empty

@@ -406,7 +406,9 @@ int fbgemm_amd_bounds_check_indices(
  * d_rows_per_table, each index read and written once. d_index_remappings_offsets
  * (T + 1 entries) may be NULL: then only the check. d_out_indices and d_out_offsets
  * have the inputs' sizes and must not overlap them; d_warning ends as the last check
- * of the separate calls would leave it. B must not be zero. */
+ * of the separate calls would leave it. B must not be zero. Calls on several streams
+ * may overlap, and captured calls be replayed beside them, as long as their outputs
+ * and warning counters are their own. */
 int fbgemm_amd_check_remap_indices(
     const int64_t* d_rows_per_table, int32_t T, const void* d_indices, const void* d_offsets, int32_t index_bits,
     int64_t indices_numel, int64_t offsets_numel, int32_t bounds_check_mode, int64_t* d_warning,

@@ -256,6 +256,42 @@ void entry_point_that_allocates_nothing() {
   hipFree(status);
 }
 
+// Checks of any size, on several streams, eager and captured, keep nothing of one call that another
+// could write: a thread's calls take no device memory from the library but what the first makes.
+void checks_share_no_scratch() {
+  const int32_t T = 8;
+  const int64_t most = 1 << 20;
+  int64_t* rows;
+  void *idx, *off, *out_idx, *out_off;
+  int64_t* warning;
+  CHECK(hipMalloc((void**)&rows, 8 * T) == hipSuccess);
+  CHECK(hipMalloc(&idx, 8 * 100) == hipSuccess);
+  CHECK(hipMalloc(&off, 8 * (most + 1)) == hipSuccess);
+  CHECK(hipMalloc(&out_idx, 8 * 100) == hipSuccess);
+  CHECK(hipMalloc(&out_off, 8 * (most + 1)) == hipSuccess);
+  CHECK(hipMalloc((void**)&warning, 8) == hipSuccess);
+  auto call = [&](int64_t bags, int mode, hipStream_t s) {
+    return fbgemm_amd_check_remap_indices(rows, T, idx, off, 64, 100, bags + 1, mode, warning, nullptr, nullptr, 32, nullptr, out_idx, out_off, s);
+  };
+  CHECK(call(64, 1, hip_stub_stream(0)) == 0);
+  const long before = hip_stub_total_allocations();
+  for (int64_t bags : {int64_t(64), int64_t(8192), most})
+    for (int mode : {1, 2})
+      for (int s = 0; s < 3; ++s) {
+        CHECK(call(bags, mode, hip_stub_stream(s)) == 0);
+        hip_stub_set_capturing(hip_stub_stream(s), true);
+        CHECK(call(bags, mode, hip_stub_stream(s)) == 0);
+        hip_stub_set_capturing(hip_stub_stream(s), false);
+      }
+  CHECK(hip_stub_total_allocations() == before);
+  hipFree(rows);
+  hipFree(idx);
+  hipFree(off);
+  hipFree(out_idx);
+  hipFree(out_off);
+  hipFree(warning);
+}
+
 void allocation_failures_in_a_first_forward() {
   const Problem p = make_problem(5);
   Buffers b(p, 16, 1 << 21);
@@ -340,6 +376,7 @@ int main() {
   remappings_twice_and_split_bags();
   thread_scratch_hand_over();
   entry_point_that_allocates_nothing();
+  checks_share_no_scratch();
   allocation_failures_in_a_first_forward();
   printf("launches %ld, device allocations %ld\n", hip_stub_launches(), hip_stub_total_allocations());
   printf("PASSED\n");
