@@ -315,9 +315,11 @@ struct DeviceScratch {
   int64_t fixed_cap = 0;
   int64_t* partial = nullptr; // bounds check: per-block maxima of the offset scan
   int64_t partial_cap = 0;
-  unsigned long long* counter = nullptr; // zero between calls (check_remap_kernel)
-  bool counter_owned = false;            // ... of one stream: its calls follow one another
-  hipStream_t counter_stream = nullptr;
+  // check_remap_kernel's counters, zero while no call has them, and the pinned words that say so. A
+  // call has a counter from its launch until its kernel clears the word, whatever its stream.
+  unsigned long long* counters = nullptr;
+  int32_t* counter_taken = nullptr;
+  int next_counter = 0;
   int64_t* seg_offsets = nullptr; // split bags: where every segment starts
   int64_t seg_offsets_cap = 0;
   float* seg_partial = nullptr;   // split bags: the segments' fp32 sums
@@ -334,6 +336,8 @@ int split_factor(int64_t waves, int64_t avg_len) {
   while (K < 32 && K * 2 * 8 <= avg_len && waves * K < 1024) K *= 2; // segments of 8 rows at least
   return K;
 }
+
+constexpr int CHECK_COUNTERS = 8; // calls in flight that take one launch; the others take two
 
 // Grow-only device buffer; the old one may still be read by an enqueued kernel.
 template <typename T>
@@ -372,7 +376,6 @@ int get_scratch(DeviceScratch** out) {
     if (!idle.empty()) {
       HIP_TRY(hipDeviceSynchronize()); // what its last owner enqueued has finished
       s = idle.back();
-      s.counter_owned = false;
       idle.pop_back();
     } else {
       int32_t* flag = nullptr;
@@ -2016,6 +2019,26 @@ int fbgemm_amd_bounds_check_indices(
   return 0;
 }
 
+namespace {
+int make_check_counters(DeviceScratch* s, hipStream_t stream) {
+  static const unsigned long long zeros[CHECK_COUNTERS] = {};
+  unsigned long long* counters = nullptr;
+  int32_t* taken = nullptr;
+  HIP_TRY(hipMalloc((void**)&counters, sizeof(zeros)));
+  hipError_t e = hipMemcpyAsync(counters, zeros, sizeof(zeros), hipMemcpyHostToDevice, stream);
+  if (e == hipSuccess) e = hipStreamSynchronize(stream);
+  if (e == hipSuccess) e = hipHostMalloc((void**)&taken, sizeof(int32_t) * CHECK_COUNTERS, hipHostMallocCoherent);
+  if (e != hipSuccess) {
+    (void)hipFree(counters);
+    return fail(FBGEMM_AMD_E_HIP, "the counters of the bounds check: %s", hipGetErrorString(e));
+  }
+  memset(taken, 0, sizeof(int32_t) * CHECK_COUNTERS);
+  s->counters = counters;
+  s->counter_taken = taken;
+  return 0;
+}
+} // namespace
+
 extern "C" int fbgemm_amd_check_remap_indices(
     const int64_t* d_rows_per_table, int32_t T, const void* d_indices, const void* d_offsets, int32_t index_bits,
     int64_t indices_numel, int64_t offsets_numel, int32_t bounds_check_mode, int64_t* d_warning,
@@ -2035,20 +2058,6 @@ extern "C" int fbgemm_amd_check_remap_indices(
   if (d_index_remappings_offsets && (!d_index_remappings || !d_logical_rows_per_table || (remap_bits != 32 && remap_bits != 64)))
     return fail(FBGEMM_AMD_E_ARG, "a mapping needs its 32- or 64-bit entries and the rows before pruning");
   hipStream_t stream = (hipStream_t)stream_;
-  std::lock_guard<std::mutex> lk(g_mu);
-  DeviceScratch* s;
-  if (int rc = get_scratch(&s)) return rc;
-  if (!s->counter) {
-    unsigned long long* counter = nullptr;
-    const unsigned long long zero = 0;
-    HIP_TRY(hipMalloc((void**)&counter, sizeof(zero)));
-    const hipError_t e = hipMemcpy(counter, &zero, sizeof(zero), hipMemcpyHostToDevice);
-    if (e != hipSuccess) {
-      (void)hipFree(counter);
-      return fail(FBGEMM_AMD_E_HIP, "hipMemcpy of a counter: %s", hipGetErrorString(e));
-    }
-    s->counter = counter;
-  }
   CheckRemapArgs a;
   memset(&a, 0, sizeof(a));
   a.rows = d_rows_per_table;
@@ -2063,19 +2072,28 @@ extern "C" int fbgemm_amd_check_remap_indices(
   a.remap = d_index_remappings;
   a.remap_offsets = d_index_remappings_offsets;
   a.warning = d_warning;
-  // The counter outlives the call, so two calls at a time would leave it wrong for good: it serves the
-  // first stream this thread comes with, and no captured call (a graph may be replayed on any stream).
-  // The others take the form of two launches, which uses no memory but the call's own outputs.
-  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-  (void)hipStreamIsCapturing(stream, &cap);
-  if (cap == hipStreamCaptureStatusNone) {
-    if (!s->counter_owned) {
-      s->counter_owned = true;
-      s->counter_stream = stream;
-    }
-    if (s->counter_stream == stream) a.counter = s->counter;
-  }
   a.mode = bounds_check_mode;
+  // A small call that counts does so in one launch with a counter of the library's, which is its alone
+  // until its kernel has left it zero. A captured call may be replayed at any time and so can have
+  // none; it takes the form of two launches, which uses no memory but the call's own outputs.
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  if (check_remap_counts(total_B, bounds_check_mode)) (void)hipStreamIsCapturing(stream, &cap);
+  if (check_remap_counts(total_B, bounds_check_mode) && cap == hipStreamCaptureStatusNone) {
+    std::lock_guard<std::mutex> lk(g_mu);
+    DeviceScratch* s;
+    if (int rc = get_scratch(&s)) return rc;
+    if (!s->counters)
+      if (int rc = make_check_counters(s, stream)) return rc;
+    for (int k = 0; k < CHECK_COUNTERS && !a.counter; ++k) {
+      const int slot = (s->next_counter + k) % CHECK_COUNTERS;
+      if (__atomic_load_n(&s->counter_taken[slot], __ATOMIC_ACQUIRE)) continue;
+      a.counter = s->counters + slot;
+      a.counter_taken = s->counter_taken + slot;
+      s->next_counter = (slot + 1) % CHECK_COUNTERS;
+      __atomic_store_n(a.counter_taken, 1, __ATOMIC_RELEASE);
+    }
+  }
+  // (an error need not mean that nothing runs: the counter stays taken until a kernel gives it back)
   HIP_TRY(launch_check_remap(a, index_bits == 64, remap_bits == 64, stream));
   return 0;
 }

@@ -56,6 +56,7 @@ hipError_t launch_bounds_check(const int64_t* rows_per_table, int32_t T, void* i
                                int64_t num_indices, int64_t total_B, int64_t B, const int32_t* B_offsets, int mode,
                                int64_t* warning, int64_t* fixed, int64_t* partial, Status* status, hipStream_t stream);
 int64_t bounds_check_partials(int64_t total_B);
+bool check_remap_counts(int64_t total_B, int mode); // whether a call can use a counter
 hipError_t launch_check_remap(CheckRemapArgs a, bool is64, bool remap64, hipStream_t stream);
 hipError_t launch_quantize_rowwise(const void* input, bool half_in, int64_t rows, int32_t cols, int32_t bits,
                                    int32_t sb_float, int32_t layout, int64_t out_stride, void* output,

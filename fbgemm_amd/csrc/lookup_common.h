@@ -201,7 +201,8 @@ struct CheckRemapArgs {
   const void* remap;
   const int64_t* remap_offsets; // T + 1, or nullptr: no mapping
   int64_t* warning;
-  unsigned long long* counter;  // zero between calls
+  unsigned long long* counter;  // zero, and this call's alone; or nullptr: a launch more
+  int32_t* counter_taken;       // pinned host word: the kernel clears it when it has left the counter zero
   int32_t carry;                // set by the launcher: what out_offsets holds of the bags before a workgroup's own
                                 // (0 nothing, 1 maxima on two levels, 2 with the second level's as running maxima)
   int32_t mode;                 // 1 WARNING, 2 IGNORE

@@ -8,6 +8,7 @@
 #include <cstring>
 #include <mutex>
 #include <set>
+#include <vector>
 
 #include "../../../fbgemm_amd/csrc/launchers.h"
 
@@ -16,6 +17,7 @@ std::mutex g_mu;
 std::set<void*> g_live;
 std::set<hipStream_t> g_capturing;
 std::atomic<long> g_total{0}, g_launches{0}, g_fail_after{-1}, g_wide4{0};
+std::vector<fbgemm_amd::CheckRemapArgs> g_checks; // those with a counter that have not finished
 std::atomic<int> g_last_lean_wide4{0};
 std::atomic<float> g_elapsed_general{1.0f}, g_elapsed_wide4{1.0f};
 struct Obj { int kind; };
@@ -138,6 +140,18 @@ void hip_stub_set_elapsed_ms(float general_ms, float wide4_ms) {
   g_elapsed_general = general_ms;
   g_elapsed_wide4 = wide4_ms;
 }
+long hip_stub_checks_in_flight(void) {
+  std::lock_guard<std::mutex> lk(g_mu);
+  return (long)g_checks.size();
+}
+void hip_stub_finish_checks(void) {
+  std::lock_guard<std::mutex> lk(g_mu);
+  for (const fbgemm_amd::CheckRemapArgs& a : g_checks) {
+    *a.counter = 0;
+    __atomic_store_n(a.counter_taken, 0, __ATOMIC_RELEASE);
+  }
+  g_checks.clear();
+}
 hipStream_t hip_stub_stream(int id) {
   static hipStubStream streams[16];
   return &streams[id & 15];
@@ -230,8 +244,16 @@ hipError_t launch_quantize_segments(const float* input, int64_t lines, int32_t, 
 }
 hipError_t launch_bounds_check(const int64_t*, int32_t, void*, void*, bool, int64_t, int64_t, int64_t, const int32_t*, int, int64_t*,
                                int64_t*, int64_t*, Status*, hipStream_t) { return LAUNCHED(); }
+bool check_remap_counts(int64_t total_B, int mode) { return mode == 1 && total_B <= 4096; }
 hipError_t launch_check_remap(CheckRemapArgs a, bool, bool, hipStream_t) {
-  if (a.counter) (void)*(volatile const unsigned long long*)a.counter;
+  std::lock_guard<std::mutex> lk(g_mu);
+  if (a.counter) { // in flight until hip_stub_finish_checks
+    for (const CheckRemapArgs& other : g_checks)
+      if (other.counter == a.counter) return hipErrorInvalidValue;
+    if (*a.counter != 0 || *a.counter_taken != 1) return hipErrorInvalidValue;
+    *a.counter = 1;
+    g_checks.push_back(a);
+  }
   return LAUNCHED();
 }
 int64_t bounds_check_partials(int64_t total_B) { return total_B / 1024 + 2; }

@@ -256,40 +256,67 @@ void entry_point_that_allocates_nothing() {
   hipFree(status);
 }
 
+struct Check {
+  const int32_t T = 8;
+  const int64_t most = 1 << 20;
+  int64_t *rows, *warning;
+  void *idx, *off, *out_idx, *out_off;
+  Check() {
+    CHECK(hipMalloc((void**)&rows, 8 * T) == hipSuccess);
+    CHECK(hipMalloc(&idx, 8 * 100) == hipSuccess);
+    CHECK(hipMalloc(&off, 8 * (most + 1)) == hipSuccess);
+    CHECK(hipMalloc(&out_idx, 8 * 100) == hipSuccess);
+    CHECK(hipMalloc(&out_off, 8 * (most + 1)) == hipSuccess);
+    CHECK(hipMalloc((void**)&warning, 8) == hipSuccess);
+  }
+  ~Check() {
+    for (void* p : {(void*)rows, idx, off, out_idx, out_off, (void*)warning}) hipFree(p);
+  }
+  int operator()(int64_t bags, int mode, hipStream_t s) {
+    return fbgemm_amd_check_remap_indices(rows, T, idx, off, 64, 100, bags + 1, mode, warning, nullptr, nullptr, 32, nullptr, out_idx, out_off, s);
+  }
+};
+
 // Checks of any size, on several streams, eager and captured, keep nothing of one call that another
 // could write: a thread's calls take no device memory from the library but what the first makes.
 void checks_share_no_scratch() {
-  const int32_t T = 8;
-  const int64_t most = 1 << 20;
-  int64_t* rows;
-  void *idx, *off, *out_idx, *out_off;
-  int64_t* warning;
-  CHECK(hipMalloc((void**)&rows, 8 * T) == hipSuccess);
-  CHECK(hipMalloc(&idx, 8 * 100) == hipSuccess);
-  CHECK(hipMalloc(&off, 8 * (most + 1)) == hipSuccess);
-  CHECK(hipMalloc(&out_idx, 8 * 100) == hipSuccess);
-  CHECK(hipMalloc(&out_off, 8 * (most + 1)) == hipSuccess);
-  CHECK(hipMalloc((void**)&warning, 8) == hipSuccess);
-  auto call = [&](int64_t bags, int mode, hipStream_t s) {
-    return fbgemm_amd_check_remap_indices(rows, T, idx, off, 64, 100, bags + 1, mode, warning, nullptr, nullptr, 32, nullptr, out_idx, out_off, s);
-  };
+  Check call;
   CHECK(call(64, 1, hip_stub_stream(0)) == 0);
+  hip_stub_finish_checks();
   const long before = hip_stub_total_allocations();
-  for (int64_t bags : {int64_t(64), int64_t(8192), most})
+  for (int64_t bags : {int64_t(64), int64_t(8192), call.most})
     for (int mode : {1, 2})
       for (int s = 0; s < 3; ++s) {
         CHECK(call(bags, mode, hip_stub_stream(s)) == 0);
+        hip_stub_finish_checks();
         hip_stub_set_capturing(hip_stub_stream(s), true);
         CHECK(call(bags, mode, hip_stub_stream(s)) == 0);
         hip_stub_set_capturing(hip_stub_stream(s), false);
       }
   CHECK(hip_stub_total_allocations() == before);
-  hipFree(rows);
-  hipFree(idx);
-  hipFree(off);
-  hipFree(out_idx);
-  hipFree(out_off);
-  hipFree(warning);
+}
+
+// The counter of a small check is its alone while it is in flight, on whatever stream (a new stream
+// may have the handle of a destroyed one whose work is still running); there are only so many, and a
+// finished check's is free again. Captured checks and those that do not count have none, and make none.
+void checks_in_flight_have_a_counter_each() {
+  Check call;
+  std::thread([&] {
+    const long before = hip_stub_total_allocations();
+    hip_stub_set_capturing(hip_stub_stream(0), true);
+    CHECK(call(64, 1, hip_stub_stream(0)) == 0);
+    hip_stub_set_capturing(hip_stub_stream(0), false);
+    CHECK(call(64, 2, hip_stub_stream(0)) == 0);
+    CHECK(call(8192, 1, hip_stub_stream(0)) == 0);
+    CHECK(hip_stub_total_allocations() == before && hip_stub_checks_in_flight() == 0);
+    for (int round = 0; round < 3; ++round) {
+      for (int n = 1; n <= 20; ++n) {
+        CHECK(call(64, 1, hip_stub_stream(n % 2)) == 0);
+        CHECK(hip_stub_checks_in_flight() == (n < 8 ? n : 8));
+      }
+      hip_stub_finish_checks();
+    }
+  }).join();
 }
 
 void allocation_failures_in_a_first_forward() {
@@ -376,6 +403,7 @@ int main() {
   remappings_twice_and_split_bags();
   thread_scratch_hand_over();
   entry_point_that_allocates_nothing();
+  checks_in_flight_have_a_counter_each();
   checks_share_no_scratch();
   allocation_failures_in_a_first_forward();
   printf("launches %ld, device allocations %ld\n", hip_stub_launches(), hip_stub_total_allocations());
