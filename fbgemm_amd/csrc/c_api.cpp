@@ -306,7 +306,7 @@ constexpr int64_t SPLIT_MIN_LEN_OVER_BURST = 256;
 struct DeviceScratch {
   FlaggedStatus* status = nullptr; // clear between the calls that use it
   int32_t* flag = nullptr;         // pinned: what a report sets besides the block
-  bool status_dirty = true;        // a call is using the block, or ended without reading it
+  bool status_dirty = true;        // something that may write the block was enqueued since it was last read
   int64_t* offsets = nullptr; // lengths -> offsets
   int64_t offsets_cap = 0;
   BagEntry* order = nullptr;  // bag order of single-table calls
@@ -365,6 +365,14 @@ struct ThreadScratch {
   }
 };
 thread_local ThreadScratch t_scratch;
+thread_local DeviceScratch* t_begun = nullptr; // whose block fbgemm_amd_status_begin handed out last
+
+// Where a call is about to enqueue something that may write `d_status`: only from here on does the
+// thread's own block have to be read before it is handed out again. A call refused before this point
+// leaves it as it was.
+void status_in_use(const void* d_status) {
+  if (t_begun && d_status == (const void*)t_begun->status) t_begun->status_dirty = true;
+}
 
 // call with g_mu held
 int get_scratch(DeviceScratch** out) {
@@ -460,13 +468,14 @@ int fbgemm_amd_status_begin(void** d_status) {
   std::lock_guard<std::mutex> lk(g_mu);
   DeviceScratch* s;
   if (int rc = get_scratch(&s)) return rc;
-  if (s->status_dirty) { // new, or left behind by a call that failed on its way: nothing may write it any more
+  if (s->status_dirty) { // new, or left behind by a call that failed after it had enqueued something
     HIP_TRY(hipDeviceSynchronize());
     const FlaggedStatus clear{Status{0, STATUS_FLAGGED, ~0ull}, s->flag};
     HIP_TRY(hipMemcpy(s->status, &clear, sizeof(clear), hipMemcpyHostToDevice));
     *s->flag = 0;
+    s->status_dirty = false;
   }
-  s->status_dirty = true; // until fbgemm_amd_status_end has looked
+  t_begun = s;
   *d_status = s->status;
   return 0;
 }
@@ -571,6 +580,7 @@ int spmdm_launch_impl(
     // the reference returns (0 == index_size) without touching anything
     if (index_size != 0 && !cfg->no_bag) {
       Status h{ERR_LENGTH_MISMATCH, 0, ~0ull};
+      status_in_use(d_status);
       HIP_TRY(hipMemcpyAsync(d_status, &h, sizeof(h), hipMemcpyHostToDevice, stream));
       HIP_TRY(hipStreamSynchronize(stream));
     }
@@ -643,11 +653,13 @@ int spmdm_launch_impl(
     if (ty == ST_FP16 || ty == ST_BF16 || ty == ST_FP32) {
       if (d.row_stride % (bits / 8)) return fail(FBGEMM_AMD_E_ARG, "rows are not aligned to their elements");
     }
+    status_in_use(d_status);
     HIP_TRY(launch_row_lookup(d, (const uint8_t*)d_input, d_indices, cfg->index_bits == 64, d_weights, output_size,
                               cfg->output_ty, d_out, out_stride_bytes, copy_bytes, a.fp8_shift, a.fp8_mult,
                               (Status*)d_status, stream));
     return 0;
   }
+  status_in_use(d_status);
   // bytes of a row that are known to be there (the last row may end with them), from data_off on
   const int64_t packed_bytes = (D * bits + 7) / 8;
   const int64_t room = has_sb && cfg->scale_bias_last ? packed_bytes + (d.sb_fp32 ? 8 : 4) : packed_bytes;
@@ -1364,6 +1376,7 @@ int tbe_forward_impl(
         voff = plan->seg_offsets;
         partial = plan->seg_partial;
       }
+      status_in_use(d_status);
       HIP_TRY(launch_split_offsets(d_offsets, offset_bits == 64, (int64_t)plan->T * B, K, false, indices_numel, voff, (Status*)d_status, stream));
       if (int rc = tbe_forward_impl(plan, d_dev_weights, d_uvm_weights, d_indices, voff, index_bits, 64, indices_numel, vbags + 1,
                                     FBGEMM_AMD_POOL_SUM, d_indice_weights, ST_FP32, partial, d_index_remappings, remap_bits,
@@ -1578,6 +1591,7 @@ int tbe_forward_impl(
     if (int rc = pooled_scratch(&tmp)) return rc;
     d_output = tmp;
   }
+  status_in_use(d_status);
   LookupArgs a;
   memset(&a, 0, sizeof(a));
   a.tables = variant == 2 ? plan->d_tables_narrow : (variant == 1 ? plan->d_tables_packed : plan->d_tables);
@@ -1837,6 +1851,7 @@ int fbgemm_amd_tbe_forward_nobag(
     if (eb > 1 && (d.weights_offset % eb || d.row_stride % eb))
       return fail(FBGEMM_AMD_E_ARG, "table %d: rows are not aligned to their elements", t);
   }
+  status_in_use(d_status);
   HIP_TRY(launch_sequence_lookup(plan->d_tables, (const uint8_t*)d_dev_weights, (const uint8_t*)d_uvm_weights, d_indices,
                                  index_bits == 64, d_offsets, (int32_t)B64, plan->T, indices_numel, D, output_ty,
                                  d_output, plan->fp8_shift, plan->fp8_mult, (Status*)d_status, (hipStream_t)stream));
@@ -1984,6 +1999,7 @@ int fbgemm_amd_compressed_indices_remap(
   // one scratch buffer: n + 1 running counts (int64), then the n mapped rows (int32)
   if (int rc = grow(&s->fixed, &s->fixed_cap, (n + 1) + (n + 1) / 2 + 1, stream)) return rc;
   if (int rc = grow(&s->partial, &s->partial_cap, prune_partials(n + 1), stream)) return rc;
+  status_in_use(d_status);
   HIP_TRY(launch_compressed_indices_remap(d_indices, index_bits == 64, d_mapping, mapping_numel, d_offsets, offsets_numel,
                                           d_weights, first, n, d_out_indices, d_out_offsets, d_out_weights, s->fixed,
                                           s->partial, reinterpret_cast<int32_t*>(s->fixed + n + 1),
@@ -2013,6 +2029,7 @@ int fbgemm_amd_bounds_check_indices(
   if (int rc = get_scratch(&s)) return rc;
   if (int rc = grow(&s->fixed, &s->fixed_cap, total_B + 1, stream)) return rc;
   if (int rc = grow(&s->partial, &s->partial_cap, bounds_check_partials(total_B), stream)) return rc;
+  status_in_use(d_status);
   HIP_TRY(launch_bounds_check(d_rows_per_table, T, d_indices, d_offsets, index_bits == 64, indices_numel, total_B,
                               d_B_offsets ? 0 : total_B / T, d_B_offsets, bounds_check_mode, d_warning, s->fixed,
                               s->partial, (Status*)d_status, stream));
@@ -2212,6 +2229,7 @@ int fbgemm_amd_tbe_inplace_update(
       return fail(FBGEMM_AMD_E_ARG, "table %d lives in a weights buffer that was not passed", t);
     max_row_bytes = std::max(max_row_bytes, d.row_stride);
   }
+  status_in_use(d_status);
   HIP_TRY(launch_inplace_update(plan->d_tables, plan->T, (uint8_t*)d_dev_weights, (uint8_t*)d_uvm_weights,
                                 (const uint8_t*)d_update_weights, update_weights_bytes, d_update_table_idx,
                                 d_update_row_idx, row_index_bits == 64, d_update_offsets, n, max_row_bytes,

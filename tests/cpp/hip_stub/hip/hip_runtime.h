@@ -62,6 +62,7 @@ long hip_stub_wide4_launches(void); // launches of the lean kernel's four-waves-
 // the general-purpose kernel, `wide4_ms` for one of the four-wave instance
 void hip_stub_set_elapsed_ms(float general_ms, float wide4_ms);
 // A stream handle that stands for a caller's stream (never dereferenced).
+long hip_stub_device_waits(void); // calls of hipDeviceSynchronize
 long hip_stub_checks_in_flight(void);
 void hip_stub_finish_checks(void);
 hipStream_t hip_stub_stream(int id);

@@ -16,7 +16,7 @@ namespace {
 std::mutex g_mu;
 std::set<void*> g_live;
 std::set<hipStream_t> g_capturing;
-std::atomic<long> g_total{0}, g_launches{0}, g_fail_after{-1}, g_wide4{0};
+std::atomic<long> g_total{0}, g_launches{0}, g_fail_after{-1}, g_wide4{0}, g_device_waits{0};
 std::vector<fbgemm_amd::CheckRemapArgs> g_checks; // those with a counter that have not finished
 std::atomic<int> g_last_lean_wide4{0};
 std::atomic<float> g_elapsed_general{1.0f}, g_elapsed_wide4{1.0f};
@@ -73,7 +73,10 @@ hipError_t hipMemsetAsync(void* dst, int value, size_t bytes, hipStream_t) {
   return hipSuccess;
 }
 hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
-hipError_t hipDeviceSynchronize(void) { return hipSuccess; }
+hipError_t hipDeviceSynchronize(void) {
+  ++g_device_waits;
+  return hipSuccess;
+}
 hipError_t hipGetDevice(int* dev) {
   *dev = 0;
   return hipSuccess;
@@ -140,6 +143,7 @@ void hip_stub_set_elapsed_ms(float general_ms, float wide4_ms) {
   g_elapsed_general = general_ms;
   g_elapsed_wide4 = wide4_ms;
 }
+long hip_stub_device_waits(void) { return g_device_waits.load(); }
 long hip_stub_checks_in_flight(void) {
   std::lock_guard<std::mutex> lk(g_mu);
   return (long)g_checks.size();

@@ -319,6 +319,37 @@ void checks_in_flight_have_a_counter_each() {
   }).join();
 }
 
+// The thread's own status block: a call that is refused, or that comes to nothing between begin and
+// its launch, does not make the next one wait for the device.
+void refused_calls_leave_the_own_status_alone() {
+  void *table, *idx, *off, *out, *st;
+  CHECK(hipMalloc(&table, 1 << 20) == hipSuccess);
+  CHECK(hipMalloc(&idx, 8 * 4000) == hipSuccess);
+  CHECK(hipMalloc(&off, 4 * 101) == hipSuccess);
+  CHECK(hipMalloc(&out, 4 * 100 * 128) == hipSuccess);
+  hipStream_t s = hip_stub_stream(3);
+  fbgemm_amd_spmdm_config c = single_table(2, 128, 1, FBGEMM_AMD_ACC_EXACT);
+  auto run = [&](int64_t rows) { return fbgemm_amd_spmdm_run(&c, 100, 4000, rows, table, idx, off, nullptr, out, nullptr, s); };
+  CHECK(run(1000) == 1);
+  const long waits = hip_stub_device_waits();
+  CHECK(run(-1) < 0);
+  CHECK(run(1000) == 1);
+  CHECK(fbgemm_amd_status_begin(&st) == 0);
+  CHECK(fbgemm_amd_spmdm_launch(&c, 100, 4000, 1000, table, nullptr, off, nullptr, out, nullptr, st, s) < 0);
+  CHECK(fbgemm_amd_status_begin(&st) == 0);
+  CHECK(run(1000) == 1);
+  CHECK(hip_stub_device_waits() == waits);
+  // one that had enqueued something does: its block may still be written
+  CHECK(fbgemm_amd_status_begin(&st) == 0);
+  CHECK(fbgemm_amd_spmdm_launch(&c, 100, 4000, 1000, table, idx, off, nullptr, out, nullptr, st, s) == 0);
+  CHECK(run(1000) == 1);
+  CHECK(hip_stub_device_waits() == waits + 1);
+  hipFree(table);
+  hipFree(idx);
+  hipFree(off);
+  hipFree(out);
+}
+
 void allocation_failures_in_a_first_forward() {
   const Problem p = make_problem(5);
   Buffers b(p, 16, 1 << 21);
@@ -404,6 +435,7 @@ int main() {
   thread_scratch_hand_over();
   entry_point_that_allocates_nothing();
   checks_in_flight_have_a_counter_each();
+  refused_calls_leave_the_own_status_alone();
   checks_share_no_scratch();
   allocation_failures_in_a_first_forward();
   printf("launches %ld, device allocations %ld\n", hip_stub_launches(), hip_stub_total_allocations());
