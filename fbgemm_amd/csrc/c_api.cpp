@@ -304,9 +304,7 @@ Burst plan_burst(int64_t bags, int32_t T, int32_t max_D, int32_t max_bits, int64
 constexpr int64_t SPLIT_MIN_LEN_OVER_BURST = 256;
 
 struct DeviceScratch {
-  FlaggedStatus* status = nullptr; // clear between the calls that use it
-  int32_t* flag = nullptr;         // pinned: what a report sets besides the block
-  bool status_dirty = true;        // something that may write the block was enqueued since it was last read
+  Status* unread = nullptr;   // where calls without a status block record what nobody reads
   int64_t* offsets = nullptr; // lengths -> offsets
   int64_t offsets_cap = 0;
   BagEntry* order = nullptr;  // bag order of single-table calls
@@ -345,11 +343,10 @@ int grow(T** buf, int64_t* cap, int64_t need, hipStream_t stream);
 
 std::mutex& g_mu = *new std::mutex();
 
-// The status block and scratch buffers behind the calls that own their scratch
-// (fbgemm_amd_spmdm_run, the lengths / bag-order / split-bag buffers of fbgemm_amd_spmdm_launch,
-// bounds checks, pruning): one set per host thread and device, so that threads calling
-// concurrently, each on a stream of its own, neither read each other's status bits nor free a
-// buffer another thread's enqueued kernel still uses. A thread that ends hands its sets to
+// The scratch buffers behind the calls that own their scratch (the lengths / bag-order / split-bag
+// buffers of fbgemm_amd_spmdm_launch, bounds checks, pruning): one set per host thread and device, so
+// that threads calling concurrently, each on a stream of its own, do not free a buffer another
+// thread's enqueued kernel still uses. A thread that ends hands its sets to
 // g_idle_scratch (no HIP call at thread exit); the next new thread adopts one after a device-wide
 // synchronize. Calls of ONE thread share its set: those must be ordered on one stream.
 // (The map and the mutex are never destroyed: threads may end, and hand their sets over, while the
@@ -361,17 +358,66 @@ struct ThreadScratch {
   ~ThreadScratch() {
     std::lock_guard<std::mutex> lk(g_mu);
     for (auto& kv : by_device)
-      if (kv.second.status) g_idle_scratch[kv.first].push_back(kv.second);
+      if (kv.second.unread) g_idle_scratch[kv.first].push_back(kv.second);
   }
 };
 thread_local ThreadScratch t_scratch;
-thread_local DeviceScratch* t_begun = nullptr; // whose block fbgemm_amd_status_begin handed out last
+
+// The status block of the calls that wait for their result (fbgemm_amd_status_begin): one per host
+// thread and device too, but apart from the scratch. It is clear and unused between calls, so a
+// thread that takes over an ended thread's, or makes its own, waits for nothing but itself: it may do
+// so while others have work under way, or capture in a mode that lets other threads wait at all.
+struct OwnStatus {
+  FlaggedStatus* block = nullptr; // clear between the calls that use it
+  int32_t* flag = nullptr;        // pinned: what a report sets besides the block
+  bool in_use = false;            // something that may write the block was enqueued since it was last read
+};
+constexpr size_t MAX_IDLE_STATUS = 64;
+std::mutex& g_status_mu = *new std::mutex();
+std::map<int, std::vector<OwnStatus>>& g_idle_status = *new std::map<int, std::vector<OwnStatus>>(); // guarded by g_status_mu; never destroyed
+struct ThreadStatus {
+  std::map<int, OwnStatus> by_device;
+  ~ThreadStatus() {
+    std::lock_guard<std::mutex> lk(g_status_mu);
+    for (auto& kv : by_device)
+      if (kv.second.block) g_idle_status[kv.first].push_back(kv.second);
+  }
+};
+thread_local ThreadStatus t_status;
+thread_local OwnStatus* t_begun = nullptr; // what fbgemm_amd_status_begin handed out last
 
 // Where a call is about to enqueue something that may write `d_status`: only from here on does the
 // thread's own block have to be read before it is handed out again. A call refused before this point
 // leaves it as it was.
 void status_in_use(const void* d_status) {
-  if (t_begun && d_status == (const void*)t_begun->status) t_begun->status_dirty = true;
+  if (t_begun && d_status == (const void*)t_begun->block) t_begun->in_use = true;
+}
+
+int clear_own_status(const OwnStatus& s, hipStream_t stream) { // waits for `stream`
+  const FlaggedStatus clear{Status{0, STATUS_FLAGGED, ~0ull}, s.flag};
+  HIP_TRY(hipMemcpyAsync(s.block, &clear, sizeof(clear), hipMemcpyHostToDevice, stream));
+  HIP_TRY(hipStreamSynchronize(stream));
+  __atomic_store_n(s.flag, 0, __ATOMIC_RELEASE);
+  return 0;
+}
+
+int make_own_status(OwnStatus* out) {
+  OwnStatus s;
+  hipStream_t stream = nullptr; // its own: the copy that clears the block is behind nobody's work
+  int rc = 0;
+  hipError_t e = hipHostMalloc((void**)&s.flag, 64, hipHostMallocCoherent);
+  if (e == hipSuccess) e = hipMalloc((void**)&s.block, sizeof(FlaggedStatus));
+  if (e == hipSuccess) e = hipStreamCreateWithFlags(&stream, hipStreamNonBlocking);
+  if (e != hipSuccess) rc = fail(FBGEMM_AMD_E_HIP, "a status block: %s", hipGetErrorString(e));
+  else rc = clear_own_status(s, stream);
+  if (stream) (void)hipStreamDestroy(stream);
+  if (rc) {
+    if (s.block) (void)hipFree(s.block);
+    if (s.flag) (void)hipHostFree(s.flag);
+    return rc;
+  }
+  *out = s;
+  return 0;
 }
 
 // call with g_mu held
@@ -379,23 +425,14 @@ int get_scratch(DeviceScratch** out) {
   int dev = 0;
   HIP_TRY(hipGetDevice(&dev));
   DeviceScratch& s = t_scratch.by_device[dev];
-  if (!s.status) {
+  if (!s.unread) {
     std::vector<DeviceScratch>& idle = g_idle_scratch[dev];
     if (!idle.empty()) {
       HIP_TRY(hipDeviceSynchronize()); // what its last owner enqueued has finished
       s = idle.back();
       idle.pop_back();
     } else {
-      int32_t* flag = nullptr;
-      HIP_TRY(hipHostMalloc((void**)&flag, 64, hipHostMallocCoherent));
-      const hipError_t e = hipMalloc((void**)&s.status, sizeof(FlaggedStatus));
-      if (e != hipSuccess) {
-        (void)hipHostFree(flag);
-        s.status = nullptr;
-        return fail(FBGEMM_AMD_E_HIP, "hipMalloc of a status block: %s", hipGetErrorString(e));
-      }
-      s.flag = flag;
-      s.status_dirty = true;
+      HIP_TRY(hipMalloc((void**)&s.unread, sizeof(Status)));
     }
   }
   *out = &s;
@@ -465,40 +502,45 @@ int fbgemm_amd_status_read(const void* d_status, void* stream, int32_t* bits, in
 
 int fbgemm_amd_status_begin(void** d_status) {
   if (!d_status) return fail(FBGEMM_AMD_E_ARG, "d_status is null");
-  std::lock_guard<std::mutex> lk(g_mu);
-  DeviceScratch* s;
-  if (int rc = get_scratch(&s)) return rc;
-  if (s->status_dirty) { // new, or left behind by a call that failed after it had enqueued something
-    HIP_TRY(hipDeviceSynchronize());
-    const FlaggedStatus clear{Status{0, STATUS_FLAGGED, ~0ull}, s->flag};
-    HIP_TRY(hipMemcpy(s->status, &clear, sizeof(clear), hipMemcpyHostToDevice));
-    *s->flag = 0;
-    s->status_dirty = false;
+  int dev = 0;
+  HIP_TRY(hipGetDevice(&dev));
+  OwnStatus& s = t_status.by_device[dev];
+  if (!s.block) {
+    std::lock_guard<std::mutex> lk(g_status_mu);
+    std::vector<OwnStatus>& idle = g_idle_status[dev];
+    // one that may still be written is taken (and waited for) only before such blocks pile up
+    const bool any = idle.size() >= MAX_IDLE_STATUS;
+    for (size_t k = idle.size(); k-- > 0 && !s.block;)
+      if (!idle[k].in_use || (any && k == 0)) {
+        s = idle[k];
+        idle.erase(idle.begin() + (std::ptrdiff_t)k);
+      }
   }
-  t_begun = s;
-  *d_status = s->status;
+  if (!s.block)
+    if (int rc = make_own_status(&s)) return rc;
+  if (s.in_use) { // left behind by a call that failed after it had enqueued something
+    HIP_TRY(hipDeviceSynchronize());
+    if (int rc = clear_own_status(s, nullptr)) return rc;
+    s.in_use = false;
+  }
+  t_begun = &s;
+  *d_status = s.block;
   return 0;
 }
 
 int fbgemm_amd_status_end(void* stream, int32_t* bits, int64_t* first_bad_pos) {
-  DeviceScratch* s;
-  {
-    std::lock_guard<std::mutex> lk(g_mu);
-    if (int rc = get_scratch(&s)) return rc;
-  }
   HIP_TRY(hipStreamSynchronize((hipStream_t)stream));
   int32_t b = 0;
   int64_t pos = -1;
-  if (__atomic_load_n(s->flag, __ATOMIC_ACQUIRE)) {
-    // cleared here, on the call's own stream, which is quiet: clearing it at the next call would have to
-    // wait for the whole device, and may not while another thread captures
-    if (int rc = fbgemm_amd_status_read(s->status, stream, &b, &pos)) return rc;
-    const FlaggedStatus clear{Status{0, STATUS_FLAGGED, ~0ull}, s->flag};
-    HIP_TRY(hipMemcpyAsync(s->status, &clear, sizeof(clear), hipMemcpyHostToDevice, (hipStream_t)stream));
-    HIP_TRY(hipStreamSynchronize((hipStream_t)stream));
-    __atomic_store_n(s->flag, 0, __ATOMIC_RELEASE);
+  if (t_begun) {
+    if (__atomic_load_n(t_begun->flag, __ATOMIC_ACQUIRE)) {
+      // cleared here, on the call's own stream, which is quiet: clearing it at the next call would have to
+      // wait for the whole device, and may not while another thread captures
+      if (int rc = fbgemm_amd_status_read(t_begun->block, stream, &b, &pos)) return rc;
+      if (int rc = clear_own_status(*t_begun, (hipStream_t)stream)) return rc;
+    }
+    t_begun->in_use = false;
   }
-  s->status_dirty = false;
   if (bits) *bits = b;
   if (first_bad_pos) *first_bad_pos = pos;
   return 0;
@@ -1995,15 +2037,18 @@ int fbgemm_amd_compressed_indices_remap(
   std::lock_guard<std::mutex> lk(g_mu);
   DeviceScratch* s;
   if (int rc = get_scratch(&s)) return rc;
-  if (!d_status) s->status_dirty = true; // what is recorded there is nobody's
   // one scratch buffer: n + 1 running counts (int64), then the n mapped rows (int32)
   if (int rc = grow(&s->fixed, &s->fixed_cap, (n + 1) + (n + 1) / 2 + 1, stream)) return rc;
   if (int rc = grow(&s->partial, &s->partial_cap, prune_partials(n + 1), stream)) return rc;
+  if (!d_status) {
+    HIP_TRY(launch_status_clear(s->unread, stream)); // it is made as any memory is
+    d_status = s->unread;
+  }
   status_in_use(d_status);
   HIP_TRY(launch_compressed_indices_remap(d_indices, index_bits == 64, d_mapping, mapping_numel, d_offsets, offsets_numel,
                                           d_weights, first, n, d_out_indices, d_out_offsets, d_out_weights, s->fixed,
                                           s->partial, reinterpret_cast<int32_t*>(s->fixed + n + 1),
-                                          d_status ? (Status*)d_status : &s->status->st, stream));
+                                          (Status*)d_status, stream));
   return 0;
 }
 

@@ -344,6 +344,23 @@ void refused_calls_leave_the_own_status_alone() {
   CHECK(fbgemm_amd_spmdm_launch(&c, 100, 4000, 1000, table, idx, off, nullptr, out, nullptr, st, s) == 0);
   CHECK(run(1000) == 1);
   CHECK(hip_stub_device_waits() == waits + 1);
+  // a thread's first waiting call, with a block of its own or with the one an ended thread has left
+  for (int k = 0; k < 3; ++k) std::thread([&] { CHECK(run(1000) == 1); }).join();
+  CHECK(hip_stub_device_waits() == waits + 1);
+  // threads that end with their block in use: the blocks do not pile up
+  const long blocks = hip_stub_total_allocations();
+  for (int k = 0; k < 200; ++k)
+    std::thread([&] {
+      CHECK(fbgemm_amd_status_begin(&st) == 0);
+      CHECK(fbgemm_amd_spmdm_launch(&c, 100, 4000, 1000, table, idx, off, nullptr, out, nullptr, st, s) == 0);
+    }).join();
+  CHECK(hip_stub_total_allocations() <= blocks + 64);
+  // what a call without a block records is nobody's: the next waiting call does not care
+  int32_t map[4] = {0, 1, 2, 3}, offs[2] = {0, 0};
+  CHECK(fbgemm_amd_compressed_indices_remap(2, idx, 32, map, 4, offs, nullptr, out, out, nullptr, nullptr, s) == 0);
+  const long now = hip_stub_device_waits();
+  CHECK(run(1000) == 1);
+  CHECK(hip_stub_device_waits() == now);
   hipFree(table);
   hipFree(idx);
   hipFree(off);

@@ -50,3 +50,52 @@ def test_rejected_accepted_in_turn(no_bag):
         t.join()
     turns()
     assert not failures, failures
+
+
+def test_first_call_of_a_thread_beside_a_capture(oracle):
+    """A thread's first waiting call makes its status block. That waits for nothing but itself, also while
+    another thread captures (in the mode that lets other threads wait); and a block that an ended thread
+    leaves is taken over the same way."""
+    assert torch.cuda.is_available(), "these tests need the GPU"
+    from fbgemm_amd import ops
+    from test_tbe_gpu import build_weights
+    rng = np.random.default_rng(4)
+    D, rows, B = 32, 50, 40
+    weights, wo, _ = build_weights(rng, [(rows, D, INT8)], 16)
+    cu = lambda a: torch.from_numpy(np.ascontiguousarray(a)).cuda()
+    meta = (cu(weights), torch.zeros(0, dtype=torch.uint8, device="cuda"), cu(np.zeros(1, np.int32)), cu(wo),
+            cu(np.array([INT8], np.uint8)), cu(np.array([0, D], np.int32)))
+    idx, off = cu(rng.integers(0, rows, size=3 * B).astype(np.int64)), cu(np.arange(B + 1, dtype=np.int64) * 3)
+    call = lambda: ops.int_nbit_split_embedding_codegen_lookup_function(
+        *meta, D, 0, 0, D, 0, 0, idx, off, ops.POOL_NONE, None, ops.FP32, row_alignment=16)
+    want = call()
+    torch.cuda.synchronize()
+    got, failures = [], []
+
+    def first():
+        try:
+            with torch.cuda.stream(streams.pop()):
+                got.append(call())
+        except BaseException as e:  # noqa: BLE001
+            failures.append(e)
+
+    for turn in range(2):  # a block of its own, then perhaps the one the first thread left
+        streams = [torch.cuda.Stream() for _ in range(2)]
+        x = torch.ones(100, device="cuda")
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=torch.cuda.Stream(), capture_error_mode="thread_local"):
+            y = x * 2
+            threads = [threading.Thread(target=first) for _ in range(2)]
+            for t in threads:
+                t.start()
+            for t in threads:
+                t.join()
+            z = y + 1
+        assert not failures, failures
+        for _ in range(3):
+            graph.replay()
+            torch.cuda.synchronize()
+            assert bool((z == 3).all())
+            x.fill_(1)
+        assert len(got) == 2 * (turn + 1) and all(torch.equal(g, want) for g in got)
