@@ -10,6 +10,7 @@
 #include <map>
 #include <memory>
 #include <mutex>
+#include <set>
 #include <vector>
 
 #include "../../include/fbgemm_amd.h"
@@ -374,6 +375,7 @@ struct OwnStatus {
 };
 constexpr size_t MAX_IDLE_STATUS = 64;
 std::mutex& g_status_mu = *new std::mutex();
+std::set<const void*>& g_own_blocks = *new std::set<const void*>(); // every thread's, guarded by g_status_mu; never destroyed
 std::map<int, std::vector<OwnStatus>>& g_idle_status = *new std::map<int, std::vector<OwnStatus>>(); // guarded by g_status_mu; never destroyed
 struct ThreadStatus {
   std::map<int, OwnStatus> by_device;
@@ -416,6 +418,8 @@ int make_own_status(OwnStatus* out) {
     if (s.flag) (void)hipHostFree(s.flag);
     return rc;
   }
+  std::lock_guard<std::mutex> lk(g_status_mu);
+  g_own_blocks.insert(s.block);
   *out = s;
   return 0;
 }
@@ -486,7 +490,12 @@ const char* fbgemm_amd_version(void) { return "0.1"; }
 
 int fbgemm_amd_status_clear(void* d_status, void* stream) {
   if (!d_status) return fail(FBGEMM_AMD_E_ARG, "d_status is null");
-  HIP_TRY(launch_status_clear((Status*)d_status, (hipStream_t)stream));
+  int32_t mark = 0;
+  {
+    std::lock_guard<std::mutex> lk(g_status_mu);
+    if (g_own_blocks.count(d_status)) mark = STATUS_FLAGGED; // without it its thread would learn of nothing any more
+  }
+  HIP_TRY(launch_status_clear((Status*)d_status, mark, (hipStream_t)stream));
   return 0;
 }
 
@@ -2041,7 +2050,7 @@ int fbgemm_amd_compressed_indices_remap(
   if (int rc = grow(&s->fixed, &s->fixed_cap, (n + 1) + (n + 1) / 2 + 1, stream)) return rc;
   if (int rc = grow(&s->partial, &s->partial_cap, prune_partials(n + 1), stream)) return rc;
   if (!d_status) {
-    HIP_TRY(launch_status_clear(s->unread, stream)); // it is made as any memory is
+    HIP_TRY(launch_status_clear(s->unread, 0, stream)); // it is made as any memory is
     d_status = s->unread;
   }
   status_in_use(d_status);

@@ -143,9 +143,9 @@ __global__ __launch_bounds__(LENGTHS_BLOCK) void lengths_to_offsets_kernel(const
   if (end == n && tid == 0) offsets[n] = carry;
 }
 
-__global__ void status_clear_kernel(Status* st) {
+__global__ void status_clear_kernel(Status* st, int32_t mark) {
   st->bits = 0;
-  st->pad = 0;
+  st->pad = mark;
   st->first_bad_pos = ~0ull;
 }
 
@@ -251,8 +251,8 @@ hipError_t launch_lengths_to_offsets(const void* lengths, bool is64, int64_t n, 
   return hipGetLastError();
 }
 
-hipError_t launch_status_clear(Status* st, hipStream_t stream) {
-  hipLaunchKernelGGL(status_clear_kernel, dim3(1), dim3(1), 0, stream, st);
+hipError_t launch_status_clear(Status* st, int32_t mark, hipStream_t stream) {
+  hipLaunchKernelGGL(status_clear_kernel, dim3(1), dim3(1), 0, stream, st, mark);
   return hipGetLastError();
 }
 

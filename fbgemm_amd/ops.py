@@ -120,7 +120,7 @@ def _make_kernel(weight_ty, block_size, normalize_by_lengths, is_weight_position
             check(lib.fbgemm_amd_spmdm_launch(
                 C.byref(cfg), output_size, index_size, data_size, _ptr(input), _ptr(indices),
                 _ptr(offsets_or_lengths), _ptr(weights), _ptr(out), _ptr(compressed_indices_table),
-                _ptr(status.buf), _stream()))
+                status.ptr, _stream()))
             return None
         rc = check(lib.fbgemm_amd_spmdm_run(
             C.byref(cfg), output_size, index_size, data_size, _ptr(input), _ptr(indices),

@@ -77,7 +77,9 @@ int fbgemm_amd_status_read(const void* d_status, void* stream, int32_t* bits, in
  * first offending position or -1). One pair at a time per thread, on one device.
  * Costs no operation on the stream unless something was recorded. A begin whose
  * launches were all refused needs no end; one whose launches were enqueued and
- * that is not ended makes the thread's next begin wait for the device. */
+ * that is not ended makes the thread's next begin wait for the device. The block
+ * is the library's: beside the launches, status_clear and status_read may be
+ * called on it, and nothing else may write it. */
 int fbgemm_amd_status_begin(void** d_status);
 int fbgemm_amd_status_end(void* stream, int32_t* bits, int64_t* first_bad_pos);
 

@@ -52,6 +52,41 @@ def test_rejected_accepted_in_turn(no_bag):
     assert not failures, failures
 
 
+def single_table_calls():
+    """A good and a bad launch of a single-table lookup into a status block, and the same as waiting calls."""
+    assert torch.cuda.is_available(), "these tests need the GPU"
+    from fbgemm_amd import ops
+    rng = np.random.default_rng(9)
+    D, rows, nb = 32, 50, 20
+    table, _ = H.make_table(rng, INT8, rows, D, True)
+    table = torch.from_numpy(table).cuda()
+    good = torch.from_numpy(rng.integers(0, rows, size=nb).astype(np.int64)).cuda()
+    bad = good.clone()
+    bad[7] = rows
+    off = torch.arange(nb + 1, dtype=torch.int32, device="cuda")
+    out = torch.empty(nb, D, device="cuda")
+    kern = ops.generate_embedding_spmdm_with_strides(ops.INT8, D, False, False)
+    return ops, lambda idx, st=None, bags=nb: kern(bags, nb, rows, table, idx, off, None, out, status=st), good, bad
+
+
+def test_own_block_cleared_by_its_user():
+    """status_clear on the block of status_begin clears it and leaves what makes it report."""
+    ops, call, good, bad = single_table_calls()
+    from fbgemm_amd import _lib
+    for reported in (False, True):
+        st = ops._OwnStatus()
+        if reported:
+            call(bad, st)
+        ops.check(_lib.lib().fbgemm_amd_status_clear(st.ptr, ops._stream()))
+        assert st.read() == (0, -1)
+        assert call(good) is True and call(bad) is False and call(good) is True
+        st = ops._OwnStatus()
+        ops.check(_lib.lib().fbgemm_amd_status_clear(st.ptr, ops._stream()))
+        call(bad, st)
+        assert st.read() == (ops.ERR_INDEX_OUT_OF_RANGE, 7)
+        assert call(good) is True and call(bad) is False
+
+
 def test_first_call_of_a_thread_beside_a_capture(oracle):
     """A thread's first waiting call makes its status block. That waits for nothing but itself, also while
     another thread captures (in the mode that lets other threads wait); and a block that an ended thread
