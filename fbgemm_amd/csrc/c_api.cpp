@@ -630,10 +630,8 @@ int spmdm_launch_impl(
   if (output_size == 0) {
     // the reference returns (0 == index_size) without touching anything
     if (index_size != 0 && !cfg->no_bag) {
-      Status h{ERR_LENGTH_MISMATCH, 0, ~0ull};
       status_in_use(d_status);
-      HIP_TRY(hipMemcpyAsync(d_status, &h, sizeof(h), hipMemcpyHostToDevice, stream));
-      HIP_TRY(hipStreamSynchronize(stream));
+      HIP_TRY(launch_status_report((Status*)d_status, ERR_LENGTH_MISMATCH, stream));
     }
     return 0;
   }

@@ -143,6 +143,9 @@ __global__ __launch_bounds__(LENGTHS_BLOCK) void lengths_to_offsets_kernel(const
   if (end == n && tid == 0) offsets[n] = carry;
 }
 
+// what a call finds wrong before it launches anything
+__global__ void status_report_kernel(Status* st, int32_t bits) { status_or(st, bits); }
+
 __global__ void status_clear_kernel(Status* st, int32_t mark) {
   st->bits = 0;
   st->pad = mark;
@@ -248,6 +251,11 @@ hipError_t launch_lengths_to_offsets(const void* lengths, bool is64, int64_t n, 
   const unsigned blocks = (unsigned)(n > 0 ? (n + run - 1) / run : 1);
   if (is64) hipLaunchKernelGGL(lengths_to_offsets_kernel<int64_t>, dim3(blocks), dim3(LENGTHS_BLOCK), 0, stream, (const int64_t*)lengths, n, run, offsets);
   else hipLaunchKernelGGL(lengths_to_offsets_kernel<int32_t>, dim3(blocks), dim3(LENGTHS_BLOCK), 0, stream, (const int32_t*)lengths, n, run, offsets);
+  return hipGetLastError();
+}
+
+hipError_t launch_status_report(Status* st, int32_t bits, hipStream_t stream) {
+  hipLaunchKernelGGL(status_report_kernel, dim3(1), dim3(1), 0, stream, st, bits);
   return hipGetLastError();
 }
 

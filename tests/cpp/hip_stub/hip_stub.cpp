@@ -192,6 +192,11 @@ hipError_t launch_lengths_to_offsets(const void*, bool, int64_t n, int64_t* offs
   for (int64_t i = 0; i <= n; ++i) offsets[i] = 0; // the whole buffer must be there
   return LAUNCHED();
 }
+hipError_t launch_status_report(Status* st, int32_t bits, hipStream_t) {
+  st->bits |= bits;
+  if (st->pad == STATUS_FLAGGED) *reinterpret_cast<FlaggedStatus*>(st)->flag = 1;
+  return LAUNCHED();
+}
 hipError_t launch_status_clear(Status* st, int32_t mark, hipStream_t) {
   st->bits = 0;
   st->pad = mark;

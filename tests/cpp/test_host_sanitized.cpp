@@ -347,6 +347,11 @@ void refused_calls_leave_the_own_status_alone() {
   // a thread's first waiting call, with a block of its own or with the one an ended thread has left
   for (int k = 0; k < 3; ++k) std::thread([&] { CHECK(run(1000) == 1); }).join();
   CHECK(hip_stub_device_waits() == waits + 1);
+  // what a call finds wrong without a kernel reaches its user
+  int32_t bits = 0;
+  CHECK(fbgemm_amd_status_begin(&st) == 0);
+  CHECK(fbgemm_amd_spmdm_launch(&c, 0, 5, 1000, table, idx, off, nullptr, out, nullptr, st, s) == 0);
+  CHECK(fbgemm_amd_status_end(s, &bits, nullptr) == 0 && bits == FBGEMM_AMD_ERR_LENGTH_MISMATCH);
   // threads that end with their block in use: the blocks do not pile up
   const long blocks = hip_stub_total_allocations();
   for (int k = 0; k < 200; ++k)

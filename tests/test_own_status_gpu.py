@@ -87,6 +87,20 @@ def test_own_block_cleared_by_its_user():
         assert call(good) is True and call(bad) is False
 
 
+def test_no_bags_but_indices():
+    """No bags but indices is an error that is known without a kernel; it is reported like any other."""
+    ops, call, good, bad = single_table_calls()
+    for _ in range(2):
+        st = ops._OwnStatus()
+        call(good, st, bags=0)
+        assert st.read() == (ops.ERR_LENGTH_MISMATCH, -1)
+        assert call(good) is True and call(bad) is False
+    st = ops.Status()
+    call(bad, st)
+    call(good, st, bags=0)
+    assert st.read() == (ops.ERR_INDEX_OUT_OF_RANGE | ops.ERR_LENGTH_MISMATCH, 7)
+
+
 def test_first_call_of_a_thread_beside_a_capture(oracle):
     """A thread's first waiting call makes its status block. That waits for nothing but itself, also while
     another thread captures (in the mode that lets other threads wait); and a block that an ended thread
