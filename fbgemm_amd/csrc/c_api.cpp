@@ -280,7 +280,6 @@ struct Burst {
 // 1 / 4: every launch it can take goes to the burst kernel with that many waves per bag, 0: none does,
 // -1: by the rule (tests: fbgemm_amd_set_burst).
 int g_burst_override = -1;
-constexpr int32_t BURST_COLS = 256;
 Burst plan_burst(int64_t bags, int32_t T, int32_t max_D, int32_t max_bits, int64_t lookups) {
   Burst b;
   const int64_t windows = ((int64_t)max_D + BURST_COLS - 1) / BURST_COLS;
@@ -293,7 +292,7 @@ Burst plan_burst(int64_t bags, int32_t T, int32_t max_D, int32_t max_bits, int64
   else if (groups <= 4096 || (windows == 1 && (groups <= 8192 ? avg_len >= 8 : groups <= 16384 && avg_len >= 24)))
     b.waves = (groups <= 1024 && avg_len >= 16) || (groups <= 2048 && avg_len >= 64) ? 4 : 1;
   // bytes of a staged row, of the widest type and table of the launch
-  const int64_t pitch = ((int64_t)std::min(max_D, BURST_COLS) * max_bits / 8 + 15) / 16 * 16;
+  const int64_t pitch = burst_pitch(max_D, max_bits);
   b.lds_bytes = b.waves == 4 ? 32768
       : groups <= 2048       ? 16384
       : groups > 4096 && 8 * pitch <= 4096 && std::min<int64_t>(avg_len, 64) * pitch <= 8192 ? 4096 : 8192;
@@ -828,7 +827,7 @@ int spmdm_launch_impl(
     return 0;
   }
   if (burst.waves)
-    HIP_TRY(launch_lookup_burst(a, cfg->index_bits == 64, d.D, burst.waves, burst.lds_bytes, stream));
+    HIP_TRY(launch_lookup_burst(a, cfg->index_bits == 64, d.D, bits, burst.waves, burst.lds_bytes, stream));
   else if (lean_enabled() && !cfg->is_weight_positional && lean_shape(d))
     HIP_TRY(launch_lookup_lean(a, cfg->index_bits == 64, cfg->accumulate != FBGEMM_AMD_ACC_FAST, false, stream));
   else
@@ -1672,7 +1671,7 @@ int tbe_forward_impl(
   // or longer bags, or the 8-bit output, and take the other kernels.
   if (burst.waves && !d_q8_out) {
     a.tables = plan->d_tables;
-    HIP_TRY(launch_lookup_burst(a, index_bits == 64, plan->max_D, burst.waves, burst.lds_bytes, stream));
+    HIP_TRY(launch_lookup_burst(a, index_bits == 64, plan->max_D, plan->max_bits, burst.waves, burst.lds_bytes, stream));
     return 0;
   }
   if (sort_bags_default() && indices_numel >= (int64_t)SORT_MIN_LOOKUPS) {

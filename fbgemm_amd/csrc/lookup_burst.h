@@ -23,8 +23,6 @@
 
 namespace fbgemm_amd {
 
-constexpr int BURST_COLS = 256; // columns of a workgroup
-
 // What a row's window of columns looks like in memory and in LDS: np pieces of `size` bytes, piece
 // k at byte k * size of the window, the last one at `last` (which is less where a whole piece there
 // would leave the row: it then overlaps its neighbour). In LDS the pieces lie end to end.
@@ -241,7 +239,7 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(WAVE
     if (quant) row_end = max(row_end, (int64_t)d.sb_off + (d.sb_fp32 ? 8 : 4));
   }
   const BurstWindow w = burst_window(d, first, row_end - in_row, (cols * bits + 7) >> 3);
-  // a multiple of 8: a window has at most 1024 bytes, and 8 of those fit
+  // a multiple of 8, and 8 at least (burst_fits)
   const int cap = min(lds_bytes / w.pitch, THREADS) & ~7;
 
   // this lane's columns: their bytes inside a staged row

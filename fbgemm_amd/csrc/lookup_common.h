@@ -189,6 +189,14 @@ struct LookupArgs {
   Status* status;
 };
 
+// The burst kernel's windows of columns, the bytes of a staged row of the widest window of a launch,
+// and what the staged rows must have at least: its loop over a bag advances by whole 8s of them.
+constexpr int32_t BURST_COLS = 256;
+constexpr int64_t burst_pitch(int32_t max_D, int32_t max_bits) {
+  return (((int64_t)(max_D < BURST_COLS ? max_D : BURST_COLS) * max_bits + 7) / 8 + 15) / 16 * 16;
+}
+constexpr bool burst_fits(int32_t max_D, int32_t max_bits, int64_t lds_bytes) { return max_D > 0 && max_bits > 0 && lds_bytes >= 8 * burst_pitch(max_D, max_bits); }
+
 // The bounds check with the pruned-row mapping (check_remap_kernel).
 struct CheckRemapArgs {
   const int64_t* rows;         // T physical row counts

@@ -222,13 +222,13 @@ hipError_t launch_lookup(const LookupArgs& a, bool idx64, hipStream_t stream) {
 hipError_t launch_lookup_burst_i64(const LookupArgs& a, dim3 grid, bool four_waves, int lds_bytes, hipStream_t stream);
 hipError_t launch_lookup_burst_i32(const LookupArgs& a, dim3 grid, bool four_waves, int lds_bytes, hipStream_t stream);
 
-// The burst kernel (lookup_burst.h): a workgroup per bag and window of 256 columns. max_D: the widest
-// table of the launch; waves: 1 or 4 per workgroup; lds_bytes: what a workgroup's
+// The burst kernel (lookup_burst.h): a workgroup per bag and window of 256 columns. max_D, max_bits: the
+// widest table and row type of the launch; waves: 1 or 4 per workgroup; lds_bytes: what a workgroup's
 // staged rows may take, at least 8 rows of the widest window.
-hipError_t launch_lookup_burst(const LookupArgs& a, bool idx64, int32_t max_D, int waves, int lds_bytes, hipStream_t stream) {
+hipError_t launch_lookup_burst(const LookupArgs& a, bool idx64, int32_t max_D, int32_t max_bits, int waves, int lds_bytes, hipStream_t stream) {
   if (a.B <= 0 || a.T <= 0) return hipSuccess;
-  const int windows = (max_D + 255) / 256;
-  if (a.T > 65535 || windows > 65535 || lds_bytes < 1024 || (waves != 1 && waves != 4)) return hipErrorInvalidValue;
+  const int windows = (max_D + BURST_COLS - 1) / BURST_COLS;
+  if (a.T > 65535 || windows > 65535 || !burst_fits(max_D, max_bits, lds_bytes) || (waves != 1 && waves != 4)) return hipErrorInvalidValue;
   const dim3 grid((unsigned)a.B, (unsigned)a.T, (unsigned)windows);
   return idx64 ? launch_lookup_burst_i64(a, grid, waves == 4, lds_bytes, stream) : launch_lookup_burst_i32(a, grid, waves == 4, lds_bytes, stream);
 }

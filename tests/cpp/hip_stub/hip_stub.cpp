@@ -184,8 +184,8 @@ hipError_t launch_lookup_lean(const LookupArgs& a, bool idx64, bool, bool wide4,
   g_last_lean_wide4 = wide4 ? 1 : 0;
   return launch_lookup(a, idx64, s);
 }
-hipError_t launch_lookup_burst(const LookupArgs& a, bool idx64, int32_t, int, int lds_bytes, hipStream_t s) {
-  if (lds_bytes < 4096) return hipErrorInvalidValue;
+hipError_t launch_lookup_burst(const LookupArgs& a, bool idx64, int32_t max_D, int32_t max_bits, int, int lds_bytes, hipStream_t s) {
+  if (!burst_fits(max_D, max_bits, lds_bytes)) return hipErrorInvalidValue;
   return launch_lookup(a, idx64, s);
 }
 hipError_t launch_lengths_to_offsets(const void*, bool, int64_t n, int64_t* offsets, hipStream_t) {

@@ -16,6 +16,7 @@
 #include <vector>
 
 #include "../../include/fbgemm_amd.h"
+#include "../../fbgemm_amd/csrc/lookup_common.h"
 #include "../../include/fbgemm_amd_bench.h"
 
 #define CHECK(cond)                                                         \
@@ -372,6 +373,30 @@ void refused_calls_leave_the_own_status_alone() {
   hipFree(out);
 }
 
+// The burst kernel goes over a bag by whole 8s of staged rows: a launch whose rows do not fit that many
+// times would never end, and is refused on the host. The rule's own sizes fit, whatever it chooses.
+void burst_launches_fit() {
+  CHECK(fbgemm_amd::burst_pitch(256, 32) == 1024 && fbgemm_amd::burst_pitch(33, 4) == 32 && fbgemm_amd::burst_pitch(1000, 8) == 256);
+  CHECK(!fbgemm_amd::burst_fits(256, 32, 1024) && !fbgemm_amd::burst_fits(300, 32, 8191) && fbgemm_amd::burst_fits(300, 32, 8192));
+  void *table, *idx, *off, *out;
+  CHECK(hipMalloc(&table, 1 << 20) == hipSuccess);
+  CHECK(hipMalloc(&idx, 64) == hipSuccess);
+  CHECK(hipMalloc(&off, 64) == hipSuccess);
+  CHECK(hipMalloc(&out, 64) == hipSuccess);
+  for (int waves : {-1, 1, 4}) {
+    fbgemm_amd_set_burst(waves);
+    for (int32_t ty : {0, 1, 2, 3, 4})
+      for (int32_t D = 4; D <= 1100; D += D < 40 ? 4 : 36)
+        for (int64_t bags : {1, 1500, 3000, 8000, 16000})
+          for (int64_t len : {1, 20, 50, 100}) {
+            fbgemm_amd_spmdm_config c = single_table(ty, D, 1, FBGEMM_AMD_ACC_EXACT);
+            CHECK(fbgemm_amd_spmdm_launch(&c, bags, bags * len, 10, table, idx, off, nullptr, out, nullptr, out, nullptr) == 0);
+          }
+  }
+  fbgemm_amd_set_burst(-1);
+  for (void* p : {table, idx, off, out}) hipFree(p);
+}
+
 void allocation_failures_in_a_first_forward() {
   const Problem p = make_problem(5);
   Buffers b(p, 16, 1 << 21);
@@ -458,6 +483,7 @@ int main() {
   entry_point_that_allocates_nothing();
   checks_in_flight_have_a_counter_each();
   refused_calls_leave_the_own_status_alone();
+  burst_launches_fit();
   checks_share_no_scratch();
   allocation_failures_in_a_first_forward();
   printf("launches %ld, device allocations %ld\n", hip_stub_launches(), hip_stub_total_allocations());
