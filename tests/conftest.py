@@ -19,16 +19,19 @@ def oracle():
     return o
 
 
-@pytest.fixture(params=["wide", "narrow", "general"])
+@pytest.fixture(params=["wide", "narrow", "general", "burst"])
 def lane_shape(request):
-    """The three routes a pooled lookup can take, for test modules that ask for this fixture:
+    """The routes a pooled lookup can take, for test modules that ask for this fixture:
     "wide" = 16-byte lanes, the lean kernel where the shape allows it (what large launches get);
-    "narrow" = 4-byte lanes (what launches too small to fill the device get by default);
-    "general" = 16-byte lanes with the lean kernel switched off (everything through the general kernel)."""
+    "narrow" = 4-byte lanes (what launches between the burst kernel's and those that fill the device get);
+    "general" = 16-byte lanes with the lean kernel switched off (everything through the general kernel);
+    "burst" = the rule as it is, which gives the burst kernel what is too small to fill the device."""
     import fbgemm_amd
     lib = fbgemm_amd.lib()
-    lib.fbgemm_amd_set_narrow_below_waves(1024 if request.param == "narrow" else 0)
+    lib.fbgemm_amd_set_narrow_below_waves({"narrow": 1024, "burst": -1}.get(request.param, 0))
+    lib.fbgemm_amd_set_burst(-1 if request.param == "burst" else 0)
     lib.fbgemm_amd_set_lean(0 if request.param == "general" else 1)
     yield request.param
     lib.fbgemm_amd_set_narrow_below_waves(-1)
+    lib.fbgemm_amd_set_burst(-1)
     lib.fbgemm_amd_set_lean(-1)

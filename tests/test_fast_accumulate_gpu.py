@@ -28,16 +28,20 @@ def ops():
     return o
 
 
-@pytest.fixture(autouse=True, params=["wide", "default"])
+@pytest.fixture(autouse=True, params=["wide", "narrow", "default"])
 def lanes(request):
-    """Test-sized launches would take 4-byte lanes (the general kernel, which is exact in either
-    mode): "wide" gives them the 16-byte lanes and the lean kernel that large launches get."""
+    """Test-sized launches would take the burst kernel (which is exact in either mode), except where the
+    rule cuts their bags into segments: "wide" gives them the 16-byte lanes and the lean kernel that large
+    launches get, "narrow" the 4-byte lanes of the general kernel (exact too)."""
     import fbgemm_amd
     lib = fbgemm_amd.lib()
     if request.param == "wide":
         lib.fbgemm_amd_set_narrow_below_waves(0)
+    elif request.param == "narrow":
+        lib.fbgemm_amd_set_burst(0)
     yield request.param
     lib.fbgemm_amd_set_narrow_below_waves(-1)
+    lib.fbgemm_amd_set_burst(-1)
 
 
 def cu(a):

@@ -32,15 +32,18 @@ def ops():
 
 @pytest.fixture
 def routes():
-    """lets a case pick its route: 16-byte or 4-byte lanes, the lean kernel on or off"""
+    """lets a case pick its route: 16-byte or 4-byte lanes or the burst kernel, the lean kernel on or off"""
     import fbgemm_amd
     lib = fbgemm_amd.lib()
 
     def choose(rng):
-        lib.fbgemm_amd_set_narrow_below_waves(1024 if rng.random() < 0.4 else 0)
+        route = rng.random()
+        lib.fbgemm_amd_set_narrow_below_waves(1024 if route < 0.4 else 0)
+        lib.fbgemm_amd_set_burst(-1 if route < 0.2 else 0)
         lib.fbgemm_amd_set_lean(0 if rng.random() < 0.3 else 1)
     yield choose
     lib.fbgemm_amd_set_narrow_below_waves(-1)
+    lib.fbgemm_amd_set_burst(-1)
     lib.fbgemm_amd_set_lean(-1)
 
 
