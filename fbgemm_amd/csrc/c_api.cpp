@@ -256,18 +256,36 @@ int wide4_mode() {
   return m < 0 ? 0 : (m > 2 ? 2 : m);
 }
 
-// Which launches the burst kernel (lookup_burst.h) takes, and in which form. `bags`: of all tables;
-// us of the single-table kernel over 1 M uniform rows, the better of the other kernels -> burst kernel:
-//                       10 bags x 100   1024 x 20      8192 x 10      8192 x 25      16384 x 10     16384 x 25
-//   4-bit, 128 wide     47.7 -> 10.8    17.3 -> 9.4    15.1 -> 14.6   21.8 -> 19.0   18.0 -> 22.2   27.4 -> 28.3
-//   8-bit, 100 wide     47.7 -> 11.2    17.4 -> 9.5    20.5 -> 14.6   29.1 -> 20.5   23.3 -> 22.1   37.5 -> 30.2
-//   8-bit, 36 wide                                     14.6 -> 13.8   20.8 -> 17.7   22.0 -> 21.4   31.9 -> 26.4
-//   fp16, 64 wide                                      18.3 -> 12.8   25.8 -> 16.8   21.2 -> 19.6   30.8 -> 24.5
-//   fp16, 200 wide                                     21.8 -> 19.3   33.7 -> 29.3   27.1 -> 28.8   48.8 -> 47.5
-//   8-bit, 512 wide     52.0 -> 13.6    18.4 -> 10.9   14.8 -> 17.1 and 20.4 -> 24.0 (4096 x 10 and x 20)
-// It is bound by how many workgroups the device holds at a time, so the line lies at workgroups:
-// 4096 (16 per compute unit: all resident at once), 8192 where a workgroup covers the whole row, and
-// 16384 for bags of three rounds and more in the other kernels.
+// Which launches the burst kernel (lookup_burst.h) takes, and in which form. It is bound by how many
+// workgroups the device holds at a time: up to 4096 (16 per compute unit, all resident at once) it
+// takes every launch. us, the better of the other kernels -> burst kernel, single tables of 1 M rows:
+//                       10 bags x 100   1024 x 20
+//   4-bit, 128 wide     47.7 -> 10.8    17.3 -> 9.4
+//   8-bit, 100 wide     47.7 -> 11.2    17.4 -> 9.5
+//   8-bit, 512 wide     52.0 -> 13.6    18.4 -> 10.9
+// Beyond, it depends on what the other kernels have against it. Burst time over theirs, for bags of 25
+// and 60 entries and tables of 200 000 rows in a table-batched launch (8 tables):
+//                       4608 bags    6144         8192         12288        16384
+//   4-bit, 64 wide      .89  .92    1.04 1.11    1.12 1.15    1.24 1.24    1.41 1.33
+//   4-bit, 128 wide     .83  .99    1.01 1.10    1.10 1.18    1.32 1.32    1.31 1.15
+//   4-bit, 256 wide     .80  .89    1.04 1.07    1.01  .97    1.18 1.12    1.16 1.05
+//   8-bit, 100 wide                               .75  .75     .87  .94    1.26 1.15
+//   8-bit, 128 wide     .79  .91    1.00 1.11     .77  .80    1.14 1.13    1.15 1.09
+//   fp16, 64 wide       .79  .79    1.01 1.05     .67  .70     .86  .86     .76  .75
+//   fp16, 128 wide                                .65  .67     .64  .67    1.24 1.08
+//   fp16, 256 wide                               1.22 1.08    1.18 1.08    1.18 1.09
+//   2-bit, 256 wide                               .81  .81     .95  .93    1.07  .99
+//   mixed types         .64  .70     .72  .79     .64  .67     .77  .78    1.19 1.00
+// * Up to 5120 workgroups (five waves per SIMD) are still one round of them.
+// * From 1024 waves of 16-byte lanes on (narrow_below_waves) the other kernels fill the device and
+//   win. Single tables with the scale and bias behind the data are the exception, an extra line per
+//   row for those kernels: 4-bit, 200 wide, 8192 x 25: .82, where the lean kernel does not take
+//   them; where it does, for long bags in more than 8192 (8-bit, 128 wide, 16384 x 25 and x 60:
+//   .98 and .83).
+// * Below, the others take 4-byte lanes, and lose once their waves exceed the 3072 that the device
+//   holds; up to there they win. (Rows that have only lanes of 4 bytes and less: the same line.)
+//   Launches of several types hold fewer of those waves, 2-bit rows cost those lanes the most.
+//   Single tables of bags that one staging takes: 5200 x 25 .83 to .93.
 // Four waves per bag pay while all such workgroups are resident together (four per compute unit:
 // 1024; 1024 bags x 100: 22.0 -> 13.9) and, for long bags, in two rounds of them (2048 x 100: 24.9 -> 21.9).
 // LDS: large launches want many workgroups resident, so they stage in 4 KB what takes at most two
@@ -277,22 +295,46 @@ struct Burst {
   int waves = 0; // 0: another kernel takes the launch
   int lds_bytes = 0;
 };
+// What the other kernels would make of a launch.
+struct BurstRivals {
+  int64_t waves = 0;        // with 16-byte lanes
+  int64_t narrow_waves = 0; // with 4-byte lanes
+  int max_vb = 0;           // the widest lanes there are
+  bool types_differ = false;
+  bool single = false;      // a single table ...
+  bool trailer = false;     // ... with the scale and bias behind the data
+  bool lean = false;        // ... whose 16-byte lanes are the lean kernel's
+};
+constexpr int64_t NARROW_WAVES_RESIDENT = 3072; // three per SIMD
+bool burst_beats(const BurstRivals& r, int64_t groups, int64_t avg_len, int64_t pitch, int32_t max_bits) { // more than 4096 workgroups
+  if (groups > 16384) return false;
+  if (groups <= 5120 && avg_len >= (r.single ? 8 : 12)) return true;
+  if (avg_len < (groups <= 8192 ? 8 : 24)) return false;
+  if (r.max_vb <= 4) return r.narrow_waves > NARROW_WAVES_RESIDENT;
+  if (max_bits == 2) return true;
+  if (r.waves < narrow_below_waves())
+    return r.narrow_waves > NARROW_WAVES_RESIDENT || r.types_differ ||
+        (r.single && groups <= 6144 && avg_len >= 24 && avg_len * pitch <= 4096);
+  return r.trailer && (!r.lean || (groups > 8192 && avg_len >= 40));
+}
 // 1 / 4: every launch it can take goes to the burst kernel with that many waves per bag, 0: none does,
 // -1: by the rule (tests: fbgemm_amd_set_burst).
 int g_burst_override = -1;
-Burst plan_burst(int64_t bags, int32_t T, int32_t max_D, int32_t max_bits, int64_t lookups) {
+// `bags`: of all tables; rivals(): a BurstRivals, asked for only where it decides.
+template <typename Rivals>
+Burst plan_burst(int64_t bags, int32_t T, int32_t max_D, int32_t max_bits, int64_t lookups, Rivals rivals) {
   Burst b;
   const int64_t windows = ((int64_t)max_D + BURST_COLS - 1) / BURST_COLS;
   if (g_burst_override == 0 || narrow_below_waves() == 0 || bags <= 0 || T > 65535 || windows > 65535 ||
       (g_burst_override < 0 && lookups >= SORT_MIN_LOOKUPS)) // those launches order their bags
     return b;
   const int64_t groups = bags * windows, avg_len = lookups / bags;
-  if (g_burst_override > 0)
-    b.waves = g_burst_override;
-  else if (groups <= 4096 || (windows == 1 && (groups <= 8192 ? avg_len >= 8 : groups <= 16384 && avg_len >= 24)))
-    b.waves = (groups <= 1024 && avg_len >= 16) || (groups <= 2048 && avg_len >= 64) ? 4 : 1;
   // bytes of a staged row, of the widest type and table of the launch
   const int64_t pitch = burst_pitch(max_D, max_bits);
+  if (g_burst_override > 0)
+    b.waves = g_burst_override;
+  else if (groups <= 4096 || (windows == 1 && groups <= 16384 && burst_beats(rivals(), groups, avg_len, pitch, max_bits)))
+    b.waves = (groups <= 1024 && avg_len >= 16) || (groups <= 2048 && avg_len >= 64) ? 4 : 1;
   b.lds_bytes = b.waves == 4 ? 32768
       : groups <= 2048       ? 16384
       : groups > 4096 && 8 * pitch <= 4096 && std::min<int64_t>(avg_len, 64) * pitch <= 8192 ? 4096 : 8192;
@@ -716,7 +758,19 @@ int spmdm_launch_impl(
   // 4- and 8-bit rows only: every other row type is summed the reference's way in either mode,
   // in one piece.
   int K = 1;
-  const Burst burst = plan_burst(output_size, 1, d.D, bits, index_size);
+  const Burst burst = plan_burst(output_size, 1, d.D, bits, index_size, [&] {
+    BurstRivals r;
+    TableDesc narrow = d;
+    plan_lanes(narrow, (uintptr_t)d_input, out_stride, has_sb, room, false, true);
+    const int wide_bags = bags_per_wave(d.lanes, d.packed), narrow_bags = bags_per_wave(narrow.lanes, narrow.packed);
+    r.waves = (output_size + wide_bags - 1) / wide_bags;
+    r.narrow_waves = (output_size + narrow_bags - 1) / narrow_bags;
+    r.max_vb = d.vb;
+    r.single = true;
+    r.trailer = has_sb && cfg->scale_bias_last;
+    r.lean = lean_shape(d);
+    return r;
+  });
   if (!noalloc && cfg->accumulate == FBGEMM_AMD_ACC_FAST && !cfg->is_weight_positional && output_size * 32 <= 0x7fffffffLL &&
       (ty == ST_INT4 || ty == ST_INT8)) {
     const int G16 = bags_per_wave(d.lanes, d.packed);
@@ -1399,7 +1453,17 @@ int tbe_forward_impl(
   // (Only when every table has rows the tolerance-grade arithmetic applies to: fp16 / fp32 / 2-bit
   // / odd-shaped tables are summed the reference's way in either mode, and a bag cut into
   // segments is not.)
-  const Burst burst = plan_burst((int64_t)plan->T * B, plan->T, plan->max_D, plan->max_bits, indices_numel);
+  const Burst burst = plan_burst((int64_t)plan->T * B, plan->T, plan->max_D, plan->max_bits, indices_numel, [&] {
+    BurstRivals r;
+    for (int t = 0; t < plan->T; ++t) {
+      const TableDesc &d = plan->tables[t], &narrow = plan->tables_narrow[t];
+      r.waves += (B + d.bags - 1) / d.bags;
+      r.narrow_waves += (B + narrow.bags - 1) / narrow.bags;
+      r.max_vb = std::max(r.max_vb, d.vb);
+      r.types_differ = r.types_differ || d.ty != plan->tables[0].ty;
+    }
+    return r;
+  });
   bool all_fast_rows = true;
   for (const TableDesc& d : plan->tables) all_fast_rows = all_fast_rows && (d.ty == ST_INT4 || d.ty == ST_INT8);
   if (allow_split && plan->accumulate == FBGEMM_AMD_ACC_FAST && all_fast_rows && (int64_t)B * 32 <= 0x7fffffffLL) {
