@@ -291,6 +291,7 @@ int wide4_mode() {
 // LDS: large launches want many workgroups resident, so they stage in 4 KB what takes at most two
 // stagings there (8-bit, 100 wide, 8192 x 60: 35.6 -> 31.2), in 8 KB otherwise (fp16, 200 wide, 16384 x 25:
 // 47.5 against 49.2); small ones stage as much as they can.
+constexpr int BURST_FOUR_WAVES_LDS = 32768;
 struct Burst {
   int waves = 0; // 0: another kernel takes the launch
   int lds_bytes = 0;
@@ -335,7 +336,7 @@ Burst plan_burst(int64_t bags, int32_t T, int32_t max_D, int32_t max_bits, int64
     b.waves = g_burst_override;
   else if (groups <= 4096 || (windows == 1 && groups <= 16384 && burst_beats(rivals(), groups, avg_len, pitch, max_bits)))
     b.waves = (groups <= 1024 && avg_len >= 16) || (groups <= 2048 && avg_len >= 64) ? 4 : 1;
-  b.lds_bytes = b.waves == 4 ? 32768
+  b.lds_bytes = b.waves == 4 ? BURST_FOUR_WAVES_LDS
       : groups <= 2048       ? 16384
       : groups > 4096 && 8 * pitch <= 4096 && std::min<int64_t>(avg_len, 64) * pitch <= 8192 ? 4096 : 8192;
   return b;
@@ -344,6 +345,23 @@ Burst plan_burst(int64_t bags, int32_t T, int32_t max_D, int32_t max_bits, int64
 // (tolerance-grade mode): 1000 bags x 100 of a 4-bit table 23.4 us in segments, 13.7 us whole; x 400
 // 46 and 38 us, 10 x 2000 42 and 111 us.
 constexpr int64_t SPLIT_MIN_LEN_OVER_BURST = 256;
+// Segments also spread a bag that is much longer than the others. Of such bags, one wave adds up a row
+// in 75 ns, four waves in 29, a segmented bag's waves together in 25 to 50: from this length on bags that
+// would be cut get four waves each. 4000 x 100 and x 200 of a 4-bit table with one bag ten times as long,
+// us in segments, with one wave and with four: 49.9, 81.6, 33.9 and 82.3, 156, 64.3 (bags of one length:
+// 34.2, 24.8, 30.2 and 48.6, 37.6, 44.2; 4000 x 60: 26.0, 16.9, 24.2, and 45.4, 51.2, 24.6 with the long
+// one). What remains: 1000 x 200 with a bag of 2000 entries 43.5 in segments, 61.1 with four waves.
+constexpr int64_t FOUR_WAVES_MIN_LEN_OVER_SPLIT = 96;
+// Bags that would be cut into K > 1 segments, where the burst kernel would take the launch: the number
+// of segments that remains.
+int split_over_burst(int K, int64_t avg_len, Burst* burst) {
+  if (!burst->waves || K <= 1 || avg_len >= SPLIT_MIN_LEN_OVER_BURST) return K;
+  if (avg_len >= FOUR_WAVES_MIN_LEN_OVER_SPLIT && g_burst_override < 0) {
+    burst->waves = 4;
+    burst->lds_bytes = BURST_FOUR_WAVES_LDS;
+  }
+  return 1;
+}
 
 struct DeviceScratch {
   Status* unread = nullptr;   // where calls without a status block record what nobody reads
@@ -758,7 +776,7 @@ int spmdm_launch_impl(
   // 4- and 8-bit rows only: every other row type is summed the reference's way in either mode,
   // in one piece.
   int K = 1;
-  const Burst burst = plan_burst(output_size, 1, d.D, bits, index_size, [&] {
+  Burst burst = plan_burst(output_size, 1, d.D, bits, index_size, [&] {
     BurstRivals r;
     TableDesc narrow = d;
     plan_lanes(narrow, (uintptr_t)d_input, out_stride, has_sb, room, false, true);
@@ -774,8 +792,7 @@ int spmdm_launch_impl(
   if (!noalloc && cfg->accumulate == FBGEMM_AMD_ACC_FAST && !cfg->is_weight_positional && output_size * 32 <= 0x7fffffffLL &&
       (ty == ST_INT4 || ty == ST_INT8)) {
     const int G16 = bags_per_wave(d.lanes, d.packed);
-    K = split_factor((output_size + G16 - 1) / G16, index_size / output_size);
-    if (burst.waves && index_size / output_size < SPLIT_MIN_LEN_OVER_BURST) K = 1;
+    K = split_over_burst(split_factor((output_size + G16 - 1) / G16, index_size / output_size), index_size / output_size, &burst);
   }
   const int64_t pooled_bags = output_size * K;       // what the lookup kernel sees as bags
   const int64_t pooled_stride = K > 1 ? D : out_stride; // segments' sums are rows of D floats
@@ -1453,7 +1470,7 @@ int tbe_forward_impl(
   // (Only when every table has rows the tolerance-grade arithmetic applies to: fp16 / fp32 / 2-bit
   // / odd-shaped tables are summed the reference's way in either mode, and a bag cut into
   // segments is not.)
-  const Burst burst = plan_burst((int64_t)plan->T * B, plan->T, plan->max_D, plan->max_bits, indices_numel, [&] {
+  Burst burst = plan_burst((int64_t)plan->T * B, plan->T, plan->max_D, plan->max_bits, indices_numel, [&] {
     BurstRivals r;
     for (int t = 0; t < plan->T; ++t) {
       const TableDesc &d = plan->tables[t], &narrow = plan->tables_narrow[t];
@@ -1469,8 +1486,8 @@ int tbe_forward_impl(
   if (allow_split && plan->accumulate == FBGEMM_AMD_ACC_FAST && all_fast_rows && (int64_t)B * 32 <= 0x7fffffffLL) {
     int64_t wide_waves = 0;
     for (const TableDesc& d : plan->tables) wide_waves += (B + d.bags - 1) / d.bags;
-    int K = split_factor(wide_waves, indices_numel / ((int64_t)plan->T * B));
-    if (burst.waves && indices_numel / ((int64_t)plan->T * B) < SPLIT_MIN_LEN_OVER_BURST) K = 1;
+    const int64_t avg_len = indices_numel / ((int64_t)plan->T * B);
+    const int K = split_over_burst(split_factor(wide_waves, avg_len), avg_len, &burst);
     if (K > 1) {
       if (int rc = shared.begin(plan, stream)) return rc;
       hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;

@@ -121,3 +121,22 @@ def test_both_sides_of_the_line(ops, oracle, bags):
     S.check_case(ops, oracle, ty=INT4, D=D, table=table, idx=idx, off_or_len=off, w=None, normalize=False, out_ty=FP32,
                  positional=False, use_offsets=True, output_stride=-1, input_stride=-1, sbl=True, data_size=rows,
                  output_size=bags, what=f"{bags} bags")
+
+
+@pytest.mark.parametrize("avg", [95, 96, 255])
+def test_whole_bags_in_the_tolerance_grade_mode(ops, avg):
+    """Bags that the burst kernel takes whole in place of segments, on both sides of the length from which
+    they get four waves, one bag much longer than the others: exact, so the bits of the exact mode."""
+    rng = np.random.default_rng(avg)
+    D, rows, bags = 64, 500, 600
+    table, _ = H.make_table(rng, INT4, rows, D, True)
+    lens = np.full(bags, avg - 10)
+    lens[17] += 10 * bags
+    off = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+    cu = lambda a: torch.from_numpy(np.ascontiguousarray(a)).cuda()
+    idx = cu(rng.integers(0, rows, size=int(off[-1])).astype(np.int32))
+    kern = ops.generate_embedding_spmdm_nbit(4, D, False, False)
+    outs = [torch.empty(bags, D, device="cuda") for _ in range(2)]
+    for out, mode in zip(outs, (ops.ACC_EXACT, ops.ACC_FAST)):
+        assert kern(bags, len(idx), rows, cu(table), idx, cu(off), None, out, accumulate=mode)
+    H.assert_same_bits(outs[1].cpu().numpy(), outs[0].cpu().numpy(), f"{avg} entries per bag")
