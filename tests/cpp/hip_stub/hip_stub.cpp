@@ -164,7 +164,36 @@ hipStream_t hip_stub_stream(int id) {
 // ---- launchers: nothing runs; the words the host reads back are written ---------------------
 namespace fbgemm_amd {
 #define LAUNCHED() (++g_launches, hipSuccess)
+// What a lookup kernel would read of every row: all of its data, on the boundaries the loads need, and
+// nothing behind what belongs to the row (of a single table, whose last row may end its buffer with
+// its last element, only the elements and the scale and bias).
+static bool reads_stay_in_the_row(const TableDesc& d, bool single, uintptr_t base) {
+  const bool quant = d.ty == ST_INT8 || d.ty == ST_INT4 || d.ty == ST_INT2;
+  int64_t end = d.row_stride;
+  if (single) {
+    end = d.data_off + d.data_bytes;
+    if (quant && d.sb_off + (d.sb_fp32 ? 8 : 4) > end) end = d.sb_off + (d.sb_fp32 ? 8 : 4);
+  }
+  if (d.inline_hdr) { // whole aligned 16-byte pieces that the row has a part of: they cross no page
+    if ((base + d.weights_offset) % 16 != 0 || d.row_stride % 16 != 0) return false;
+    end = (end + 15) / 16 * 16;
+  }
+  const int64_t first = d.inline_hdr ? 0 : d.data_off, bytes = d.inline_hdr ? d.data_bytes + d.data_off : d.data_bytes;
+  const int64_t chunks = (bytes + d.vb - 1) / d.vb, last = d.inline_hdr ? (chunks - 1) * d.vb : d.last_chunk;
+  if (d.vb < 1 || d.vb > 16 || (int64_t)d.lanes * d.chunks * d.passes < chunks) return false;
+  if (d.vb >= 4 && (base + d.weights_offset + first + last) % 4 != 0) return false;
+  if (d.vb >= 4 && d.row_stride % 4 != 0) return false;
+  int64_t covered = 0;
+  for (int64_t k = 0; k < chunks; ++k) {
+    const int64_t at = k * d.vb < last ? k * d.vb : last;
+    if (at < 0 || at > covered || first + at + d.vb > end) return false;
+    covered = at + d.vb;
+  }
+  return covered >= bytes;
+}
 hipError_t launch_lookup(const LookupArgs& a, bool, hipStream_t) {
+  for (int t = 0; t < (a.tables ? a.T : 1); ++t)
+    if (!reads_stay_in_the_row(a.tables ? a.tables[t] : a.single, !a.tables, a.tables ? 0 : (uintptr_t)a.weights[0])) return hipErrorInvalidValue;
   // what a kernel would dereference must still be alive: touch the first bytes of each list
   if (a.work) (void)*(volatile const int32_t*)&a.work[0].table;
   if (a.xcd_start) (void)*(volatile const int64_t*)&a.xcd_start[8];

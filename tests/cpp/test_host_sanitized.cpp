@@ -373,6 +373,59 @@ void refused_calls_leave_the_own_status_alone() {
   hipFree(out);
 }
 
+// Every width, type, row layout, row stride and base alignment, in launches that take 16-byte lanes and
+// such that take 4-byte ones: the loads of a row stay inside it (the stand-in's launches check that).
+void row_reads_stay_in_the_row() {
+  void *table, *idx, *off, *out;
+  CHECK(hipMalloc(&table, 1 << 20) == hipSuccess);
+  CHECK(hipMalloc(&idx, 64) == hipSuccess);
+  CHECK(hipMalloc(&off, 64) == hipSuccess);
+  CHECK(hipMalloc(&out, 64) == hipSuccess);
+  fbgemm_amd_set_burst(0);
+  for (int32_t lean : {0, 1}) {
+    fbgemm_amd_set_lean(lean);
+    for (int32_t ty : {0, 1, 2, 3, 4, 5})
+      for (int32_t D = 1; D <= 1100; D += D < 300 ? 1 : 7)
+        for (int32_t trailer : {0, 1})
+          for (int32_t pad : {0, 1, 2, 4, 12})
+            for (int32_t at : {0, 1, 2, 4}) {
+              const int32_t elem = ty == 0 ? 4 : ty == 1 || ty == 5 ? 2 : 1;
+              if (at % elem) continue;
+              const int32_t bits = ty == 0 ? 32 : ty == 1 || ty == 5 ? 16 : ty == 2 ? 8 : ty == 3 ? 4 : 2;
+              const int32_t row = elem > 1 ? D : (D * bits + 7) / 8 + (ty == 2 && trailer ? 8 : 4);
+              fbgemm_amd_spmdm_config c = single_table(ty, D, 1, FBGEMM_AMD_ACC_EXACT);
+              c.scale_bias_last = trailer;
+              c.input_stride = pad ? row + pad : -1;
+              for (int64_t bags : {100, 100000})
+                CHECK(fbgemm_amd_spmdm_launch(&c, bags, 10, 10, (char*)table + at, idx, off, nullptr, out, nullptr, out, nullptr) == 0);
+            }
+  }
+  fbgemm_amd_set_lean(0); // all tables in one launch of the general kernel
+  for (int32_t align : {1, 4, 16}) {
+    std::vector<int64_t> wo;
+    std::vector<uint8_t> tys;
+    std::vector<int32_t> Ds{0};
+    int64_t bytes = 0;
+    for (uint8_t ty : {0, 1, 2, 3, 4})
+      for (int32_t D = 4; D <= 600; D += 4) {
+        wo.push_back(bytes);
+        tys.push_back(ty);
+        Ds.push_back(Ds.back() + D);
+        bytes += (fbgemm_amd_padded_row_size_in_bytes(D, ty, align, 4) * 10 + 127) / 128 * 128;
+      }
+    fbgemm_amd_tbe_plan* plan = nullptr;
+    const int32_t T = (int32_t)tys.size();
+    CHECK(fbgemm_amd_tbe_plan_create(&plan, T, wo.data(), tys.data(), Ds.data(), nullptr, bytes, 0, align) == 0);
+    for (int64_t B : {1, 2000})
+      for (int64_t n : {T * B, 40 * T * B}) // bags end to end in the wave, too
+        CHECK(fbgemm_amd_tbe_forward(plan, table, nullptr, idx, off, 64, n, T * B + 1, 0, nullptr, 0, out, out, nullptr) == 0);
+    fbgemm_amd_tbe_plan_destroy(plan);
+  }
+  fbgemm_amd_set_lean(-1);
+  fbgemm_amd_set_burst(-1);
+  for (void* p : {table, idx, off, out}) hipFree(p);
+}
+
 // The burst kernel goes over a bag by whole 8s of staged rows: a launch whose rows do not fit that many
 // times would never end, and is refused on the host. The rule's own sizes fit, whatever it chooses.
 void burst_launches_fit() {
@@ -484,6 +537,7 @@ int main() {
   checks_in_flight_have_a_counter_each();
   refused_calls_leave_the_own_status_alone();
   burst_launches_fit();
+  row_reads_stay_in_the_row();
   checks_share_no_scratch();
   allocation_failures_in_a_first_forward();
   printf("launches %ld, device allocations %ld\n", hip_stub_launches(), hip_stub_total_allocations());
