@@ -54,3 +54,68 @@ def test_dequantize(ops, out_ty, dtype, bits_dtype, np_bits, bits, sb_float, lay
             want = oracle.dequantize_rowwise(q, cols, bits, sb_float, layout, out_ty).view(np_bits)
             got = ops.dequantize_rowwise(torch.from_numpy(q).cuda(), cols, bits, sb_float, layout, dtype)
             assert (got.cpu().view(bits_dtype).numpy() == want).all(), (cols, rows)
+
+
+def special_rows(cols, dtype):
+    """Rows whose extremes or elements are not ordinary numbers, and rows of one value."""
+    rng = np.random.default_rng(cols)
+    rows = rng.normal(size=(24, cols)).astype(dtype)
+    inf, nan, big = np.inf, np.nan, np.finfo(dtype).max
+    for r, (at, v) in enumerate([(0, nan), (cols // 2, nan), (cols - 1, nan), (0, inf), (cols - 1, inf), (0, -inf), (cols // 2, -inf),
+                                 (slice(None), nan), (slice(None), inf), (slice(None), -inf), (slice(None), 0.0), (slice(None), -0.0),
+                                 (slice(None), 1.25), (slice(None), -3.0), (0, big), (cols - 1, -big)]):
+        rows[r, at] = v
+    rows[16, 0], rows[16, -1] = inf, -inf
+    rows[17, 0], rows[17, -1] = big, -big
+    rows[18, 1], rows[18, -1] = nan, inf
+    rows[19] *= dtype(np.finfo(dtype).tiny)          # subnormal ranges
+    rows[20] = np.finfo(dtype).smallest_subnormal
+    rows[21, :] = 0.0
+    rows[21, 3] = nan                                # a zero extreme: the search with positions
+    rows[22] = np.abs(rows[22])
+    rows[22, ::2] = -0.0
+    return rows
+
+
+@pytest.mark.parametrize("bits,sb_float,layout", FORMATS)
+@pytest.mark.parametrize("dtype", [np.float32, np.float16])
+def test_quantize_special_values(ops, dtype, bits, sb_float, layout):
+    """The bytes of the general form, which takes the same rows one element off the 16-byte grid; those of
+    the oracle where a row and its range are finite."""
+    for cols in (8, 40, 128, 512):
+        x = special_rows(cols, dtype)
+        d = torch.from_numpy(x).cuda()
+        off = torch.empty(x.size + 1, dtype=d.dtype, device="cuda")[1:].view(x.shape)
+        off.copy_(d)
+        got = ops.quantize_rowwise(d, bits, sb_float, layout).cpu().numpy()
+        assert (got == ops.quantize_rowwise(off, bits, sb_float, layout).cpu().numpy()).all(), cols
+        with np.errstate(over="ignore", invalid="ignore"):
+            finite = np.isfinite(x).all(1) & np.isfinite(x.astype(np.float32).max(1) - x.astype(np.float32).min(1))
+            if not sb_float:  # the pair is stored in fp16
+                finite &= np.isfinite(x.astype(np.float16)).all(1) & (x.astype(np.float32).max(1) - x.astype(np.float32).min(1) < 6e4)
+        assert finite.sum() >= 6
+        assert (got[finite] == oracle.quantize_rowwise(x[finite], bits, sb_float, layout)).all(), cols
+
+
+@pytest.mark.parametrize("bits,sb_float,layout", FORMATS)
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+def test_dequantize_special_values(ops, dtype, bits, sb_float, layout):
+    """Scales and biases that are infinite, no numbers, zero or subnormal: the bits of the general form, which
+    takes the same rows off the dword grid."""
+    pair_type = np.float32 if sb_float and not layout else np.float16
+    special = np.array([np.inf, -np.inf, np.nan, 0.0, -0.0, np.finfo(pair_type).max, np.finfo(pair_type).smallest_subnormal, 0.5], pair_type)
+    rows = len(special) ** 2
+    for cols in (8, 40, 128):
+        rng = np.random.default_rng(cols)
+        data = (cols * bits + 7) // 8
+        stride = oracle.quantized_row_bytes(cols, bits, sb_float, layout)
+        q = rng.integers(0, 256, size=(rows, stride), dtype=np.uint8)
+        at = 0 if layout else data
+        pair = np.ascontiguousarray(np.stack(np.meshgrid(special, special), -1).reshape(rows, 2))
+        q[:, at:at + pair.view(np.uint8).shape[1]] = pair.view(np.uint8)
+        off = torch.empty(rows, stride + 1, dtype=torch.uint8, device="cuda")
+        off[:, :stride] = torch.from_numpy(q).cuda()
+        got = ops.dequantize_rowwise(torch.from_numpy(q).cuda(), cols, bits, sb_float, layout, dtype)
+        want = ops.dequantize_rowwise(off, cols, bits, sb_float, layout, dtype)
+        as_int = torch.int32 if dtype == torch.float32 else torch.int16
+        assert torch.equal(got.view(as_int), want.view(as_int)), cols
