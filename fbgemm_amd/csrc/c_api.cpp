@@ -285,7 +285,8 @@ int wide4_mode() {
 // * Below, the others take 4-byte lanes, and lose once their waves exceed the 3072 that the device
 //   holds; up to there they win. (Rows that have only lanes of 4 bytes and less: the same line.)
 //   Launches of several types hold fewer of those waves, 2-bit rows cost those lanes the most.
-//   Single tables of bags that one staging takes: 5200 x 25 .83 to .93.
+//   Single tables of bags that one staging takes: 5200 x 25 .83 to .93, x 12 .90 to .95 where rows are
+//   not the smallest.
 // Four waves per bag pay while all such workgroups are resident together (four per compute unit:
 // 1024; 1024 bags x 100: 22.0 -> 13.9) and, for long bags, in two rounds of them (2048 x 100: 24.9 -> 21.9).
 // LDS: large launches want many workgroups resident, so they stage in 4 KB what takes at most two
@@ -315,7 +316,7 @@ bool burst_beats(const BurstRivals& r, int64_t groups, int64_t avg_len, int64_t 
   if (max_bits == 2) return true;
   if (r.waves < narrow_below_waves())
     return r.narrow_waves > NARROW_WAVES_RESIDENT || r.types_differ ||
-        (r.single && groups <= 6144 && avg_len >= 24 && avg_len * pitch <= 4096);
+        (r.single && groups <= 6144 && avg_len >= (pitch >= 64 ? 10 : 24) && avg_len * pitch <= 4096);
   return r.trailer && (!r.lean || (groups > 8192 && avg_len >= 40));
 }
 // 1 / 4: every launch it can take goes to the burst kernel with that many waves per bag, 0: none does,
