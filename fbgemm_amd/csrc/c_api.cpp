@@ -1748,9 +1748,10 @@ int tbe_forward_impl(
   a.status = (Status*)d_status;
   a.fp8_shift = plan->fp8_shift;
   a.fp8_mult = plan->fp8_mult;
-  // The burst kernel needs none of the work set. The set is there all the same: whether a forward may
-  // be captured must depend on its batch size alone, and a later one of the same size may have shorter
-  // or longer bags, or the 8-bit output, and take the other kernels.
+  // The burst kernel needs none of the work set. The set is there all the same, so that whether a forward
+  // may be captured depends on nothing the burst rule looks at: a later one of the same batch size may
+  // have shorter or longer bags, or the 8-bit output, and take the other kernels. (The set does depend
+  // on the lane shapes, which the average bag length enters: see the key above.)
   if (burst.waves && !d_q8_out) {
     a.tables = plan->d_tables;
     HIP_TRY(launch_lookup_burst(a, index_bits == 64, plan->max_D, plan->max_bits, burst.waves, burst.lds_bytes, stream));

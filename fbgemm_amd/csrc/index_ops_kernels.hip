@@ -225,7 +225,7 @@ __global__ __launch_bounds__(256) void bounds_check_bags_kernel(
 // makes the running maximum of their offsets, which decides what the bags are, and then walks
 // their indices as one range, 8 loads in flight per thread: the mapping is a random gather, bound
 // by round trips unless many of them overlap.
-//   64 tables x 32 bags x 30 entries: 16 us of copies and check -> 8.8 us (its chain of five round
+//   64 tables x 32 bags x 30 entries: 16 us of copies and check -> 9.5 us (its chain of five round
 //   trips). 32 pruned tables x 4096 bags x 27: 121 us of copies, check, mapping (64.6) and check ->
 //   78 us: the random 4-byte reads of 256 MB of mappings, a line each, 6 TB/s of lines.
 // The warning counter is what the last of the separate checks leaves there: with a mapping the

@@ -12,8 +12,8 @@
 // WAVES = 1: a wave per bag, a lane owns 4 columns (64 lanes * 4 = the 256 columns), up to 64 rows
 // at a time in 4, 8 or 16 KB of LDS. Large launches are bound by how many workgroups are resident, so
 // this form keeps 4 loads per thread and adds 4 rows per turn, which fits 5 waves per SIMD without
-// spills (8 and 8 need 128 registers, 4 waves: 5000 bags x 25 of a 4-bit table 16.0 us, so 14.6; 6 and
-// 8 waves per SIMD spill: 16.8 and 16.0). WAVES = 4: four waves per bag, a lane
+// spills: 5000 bags x 25 of a 4-bit table in 14.6 us. With 8 loads and 8 rows it needs 128 registers, 4
+// waves per SIMD: 16.0; held to 6 and to 8 waves per SIMD it spills: 16.8 and 16.0. WAVES = 4: four waves per bag, a lane
 // owns one column, up to 256 rows at a time in 32 KB: for fewer bags than compute units have room
 // for, whose rows one wave would need many loads each for, and whose summing loop (a dependent add
 // and fma per row and column) is the longest part left. Which of them, and from where on the other
