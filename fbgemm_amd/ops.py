@@ -34,6 +34,8 @@ def _stream():
 
 
 def _ptr(t):
+    """The address of a tensor that the caller holds until the call it is for has been made: the memory of
+    a temporary goes to the next one."""
     return None if t is None else C.c_void_p(t.data_ptr())
 
 
@@ -366,8 +368,9 @@ def int_nbit_split_embedding_codegen_lookup_function(
             return out.zero_()
         own = status is None
         st = _OwnStatus() if own else status
+        indices, offsets = indices.contiguous(), offsets.contiguous()
         check(_lib.lib().fbgemm_amd_tbe_forward_nobag(
-            plan.handle, _ptr(dev_weights), _ptr(uvm_weights), _ptr(indices.contiguous()), _ptr(offsets.contiguous()),
+            plan.handle, _ptr(dev_weights), _ptr(uvm_weights), _ptr(indices), _ptr(offsets),
             _bits(indices), indices.numel(), offsets.numel(), D, output_dtype, _ptr(out), st.ptr, _stream()))
         if own:
             bits, pos = st.read()
@@ -378,8 +381,9 @@ def int_nbit_split_embedding_codegen_lookup_function(
         raise NotImplementedError(f"output_dtype {output_dtype} is not on this path")
     if indice_weights is not None and indice_weights.numel() == 0:
         indice_weights = None
-    if indice_weights is not None and indice_weights.dtype != torch.float32:
-        indice_weights = indice_weights.float()  # embedding_forward_quantized_host.cpp:345
+    if indice_weights is not None:
+        indice_weights = indice_weights.float().contiguous()  # embedding_forward_quantized_host.cpp:345
+    indices, offsets = indices.contiguous(), offsets.contiguous()
     if row_alignment is None:
         row_alignment = 16  # the GPU operator's default (embedding_forward_quantized_host.cpp:310)
     if plan is None:
@@ -420,8 +424,8 @@ def int_nbit_split_embedding_codegen_lookup_function(
             else:
                 plan.set_index_remappings(index_remappings, index_remappings_offsets)
     check(_lib.lib().fbgemm_amd_tbe_forward_pruned(
-        plan.handle, _ptr(dev_weights), _ptr(uvm_weights), _ptr(indices.contiguous()),
-        _ptr(offsets.contiguous()), _bits(indices), indices.numel(), offsets.numel(), pooling_mode,
+        plan.handle, _ptr(dev_weights), _ptr(uvm_weights), _ptr(indices),
+        _ptr(offsets), _bits(indices), indices.numel(), offsets.numel(), pooling_mode,
         _ptr(indice_weights), output_dtype, _ptr(out), _ptr(index_remappings),
         32 if index_remappings is None else _bits(index_remappings), _ptr(ro), 0 if ro is None else ro.numel(),
         st.ptr, _stream()))
@@ -460,8 +464,9 @@ def pruned_array_lookup(indices, offsets, index_remappings, index_remappings_off
     T = index_remappings_offsets.numel() - 1
     dense = torch.empty_like(indices)
     ro = index_remappings_offsets.to(torch.int64).contiguous()
+    indices, offsets, index_remappings = indices.contiguous(), offsets.contiguous(), index_remappings.contiguous()
     check(_lib.lib().fbgemm_amd_pruned_array_lookup(
-        _ptr(indices.contiguous()), _ptr(offsets.contiguous()), _bits(indices), offsets.numel(),
+        _ptr(indices), _ptr(offsets), _bits(indices), offsets.numel(),
         _ptr(index_remappings), _bits(index_remappings), _ptr(ro), T, _ptr(dense), _stream()))
     return dense
 
@@ -478,8 +483,9 @@ def pruned_array_lookup_from_row_idx(update_row_indices, update_table_indices, i
     T = index_remappings_offsets.numel() - 1
     dense = torch.empty_like(update_row_indices)
     ro = index_remappings_offsets.to(torch.int64).contiguous()
+    rows, tables, index_remappings = update_row_indices.contiguous(), update_table_indices.contiguous(), index_remappings.contiguous()
     check(_lib.lib().fbgemm_amd_pruned_array_lookup_from_row_idx(
-        _ptr(update_row_indices.contiguous()), _bits(update_row_indices), _ptr(update_table_indices.contiguous()),
+        _ptr(rows), _bits(update_row_indices), _ptr(tables),
         update_row_indices.numel(), _ptr(index_remappings), _bits(index_remappings), _ptr(ro), T, _ptr(dense),
         _stream()))
     return dense
@@ -506,11 +512,12 @@ def emb_inplace_update(dev_weights, uvm_weights, weights_placements, weights_off
                          row_alignment)
     own = status is None
     st = _OwnStatus() if own else status
-    update_weights = update_weights.contiguous()
+    update_weights, update_offsets = update_weights.contiguous(), update_offsets.contiguous()
+    update_table_indices, update_row_indices = update_table_indices.contiguous(), update_row_indices.contiguous()
     check(_lib.lib().fbgemm_amd_tbe_inplace_update(
         plan.handle, _ptr(dev_weights), _ptr(uvm_weights), _ptr(update_weights), update_weights.numel(),
-        _ptr(update_table_indices.contiguous()), _ptr(update_row_indices.contiguous()), _bits(update_row_indices),
-        _ptr(update_offsets.contiguous()), n, st.ptr, _stream()))
+        _ptr(update_table_indices), _ptr(update_row_indices), _bits(update_row_indices),
+        _ptr(update_offsets), n, st.ptr, _stream()))
     if own:
         bits, pos = st.read()
         if bits & ERR_INDEX_OUT_OF_RANGE:
@@ -609,9 +616,10 @@ def pruned_hashmap_lookup(indices, offsets, hash_table, hash_table_offsets):
         raise RuntimeError("pruned_hashmap_lookup needs B > 0")  # TORCH_CHECK(B > 0), :537
     dense = torch.empty_like(indices)
     hto = hash_table_offsets.to(torch.int64).contiguous()
+    indices, offsets, hash_table = indices.contiguous(), offsets.contiguous(), hash_table.contiguous()
     check(_lib.lib().fbgemm_amd_pruned_hashmap_lookup(
-        _ptr(indices.contiguous()), _ptr(offsets.contiguous()), _bits(indices), offsets.numel(),
-        _ptr(hash_table.contiguous()), _bits(hash_table), _ptr(hto), T, _ptr(dense), _stream()))
+        _ptr(indices), _ptr(offsets), _bits(indices), offsets.numel(),
+        _ptr(hash_table), _bits(hash_table), _ptr(hto), T, _ptr(dense), _stream()))
     return dense
 
 
@@ -706,10 +714,11 @@ def compressed_indices_remap(indices, compressed_indices_mapping, offsets, weigh
     out_indices = torch.empty_like(indices)
     out_offsets = torch.empty_like(offsets)
     out_weights = None if weights is None else torch.empty_like(weights)
+    weights = None if weights is None else weights.contiguous()
     st = _OwnStatus()
     check(_lib.lib().fbgemm_amd_compressed_indices_remap(
         offsets.numel(), _ptr(indices), _bits(indices), _ptr(mapping), mapping.numel(), _ptr(offsets),
-        _ptr(None if weights is None else weights.contiguous()), _ptr(out_indices), _ptr(out_offsets), _ptr(out_weights),
+        _ptr(weights), _ptr(out_indices), _ptr(out_offsets), _ptr(out_weights),
         st.ptr, _stream()))
     bits, pos = st.read()
     if bits:
