@@ -263,7 +263,15 @@ int wide4_mode() {
 //   4-bit, 128 wide     47.7 -> 10.8    17.3 -> 9.4
 //   8-bit, 100 wide     47.7 -> 11.2    17.4 -> 9.5
 //   8-bit, 512 wide     52.0 -> 13.6    18.4 -> 10.9
-// Beyond, it depends on what the other kernels have against it. Burst time over theirs, for bags of 25
+// and rows of several windows in 1024 to 4096 workgroups, one launch behind the other (1 entry per bag: a
+// launch is all there is):
+//                       2048 x 1        2048 x 10       2048 x 60       1024 x 200
+//   4-bit, 260 wide     10.9 -> 7.8     15.4 -> 9.6     44.5 -> 28.9    123 -> 38.9
+//   4-bit, 512 wide      7.8 -> 7.9      9.9 -> 7.8     21.5 -> 17.9    49.6 -> 31.7
+//   8-bit, 512 wide      9.9 -> 7.8     13.9 -> 8.1     34.6 -> 18.3    85.9 -> 36.6
+//   fp16, 512 wide      12.9 -> 7.9     19.3 -> 9.6     54.8 -> 24.4    145 -> 43.1
+// (table batches of 2, 8 and 40 tables of mixed widths, whose widest decides the count: .14 to 1.0 of the
+// other kernels' time over 2 to 100 entries per bag). Beyond, it depends on what the other kernels have against it. Burst time over theirs, for bags of 25
 // and 60 entries and tables of 200 000 rows in a table-batched launch (8 tables):
 //                       4608 bags    6144         8192         12288        16384
 //   4-bit, 64 wide      .89  .92    1.04 1.11    1.12 1.15    1.24 1.24    1.41 1.33
