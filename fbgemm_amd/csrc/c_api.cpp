@@ -1980,6 +1980,8 @@ int fbgemm_amd_tbe_forward_nobag(
   if (!d_offsets || !d_output || !d_indices) return fail(FBGEMM_AMD_E_ARG, "null data pointer");
   if (plan->has_fp8 && plan->fp8_shift == 0)
     return fail(FBGEMM_AMD_E_ARG, "the plan holds FP8 tables: set their exponent bits and bias first (fbgemm_amd_tbe_plan_set_fp8)");
+  bool aligned = (uintptr_t)d_dev_weights % 16 == 0 && (uintptr_t)d_uvm_weights % 16 == 0;
+  int32_t max_pieces = 0;
   for (int t = 0; t < plan->T; ++t) {
     const TableDesc& d = plan->tables[t];
     if (d.D != D) return fail(FBGEMM_AMD_E_ARG, "table %d has D = %d: without pooling all tables share D = %d", t, d.D, D);
@@ -1989,8 +1991,18 @@ int fbgemm_amd_tbe_forward_nobag(
     const int eb = type_bits(d.ty) / 8;
     if (eb > 1 && (d.weights_offset % eb || d.row_stride % eb))
       return fail(FBGEMM_AMD_E_ARG, "table %d: rows are not aligned to their elements", t);
+    aligned = aligned && d.weights_offset % 16 == 0 && d.row_stride % 16 == 0;
+    max_pieces = std::max(max_pieces, (d.data_off + d.data_bytes + 15) / 16);
   }
   status_in_use(d_status);
+  // rows on 16-byte boundaries and output in whole 16-byte pieces: never slower there, from 2 positions to 3.5 M
+  // (sequence_stream.hip has both sides); the lean kernel's switch turns it off too
+  if (lean_enabled() && aligned && sequence_stream_takes(D, output_ty, d_output, max_pieces)) {
+    HIP_TRY(launch_sequence_stream(plan->d_tables, (const uint8_t*)d_dev_weights, (const uint8_t*)d_uvm_weights, d_indices,
+                                   index_bits == 64, d_offsets, (int32_t)B64, plan->T, indices_numel, D, output_ty, d_output,
+                                   max_pieces, plan->fp8_shift, plan->fp8_mult, (Status*)d_status, (hipStream_t)stream));
+    return 0;
+  }
   HIP_TRY(launch_sequence_lookup(plan->d_tables, (const uint8_t*)d_dev_weights, (const uint8_t*)d_uvm_weights, d_indices,
                                  index_bits == 64, d_offsets, (int32_t)B64, plan->T, indices_numel, D, output_ty,
                                  d_output, plan->fp8_shift, plan->fp8_mult, (Status*)d_status, (hipStream_t)stream));

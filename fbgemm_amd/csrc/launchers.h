@@ -19,6 +19,14 @@ hipError_t launch_sequence_lookup(const TableDesc* tables, const uint8_t* w0, co
                                   bool idx64, const void* offsets, int32_t B, int32_t T, int64_t total_L, int32_t D,
                                   int32_t out_ty, void* out, int32_t fp8_shift, float fp8_mult, Status* status,
                                   hipStream_t stream);
+// Rows on 16-byte boundaries, at most max_pieces 16-byte pieces each (header and elements) and 64 of them, whole pieces of output
+inline bool sequence_stream_takes(int32_t D, int32_t out_ty, const void* out, int32_t max_pieces) {
+  return max_pieces > 0 && max_pieces <= 64 && (uintptr_t)out % 16 == 0 &&
+      (out_ty == ST_FP32 ? D % 4 == 0 : (out_ty == ST_FP16 || out_ty == ST_BF16) && D % 8 == 0);
+}
+hipError_t launch_sequence_stream(const TableDesc* tables, const uint8_t* w0, const uint8_t* w1, const void* indices, bool idx64,
+                                  const void* offsets, int32_t B, int32_t T, int64_t total_L, int32_t D, int32_t out_ty, void* out,
+                                  int32_t max_pieces, int32_t fp8_shift, float fp8_mult, Status* status, hipStream_t stream);
 hipError_t launch_row_lookup(const TableDesc& d, const uint8_t* table, const void* indices, bool idx64,
                              const float* weights, int64_t n, int32_t out_ty, void* out, int64_t out_stride_bytes,
                              int64_t copy_bytes, int32_t fp8_shift, float fp8_mult, Status* status, hipStream_t stream);

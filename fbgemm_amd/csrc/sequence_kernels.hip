@@ -1,6 +1,8 @@
 // gfx950 kernels that write one output row per index: the table-batched
 // forward without pooling (PoolingMode.NONE, "sequence" output) and, at the end
-// of the file, the no_bag mode of the single-table kernels.
+// of the file, the no_bag mode of the single-table kernels. Forwards over rows on
+// 16-byte boundaries take sequence_stream_kernel (sequence_stream.hip) instead; what is
+// left here is every other alignment, width and the outputs that copy rows.
 //
 // What the reference's CPU operator does for this mode
 // (fbgemm_gpu/codegen/inference/embedding_forward_quantized_cpu_template.cpp:283-296,390-420):

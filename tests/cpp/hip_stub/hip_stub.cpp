@@ -238,6 +238,8 @@ hipError_t launch_bag_order(const void*, bool, int32_t B, int32_t T, BagEntry* o
 }
 hipError_t launch_sequence_lookup(const TableDesc*, const uint8_t*, const uint8_t*, const void*, bool, const void*, int32_t, int32_t,
                                   int64_t, int32_t, int32_t, void*, int32_t, float, Status*, hipStream_t) { return LAUNCHED(); }
+hipError_t launch_sequence_stream(const TableDesc*, const uint8_t*, const uint8_t*, const void*, bool, const void*, int32_t, int32_t,
+                                  int64_t, int32_t, int32_t, void*, int32_t, int32_t, float, Status*, hipStream_t) { return LAUNCHED(); }
 hipError_t launch_row_lookup(const TableDesc&, const uint8_t*, const void*, bool, const float*, int64_t, int32_t, void*, int64_t,
                              int64_t, int32_t, float, Status*, hipStream_t) { return LAUNCHED(); }
 hipError_t launch_float_to_hfp8(const float*, int64_t, int32_t, int32_t, float, uint8_t*, hipStream_t) { return LAUNCHED(); }

@@ -370,6 +370,19 @@ def test_no_pooling_random_shapes(ops, oracle, seed):
                          f"seed {seed}: T={T} D={D} tys={tys} B={B} L<={max_len} align={align} out={out_ty}")
 
 
+@pytest.mark.parametrize("out_ty", [FP32, FP16, BF16])
+@pytest.mark.parametrize("D", [8, 24, 248, 256, 264])
+def test_no_pooling_at_the_edges_of_what_a_wave_takes(ops, oracle, D, out_ty):
+    """Runs of positions that end at, just before and just behind the 4, 16 and 32 a wave takes, from tables of
+    five row types side by side; rows of one 16-byte piece up to the 64 pieces the kernel takes (fp32 x 256), and of 66."""
+    rng = np.random.default_rng(7700 + D)
+    for n in (1, 3, 4, 5, 15, 16, 17, 31, 32, 33, 65):
+        specs = [(int(rng.integers(1, 40)), D, ty) for ty in (INT4, INT8, FP16, INT2, FP32)]
+        _no_pooling_case(ops, oracle, rng, specs, n, 1, np.int64 if n & 1 else np.int32, 16, out_ty, f"D={D} out={out_ty} n={n}")
+    specs = [(500, D, INT4), (3, D, INT8)]  # 32 positions a wave
+    _no_pooling_case(ops, oracle, rng, specs, 9001, 12, np.int64, 16, out_ty, f"D={D} out={out_ty} large")
+
+
 def test_no_pooling_more_positions_than_one_pass_of_the_grid(ops, oracle):
     """Rows of 512 columns take a whole wave; 300 K positions are more than the largest grid covers at once, so
     every wave walks several groups and uses the indices it fetched one group ahead."""
