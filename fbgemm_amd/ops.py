@@ -30,7 +30,8 @@ ERR_INDEX_OUT_OF_RANGE, ERR_BAG_OVERRUN, ERR_LENGTH_MISMATCH, ERR_NEGATIVE_LENGT
 
 
 def _stream():
-    return C.c_void_p(torch.cuda.current_stream().cuda_stream)
+    # torch.cuda.current_stream().cuda_stream without the Stream object around it: 2 us a call
+    return C.c_void_p(torch._C._cuda_getCurrentRawStream(torch.cuda.current_device()))
 
 
 def _ptr(t):

@@ -75,7 +75,7 @@ int fbgemm_amd_status_read(const void* d_status, void* stream, int32_t* bits, in
  * out the block (cleared), the launches of this thread that follow take it as their
  * d_status, end waits for `stream` and returns what they recorded (bits, and the
  * first offending position or -1). One pair at a time per thread, on one device.
- * Costs no operation on the stream unless something was recorded. A begin whose
+ * Costs a one-thread kernel on the stream, and more only if something was recorded. A begin whose
  * launches were all refused needs no end; one whose launches were enqueued and
  * that is not ended makes the thread's next begin wait for the device. The block
  * is the library's: beside the launches, status_clear and status_read may be

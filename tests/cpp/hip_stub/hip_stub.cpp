@@ -232,6 +232,10 @@ hipError_t launch_status_clear(Status* st, int32_t mark, hipStream_t) {
   st->first_bad_pos = ~0ull;
   return LAUNCHED();
 }
+hipError_t launch_status_done(int32_t* word, int32_t number, hipStream_t) {
+  *word = number;
+  return LAUNCHED();
+}
 hipError_t launch_bag_order(const void*, bool, int32_t B, int32_t T, BagEntry* order, hipStream_t) {
   memset(order, 0, sizeof(BagEntry) * (size_t)B * (size_t)T);
   return LAUNCHED();

@@ -148,3 +148,23 @@ def test_first_call_of_a_thread_beside_a_capture(oracle):
             assert bool((z == 3).all())
             x.fill_(1)
         assert len(got) == 2 * (turn + 1) and all(torch.equal(g, want) for g in got)
+
+
+@pytest.mark.parametrize("products", [0, 40])
+def test_waiting_call_behind_other_work(products):
+    """A waiting call returns when its stream has come to its end, also where that takes longer than the host
+    watches for it (40 products of 4096 x 4096 floats are several milliseconds): what it read and wrote is then
+    free for any other stream."""
+    ops, call, good, bad = single_table_calls()
+    x = torch.ones(4096, 4096, device="cuda") / 4096
+    y, other = torch.empty_like(x), torch.cuda.Stream()
+    torch.cuda.synchronize()
+    for _ in range(3):
+        y.zero_()
+        for _ in range(products):
+            torch.mm(x, x, out=y)
+        assert call(good) is True
+        with torch.cuda.stream(other):
+            # row sums of the product of two matrices of 1 / 4096: 4096 / 4096 per row
+            assert float(y.sum(1).max()) == pytest.approx(1.0 if products else 0.0, abs=1e-5)
+        assert call(bad) is False
