@@ -65,6 +65,9 @@ SYMBOLS = {
     "fbgemm_amd_tbe_plan_num_rows": (_I64, [_P, _I32]),
     "fbgemm_amd_tbe_plan_row_bytes": (_I64, [_P, _I32]),
     "fbgemm_amd_check_remap_indices": (C.c_int, [_P, _I32, _P, _P, _I32, _I64, _I64, _I32, _P, _P, _P, _I32, _P, _P, _P, _P]),
+    "fbgemm_amd_check_remap_indices_ranked": (C.c_int, [_P, _P, _I32, _P, _P, _I32, _I64, _I64, _I32, _P, _P, _P, _I32, _P, _P, _P, _P]),
+    "fbgemm_amd_rank_records_create": (C.c_int, [C.POINTER(_P), _P, _I32, _P, _I64, _P]),
+    "fbgemm_amd_rank_records_destroy": (None, [_P]),
     "fbgemm_amd_pruned_array_lookup": (C.c_int, [_P, _P, _I32, _I64, _P, _I32, _P, _I32, _P, _P]),
     "fbgemm_amd_tbe_inplace_update": (C.c_int, [_P, _P, _P, _P, _I64, _P, _P, _I32, _P, _I64, _P, _P]),
     "fbgemm_amd_pruned_array_lookup_from_row_idx": (C.c_int, [_P, _I32, _P, _I64, _P, _I32, _P, _I32, _P, _P]),

@@ -1018,6 +1018,30 @@ int fbgemm_amd_spmdm_run(
 
 // ---- table-batched forward ---------------------------------------------------
 
+namespace {
+// The compact form of the mappings of T tables (remap_rank_kernels.hip), where any of them preserves the order.
+struct RankSet {
+  RankRecord* records = nullptr;  // null: no table has it
+  int64_t* offsets = nullptr;     // T entries: first record of the table, or -1
+  int64_t* remap_offsets = nullptr; // T + 1: the mapping offsets it was made for
+  const void* source = nullptr;   // the mapping array, and the width of its entries
+  int32_t bits = 0;
+  int32_t tables = 0;             // that have it
+};
+
+void free_ranks(RankSet* r) {
+  if (r->records) (void)hipFree(r->records);
+  if (r->offsets) (void)hipFree(r->offsets);
+  if (r->remap_offsets) (void)hipFree(r->remap_offsets);
+  *r = RankSet();
+}
+} // namespace
+
+struct fbgemm_amd_rank_records {
+  RankSet set;
+  int32_t T = 0;
+};
+
 struct fbgemm_amd_tbe_plan {
   int32_t T = 0;
   int64_t total_D = 0;
@@ -1108,14 +1132,7 @@ struct fbgemm_amd_tbe_plan {
   uint64_t use_clock = 0;
   int32_t accumulate = FBGEMM_AMD_ACC_EXACT;
   // compact form of the pruned-row mappings (fbgemm_amd_tbe_plan_set_index_remappings)
-  RankRecord* d_rank_records = nullptr;
-  int64_t* d_rank_offsets = nullptr; // T entries: first record of the table, or -1
-  // the T + 1 mapping offsets the records were built for (device copy): forwards that use the
-  // records bound and slice the mappings with these, whatever offsets they are handed
-  int64_t* d_rank_remap_offsets = nullptr;
-  const void* rank_source = nullptr; // the mapping array the records were made from
-  int32_t rank_bits = 0;
-  int32_t rank_tables = 0;           // tables that use the records
+  RankSet ranks; // forwards that use it bound and slice the mappings with its offsets, whatever they are handed
   // lane-shape choice of the last forward, per (B, indices_numel >> 16)
   int32_t shape_B = -1;
   int64_t shape_bucket = -1;
@@ -1352,9 +1369,7 @@ void fbgemm_amd_tbe_plan_destroy(fbgemm_amd_tbe_plan* plan) {
   if (plan->seg_offsets) (void)hipFree(plan->seg_offsets);
   if (plan->seg_partial) (void)hipFree(plan->seg_partial);
   if (plan->shared_done) (void)hipEventDestroy(plan->shared_done);
-  if (plan->d_rank_records) (void)hipFree(plan->d_rank_records);
-  if (plan->d_rank_offsets) (void)hipFree(plan->d_rank_offsets);
-  if (plan->d_rank_remap_offsets) (void)hipFree(plan->d_rank_remap_offsets);
+  free_ranks(&plan->ranks);
   delete plan;
 }
 
@@ -1724,10 +1739,10 @@ int tbe_forward_impl(
     }
     w = W;
     exact = plan->accumulate != FBGEMM_AMD_ACC_FAST;
-    if (d_index_remappings && plan->d_rank_records && plan->rank_source == d_index_remappings && plan->rank_bits == remap_bits) {
-      rank_records = plan->d_rank_records;
-      rank_offsets = plan->d_rank_offsets;
-      d_index_remappings_offsets = plan->d_rank_remap_offsets;
+    if (d_index_remappings && plan->ranks.records && plan->ranks.source == d_index_remappings && plan->ranks.bits == remap_bits) {
+      rank_records = plan->ranks.records;
+      rank_offsets = plan->ranks.offsets;
+      d_index_remappings_offsets = plan->ranks.remap_offsets;
     }
     reuse_order = plan->reuse_order;
   }
@@ -1877,29 +1892,11 @@ int fbgemm_amd_tbe_plan_set_accumulate(fbgemm_amd_tbe_plan* plan, int32_t mode) 
   return 0;
 }
 
-int fbgemm_amd_tbe_plan_set_index_remappings(
-    fbgemm_amd_tbe_plan* plan, const void* d_index_remappings, int32_t remap_bits,
-    const int64_t* index_remappings_offsets, int64_t index_remappings_offsets_numel, void* stream_) {
-  if (!plan) return fail(FBGEMM_AMD_E_ARG, "plan is null");
-  hipStream_t stream = (hipStream_t)stream_;
-  std::lock_guard<std::mutex> lk(plan->mu);
-  // forget what was made from an earlier array (after the forwards that may still read it)
-  if (plan->d_rank_records || plan->d_rank_offsets || plan->d_rank_remap_offsets) {
-    HIP_TRY(hipDeviceSynchronize());
-    if (plan->d_rank_records) (void)hipFree(plan->d_rank_records);
-    if (plan->d_rank_offsets) (void)hipFree(plan->d_rank_offsets);
-    if (plan->d_rank_remap_offsets) (void)hipFree(plan->d_rank_remap_offsets);
-    plan->d_rank_records = nullptr;
-    plan->d_rank_offsets = nullptr;
-    plan->d_rank_remap_offsets = nullptr;
-  }
-  plan->rank_source = nullptr;
-  plan->rank_tables = 0;
-  if (!d_index_remappings) return 0;
-  if (remap_bits != 32 && remap_bits != 64) return fail(FBGEMM_AMD_E_ARG, "remap entries are 32 or 64 bits wide");
-  if (!index_remappings_offsets || index_remappings_offsets_numel != (int64_t)plan->T + 1)
-    return fail(FBGEMM_AMD_E_ARG, "index_remappings_offsets must hold T+1 = %d entries (on the host)", plan->T + 1);
-  const int T = plan->T;
+} // extern "C"
+namespace {
+// index_remappings_offsets: T + 1 entries on the host. Waits for `stream`.
+int build_ranks(const void* d_index_remappings, int32_t remap_bits, const int64_t* index_remappings_offsets, int T, hipStream_t stream,
+                RankSet* out) {
   std::vector<int64_t> first(T, -1);
   int64_t words = 0, max_partials = 1;
   for (int t = 0; t < T; ++t) {
@@ -1959,20 +1956,58 @@ int fbgemm_amd_tbe_plan_set_index_remappings(
       drop();
       return fail(FBGEMM_AMD_E_HIP, "rank offsets: %s", hipGetErrorString(e));
     }
-    plan->d_rank_records = records;
+    *out = RankSet{records, d_first, d_offs, d_index_remappings, remap_bits, used};
     records = nullptr;
-    plan->d_rank_offsets = d_first;
-    plan->d_rank_remap_offsets = d_offs;
-    plan->rank_source = d_index_remappings;
-    plan->rank_bits = remap_bits;
-    plan->rank_tables = used;
   }
   drop();
 #undef HIP_TRY_DROP
   return 0;
 }
+} // namespace
+extern "C" {
 
-int32_t fbgemm_amd_tbe_plan_rank_tables(const fbgemm_amd_tbe_plan* plan) { return plan ? plan->rank_tables : -1; }
+int fbgemm_amd_tbe_plan_set_index_remappings(
+    fbgemm_amd_tbe_plan* plan, const void* d_index_remappings, int32_t remap_bits,
+    const int64_t* index_remappings_offsets, int64_t index_remappings_offsets_numel, void* stream_) {
+  if (!plan) return fail(FBGEMM_AMD_E_ARG, "plan is null");
+  hipStream_t stream = (hipStream_t)stream_;
+  std::lock_guard<std::mutex> lk(plan->mu);
+  // forget what was made from an earlier array (after the forwards that may still read it)
+  if (plan->ranks.records) {
+    HIP_TRY(hipDeviceSynchronize());
+    free_ranks(&plan->ranks);
+  }
+  if (!d_index_remappings) return 0;
+  if (remap_bits != 32 && remap_bits != 64) return fail(FBGEMM_AMD_E_ARG, "remap entries are 32 or 64 bits wide");
+  if (!index_remappings_offsets || index_remappings_offsets_numel != (int64_t)plan->T + 1)
+    return fail(FBGEMM_AMD_E_ARG, "index_remappings_offsets must hold T+1 = %d entries (on the host)", plan->T + 1);
+  return build_ranks(d_index_remappings, remap_bits, index_remappings_offsets, plan->T, stream, &plan->ranks);
+}
+
+int fbgemm_amd_rank_records_create(
+    fbgemm_amd_rank_records** out, const void* d_index_remappings, int32_t remap_bits, const int64_t* index_remappings_offsets,
+    int64_t index_remappings_offsets_numel, void* stream) {
+  if (!out) return fail(FBGEMM_AMD_E_ARG, "out is null");
+  *out = nullptr;
+  if (remap_bits != 32 && remap_bits != 64) return fail(FBGEMM_AMD_E_ARG, "remap entries are 32 or 64 bits wide");
+  if (!index_remappings_offsets || index_remappings_offsets_numel < 2 || index_remappings_offsets_numel - 1 > 0x7fffffffLL)
+    return fail(FBGEMM_AMD_E_ARG, "index_remappings_offsets must hold T+1 entries (on the host)");
+  if (!d_index_remappings) return 0;
+  std::unique_ptr<fbgemm_amd_rank_records> r(new fbgemm_amd_rank_records());
+  r->T = (int32_t)(index_remappings_offsets_numel - 1);
+  if (int rc = build_ranks(d_index_remappings, remap_bits, index_remappings_offsets, r->T, (hipStream_t)stream, &r->set)) return rc;
+  const int32_t tables = r->set.tables;
+  if (tables > 0) *out = r.release();
+  return tables;
+}
+
+void fbgemm_amd_rank_records_destroy(fbgemm_amd_rank_records* ranks) {
+  if (!ranks) return;
+  free_ranks(&ranks->set); // waits for the kernels that may still read it
+  delete ranks;
+}
+
+int32_t fbgemm_amd_tbe_plan_rank_tables(const fbgemm_amd_tbe_plan* plan) { return plan ? plan->ranks.tables : -1; }
 
 int fbgemm_amd_tbe_plan_trim(fbgemm_amd_tbe_plan* plan) {
   if (!plan) return fail(FBGEMM_AMD_E_ARG, "plan is null");
@@ -2249,6 +2284,17 @@ extern "C" int fbgemm_amd_check_remap_indices(
     const int64_t* d_rows_per_table, int32_t T, const void* d_indices, const void* d_offsets, int32_t index_bits,
     int64_t indices_numel, int64_t offsets_numel, int32_t bounds_check_mode, int64_t* d_warning,
     const int64_t* d_logical_rows_per_table, const void* d_index_remappings, int32_t remap_bits,
+    const int64_t* d_index_remappings_offsets, void* d_out_indices, void* d_out_offsets, void* stream) {
+  return fbgemm_amd_check_remap_indices_ranked(nullptr, d_rows_per_table, T, d_indices, d_offsets, index_bits, indices_numel, offsets_numel,
+                                               bounds_check_mode, d_warning, d_logical_rows_per_table, d_index_remappings, remap_bits,
+                                               d_index_remappings_offsets, d_out_indices, d_out_offsets, stream);
+}
+
+extern "C" int fbgemm_amd_check_remap_indices_ranked(
+    const fbgemm_amd_rank_records* ranks,
+    const int64_t* d_rows_per_table, int32_t T, const void* d_indices, const void* d_offsets, int32_t index_bits,
+    int64_t indices_numel, int64_t offsets_numel, int32_t bounds_check_mode, int64_t* d_warning,
+    const int64_t* d_logical_rows_per_table, const void* d_index_remappings, int32_t remap_bits,
     const int64_t* d_index_remappings_offsets, void* d_out_indices, void* d_out_offsets, void* stream_) {
   if (T <= 0 || !d_rows_per_table) return fail(FBGEMM_AMD_E_ARG, "rows_per_table must hold T >= 1 entries");
   if (index_bits != 32 && index_bits != 64) return fail(FBGEMM_AMD_E_ARG, "index_bits must be 32 or 64");
@@ -2279,11 +2325,18 @@ extern "C" int fbgemm_amd_check_remap_indices(
   a.remap_offsets = d_index_remappings_offsets;
   a.warning = d_warning;
   a.mode = bounds_check_mode;
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  if (ranks || check_remap_counts(total_B, bounds_check_mode)) (void)hipStreamIsCapturing(stream, &cap);
+  // a graph reads the mapping itself: it may be replayed after the mapping has changed in place
+  if (ranks && cap == hipStreamCaptureStatusNone && d_index_remappings_offsets && ranks->T == T && ranks->set.source == d_index_remappings &&
+      ranks->set.bits == remap_bits) {
+    a.rank_records = ranks->set.records;
+    a.rank_offsets = ranks->set.offsets;
+    a.remap_offsets = ranks->set.remap_offsets;
+  }
   // A small call that counts does so in one launch with a counter of the library's, which is its alone
   // until its kernel has left it zero. A captured call may be replayed at any time and so can have
   // none; it takes the form of two launches, which uses no memory but the call's own outputs.
-  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-  if (check_remap_counts(total_B, bounds_check_mode)) (void)hipStreamIsCapturing(stream, &cap);
   if (check_remap_counts(total_B, bounds_check_mode) && cap == hipStreamCaptureStatusNone) {
     std::lock_guard<std::mutex> lk(g_mu);
     DeviceScratch* s;

@@ -312,15 +312,20 @@ __global__ __launch_bounds__(SCAN_THREADS) void check_remap_carry_kernel(void* o
   }
 }
 
-template <typename index_t, typename remap_t>
+template <typename index_t, typename remap_t, bool RANKED>
 __global__ __launch_bounds__(CR_BAGS) void check_remap_kernel(CheckRemapArgs a) {
   constexpr bool IS64 = sizeof(index_t) == 8;
   __shared__ int64_t fixed[CR_BAGS + 1];
   __shared__ int64_t t_rows[CR_BAGS], t_logical[CR_BAGS], t_remap[CR_BAGS], t_cap[CR_BAGS];
+  __shared__ int64_t t_rank[RANKED ? CR_BAGS : 1];
   __shared__ int64_t lds[CR_BAGS / 64];
   __shared__ int bad_count;
   const int tid = threadIdx.x;
-  const int64_t k0 = (int64_t)blockIdx.x * CR_BAGS;
+  // Workgroups (x, *) run on XCD x % 8. With the grid of more than one launch, a multiple of 8 wide, each
+  // XCD takes consecutive bags, an eighth of the tables, whose compact mappings then stay in its L2.
+  const unsigned block = a.carry ? (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3) : blockIdx.x;
+  const int64_t k0 = (int64_t)block * CR_BAGS;
+  if (k0 >= a.total_B) return;
   const int nb = (int)(a.total_B - k0 < CR_BAGS ? a.total_B - k0 : CR_BAGS);
   // every load the walk over the offsets needs, before anything waits: this bag's offset, the one
   // behind the last bag, and what the bags before these leave
@@ -358,6 +363,7 @@ __global__ __launch_bounds__(CR_BAGS) void check_remap_kernel(CheckRemapArgs a) 
       t_logical[tid] = a.logical_rows[t0 + tid];
       t_remap[tid] = a.remap_offsets[t0 + tid];
       t_cap[tid] = a.remap_offsets[t0 + tid + 1] - t_remap[tid];
+      if (RANKED) t_rank[tid] = a.rank_offsets[t0 + tid];
     }
   }
   carry = cr_block_max(carry, lds);
@@ -392,7 +398,7 @@ __global__ __launch_bounds__(CR_BAGS) void check_remap_kernel(CheckRemapArgs a) 
     if (a.remap_offsets) bad = 0; // the second check starts from zero, and from offsets that are in order
   }
   // the indices of these bags; what lies before the first bag is nobody's and passes through
-  const int64_t lo0 = blockIdx.x == 0 ? 0 : fixed[0], hi0 = fixed[nb], own = fixed[0];
+  const int64_t lo0 = block == 0 ? 0 : fixed[0], hi0 = fixed[nb], own = fixed[0];
   const int64_t share = (hi0 - lo0 + gridDim.y - 1) / gridDim.y;
   const int64_t lo = lo0 + share * blockIdx.y;
   const int64_t hi = lo + share < hi0 ? lo + share : hi0;
@@ -430,12 +436,27 @@ __global__ __launch_bounds__(CR_BAGS) void check_remap_kernel(CheckRemapArgs a) 
     }
     if (a.remap_offsets) {
       remap_t m[CR_LOADS];
+      RankRecord rec[CR_LOADS];
+      bool ranked[CR_LOADS];
 #pragma unroll
-      for (int u = 0; u < CR_LOADS; ++u)
-        if (gather[u]) m[u] = remap[t_remap[t[u]] + (int64_t)v[u]];
+      for (int u = 0; u < CR_LOADS; ++u) {
+        ranked[u] = false;
+        if (gather[u]) {
+          const int64_t rank = RANKED ? t_rank[t[u]] : -1;
+          ranked[u] = rank >= 0;
+          if (RANKED && ranked[u]) rec[u] = a.rank_records[rank + ((int64_t)v[u] >> 5)];
+          else m[u] = remap[t_remap[t[u]] + (int64_t)v[u]];
+        }
+      }
 #pragma unroll
-      for (int u = 0; u < CR_LOADS; ++u)
-        if (gather[u]) v[u] = (index_t)m[u];
+      for (int u = 0; u < CR_LOADS; ++u) {
+        if (RANKED && ranked[u]) { // the rank among the kept rows (remap_rank_kernels.hip)
+          const uint32_t bit = (uint32_t)v[u] & 31u;
+          v[u] = ((rec[u].bits >> bit) & 1u) ? (index_t)(rec[u].before + (uint32_t)__builtin_popcount(rec[u].bits & ((1u << bit) - 1u))) : (index_t)-1;
+        } else if (gather[u]) {
+          v[u] = (index_t)m[u];
+        }
+      }
     }
 #pragma unroll
     for (int u = 0; u < CR_LOADS; ++u) {
@@ -575,11 +596,18 @@ hipError_t launch_check_remap(CheckRemapArgs a, bool is64, bool remap64, hipStre
   const int64_t per = a.N < (int64_t)256 * CR_LOADS * CR_BAGS ? 2 * CR_BAGS : CR_LOADS * CR_BAGS;
   int64_t shares = (a.N / blocks + per - 1) / per;
   shares = shares < 1 ? 1 : (shares > 1024 ? 1024 : shares);
-  const dim3 grid((unsigned)blocks, (unsigned)shares), block(CR_BAGS);
-  if (is64 && remap64) hipLaunchKernelGGL((check_remap_kernel<int64_t, int64_t>), grid, block, 0, stream, a);
-  else if (is64) hipLaunchKernelGGL((check_remap_kernel<int64_t, int32_t>), grid, block, 0, stream, a);
-  else if (remap64) hipLaunchKernelGGL((check_remap_kernel<int32_t, int64_t>), grid, block, 0, stream, a);
-  else hipLaunchKernelGGL((check_remap_kernel<int32_t, int32_t>), grid, block, 0, stream, a);
+  const dim3 grid((unsigned)(a.carry ? (blocks + 7) / 8 * 8 : blocks), (unsigned)shares), block(CR_BAGS);
+  const bool ranked = a.remap_offsets && a.rank_records && a.rank_offsets;
+#define FBGEMM_AMD_CHECK_REMAP(INDEX_T, REMAP_T)                                                                          \
+  do {                                                                                                                    \
+    if (ranked) hipLaunchKernelGGL((check_remap_kernel<INDEX_T, REMAP_T, true>), grid, block, 0, stream, a);              \
+    else hipLaunchKernelGGL((check_remap_kernel<INDEX_T, REMAP_T, false>), grid, block, 0, stream, a);                    \
+  } while (0)
+  if (is64 && remap64) FBGEMM_AMD_CHECK_REMAP(int64_t, int64_t);
+  else if (is64) FBGEMM_AMD_CHECK_REMAP(int64_t, int32_t);
+  else if (remap64) FBGEMM_AMD_CHECK_REMAP(int32_t, int64_t);
+  else FBGEMM_AMD_CHECK_REMAP(int32_t, int32_t);
+#undef FBGEMM_AMD_CHECK_REMAP
   return hipGetLastError();
 }
 

@@ -208,6 +208,8 @@ struct CheckRemapArgs {
   int64_t N, total_B, B;       // total_B = T * B
   const void* remap;
   const int64_t* remap_offsets; // T + 1, or nullptr: no mapping
+  const RankRecord* rank_records; // nullptr, or the compact form of order-preserving mappings
+  const int64_t* rank_offsets;    // T entries: first record of table t, or -1: its mapping is read from `remap`
   int64_t* warning;
   unsigned long long* counter;  // zero, and this call's alone; or nullptr: a launch more
   int32_t* counter_taken;       // pinned host word: the kernel clears it when it has left the counter zero

@@ -294,6 +294,33 @@ class TbePlan:
                 pass
 
 
+class RankRecords:
+    """The compact form of array-based pruned-row mappings for ``check_remap_indices`` (fbgemm_amd_rank_records_create),
+    from the contents they have now: ``key`` says what they were, and whoever keeps one makes it anew when they change.
+    A copied or unpickled holder gets ``None`` in its place."""
+
+    def __init__(self, index_remappings, index_remappings_offsets):
+        self.key = TbePlan.rank_key(index_remappings, index_remappings_offsets)
+        self.handle = None
+        if index_remappings.numel() and index_remappings.is_contiguous():
+            offsets = index_remappings_offsets.detach().to("cpu", torch.int64).contiguous()
+            handle = C.c_void_p()
+            check(_lib.lib().fbgemm_amd_rank_records_create(
+                C.byref(handle), _ptr(index_remappings), _bits(index_remappings), _ptr(offsets), offsets.numel(), _stream()))
+            self.handle = handle if handle.value else None
+
+    def __reduce__(self):
+        return type(None), ()
+
+    def __del__(self):
+        h, self.handle = getattr(self, "handle", None), None
+        if h:
+            try:
+                _lib.lib().fbgemm_amd_rank_records_destroy(h)
+            except Exception:
+                pass
+
+
 _plans = collections.OrderedDict()  # least recently used first
 MAX_CACHED_PLANS = 64
 
@@ -574,10 +601,11 @@ def bounds_check_indices(rows_per_table, indices, offsets, bounds_check_mode, wa
 
 
 def check_remap_indices(rows_per_table, indices, offsets, bounds_check_mode, warning, weights=None,
-                        logical_rows_per_table=None, index_remappings=None, index_remappings_offsets=None):
+                        logical_rows_per_table=None, index_remappings=None, index_remappings_offsets=None, ranks=None):
     """``bounds_check_indices`` (WARNING or IGNORE) on copies of ``indices`` and ``offsets``, which are returned;
     with ``index_remappings`` the check against the logical rows, ``pruned_array_lookup`` and the check against
-    ``rows_per_table`` in one pass. ``warning`` ends as the last of those checks would leave it."""
+    ``rows_per_table`` in one pass. ``warning`` ends as the last of those checks would leave it. ``ranks`` (RankRecords
+    of these mappings as they are now) answers in the array's place."""
     _require_cuda(rows_per_table, indices, offsets, warning, weights, logical_rows_per_table, index_remappings,
                   index_remappings_offsets)
     if indices.dtype != offsets.dtype:
@@ -598,8 +626,8 @@ def check_remap_indices(rows_per_table, indices, offsets, bounds_check_mode, war
         if logical.numel() != rows.numel() or offs.numel() != rows.numel() + 1:
             raise ValueError("the mappings do not belong to these tables")
     out_indices, out_offsets = torch.empty_like(indices), torch.empty_like(offsets)
-    check(_lib.lib().fbgemm_amd_check_remap_indices(
-        _ptr(rows), rows.numel(), _ptr(indices), _ptr(offsets), _bits(indices), indices.numel(), offsets.numel(),
+    check(_lib.lib().fbgemm_amd_check_remap_indices_ranked(
+        None if ranks is None else ranks.handle, _ptr(rows), rows.numel(), _ptr(indices), _ptr(offsets), _bits(indices), indices.numel(), offsets.numel(),
         int(bounds_check_mode), _ptr(warning), _ptr(logical), _ptr(index_remappings),
         32 if index_remappings is None else _bits(index_remappings), _ptr(offs), _ptr(out_indices), _ptr(out_offsets),
         _stream()))

@@ -419,6 +419,26 @@ int fbgemm_amd_check_remap_indices(
     const int64_t* d_logical_rows_per_table, const void* d_index_remappings, int32_t remap_bits,
     const int64_t* d_index_remappings_offsets, void* d_out_indices, void* d_out_offsets, void* stream);
 
+/* The compact form of pruned-row mappings that keep the rows' order, 2 bits per logical
+ * row, for the check above: made once from d_index_remappings (T + 1 offsets on the
+ * host; waits for `stream`) and made anew by the caller whenever its contents change.
+ * Returns for how many tables there is one; *out is NULL where there is none. destroy
+ * waits for the device. The ranked check is the check above and, where `ranks`
+ * (NULL: none) was made from the very array it is handed, asks it instead of the
+ * array, whose random 4-byte reads cost a line each: the same results. A call under
+ * stream capture reads the array. */
+typedef struct fbgemm_amd_rank_records fbgemm_amd_rank_records;
+int fbgemm_amd_rank_records_create(
+    fbgemm_amd_rank_records** out, const void* d_index_remappings, int32_t remap_bits,
+    const int64_t* index_remappings_offsets, int64_t index_remappings_offsets_numel, void* stream);
+void fbgemm_amd_rank_records_destroy(fbgemm_amd_rank_records* ranks);
+int fbgemm_amd_check_remap_indices_ranked(
+    const fbgemm_amd_rank_records* ranks,
+    const int64_t* d_rows_per_table, int32_t T, const void* d_indices, const void* d_offsets, int32_t index_bits,
+    int64_t indices_numel, int64_t offsets_numel, int32_t bounds_check_mode, int64_t* d_warning,
+    const int64_t* d_logical_rows_per_table, const void* d_index_remappings, int32_t remap_bits,
+    const int64_t* d_index_remappings_offsets, void* d_out_indices, void* d_out_offsets, void* stream);
+
 /* pruned_hashmap_lookup (embedding_forward_quantized_cpu_template.cpp:524-603; GPU
  * embedding_forward_quantized_split_lookup.cu:19-118): d_hash_table holds
  * [slots][2] (sparse id, dense id) pairs of hash_bits each, -1 = empty, built by

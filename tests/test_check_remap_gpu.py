@@ -141,3 +141,108 @@ def test_streams_and_captured_calls(ops, bags):
     t.start()
     t.join()
     assert not failures, failures
+
+
+def order_preserving(rng, rows, keep):
+    """A mapping of `rows` logical rows that numbers the kept ones in order, and how many it keeps."""
+    kept = rng.random(rows) < keep
+    return np.where(kept, np.cumsum(kept) - 1, -1), int(kept.sum())
+
+
+@pytest.mark.parametrize("dtype", [torch.int32, torch.int64])
+@pytest.mark.parametrize("mapped", [torch.int32, torch.int64])
+def test_compact_mappings(ops, mapped, dtype):
+    """Tables with order-preserving mappings (around the 32 rows of a record: none kept, all kept, some), others and
+    none side by side: the compact form answers as the arrays do."""
+    rng = np.random.default_rng(8)
+    cu = lambda a, dt=torch.int64: torch.from_numpy(np.ascontiguousarray(a)).cuda().to(dt)
+    maps, rows, logical = [], [], []
+    for n in (1, 31, 32, 33, 64, 255, 1000, 8191, 8193, 40_000):
+        for keep in (0.0, 0.5, 1.0):
+            m, kept = order_preserving(rng, n, keep)
+            maps.append(m)
+            rows.append(max(kept - (n % 2), 0))  # odd ones: the last kept row lies outside the table
+            logical.append(n)
+    for n in (50, 300):
+        maps += [rng.integers(-1, n, size=n), np.zeros(0, np.int64)]
+        rows += [n, n]
+        logical += [n, n]
+    T = len(maps)
+    rows, logical = cu(rows), cu(logical)
+    offs = cu(np.concatenate([[0], np.cumsum([len(m) for m in maps])]))
+    remap = cu(np.concatenate(maps), mapped)
+    ranks = ops.RankRecords(remap, offs)
+    assert ranks.handle is not None
+    for B, avg in ((1, 40), (300, 7)):
+        lens = rng.integers(0, 2 * avg, size=T * B)
+        off = np.concatenate([[0], np.cumsum(lens)])
+        idx = rng.integers(-2, int(logical.max()) + 40, size=int(off[-1]))
+        idx = np.where(rng.random(len(idx)) < 0.9, idx % np.repeat(logical.cpu().numpy(), lens.reshape(T, B).sum(1)), idx)
+        for mode in (1, 2):
+            args = (rows, cu(idx, dtype), cu(off, dtype), mode)
+            w0, w1 = torch.zeros(1, dtype=torch.int64, device="cuda"), torch.zeros(1, dtype=torch.int64, device="cuda")
+            want = one_after_the_other(ops, *args, w0, logical, remap, offs)
+            got = ops.check_remap_indices(*args, w1, None, logical, remap, offs, ranks)
+            assert all(torch.equal(g, w) for g, w in zip(got, want)) and torch.equal(w0, w1), (B, mode)
+
+
+def test_module_follows_its_mappings():
+    """A pruned module's forward with the compact form of its mappings, after they have been edited in place, set anew,
+    and in copies and saved modules."""
+    import copy
+    import io
+
+    from fbgemm_amd import module as M
+    rng = np.random.default_rng(2)
+    rows, D, B = 400, 32, 64
+    m = M.IntNBitTableBatchedEmbeddingBagsCodegen([("", rows, D, M.SparseType.INT8, M.EmbeddingLocation.DEVICE)] * 2,
+                                                  bounds_check_mode=M.BoundsCheckMode.WARNING, output_dtype=M.SparseType.FP32)
+    m.fill_random_weights()
+    for _, sb in m.split_embedding_weights():
+        sb.view(torch.float16).copy_(torch.rand(rows, 2, device="cuda").half())
+    mapping = lambda: torch.from_numpy(order_preserving(rng, 2 * rows, 0.4)[0]).cuda()
+    off = torch.arange(2 * B + 1, dtype=torch.int64, device="cuda") * 5
+    idx = torch.from_numpy(rng.integers(0, 2 * rows, size=10 * B)).cuda()
+    plain = copy.deepcopy(m)
+
+    def check(mod, maps):
+        flat = torch.cat(maps).to(idx.device)
+        where = torch.cat([idx[:5 * B], idx[5 * B:] + 2 * rows])
+        want = plain(flat[where].to(torch.int64), off)
+        for _ in range(3):
+            assert torch.equal(mod(idx, off), want)
+
+    maps = [mapping(), mapping()]
+    m.set_index_remappings(maps)
+    assert m._rank_records is not None and m._rank_records.handle is not None
+    check(m, maps)
+    maps = [mapping(), mapping()]
+    m.index_remappings_array.copy_(torch.cat(maps))
+    check(m, maps)
+    assert m._rank_records is not None
+    buf = io.BytesIO()
+    torch.save(m, buf)
+    buf.seek(0)
+    for other in (copy.deepcopy(m), torch.load(buf, weights_only=False)):
+        check(other, maps)
+        changed = [maps[1], maps[0]]
+        other.index_remappings_array.copy_(torch.cat(changed))
+        check(other, changed)
+        check(m, maps)
+    # a graph reads the array: it sees what is written there between its replays
+    graph, s = torch.cuda.CUDAGraph(), torch.cuda.Stream()
+    with torch.cuda.stream(s):
+        call = lambda: M.ops.check_remap_indices(m.rows_per_table, idx, off, 1, m.bounds_check_warning, None, m.original_rows_per_table,
+                                                 m._feature_remap_array, m._feature_remap_offsets, m._ranks())
+        call()
+        torch.cuda.synchronize()
+        with torch.cuda.graph(graph, stream=s):
+            out, _ = call()
+    for maps in ([mapping(), mapping()], [mapping(), mapping()]):
+        m.index_remappings_array.copy_(torch.cat(maps))
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        flat = torch.cat(maps)
+        assert torch.equal(out, torch.where(flat < rows, flat, 0)[torch.cat([idx[:5 * B], idx[5 * B:] + 2 * rows])])
+        check(m, maps)
