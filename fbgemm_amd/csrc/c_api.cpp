@@ -1706,7 +1706,8 @@ int tbe_forward_impl(
           }
     }
     // the slot's side stream (default priority, like every stream here) and its two events
-    if (!capturing && !W.side_stream[order_slot] && W.lean.num_waves > 0 && W.general.num_waves > 0) {
+    if (!capturing && !W.side_stream[order_slot] && W.lean.num_waves > 0 && W.general.num_waves > 0 &&
+        (W.lean_wide4 || d_index_remappings || d_q8_out)) {
       hipStream_t s2 = nullptr;
       hipEvent_t e1 = nullptr, e2 = nullptr;
       if (hipStreamCreateWithFlags(&s2, hipStreamNonBlocking) == hipSuccess &&
@@ -1819,9 +1820,23 @@ int tbe_forward_impl(
     if (!reuse_order) HIP_TRY(launch_bag_order(d_offsets, offset_bits == 64, B, plan->T, w.d_order[order_slot], stream));
     a.order = w.d_order[order_slot];
   }
-  // Tables for both kernels, and a forward long enough not to notice two events (the size from
-  // which the bags are ordered): the general kernel runs on the slot's side stream, beside the
-  // lean one, forked off behind the scheduler and joined before the forward's stream goes on.
+  // Tables for both kernels: one launch of both (lookup_both.h). us with two launches in a row (from 2^21 lookups on: side
+  // by side on two streams) and with one, tables of all row types and odd widths:
+  //   40 tables x 1000 bags x 12   63.6 -> 45.6        7 x 2960 x 10    40.7 -> 24.9
+  //   83 x 618 x 20                82.8 -> 62.4        48 x 2547 x 19  100.3 -> 81.6
+  //   69 x 2201 x 3                90.1 -> 76.0        37 x 5521 x 29    271 -> 224
+  // (of 40 such shapes none slower by more than 1 %). Two streams stay where the lean tables are wide 4-bit bags whose bags
+  // are ordered (55 x 3872 x 21 with a sixth of 2-bit rows: 182 against 189 us), with a mapping and with the 8-bit output.
+  if (w.lean.num_waves > 0 && w.general.num_waves > 0 && !d_index_remappings && !d_q8_out && !(w.lean_wide4 && a.order)) {
+    a.work = w.general.d_work;
+    a.xcd_start = w.general.d_xcd_start;
+    a.num_waves = w.general.num_waves;
+    HIP_TRY(launch_lookup_both(a, WorkRun{w.lean.d_work, w.lean.d_xcd_start, w.lean.num_waves}, index_bits == 64, exact, stream));
+    return 0;
+  }
+  // Otherwise, in a forward long enough not to notice two events (the size from which the bags are ordered), the
+  // general kernel runs on the slot's side stream, beside the lean one, forked off behind the scheduler and joined
+  // before the forward's stream goes on.
   static const int side_enabled = env_int("FBGEMM_AMD_SIDE_STREAM", 1);
   hipStream_t side = (side_enabled && w.lean.num_waves > 0 && w.general.num_waves > 0 && a.order) ? w.side_stream[order_slot] : nullptr;
   if (w.general.num_waves > 0) {

@@ -144,6 +144,13 @@ struct WaveWork {
   int32_t first_bag;
 };
 
+// A work list of a table-batched launch: 8 runs, one per XCD (see LookupArgs::xcd_start).
+struct WorkRun {
+  const WaveWork* work;
+  const int64_t* xcd_start;
+  int64_t num_waves; // of the longest run
+};
+
 struct LookupArgs {
   const TableDesc* tables;   // device array, or nullptr when `single` is used
   TableDesc single;

@@ -454,6 +454,22 @@ __device__ __forceinline__ void pool_dispatch_vb(const LookupArgs& a, const Tabl
 #define FBGEMM_AMD_MIN_WAVES 3 // waves per SIMD the register allocation must leave room for
 #endif
 
+// The bags of table `table` from position `first_slot` of its order on, as many as a wave takes.
+template <typename index_t, bool GENERAL>
+__device__ __forceinline__ void run_table(const LookupArgs& a, const TableDesc& d, int table, int first_slot, int lane, StageRow* stage_row,
+                                          StageMul* stage_mul) {
+  switch (d.ty) {
+    case ST_INT4: pool_dispatch_vb<index_t, GENERAL, ST_INT4>(a, d, table, first_slot, lane, stage_row, stage_mul); break;
+    case ST_INT8: pool_dispatch_vb<index_t, GENERAL, ST_INT8>(a, d, table, first_slot, lane, stage_row, stage_mul); break;
+    case ST_FP16: pool_dispatch_vb<index_t, GENERAL, ST_FP16>(a, d, table, first_slot, lane, stage_row, stage_mul); break;
+    case ST_INT2: pool_dispatch_vb<index_t, GENERAL, ST_INT2>(a, d, table, first_slot, lane, stage_row, stage_mul); break;
+    case ST_FP32: pool_dispatch_vb<index_t, GENERAL, ST_FP32>(a, d, table, first_slot, lane, stage_row, stage_mul); break;
+    case ST_BF16: pool_dispatch_vb<index_t, GENERAL, ST_BF16>(a, d, table, first_slot, lane, stage_row, stage_mul); break;
+    case ST_FP8: pool_dispatch_vb<index_t, GENERAL, ST_FP8>(a, d, table, first_slot, lane, stage_row, stage_mul); break;
+    default: break;
+  }
+}
+
 // One item of the work list: `wave` is the position in the list (or the wave's
 // number for a single-table call).
 template <typename index_t, bool GENERAL>
@@ -467,16 +483,7 @@ __device__ __forceinline__ void run_item(const LookupArgs& a, int64_t wave, int 
     first_slot = (int)(wave * a.single.bags);
   }
   const TableDesc d = a.tables ? a.tables[table] : a.single;
-  switch (d.ty) {
-    case ST_INT4: pool_dispatch_vb<index_t, GENERAL, ST_INT4>(a, d, table, first_slot, lane, stage_row, stage_mul); break;
-    case ST_INT8: pool_dispatch_vb<index_t, GENERAL, ST_INT8>(a, d, table, first_slot, lane, stage_row, stage_mul); break;
-    case ST_FP16: pool_dispatch_vb<index_t, GENERAL, ST_FP16>(a, d, table, first_slot, lane, stage_row, stage_mul); break;
-    case ST_INT2: pool_dispatch_vb<index_t, GENERAL, ST_INT2>(a, d, table, first_slot, lane, stage_row, stage_mul); break;
-    case ST_FP32: pool_dispatch_vb<index_t, GENERAL, ST_FP32>(a, d, table, first_slot, lane, stage_row, stage_mul); break;
-    case ST_BF16: pool_dispatch_vb<index_t, GENERAL, ST_BF16>(a, d, table, first_slot, lane, stage_row, stage_mul); break;
-    case ST_FP8: pool_dispatch_vb<index_t, GENERAL, ST_FP8>(a, d, table, first_slot, lane, stage_row, stage_mul); break;
-    default: break;
-  }
+  run_table<index_t, GENERAL>(a, d, table, first_slot, lane, stage_row, stage_mul);
 }
 
 

@@ -224,6 +224,22 @@ hipError_t launch_lookup(const LookupArgs& a, bool idx64, hipStream_t stream) {
   return idx64 ? launch_lookup_i64(a, (unsigned)blocks, stream) : launch_lookup_i32(a, (unsigned)blocks, stream);
 }
 
+hipError_t launch_lookup_both_i64_exact(const LookupArgs& a, const WorkRun& lean, unsigned general_blocks, unsigned blocks, hipStream_t stream);
+hipError_t launch_lookup_both_i64_fast(const LookupArgs& a, const WorkRun& lean, unsigned general_blocks, unsigned blocks, hipStream_t stream);
+hipError_t launch_lookup_both_i32_exact(const LookupArgs& a, const WorkRun& lean, unsigned general_blocks, unsigned blocks, hipStream_t stream);
+hipError_t launch_lookup_both_i32_fast(const LookupArgs& a, const WorkRun& lean, unsigned general_blocks, unsigned blocks, hipStream_t stream);
+
+// Both kernels in one launch (lookup_both.h): `a` with the general tables' list, `lean` the lean tables'.
+hipError_t launch_lookup_both(const LookupArgs& a, const WorkRun& lean, bool idx64, bool exact, hipStream_t stream) {
+  const int64_t general = 8 * a.num_waves, blocks = general + 8 * lean.num_waves;
+  if (blocks <= 0) return hipSuccess;
+  if (blocks > 0x7fffffffLL || !a.tables || !a.work || !a.xcd_start || !lean.work || !lean.xcd_start || a.remap || a.positional || a.check_total ||
+      a.out_ty == ST_INT8)
+    return hipErrorInvalidValue;
+  if (exact) return idx64 ? launch_lookup_both_i64_exact(a, lean, (unsigned)general, (unsigned)blocks, stream) : launch_lookup_both_i32_exact(a, lean, (unsigned)general, (unsigned)blocks, stream);
+  return idx64 ? launch_lookup_both_i64_fast(a, lean, (unsigned)general, (unsigned)blocks, stream) : launch_lookup_both_i32_fast(a, lean, (unsigned)general, (unsigned)blocks, stream);
+}
+
 hipError_t launch_lookup_burst_i64(const LookupArgs& a, dim3 grid, bool four_waves, int lds_bytes, hipStream_t stream);
 hipError_t launch_lookup_burst_i32(const LookupArgs& a, dim3 grid, bool four_waves, int lds_bytes, hipStream_t stream);
 

@@ -213,6 +213,12 @@ hipError_t launch_lookup_lean(const LookupArgs& a, bool idx64, bool, bool wide4,
   g_last_lean_wide4 = wide4 ? 1 : 0;
   return launch_lookup(a, idx64, s);
 }
+hipError_t launch_lookup_both(const LookupArgs& a, const WorkRun& lean, bool idx64, bool, hipStream_t s) {
+  if (!a.work || !a.xcd_start || !lean.work || !lean.xcd_start) return hipErrorInvalidValue;
+  (void)*(volatile const int32_t*)&lean.work[0].table;
+  (void)*(volatile const int64_t*)&lean.xcd_start[8];
+  return launch_lookup(a, idx64, s);
+}
 hipError_t launch_lookup_burst(const LookupArgs& a, bool idx64, int32_t max_D, int32_t max_bits, int, int lds_bytes, hipStream_t s) {
   if (!burst_fits(max_D, max_bits, lds_bytes)) return hipErrorInvalidValue;
   return launch_lookup(a, idx64, s);

@@ -370,6 +370,41 @@ def test_no_pooling_random_shapes(ops, oracle, seed):
                          f"seed {seed}: T={T} D={D} tys={tys} B={B} L<={max_len} align={align} out={out_ty}")
 
 
+@pytest.mark.parametrize("dt", [np.int32, np.int64])
+@pytest.mark.parametrize("fast", [False, True])
+def test_tables_of_both_kernels(ops, oracle, fast, dt):
+    """Tables for the lean and for the general kernel in one launch: batch sizes that leave some of the 8 runs of either
+    work list empty, and one that orders its bags. Tolerance-grade mode with fp16 rows, which it sums the exact way."""
+    rng = np.random.default_rng(61)
+    lean = [(300, 64, FP16), (90, 32, FP16)] if fast else [(300, 128, INT4), (90, 64, FP16), (200, 64, INT8)]
+    general = [(50, 32, INT2), (70, 20, FP32), (40, 36, INT8)] if not fast else [(50, 32, INT2), (70, 20, FP32), (40, 36, FP16)]
+    for k, (B, avg) in enumerate(((1, 9), (7, 5), (8, 30), (33, 12), (400, 6), (9000, 45))):
+        specs = [t for pair in zip(general, lean) for t in pair] if k % 2 else lean[:1] + general[k % 3:k % 3 + 1]
+        if B == 9000:
+            specs = specs + specs[:2]
+        T = len(specs)
+        weights, wo, _ = build_weights(rng, specs, 16)
+        lens = rng.integers(0, 2 * avg + 1, size=T * B)
+        off = np.concatenate([[0], np.cumsum(lens)]).astype(dt)
+        idx = np.concatenate([rng.integers(0, specs[t][0], size=int(off[(t + 1) * B] - off[t * B])) for t in range(T)]).astype(dt)
+        idx[rng.random(len(idx)) < 0.03] = -1
+        if B == 9000:
+            assert len(idx) >= 1 << 21
+        psw = rng.uniform(0.5, 1.5, size=len(idx)).astype(np.float32) if k % 2 else None
+        if not fast:
+            got, want = run_both(ops, oracle, weights, wo, specs, idx, off, k % 2, psw, FP32 if k % 3 else FP16, 16)
+        else:
+            tys, D_offsets = np.array([s[2] for s in specs], np.uint8), np.concatenate([[0], np.cumsum([s[1] for s in specs])]).astype(np.int32)
+            total, maxd = int(D_offsets[-1]), lambda ty: max([s[1] for s in specs if s[2] == ty], default=0)
+            got = ops.int_nbit_split_embedding_codegen_lookup_function(
+                cu(weights), torch.zeros(0, dtype=torch.uint8, device="cuda"), cu(np.zeros(T, np.int32)), cu(wo), cu(tys), cu(D_offsets), total,
+                maxd(INT2), maxd(INT4), maxd(INT8), maxd(FP16), maxd(FP32), cu(idx), cu(off), 0, None if psw is None else cu(psw), FP32,
+                row_alignment=16, accumulate=ops.ACC_FAST).cpu().numpy()
+            rc, want = oracle.tbe_forward(weights, wo, tys, D_offsets, total, idx, off, 0, psw, FP32, 16)
+            assert rc == 0
+        H.assert_same_bits(got, want, f"B={B} T={T} fast={fast} {dt}")
+
+
 @pytest.mark.parametrize("out_ty", [FP32, FP16, BF16])
 @pytest.mark.parametrize("D", [8, 24, 248, 256, 264])
 def test_no_pooling_at_the_edges_of_what_a_wave_takes(ops, oracle, D, out_ty):
