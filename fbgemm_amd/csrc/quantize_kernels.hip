@@ -322,39 +322,42 @@ __global__ __launch_bounds__(256) void quantize_rowwise_kernel(
 }
 
 // The common form of the above: whole rows of at most 64 runs, a multiple of 8 columns, 16-byte
-// aligned, extremes from the row. Streaming, so bound by memory: what counts is bytes in flight and
-// few instructions per element. A wave takes QROWS groups of rows at a time with all their loads
-// issued first (64 or 128 bytes per lane in flight), rows stay in registers, and nothing is predicated by
-// column. 1 M fp32 rows of 128 columns to 4 bits (608 MB): 158 -> 119 us.
-constexpr int QROWS = 2;
-template <bool HALF_IN, int BITS>
+// aligned, extremes from the row. Streaming, so bound by memory: what counts is bytes in flight,
+// whole lines per request and few instructions per element. A wave takes GROUPS groups of rows at a time with all
+// their loads issued first (up to 128 bytes per lane in flight), rows stay in registers, and nothing is predicated by
+// column. QUADS (fp32 rows to 4 and 8 bits): a lane's 8 columns are two quads, lpr quads apart, so that a load
+// instruction takes whole lines, where two loads of 8 consecutive columns each take every line's half; else they are
+// consecutive. 1 M fp32 rows of 128 columns to 4 bits (608 MB): 119 -> 111 us (5.5 TB/s).
+template <bool HALF_IN, int BITS, bool QUADS, int GROUPS>
 __global__ __launch_bounds__(256) void quantize_rows_kernel(const void* input, int64_t rows, int32_t cols, int32_t sb_float,
                                                             int32_t layout, int64_t out_stride, uint8_t* output, int32_t lpr_log) {
+  static_assert(!QUADS || (!HALF_IN && BITS >= 4), "quads of fp32 columns");
   const int lane = threadIdx.x & 63;
   const int lpr = 1 << lpr_log, sub = lane & (lpr - 1);
   const int rows_per_group = 64 >> lpr_log;
-  const int j0 = sub * RUN;
-  const bool on = j0 < cols;
+  const int j0 = QUADS ? sub * 4 : sub * RUN, j1 = QUADS ? (sub + lpr) * 4 : j0 + 4; // first column of either half
+  const bool on = j0 < cols, on1 = j1 < cols; // QUADS: `on` holds for all lanes
   const int data_bytes = cols * BITS / 8;
-  const int64_t step = (int64_t)gridDim.x * (blockDim.x >> 6) * (QROWS * rows_per_group);
-  for (int64_t first = ((int64_t)blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6)) * (QROWS * rows_per_group); first < rows;
+  const int64_t step = (int64_t)gridDim.x * (blockDim.x >> 6) * (GROUPS * rows_per_group);
+  for (int64_t first = ((int64_t)blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6)) * (GROUPS * rows_per_group); first < rows;
        first += step) {
-    float x[QROWS][RUN];
+    float x[GROUPS][RUN];
 #pragma unroll
-    for (int u = 0; u < QROWS; ++u) {
+    for (int u = 0; u < GROUPS; ++u) {
       const int64_t row_raw = first + u * rows_per_group + (lane >> lpr_log);
       const int64_t row = row_raw < rows ? row_raw : rows - 1; // lanes past the end shadow the last row and store nothing
-      const uint8_t* p = reinterpret_cast<const uint8_t*>(input) + (row * (int64_t)cols + (on ? j0 : 0)) * (HALF_IN ? 2 : 4);
+      const uint8_t* in_row = reinterpret_cast<const uint8_t*>(input) + row * (int64_t)cols * (HALF_IN ? 2 : 4);
+      // columns behind the row's last read its first: the same extremes
       if (HALF_IN) {
-        const stream_u32x4 v = __builtin_nontemporal_load(reinterpret_cast<const stream_u32x4*>(p));
+        const stream_u32x4 v = __builtin_nontemporal_load(reinterpret_cast<const stream_u32x4*>(in_row + (on ? j0 : 0) * 2));
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
           x[u][2 * k] = half_bits_to_float((uint16_t)v[k]);
           x[u][2 * k + 1] = half_bits_to_float((uint16_t)(v[k] >> 16));
         }
       } else {
-        const stream_u32x4 a = __builtin_nontemporal_load(reinterpret_cast<const stream_u32x4*>(p));
-        const stream_u32x4 b = __builtin_nontemporal_load(reinterpret_cast<const stream_u32x4*>(p) + 1);
+        const stream_u32x4 a = __builtin_nontemporal_load(reinterpret_cast<const stream_u32x4*>(in_row + (on ? j0 : 0) * 4));
+        const stream_u32x4 b = __builtin_nontemporal_load(reinterpret_cast<const stream_u32x4*>(in_row + (on1 ? j1 : 0) * 4));
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
           x[u][k] = q_bits_to_float(a[k]);
@@ -363,9 +366,8 @@ __global__ __launch_bounds__(256) void quantize_rows_kernel(const void* input, i
       }
     }
 #pragma unroll
-    for (int u = 0; u < QROWS; ++u) {
+    for (int u = 0; u < GROUPS; ++u) {
       const int64_t row = first + u * rows_per_group + (lane >> lpr_log);
-      // lanes behind the row's last run read its first run: the same extremes
       float lo = __builtin_inff(), hi = -__builtin_inff();
 #pragma unroll
       for (int k = 0; k < RUN; ++k) {
@@ -379,10 +381,10 @@ __global__ __launch_bounds__(256) void quantize_rows_kernel(const void* input, i
       }
       if (__builtin_amdgcn_ballot_w64(lo == 0.0f || hi == 0.0f) != 0ull) { // see quantize_rowwise_kernel
         Extreme mn{0.0f, 0x7fffffff}, mx{0.0f, 0x7fffffff};
-        if (on) {
 #pragma unroll
-          for (int k = 0; k < RUN; ++k) {
-            const Extreme e{x[u][k], j0 + k};
+        for (int k = 0; k < RUN; ++k) {
+          if (k < 4 ? on : on1) {
+            const Extreme e{x[u][k], k < 4 ? j0 + k : j1 + k - 4};
             mn = mn.idx == 0x7fffffff ? e : first_min(mn, e);
             mx = mx.idx == 0x7fffffff ? e : first_max(mx, e);
           }
@@ -396,23 +398,38 @@ __global__ __launch_bounds__(256) void quantize_rows_kernel(const void* input, i
         hi = mx.v;
       }
       const RowCode code = row_code<BITS>(lo, hi, sb_float, layout);
-      uint32_t w0 = 0, w1 = 0;
+      uint32_t w0 = 0, w1 = 0; // the bytes of the first and of the second four columns (below 8 bits without QUADS: all in w0)
 #pragma unroll
       for (int k = 0; k < RUN; ++k) {
         float r = __builtin_rintf((x[u][k] - code.minimum) * code.inverse_scale); // lrintf: to nearest, ties to even
         if (!sb_float) r = r < 0.0f ? 0.0f : (r > (float)((1 << BITS) - 1) ? (float)((1 << BITS) - 1) : r);
         const uint32_t q = (uint32_t)(int)r & 0xffu;
-        if (BITS == 8 && k >= 4) w1 |= q << ((k - 4) * 8);
+        if ((QUADS || BITS == 8) && k >= 4) w1 |= q << ((k - 4) * BITS);
         else w0 |= q << (k * BITS);
       }
-      if (row < rows && on) {
-        uint8_t* out_row = output + row * out_stride;
-        if (sub == 0) {
-          uint8_t* sb = layout == 1 ? out_row : out_row + data_bytes;
-          if (code.sb_bytes == 8) store_run(sb, (uint64_t)code.sb0 | ((uint64_t)code.sb1 << 32), 8);
-          else store_run(sb, (uint64_t)(code.sb0 & 0xffffu) | ((uint64_t)(code.sb1 & 0xffffu) << 16), 4);
+      uint8_t* out_row = output + row * out_stride;
+      uint8_t* data = layout == 1 ? out_row + 4 : out_row;
+      if (row < rows && on && sub == 0) {
+        uint8_t* sb = layout == 1 ? out_row : out_row + data_bytes;
+        if (code.sb_bytes == 8) store_run(sb, (uint64_t)code.sb0 | ((uint64_t)code.sb1 << 32), 8);
+        else store_run(sb, (uint64_t)(code.sb0 & 0xffffu) | ((uint64_t)(code.sb1 & 0xffffu) << 16), 4);
+      }
+      if constexpr (!QUADS) {
+        if (row < rows && on) store_run(data + j0 * BITS / 8, (uint64_t)w0 | ((uint64_t)w1 << 32), RUN * BITS / 8);
+      } else if constexpr (BITS == 8) {
+        if (row < rows) store_run(data + j0, w0, 4);
+        if (row < rows && on1) store_run(data + j1, w1, 4);
+      } else {
+        // two lanes' quads make 4 bytes: the even lane takes both first ones, the odd lane both second ones
+        // (a row has an even number of quads, and lpr is even or the row is one lane's)
+        if (lpr == 1) {
+          if (row < rows) store_run(data, w0 | w1 << 16, 4);
+        } else {
+          const bool odd = sub & 1;
+          const uint32_t other = (uint32_t)__builtin_amdgcn_mov_dpp((int)(odd ? w0 : w1), 0xb1, 0xf, 0xf, true); // lane ^ 1
+          const uint32_t w = odd ? other | w1 << 16 : w0 | other << 16;
+          if (row < rows && (odd ? on1 : on)) store_run(data + (odd ? j1 - 4 : j0) / 2, w, 4);
         }
-        store_run((layout == 1 ? out_row + 4 : out_row) + j0 * BITS / 8, (uint64_t)w0 | ((uint64_t)w1 << 32), RUN * BITS / 8);
       }
     }
   }
@@ -672,17 +689,30 @@ hipError_t launch_quantize_rowwise(const void* input, bool half_in, int64_t rows
   if (!min_max && cols % RUN == 0 && cols <= 64 * RUN && reinterpret_cast<uintptr_t>(input) % 16 == 0) {
     int log = 0;
     while ((1 << log) < lpr) ++log;
-    const dim3 fast(stream_blocks((blocks + QROWS - 1) / QROWS));
-#define FBGEMM_AMD_LAUNCH_QR(H, B) \
-  hipLaunchKernelGGL((quantize_rows_kernel<H, B>), fast, block, 0, stream, input, rows, cols, sb_float, layout, out_stride, (uint8_t*)output, log)
+    // Quads from 64 columns on; four row groups at a time but for the quads of rows that leave lanes idle (us, 512 MB of fp32):
+    //           runs of 8, 2 groups -> the choice             2 groups -> the choice
+    //   4 bits  x 32  125.2 -> 118.0   x 128  122.5 -> 112.5    x 72  160.3 -> 157.6    x 200  134.4 -> 126.4
+    //   8 bits  x 64  133.5 -> 119.1   x 512  133.5 -> 122.6    x 96  135.2 -> 132.5    x 136  176.0 -> 169.2
+    // and of fp16 to 4 bits x 128  95.0 -> 91.1, to 8 bits x 256  97.9 -> 96.8.
+    const bool full = cols == lpr * RUN, quads = !half_in && bits >= 4 && cols >= 64;
+    const int groups = quads && !full ? 2 : 4;
+    const dim3 fast(stream_blocks((blocks + groups - 1) / groups));
+#define FBGEMM_AMD_LAUNCH_QR(H, B, QUADS, GROUPS) \
+  hipLaunchKernelGGL((quantize_rows_kernel<H, B, QUADS, GROUPS>), fast, block, 0, stream, input, rows, cols, sb_float, layout, out_stride, (uint8_t*)output, log)
     if (half_in) {
-      if (bits == 2) FBGEMM_AMD_LAUNCH_QR(true, 2);
-      else if (bits == 4) FBGEMM_AMD_LAUNCH_QR(true, 4);
-      else FBGEMM_AMD_LAUNCH_QR(true, 8);
+      if (bits == 2) FBGEMM_AMD_LAUNCH_QR(true, 2, false, 4);
+      else if (bits == 4) FBGEMM_AMD_LAUNCH_QR(true, 4, false, 4);
+      else FBGEMM_AMD_LAUNCH_QR(true, 8, false, 4);
+    } else if (!quads) {
+      if (bits == 2) FBGEMM_AMD_LAUNCH_QR(false, 2, false, 4);
+      else if (bits == 4) FBGEMM_AMD_LAUNCH_QR(false, 4, false, 4);
+      else FBGEMM_AMD_LAUNCH_QR(false, 8, false, 4);
+    } else if (full) {
+      if (bits == 4) FBGEMM_AMD_LAUNCH_QR(false, 4, true, 4);
+      else FBGEMM_AMD_LAUNCH_QR(false, 8, true, 4);
     } else {
-      if (bits == 2) FBGEMM_AMD_LAUNCH_QR(false, 2);
-      else if (bits == 4) FBGEMM_AMD_LAUNCH_QR(false, 4);
-      else FBGEMM_AMD_LAUNCH_QR(false, 8);
+      if (bits == 4) FBGEMM_AMD_LAUNCH_QR(false, 4, true, 2);
+      else FBGEMM_AMD_LAUNCH_QR(false, 8, true, 2);
     }
 #undef FBGEMM_AMD_LAUNCH_QR
     return hipGetLastError();

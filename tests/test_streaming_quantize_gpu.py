@@ -40,6 +40,25 @@ def test_quantize(ops, dtype, bits, sb_float, layout):
 
 
 @pytest.mark.parametrize("bits,sb_float,layout", FORMATS)
+def test_quantize_quads(ops, bits, sb_float, layout):
+    """fp32 rows whose lanes hold two quads apart: the widths where that begins, powers of two (four row groups at a
+    time) and widths with one lane's second quad, or all but one's, behind the row; rows off the dword grid; padded rows."""
+    for cols in (56, 64, 72, 120, 128, 136, 248, 256):
+        for rows in (1, 15, 16, 17, 130):
+            rng = np.random.default_rng(100 * cols + rows)
+            x = rng.normal(size=(rows, cols)).astype(np.float32)
+            x[rng.random(x.shape) < 0.1] *= 0
+            x[rows // 2, cols // 2:] = np.abs(x[rows // 2, cols // 2:]) + 9  # extremes in the one and in the other quad
+            want = oracle.quantize_rowwise(x, bits, sb_float, layout)
+            d = torch.from_numpy(x).cuda()
+            assert (ops.quantize_rowwise(d, bits, sb_float, layout).cpu().numpy() == want).all(), (cols, rows)
+            for pad in (1, 8):
+                out = torch.full((rows, want.shape[1] + pad), 7, dtype=torch.uint8, device="cuda")
+                ops.quantize_rowwise(d, bits, sb_float, layout, out=out)
+                assert (out[:, :-pad].cpu().numpy() == want).all() and bool((out[:, -pad:] == 7).all()), (cols, rows, pad)
+
+
+@pytest.mark.parametrize("bits,sb_float,layout", FORMATS)
 @pytest.mark.parametrize("out_ty,dtype,bits_dtype,np_bits", OUT)
 def test_dequantize(ops, out_ty, dtype, bits_dtype, np_bits, bits, sb_float, layout):
     for n, cols in enumerate((4, 8, 16, 24, 40, 48, 100, 128, 264, 2056, 65536, 65544)):
