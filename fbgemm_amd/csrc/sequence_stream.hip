@@ -8,8 +8,8 @@
 // lane's pieces in flight at once (2.5 KB a wave for 32 rows of 4 bits x 128, where four rows per
 // group of lanes are 1 KB). The decoding lanes take the output's 16-byte pieces in order, so that a
 // store instruction writes 1 KB in a row whatever the width, and unpack through half-precision
-// denormals as the pooled kernels do: 30 vector instructions per piece where sequence_lookup_kernel
-// spends 90. Waves of one segment and no more: a grid of resident waves that fetched the next rows
+// denormals as the pooled kernels do: 52 vector instructions per piece, all told, where
+// sequence_lookup_kernel spends 174. Waves of one segment and no more: a grid of resident waves that fetched the next rows
 // behind the current ones took 300 us where this takes 281.
 //   32 tables x 1 M rows of 4 bits x 128, 3.5 M positions to fp16: 431 -> 281 us; to fp32 453 us;
 //   4-bit, 8-bit and fp16 tables mixed 440 -> 315 us; 442 368 positions 56 -> 23 us, 65 536 14.8 -> 6.8.
