@@ -482,18 +482,18 @@ int clear_own_status(const OwnStatus& s, hipStream_t stream) { // waits for `str
 constexpr auto WATCH_FOR = std::chrono::milliseconds(1);
 int wait_for_stream(OwnStatus& s, hipStream_t stream) {
   hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-  if (hipStreamIsCapturing(stream, &cap) == hipSuccess && cap == hipStreamCaptureStatusNone) {
+  bool watch = hipStreamIsCapturing(stream, &cap) == hipSuccess;
+  if (watch && cap == hipStreamCaptureStatusNone) {
     s.calls = (int32_t)((uint32_t)s.calls + 1u);
-    if (launch_status_done(s.done, s.calls, stream) == hipSuccess) {
-      const auto until = std::chrono::steady_clock::now() + WATCH_FOR;
-      for (int turn = 0;; ++turn) {
-        if (__atomic_load_n(s.done, __ATOMIC_ACQUIRE) == s.calls) return 0;
-        __builtin_ia32_pause();
-        if ((turn & 63) == 63 && std::chrono::steady_clock::now() >= until) break;
-      }
+    watch = launch_status_done(s.done, s.calls, stream) == hipSuccess;
+    const auto until = std::chrono::steady_clock::now() + WATCH_FOR;
+    for (int turn = 0; watch; ++turn) {
+      if (__atomic_load_n(s.done, __ATOMIC_ACQUIRE) == s.calls) return 0;
+      __builtin_ia32_pause();
+      if ((turn & 63) == 63 && std::chrono::steady_clock::now() >= until) break;
     }
   }
-  (void)hipGetLastError();
+  if (!watch) (void)hipGetLastError(); // this function's own
   HIP_TRY(hipStreamSynchronize(stream));
   return 0;
 }
