@@ -272,35 +272,6 @@ class IntNBitTableBatchedEmbeddingBagsCodegen(torch.nn.Module):
                 foffs.append(foffs[-1] + (index_remapping[t].numel() if index_remapping[t] is not None else 0))
             self._feature_remap_array = torch.cat(parts)
             self._feature_remap_offsets = torch.tensor(foffs, device=dev, dtype=torch.int64)
-        self._rank_records, self._rank_key = None, None
-        if kept and self.bounds_check_mode_int in (BoundsCheckMode.WARNING.value, BoundsCheckMode.IGNORE.value):
-            self._ranks()
-            self._ranks()
-
-    # the compact form of the mappings (not state: copies and saved modules make their own), and what they were
-    # at the last forward
-    _rank_records = None
-    _rank_key = None
-
-    def _ranks(self):
-        """The mappings in the form the checked forward asks (ops.RankRecords), or None. They are told by address and
-        version; contents that two forwards have found the same are worth the making, those of every step are not.
-        Tensors that have no version (inference mode) have no compact form either. What is written behind the version's
-        back (``.data``, a kernel of the caller's) takes ``set_index_remappings`` to be seen."""
-        mapping, offsets = self._feature_remap_array, self._feature_remap_offsets
-        if mapping.is_inference() or offsets.is_inference():
-            return None
-        key = ops.TbePlan.rank_key(mapping, offsets)
-        ranks = self._rank_records
-        if ranks is not None and ranks.key == key:
-            return ranks
-        if self._rank_key != key:
-            self._rank_key, self._rank_records = key, None
-            return None
-        if torch.cuda.is_current_stream_capturing():
-            return None
-        self._rank_records = ranks = ops.RankRecords(mapping, offsets)
-        return ranks
 
     def set_index_remappings(self, index_remapping, pruning_hash_load_factor=0.5, use_array_for_index_remapping=True):
         if use_array_for_index_remapping:
@@ -379,7 +350,7 @@ class IntNBitTableBatchedEmbeddingBagsCodegen(torch.nn.Module):
             indices, offsets = ops.check_remap_indices(
                 self.rows_per_table, indices, offsets, self.bounds_check_mode_int, self.bounds_check_warning, per_sample_weights,
                 self.original_rows_per_table if arrayed else None, self._feature_remap_array if arrayed else None,
-                self._feature_remap_offsets if arrayed else None, self._ranks() if arrayed else None)
+                self._feature_remap_offsets if arrayed else None)
         else:
             indices, offsets = self._check_and_remap(indices, offsets, per_sample_weights, check, hashed, arrayed, fuse_remap)
         return ops.int_nbit_split_embedding_codegen_lookup_function(

@@ -296,8 +296,10 @@ class TbePlan:
 
 class RankRecords:
     """The compact form of array-based pruned-row mappings for ``check_remap_indices`` (fbgemm_amd_rank_records_create),
-    from the contents they have now: ``key`` says what they were, and whoever keeps one makes it anew when they change.
-    A copied or unpickled holder gets ``None`` in its place."""
+    from the contents they have now. Whoever makes one says with it that they stay as they are, and makes it anew when
+    they change: a write that raises the tensor's version is noticed (``key``; the array is read again), one that does
+    not (``.data``, a collective, a graph's replay, a kernel of the caller's) is not. The module keeps none: its forward
+    reads the array. A copied or unpickled holder gets ``None`` in its place."""
 
     def __init__(self, index_remappings, index_remappings_offsets):
         self.key = TbePlan.rank_key(index_remappings, index_remappings_offsets)
@@ -605,7 +607,8 @@ def check_remap_indices(rows_per_table, indices, offsets, bounds_check_mode, war
     """``bounds_check_indices`` (WARNING or IGNORE) on copies of ``indices`` and ``offsets``, which are returned;
     with ``index_remappings`` the check against the logical rows, ``pruned_array_lookup`` and the check against
     ``rows_per_table`` in one pass. ``warning`` ends as the last of those checks would leave it. ``ranks`` (RankRecords
-    of these mappings as they are now) answers in the array's place."""
+    of these mappings as they are now) answers in the array's place; made from another array, or from an earlier version
+    of this one, it is left aside."""
     _require_cuda(rows_per_table, indices, offsets, warning, weights, logical_rows_per_table, index_remappings,
                   index_remappings_offsets)
     if indices.dtype != offsets.dtype:
@@ -619,6 +622,9 @@ def check_remap_indices(rows_per_table, indices, offsets, bounds_check_mode, war
         raise RuntimeError(f"weights size {weights.size(0)} is not equal to indices size {indices.numel()}")
     rows = rows_per_table.to(torch.int64).contiguous()
     logical = offs = None
+    if ranks is not None and (index_remappings is None or index_remappings.is_inference() or index_remappings_offsets.is_inference()
+                              or ranks.key != TbePlan.rank_key(index_remappings, index_remappings_offsets)):
+        ranks = None
     if index_remappings is not None:
         logical = logical_rows_per_table.to(torch.int64).contiguous()
         offs = index_remappings_offsets.to(torch.int64).contiguous()

@@ -186,9 +186,10 @@ def test_compact_mappings(ops, mapped, dtype):
             assert all(torch.equal(g, w) for g, w in zip(got, want)) and torch.equal(w0, w1), (B, mode)
 
 
-def test_module_follows_its_mappings():
-    """A pruned module's forward with the compact form of its mappings, after they have been edited in place, set anew,
-    and in copies and saved modules."""
+@pytest.mark.parametrize("edited", [False, True])
+def test_module_follows_its_mappings(edited):
+    """A pruned module's forward after its mappings have been edited in place, set anew, and in copies and saved
+    modules; and a captured check that was handed the compact form of earlier contents."""
     import copy
     import io
 
@@ -214,12 +215,10 @@ def test_module_follows_its_mappings():
 
     maps = [mapping(), mapping()]
     m.set_index_remappings(maps)
-    assert m._rank_records is not None and m._rank_records.handle is not None
     check(m, maps)
     maps = [mapping(), mapping()]
     m.index_remappings_array.copy_(torch.cat(maps))
     check(m, maps)
-    assert m._rank_records is not None
     buf = io.BytesIO()
     torch.save(m, buf)
     buf.seek(0)
@@ -229,12 +228,17 @@ def test_module_follows_its_mappings():
         other.index_remappings_array.copy_(torch.cat(changed))
         check(other, changed)
         check(m, maps)
-    # a graph reads the array: it sees what is written there between its replays
+    # a graph reads the array: it sees what is written there between its replays; compact forms of the contents at the
+    # capture and of those before the last edit, which a capture right behind that edit leaves aside
     graph, s = torch.cuda.CUDAGraph(), torch.cuda.Stream()
     with torch.cuda.stream(s):
+        ranks = [M.ops.RankRecords(m._feature_remap_array, m._feature_remap_offsets)]
         call = lambda: M.ops.check_remap_indices(m.rows_per_table, idx, off, 1, m.bounds_check_warning, None, m.original_rows_per_table,
-                                                 m._feature_remap_array, m._feature_remap_offsets, m._ranks())
+                                                 m._feature_remap_array, m._feature_remap_offsets, ranks[0])
         call()
+        if edited:
+            maps = [mapping(), mapping()]
+            m.index_remappings_array.copy_(torch.cat(maps))
         torch.cuda.synchronize()
         with torch.cuda.graph(graph, stream=s):
             out, _ = call()
@@ -246,3 +250,45 @@ def test_module_follows_its_mappings():
         flat = torch.cat(maps)
         assert torch.equal(out, torch.where(flat < rows, flat, 0)[torch.cat([idx[:5 * B], idx[5 * B:] + 2 * rows])])
         check(m, maps)
+
+
+@pytest.mark.parametrize("mode", [1, 2])
+@pytest.mark.parametrize("write", ["data", "dlpack", "replay"])
+def test_module_sees_writes_without_a_version(write, mode):
+    """What writes the mappings without raising the tensor's version (``.data``, another view of the memory, a graph that
+    refreshes them, as collectives and kernels of the caller's do too) is seen by the next checked forward, also after
+    forwards on unchanged mappings."""
+    from fbgemm_amd import module as M
+    rng = np.random.default_rng(5)
+    rows, D, B = 300, 32, 64
+    m = M.IntNBitTableBatchedEmbeddingBagsCodegen([("", rows, D, M.SparseType.INT8, M.EmbeddingLocation.DEVICE)] * 2,
+                                                  bounds_check_mode=M.BoundsCheckMode(mode), output_dtype=M.SparseType.FP32)
+    m.fill_random_weights()
+    for _, sb in m.split_embedding_weights():
+        sb.view(torch.float16).copy_(torch.rand(rows, 2, device="cuda").half())
+    off = torch.arange(2 * B + 1, dtype=torch.int64, device="cuda") * 5
+    idx = torch.from_numpy(rng.integers(0, 2 * rows, size=10 * B)).cuda()
+    where = torch.cat([idx[:5 * B], idx[5 * B:] + 2 * rows])
+    plain = M.IntNBitTableBatchedEmbeddingBagsCodegen([("", rows, D, M.SparseType.INT8, M.EmbeddingLocation.DEVICE)] * 2,
+                                                      bounds_check_mode=M.BoundsCheckMode(mode), output_dtype=M.SparseType.FP32)
+    plain.initialize_weights()
+    plain.weights_dev.copy_(m.weights_dev)
+    maps = lambda: [torch.from_numpy(order_preserving(rng, 2 * rows, 0.4)[0]).cuda() for _ in range(2)]
+    first = maps()
+    m.set_index_remappings(first)
+    array = m.index_remappings_array
+    fresh = torch.cat(first).to(array.dtype)
+    if write == "replay":
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            array.copy_(fresh)
+        torch.cuda.synchronize()
+    for turn in range(3):
+        if turn:
+            fresh.copy_(torch.cat(maps()))
+            version = array._version
+            {"data": lambda: array.data.copy_(fresh), "dlpack": lambda: torch.from_dlpack(array).copy_(fresh),
+             "replay": lambda: graph.replay()}[write]()
+            assert array._version == version
+        for _ in range(3):
+            assert torch.equal(m(idx, off), plain(fresh[where].to(torch.int64), off)), turn
