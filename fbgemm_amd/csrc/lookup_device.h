@@ -258,11 +258,15 @@ __device__ __forceinline__ uint32_t to_bf16_bits(float f) { return (float_to_bit
 __device__ __forceinline__ uint32_t pack_bf16x2(float lo, float hi) {
   return __builtin_amdgcn_perm(float_to_bits(hi) + 0x8000u, float_to_bits(lo) + 0x8000u, 0x07060302u);
 }
-// one v_cvt_pk_f16_f32 (round to nearest even): the bits of two to_half_bits
+// One v_cvt_pk_f16_f32 (round to nearest even): the bits of two to_half_bits. A translation unit may take the two apart.
 typedef float f32x2 __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ uint32_t pack_half2(float lo, float hi) {
+#ifdef FBGEMM_AMD_HALVES_APART
+  return to_half_bits(lo) | (to_half_bits(hi) << 16);
+#else
   const f32x2 v = {lo, hi};
   return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, f16x2));
+#endif
 }
 
 // `p` on a dword boundary (2-byte stores: on their own)
