@@ -228,8 +228,11 @@ __global__ __launch_bounds__(256) void bounds_check_bags_kernel(
 //   64 tables x 32 bags x 30 entries: 16 us of copies and check -> 9.5 us (its chain of five round
 //   trips). 32 pruned tables x 4096 bags x 27: 121 us of copies, check, mapping (64.6) and check ->
 //   78 us: the random 4-byte reads of 256 MB of mappings, a line each, 6 TB/s of lines. With the
-//   compact mappings (RANKED, 8 bytes per 32 logical rows, 16 MB) 55 us, and 33 with consecutive bags
-//   on one XCD, whose L2 then holds the records of its tables.
+//   compact mappings (RANKED, 8 bytes per 32 logical rows, 16 MB) 55 us.
+// Workgroups take the bags in their order and so go round the XCDs. An eighth of the bags per XCD, whose
+// L2 would then hold its tables' records, takes 33 us there, but as long as the longest eighth takes:
+// 64 tables x 2048 bags x 30 with 50 times longer bags in the first 8 tables 25 -> 54 us without a
+// mapping, 117 -> 379 with the array, 88 -> 274 with records.
 // The warning counter is what the last of the separate checks leaves there: with a mapping the
 // second check's, which starts from zero and whose offsets are already in order.
 //
@@ -323,11 +326,7 @@ __global__ __launch_bounds__(CR_BAGS) void check_remap_kernel(CheckRemapArgs a) 
   __shared__ int64_t lds[CR_BAGS / 64];
   __shared__ int bad_count;
   const int tid = threadIdx.x;
-  // Workgroups (x, *) run on XCD x % 8. With the grid of more than one launch, a multiple of 8 wide, each
-  // XCD takes consecutive bags, an eighth of the tables, whose compact mappings then stay in its L2.
-  const unsigned block = a.carry ? (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3) : blockIdx.x;
-  const int64_t k0 = (int64_t)block * CR_BAGS;
-  if (k0 >= a.total_B) return;
+  const int64_t k0 = (int64_t)blockIdx.x * CR_BAGS;
   const int nb = (int)(a.total_B - k0 < CR_BAGS ? a.total_B - k0 : CR_BAGS);
   // every load the walk over the offsets needs, before anything waits: this bag's offset, the one
   // behind the last bag, and what the bags before these leave
@@ -400,7 +399,7 @@ __global__ __launch_bounds__(CR_BAGS) void check_remap_kernel(CheckRemapArgs a) 
     if (a.remap_offsets) bad = 0; // the second check starts from zero, and from offsets that are in order
   }
   // the indices of these bags; what lies before the first bag is nobody's and passes through
-  const int64_t lo0 = block == 0 ? 0 : fixed[0], hi0 = fixed[nb], own = fixed[0];
+  const int64_t lo0 = blockIdx.x == 0 ? 0 : fixed[0], hi0 = fixed[nb], own = fixed[0];
   const int64_t share = (hi0 - lo0 + gridDim.y - 1) / gridDim.y;
   const int64_t lo = lo0 + share * blockIdx.y;
   const int64_t hi = lo + share < hi0 ? lo + share : hi0;
@@ -598,7 +597,7 @@ hipError_t launch_check_remap(CheckRemapArgs a, bool is64, bool remap64, hipStre
   const int64_t per = a.N < (int64_t)256 * CR_LOADS * CR_BAGS ? 2 * CR_BAGS : CR_LOADS * CR_BAGS;
   int64_t shares = (a.N / blocks + per - 1) / per;
   shares = shares < 1 ? 1 : (shares > 1024 ? 1024 : shares);
-  const dim3 grid((unsigned)(a.carry ? (blocks + 7) / 8 * 8 : blocks), (unsigned)shares), block(CR_BAGS);
+  const dim3 grid((unsigned)blocks, (unsigned)shares), block(CR_BAGS);
   const bool ranked = a.remap_offsets && a.rank_records && a.rank_offsets;
 #define FBGEMM_AMD_CHECK_REMAP(INDEX_T, REMAP_T)                                                                          \
   do {                                                                                                                    \
