@@ -324,10 +324,11 @@ __global__ __launch_bounds__(256) void quantize_rowwise_kernel(
 // The common form of the above: whole rows of at most 64 runs, a multiple of 8 columns, 16-byte
 // aligned, extremes from the row. Streaming, so bound by memory: what counts is bytes in flight,
 // whole lines per request and few instructions per element. A wave takes GROUPS groups of rows at a time with all
-// their loads issued first (up to 128 bytes per lane in flight), rows stay in registers, and nothing is predicated by
-// column. QUADS (fp32 rows to 4 and 8 bits): a lane's 8 columns are two quads, lpr quads apart, so that a load
-// instruction takes whole lines, where two loads of 8 consecutive columns each take every line's half; else they are
-// consecutive. 1 M fp32 rows of 128 columns to 4 bits (608 MB): 119 -> 111 us (5.5 TB/s).
+// their loads issued first (64 or 128 bytes per lane in flight), rows stay in registers, and nothing is predicated by
+// column. QUADS (fp32 rows to 4 and 8 bits that use every lane): a lane's 8 columns are two quads, lpr quads apart, so
+// that a load instruction takes whole lines, where two loads of 8 consecutive columns each take every line's half; else
+// they are consecutive. 1 M fp32 rows of 128 columns to 4 bits (608 MB), other rows in every call: 114.6 -> 106.6 us
+// (5.7 TB/s); the launcher has the sizes at which either does not pay.
 template <bool HALF_IN, int BITS, bool QUADS, int GROUPS>
 __global__ __launch_bounds__(256) void quantize_rows_kernel(const void* input, int64_t rows, int32_t cols, int32_t sb_float,
                                                             int32_t layout, int64_t out_stride, uint8_t* output, int32_t lpr_log) {
@@ -336,7 +337,7 @@ __global__ __launch_bounds__(256) void quantize_rows_kernel(const void* input, i
   const int lpr = 1 << lpr_log, sub = lane & (lpr - 1);
   const int rows_per_group = 64 >> lpr_log;
   const int j0 = QUADS ? sub * 4 : sub * RUN, j1 = QUADS ? (sub + lpr) * 4 : j0 + 4; // first column of either half
-  const bool on = j0 < cols, on1 = j1 < cols; // QUADS: `on` holds for all lanes
+  const bool on = QUADS || j0 < cols;
   const int data_bytes = cols * BITS / 8;
   const int64_t step = (int64_t)gridDim.x * (blockDim.x >> 6) * (GROUPS * rows_per_group);
   for (int64_t first = ((int64_t)blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6)) * (GROUPS * rows_per_group); first < rows;
@@ -347,7 +348,7 @@ __global__ __launch_bounds__(256) void quantize_rows_kernel(const void* input, i
       const int64_t row_raw = first + u * rows_per_group + (lane >> lpr_log);
       const int64_t row = row_raw < rows ? row_raw : rows - 1; // lanes past the end shadow the last row and store nothing
       const uint8_t* in_row = reinterpret_cast<const uint8_t*>(input) + row * (int64_t)cols * (HALF_IN ? 2 : 4);
-      // columns behind the row's last read its first: the same extremes
+      // lanes behind the row's last run read its first: the same extremes
       if (HALF_IN) {
         const stream_u32x4 v = __builtin_nontemporal_load(reinterpret_cast<const stream_u32x4*>(in_row + (on ? j0 : 0) * 2));
 #pragma unroll
@@ -357,7 +358,7 @@ __global__ __launch_bounds__(256) void quantize_rows_kernel(const void* input, i
         }
       } else {
         const stream_u32x4 a = __builtin_nontemporal_load(reinterpret_cast<const stream_u32x4*>(in_row + (on ? j0 : 0) * 4));
-        const stream_u32x4 b = __builtin_nontemporal_load(reinterpret_cast<const stream_u32x4*>(in_row + (on1 ? j1 : 0) * 4));
+        const stream_u32x4 b = __builtin_nontemporal_load(reinterpret_cast<const stream_u32x4*>(in_row + (on ? j1 : 4) * 4));
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
           x[u][k] = q_bits_to_float(a[k]);
@@ -383,7 +384,7 @@ __global__ __launch_bounds__(256) void quantize_rows_kernel(const void* input, i
         Extreme mn{0.0f, 0x7fffffff}, mx{0.0f, 0x7fffffff};
 #pragma unroll
         for (int k = 0; k < RUN; ++k) {
-          if (k < 4 ? on : on1) {
+          if (on) {
             const Extreme e{x[u][k], k < 4 ? j0 + k : j1 + k - 4};
             mn = mn.idx == 0x7fffffff ? e : first_min(mn, e);
             mx = mx.idx == 0x7fffffff ? e : first_max(mx, e);
@@ -418,7 +419,7 @@ __global__ __launch_bounds__(256) void quantize_rows_kernel(const void* input, i
         if (row < rows && on) store_run(data + j0 * BITS / 8, (uint64_t)w0 | ((uint64_t)w1 << 32), RUN * BITS / 8);
       } else if constexpr (BITS == 8) {
         if (row < rows) store_run(data + j0, w0, 4);
-        if (row < rows && on1) store_run(data + j1, w1, 4);
+        if (row < rows) store_run(data + j1, w1, 4);
       } else {
         // two lanes' quads make 4 bytes: the even lane takes both first ones, the odd lane both second ones
         // (a row has an even number of quads, and lpr is even or the row is one lane's)
@@ -428,7 +429,7 @@ __global__ __launch_bounds__(256) void quantize_rows_kernel(const void* input, i
           const bool odd = sub & 1;
           const uint32_t other = (uint32_t)__builtin_amdgcn_mov_dpp((int)(odd ? w0 : w1), 0xb1, 0xf, 0xf, true); // lane ^ 1
           const uint32_t w = odd ? other | w1 << 16 : w0 | other << 16;
-          if (row < rows && (odd ? on1 : on)) store_run(data + (odd ? j1 - 4 : j0) / 2, w, 4);
+          if (row < rows) store_run(data + (odd ? j1 - 4 : j0) / 2, w, 4);
         }
       }
     }
@@ -689,31 +690,37 @@ hipError_t launch_quantize_rowwise(const void* input, bool half_in, int64_t rows
   if (!min_max && cols % RUN == 0 && cols <= 64 * RUN && reinterpret_cast<uintptr_t>(input) % 16 == 0) {
     int log = 0;
     while ((1 << log) < lpr) ++log;
-    // Quads from 64 columns on; four row groups at a time but for the quads of rows that leave lanes idle (us, 512 MB of fp32):
-    //           runs of 8, 2 groups -> the choice             2 groups -> the choice
-    //   4 bits  x 32  125.2 -> 118.0   x 128  122.5 -> 112.5    x 72  160.3 -> 157.6    x 200  134.4 -> 126.4
-    //   8 bits  x 64  133.5 -> 119.1   x 512  133.5 -> 122.6    x 96  135.2 -> 132.5    x 136  176.0 -> 169.2
-    // and of fp16 to 4 bits x 128  95.0 -> 91.1, to 8 bits x 256  97.9 -> 96.8.
-    const bool full = cols == lpr * RUN, quads = !half_in && bits >= 4 && cols >= 64;
-    const int groups = quads && !full ? 2 : 4;
+    // Two row groups at a time, but four in long streams of fp16 rows and of short fp32 ones; quads for fp32 rows that use
+    // all lanes, unless few. us, inputs that change from call to call, runs of 8 and 2 groups -> 4 groups / quads:
+    //   4 groups  fp16 to 4 bits   1000 x 128  4.5 -> 6.1    1 M x 64  48.0 -> 49.2    508 k x 264  177.8 -> 172.4
+    //             fp32 to 2 bits   1000 x 128  4.4 -> 6.1    1 M x 64  57.4 -> 58.7    2 M x 64     120.0 -> 112.6
+    //             fp32 to 4 bits   100 k x 128  16.2 -> 17.9 (no quads)                4 M x 32     122.6 -> 119.4
+    //   quads     fp32 to 8 bits   1000 x 128  4.35 -> 4.62  10 k x 128  5.41 -> 5.41  1 M x 128    124.9 -> 115.1
+    //             fp32 to 4 bits   1000 x 128  4.37 -> 4.41  10 k x 128  5.35 -> 5.27  1 M x 128    114.6 -> 106.6
+    //             fp32 to 8 bits   1000 x 72   4.37 -> 4.92  100 k x 72  13.6 -> 13.7  1.9 M x 72   163.2 -> 167.2
+    const int64_t elements = rows > INT64_MAX / cols ? INT64_MAX : rows * cols;
+    const bool quads = !half_in && bits >= 4 && cols >= 64 && cols == lpr * RUN && elements >= (1 << 20);
+    const int groups = !quads && (half_in || cols <= 64) && elements > (1 << 26) ? 4 : 2;
     const dim3 fast(stream_blocks((blocks + groups - 1) / groups));
 #define FBGEMM_AMD_LAUNCH_QR(H, B, QUADS, GROUPS) \
   hipLaunchKernelGGL((quantize_rows_kernel<H, B, QUADS, GROUPS>), fast, block, 0, stream, input, rows, cols, sb_float, layout, out_stride, (uint8_t*)output, log)
-    if (half_in) {
-      if (bits == 2) FBGEMM_AMD_LAUNCH_QR(true, 2, false, 4);
-      else if (bits == 4) FBGEMM_AMD_LAUNCH_QR(true, 4, false, 4);
-      else FBGEMM_AMD_LAUNCH_QR(true, 8, false, 4);
-    } else if (!quads) {
-      if (bits == 2) FBGEMM_AMD_LAUNCH_QR(false, 2, false, 4);
-      else if (bits == 4) FBGEMM_AMD_LAUNCH_QR(false, 4, false, 4);
-      else FBGEMM_AMD_LAUNCH_QR(false, 8, false, 4);
-    } else if (full) {
-      if (bits == 4) FBGEMM_AMD_LAUNCH_QR(false, 4, true, 4);
-      else FBGEMM_AMD_LAUNCH_QR(false, 8, true, 4);
-    } else {
+#define FBGEMM_AMD_LAUNCH_QR_BITS(H, GROUPS)              \
+  do {                                                    \
+    if (bits == 2) FBGEMM_AMD_LAUNCH_QR(H, 2, false, GROUPS); \
+    else if (bits == 4) FBGEMM_AMD_LAUNCH_QR(H, 4, false, GROUPS); \
+    else FBGEMM_AMD_LAUNCH_QR(H, 8, false, GROUPS);       \
+  } while (0)
+    if (quads) {
       if (bits == 4) FBGEMM_AMD_LAUNCH_QR(false, 4, true, 2);
       else FBGEMM_AMD_LAUNCH_QR(false, 8, true, 2);
+    } else if (half_in) {
+      if (groups == 4) FBGEMM_AMD_LAUNCH_QR_BITS(true, 4);
+      else FBGEMM_AMD_LAUNCH_QR_BITS(true, 2);
+    } else {
+      if (groups == 4) FBGEMM_AMD_LAUNCH_QR_BITS(false, 4);
+      else FBGEMM_AMD_LAUNCH_QR_BITS(false, 2);
     }
+#undef FBGEMM_AMD_LAUNCH_QR_BITS
 #undef FBGEMM_AMD_LAUNCH_QR
     return hipGetLastError();
   }

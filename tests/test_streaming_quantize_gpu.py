@@ -41,8 +41,8 @@ def test_quantize(ops, dtype, bits, sb_float, layout):
 
 @pytest.mark.parametrize("bits,sb_float,layout", FORMATS)
 def test_quantize_quads(ops, bits, sb_float, layout):
-    """fp32 rows whose lanes hold two quads apart: the widths where that begins, powers of two (four row groups at a
-    time) and widths with one lane's second quad, or all but one's, behind the row; rows off the dword grid; padded rows."""
+    """The widths where lanes hold two quads of an fp32 row in streams long enough (below: those), and their neighbours;
+    rows off the dword grid; padded rows."""
     for cols in (56, 64, 72, 120, 128, 136, 248, 256):
         for rows in (1, 15, 16, 17, 130):
             rng = np.random.default_rng(100 * cols + rows)
@@ -56,6 +56,32 @@ def test_quantize_quads(ops, bits, sb_float, layout):
                 out = torch.full((rows, want.shape[1] + pad), 7, dtype=torch.uint8, device="cuda")
                 ops.quantize_rowwise(d, bits, sb_float, layout, out=out)
                 assert (out[:, :-pad].cpu().numpy() == want).all() and bool((out[:, -pad:] == 7).all()), (cols, rows, pad)
+
+
+@pytest.mark.parametrize("bits,sb_float,layout", FORMATS)
+def test_quantize_quads_of_long_streams(ops, bits, sb_float, layout):
+    """The same at the sizes from which rows that use every lane are held as quads (2^20 elements), one row fewer, and a
+    last group of one row and of all but one; zeros of both signs as the extremes of either quad."""
+    for cols in (64, 128, 256, 512):
+        for rows in ((1 << 20) // cols - 1, (1 << 20) // cols, (1 << 20) // cols + 1, (1 << 20) // cols + 16 * 512 // cols - 1):
+            rng = np.random.default_rng(cols + rows)
+            x = np.abs(rng.normal(size=(rows, cols))).astype(np.float32)
+            x[rng.random(x.shape) < 0.05] *= 0
+            x[rng.random(x.shape) < 0.02] = -0.0
+            want = oracle.quantize_rowwise(x, bits, sb_float, layout)
+            for pad in (1, 8):
+                out = torch.full((rows, want.shape[1] + pad), 7, dtype=torch.uint8, device="cuda")
+                ops.quantize_rowwise(torch.from_numpy(x).cuda(), bits, sb_float, layout, out=out)
+                assert (out[:, :-pad].cpu().numpy() == want).all() and bool((out[:, -pad:] == 7).all()), (cols, rows, pad)
+
+
+@pytest.mark.parametrize("bits,sb_float,layout", FORMATS)
+@pytest.mark.parametrize("dtype,cols", [(torch.float16, 200), (torch.float16, 64), (torch.float32, 32)])
+def test_quantize_four_groups(ops, dtype, cols, bits, sb_float, layout):
+    """Streams of more than 2^26 elements take four row groups at a time: the bytes of their parts, which take two."""
+    x = torch.randn((1 << 26) // cols + 19, cols, device="cuda", generator=torch.Generator("cuda").manual_seed(cols)).to(dtype)
+    got = ops.quantize_rowwise(x, bits, sb_float, layout)
+    assert torch.equal(got, torch.cat([ops.quantize_rowwise(part, bits, sb_float, layout) for part in x.split(x.size(0) // 3 // 8 * 8)]))
 
 
 @pytest.mark.parametrize("bits,sb_float,layout", FORMATS)
