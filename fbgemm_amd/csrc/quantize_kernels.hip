@@ -421,16 +421,11 @@ __global__ __launch_bounds__(256) void quantize_rows_kernel(const void* input, i
         if (row < rows) store_run(data + j0, w0, 4);
         if (row < rows) store_run(data + j1, w1, 4);
       } else {
-        // two lanes' quads make 4 bytes: the even lane takes both first ones, the odd lane both second ones
-        // (a row has an even number of quads, and lpr is even or the row is one lane's)
-        if (lpr == 1) {
-          if (row < rows) store_run(data, w0 | w1 << 16, 4);
-        } else {
-          const bool odd = sub & 1;
-          const uint32_t other = (uint32_t)__builtin_amdgcn_mov_dpp((int)(odd ? w0 : w1), 0xb1, 0xf, 0xf, true); // lane ^ 1
-          const uint32_t w = odd ? other | w1 << 16 : w0 | other << 16;
-          if (row < rows) store_run(data + (odd ? j1 - 4 : j0) / 2, w, 4);
-        }
+        // two lanes' quads make 4 bytes: the even lane takes both first ones, the odd lane both second ones (lpr is at least 8)
+        const bool odd = sub & 1;
+        const uint32_t other = (uint32_t)__builtin_amdgcn_mov_dpp((int)(odd ? w0 : w1), 0xb1, 0xf, 0xf, true); // lane ^ 1
+        const uint32_t w = odd ? other | w1 << 16 : w0 | other << 16;
+        if (row < rows) store_run(data + (odd ? j1 - 4 : j0) / 2, w, 4);
       }
     }
   }
