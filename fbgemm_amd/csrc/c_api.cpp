@@ -1826,8 +1826,10 @@ int tbe_forward_impl(
   //   83 x 618 x 20                82.8 -> 62.4        48 x 2547 x 19  100.3 -> 81.6
   //   69 x 2201 x 3                90.1 -> 76.0        37 x 5521 x 29    271 -> 224
   // (of 40 such shapes none slower by more than 1 %). Two streams stay where the lean tables are wide 4-bit bags whose bags
-  // are ordered (55 x 3872 x 21 with a sixth of 2-bit rows: 182 against 189 us), with a mapping and with the 8-bit output.
-  if (w.lean.num_waves > 0 && w.general.num_waves > 0 && !d_index_remappings && !d_q8_out && !(w.lean_wide4 && a.order)) {
+  // are ordered (55 x 3872 x 21 with a sixth of 2-bit rows: 182 against 189 us), with a mapping and with the 8-bit output; and
+  // lists that one grid cannot hold are launched one behind the other.
+  if (w.lean.num_waves > 0 && w.general.num_waves > 0 && !d_index_remappings && !d_q8_out && !(w.lean_wide4 && a.order) &&
+      lookup_both_fits(w.general.num_waves, w.lean.num_waves)) {
     a.work = w.general.d_work;
     a.xcd_start = w.general.d_xcd_start;
     a.num_waves = w.general.num_waves;

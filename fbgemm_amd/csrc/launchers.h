@@ -10,6 +10,8 @@
 namespace fbgemm_amd {
 hipError_t launch_lookup(const LookupArgs& a, bool idx64, hipStream_t stream);
 hipError_t launch_lookup_lean(const LookupArgs& a, bool idx64, bool exact, bool wide4, hipStream_t stream);
+// A grid that holds both kernels' lists, of which each may be as long as a grid can be
+inline bool lookup_both_fits(int64_t general_waves, int64_t lean_waves) { return 8 * (general_waves + lean_waves) <= 0x7fffffffLL; }
 hipError_t launch_lookup_both(const LookupArgs& a, const WorkRun& lean, bool idx64, bool exact, hipStream_t stream);
 hipError_t launch_lookup_burst(const LookupArgs& a, bool idx64, int32_t max_D, int32_t max_bits, int waves, int lds_bytes, hipStream_t stream);
 hipError_t launch_lengths_to_offsets(const void* lengths, bool is64, int64_t n, int64_t* offsets, hipStream_t stream);

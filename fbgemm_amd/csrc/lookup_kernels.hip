@@ -2,6 +2,7 @@
 // offsets, the status block, pruned_array_lookup, and
 // the launchers the C ABI calls. The lookup kernels themselves are in
 // lookup_general.h (any shape) and compiled one instance per translation unit.
+#include "launchers.h"
 #include "lookup_device.h"
 
 namespace fbgemm_amd {
@@ -233,7 +234,7 @@ hipError_t launch_lookup_both_i32_fast(const LookupArgs& a, const WorkRun& lean,
 hipError_t launch_lookup_both(const LookupArgs& a, const WorkRun& lean, bool idx64, bool exact, hipStream_t stream) {
   const int64_t general = 8 * a.num_waves, blocks = general + 8 * lean.num_waves;
   if (blocks <= 0) return hipSuccess;
-  if (blocks > 0x7fffffffLL || !a.tables || !a.work || !a.xcd_start || !lean.work || !lean.xcd_start || a.remap || a.positional || a.check_total ||
+  if (!lookup_both_fits(a.num_waves, lean.num_waves) || !a.tables || !a.work || !a.xcd_start || !lean.work || !lean.xcd_start || a.remap || a.positional || a.check_total ||
       a.out_ty == ST_INT8)
     return hipErrorInvalidValue;
   if (exact) return idx64 ? launch_lookup_both_i64_exact(a, lean, (unsigned)general, (unsigned)blocks, stream) : launch_lookup_both_i32_exact(a, lean, (unsigned)general, (unsigned)blocks, stream);

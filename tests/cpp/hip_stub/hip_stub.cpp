@@ -214,7 +214,7 @@ hipError_t launch_lookup_lean(const LookupArgs& a, bool idx64, bool, bool wide4,
   return launch_lookup(a, idx64, s);
 }
 hipError_t launch_lookup_both(const LookupArgs& a, const WorkRun& lean, bool idx64, bool, hipStream_t s) {
-  if (!a.work || !a.xcd_start || !lean.work || !lean.xcd_start) return hipErrorInvalidValue;
+  if (!lookup_both_fits(a.num_waves, lean.num_waves) || !a.work || !a.xcd_start || !lean.work || !lean.xcd_start) return hipErrorInvalidValue;
   (void)*(volatile const int32_t*)&lean.work[0].table;
   (void)*(volatile const int64_t*)&lean.xcd_start[8];
   return launch_lookup(a, idx64, s);

@@ -16,6 +16,7 @@
 #include <vector>
 
 #include "../../include/fbgemm_amd.h"
+#include "../../fbgemm_amd/csrc/launchers.h"
 #include "../../fbgemm_amd/csrc/lookup_common.h"
 #include "../../include/fbgemm_amd_bench.h"
 
@@ -525,9 +526,17 @@ void plan_of_wide_4bit_tables() {
   }
 }
 
+// Both pooled-lookup kernels in one launch: lists that fit a grid each, and only apart
+void lists_that_one_grid_cannot_hold() {
+  const int64_t most = 0x7fffffffLL / 8; // waves of the longest run that a grid holds
+  CHECK(fbgemm_amd::lookup_both_fits(most, 0) && fbgemm_amd::lookup_both_fits(0, most) && fbgemm_amd::lookup_both_fits(most - 1, 1) && fbgemm_amd::lookup_both_fits(1000, 1000));
+  CHECK(!fbgemm_amd::lookup_both_fits(most, 1) && !fbgemm_amd::lookup_both_fits(1, most) && !fbgemm_amd::lookup_both_fits(most, most));
+}
+
 } // namespace
 
 int main() {
+  lists_that_one_grid_cannot_hold();
   plan_of_wide_4bit_tables();
   plan_create_failures();
   work_list_cache_and_graphs();
