@@ -1030,9 +1030,10 @@ struct RankSet {
 };
 
 void free_ranks(RankSet* r) {
-  if (r->records) (void)hipFree(r->records);
-  if (r->offsets) (void)hipFree(r->offsets);
-  if (r->remap_offsets) (void)hipFree(r->remap_offsets);
+  bool freed = true;
+  for (void* p : {(void*)r->records, (void*)r->offsets, (void*)r->remap_offsets})
+    if (p && hipFree(p) != hipSuccess) freed = false;
+  if (!freed) (void)hipGetLastError(); // not the next launch's
   *r = RankSet();
 }
 } // namespace
@@ -1933,11 +1934,13 @@ int build_ranks(const void* d_index_remappings, int32_t remap_bits, const int64_
     if (partial) (void)hipFree(partial);
     if (flags) (void)hipFree(flags);
   };
+  // an error is this call's result and not the next launch's: nobody needs the records
 #define HIP_TRY_DROP(expr)                                                              \
   do {                                                                                  \
     hipError_t e_ = (expr);                                                             \
     if (e_ != hipSuccess) {                                                             \
       drop();                                                                           \
+      (void)hipGetLastError();                                                          \
       return fail(FBGEMM_AMD_E_HIP, "%s: %s", #expr, hipGetErrorString(e_));            \
     }                                                                                   \
   } while (0)
@@ -1971,6 +1974,7 @@ int build_ranks(const void* d_index_remappings, int32_t remap_bits, const int64_
       if (d_first) (void)hipFree(d_first);
       if (d_offs) (void)hipFree(d_offs);
       drop();
+      (void)hipGetLastError();
       return fail(FBGEMM_AMD_E_HIP, "rank offsets: %s", hipGetErrorString(e));
     }
     *out = RankSet{records, d_first, d_offs, d_index_remappings, remap_bits, used};

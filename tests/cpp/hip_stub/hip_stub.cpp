@@ -18,6 +18,7 @@ std::set<void*> g_live;
 std::set<hipStream_t> g_capturing;
 std::atomic<long> g_total{0}, g_launches{0}, g_fail_after{-1}, g_wide4{0}, g_device_waits{0};
 std::vector<fbgemm_amd::CheckRemapArgs> g_checks; // those with a counter that have not finished
+thread_local hipError_t t_last_error = hipSuccess; // of an allocation that was made to fail
 std::atomic<int> g_last_lean_wide4{0};
 std::atomic<float> g_elapsed_general{1.0f}, g_elapsed_wide4{1.0f};
 struct Obj { int kind; };
@@ -32,6 +33,7 @@ hipError_t hipMalloc(void** p, size_t bytes) {
     g_fail_after.store(f - 1);
     if (f == 0) {
       *p = nullptr;
+      t_last_error = hipErrorOutOfMemory;
       return hipErrorOutOfMemory;
     }
   }
@@ -81,7 +83,11 @@ hipError_t hipGetDevice(int* dev) {
   *dev = 0;
   return hipSuccess;
 }
-hipError_t hipGetLastError(void) { return hipSuccess; }
+hipError_t hipGetLastError(void) {
+  const hipError_t e = t_last_error;
+  t_last_error = hipSuccess;
+  return e;
+}
 const char* hipGetErrorString(hipError_t e) { return e == hipSuccess ? "no error" : e == hipErrorOutOfMemory ? "out of memory" : "error"; }
 hipError_t hipStreamIsCapturing(hipStream_t stream, hipStreamCaptureStatus* status) {
   std::lock_guard<std::mutex> lk(g_mu);

@@ -526,6 +526,36 @@ void plan_of_wide_4bit_tables() {
   }
 }
 
+// Records of mappings, a plan's and a caller's, where an allocation fails: the call says so, leaves nothing behind, no
+// error for the next launch to find either, and works once memory is there
+void records_without_memory() {
+  const std::vector<int64_t> offs = {0, 1000, 1000, 3000};
+  void* remap = nullptr;
+  CHECK(hipMalloc(&remap, 4 * 3000) == hipSuccess);
+  Problem p = make_problem(3);
+  fbgemm_amd_tbe_plan* plan = nullptr;
+  CHECK(fbgemm_amd_tbe_plan_create(&plan, p.T, p.wo.data(), p.tys.data(), p.D_offsets.data(), nullptr, p.bytes, 0, 16) == 0);
+  const long base = hip_stub_live_allocations();
+  hipStream_t s = hip_stub_stream(2);
+  for (long k = 0; k < 5; ++k) {
+    fbgemm_amd_rank_records* ranks = nullptr;
+    hip_stub_fail_malloc_after(k);
+    CHECK(fbgemm_amd_rank_records_create(&ranks, remap, 32, offs.data(), 4, s) < 0 && !ranks);
+    CHECK(hipGetLastError() == hipSuccess);
+    hip_stub_fail_malloc_after(k);
+    CHECK(fbgemm_amd_tbe_plan_set_index_remappings(plan, remap, 32, offs.data(), 4, s) < 0);
+    hip_stub_fail_malloc_after(-1);
+    CHECK(hipGetLastError() == hipSuccess);
+    CHECK(fbgemm_amd_tbe_plan_rank_tables(plan) == 0 && hip_stub_live_allocations() == base);
+  }
+  fbgemm_amd_rank_records* ranks = nullptr;
+  CHECK(fbgemm_amd_rank_records_create(&ranks, remap, 32, offs.data(), 4, s) == 2 && ranks);
+  CHECK(fbgemm_amd_tbe_plan_set_index_remappings(plan, remap, 32, offs.data(), 4, s) == 0);
+  fbgemm_amd_rank_records_destroy(ranks);
+  fbgemm_amd_tbe_plan_destroy(plan);
+  hipFree(remap);
+}
+
 // Both pooled-lookup kernels in one launch: lists that fit a grid each, and only apart
 void lists_that_one_grid_cannot_hold() {
   const int64_t most = 0x7fffffffLL / 8; // waves of the longest run that a grid holds
@@ -537,6 +567,7 @@ void lists_that_one_grid_cannot_hold() {
 
 int main() {
   lists_that_one_grid_cannot_hold();
+  records_without_memory();
   plan_of_wide_4bit_tables();
   plan_create_failures();
   work_list_cache_and_graphs();
