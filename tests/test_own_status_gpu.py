@@ -1,6 +1,7 @@
 """Calls that wait for their result share a status block per thread that is clear between them: a
 rejected call must not be seen by the next one, nor a call that failed on its way."""
 import threading
+import time
 
 import numpy as np
 import pytest
@@ -153,18 +154,28 @@ def test_first_call_of_a_thread_beside_a_capture(oracle):
 @pytest.mark.parametrize("products", [0, 40])
 def test_waiting_call_behind_other_work(products):
     """A waiting call returns when its stream has come to its end, also where that takes longer than the host
-    watches for it (40 products of 4096 x 4096 floats are several milliseconds): what it read and wrote is then
-    free for any other stream."""
+    watches for it (40 products of 4096 x 4096 floats are tens of milliseconds): an event recorded before the call is
+    over, and what the last of the work before it wrote is there for a kernel and for a copy of another stream."""
     ops, call, good, bad = single_table_calls()
     x = torch.ones(4096, 4096, device="cuda") / 4096
-    y, other = torch.empty_like(x), torch.cuda.Stream()
+    product, y, other = torch.empty_like(x), torch.zeros_like(x), torch.cuda.Stream()
+    host = torch.empty(x.shape, pin_memory=True)
     torch.cuda.synchronize()
-    for _ in range(3):
-        y.zero_()
+    for turn in range(1, 4):
         for _ in range(products):
-            torch.mm(x, x, out=y)
+            torch.mm(x, x, out=product)
+        y.fill_(turn)
+        before = torch.cuda.Event()
+        before.record()
         assert call(good) is True
+        # the event's signal is written before the word the call waits for, by another unit: far less than a product apart
+        until = time.perf_counter() + 1e-4
+        while not before.query() and time.perf_counter() < until:
+            pass
+        assert before.query()
         with torch.cuda.stream(other):
-            # row sums of the product of two matrices of 1 / 4096: 4096 / 4096 per row
-            assert float(y.sum(1).max()) == pytest.approx(1.0 if products else 0.0, abs=1e-5)
+            host.copy_(y, non_blocking=True)
+            assert bool((y == turn).all())
+            other.synchronize()
+        assert bool((host == turn).all())
         assert call(bad) is False
