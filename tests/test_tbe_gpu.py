@@ -418,22 +418,26 @@ def test_no_pooling_at_the_edges_of_what_a_wave_takes(ops, oracle, D, out_ty):
     _no_pooling_case(ops, oracle, rng, specs, 9001, 12, np.int64, 16, out_ty, f"D={D} out={out_ty} large")
 
 
-def test_no_pooling_more_positions_than_one_pass_of_the_grid(ops, oracle):
-    """Rows of 512 columns take a whole wave; 300 K positions are more than the largest grid covers at once, so
-    every wave walks several groups and uses the indices it fetched one group ahead."""
+@pytest.mark.parametrize("row_alignment", [4, 16])
+def test_no_pooling_more_positions_than_one_pass_of_the_grid(ops, oracle, row_alignment):
+    """Rows of 512 columns off the 16-byte grid (sequence_lookup_kernel) take a whole wave; 300 K positions are more than
+    the largest grid covers at once, so every wave walks several groups and uses the indices it fetched one group ahead.
+    Rows on that grid (sequence_stream_kernel) take as many waves as there are positions."""
     rng = np.random.default_rng(31)
     specs = [(500, 512, INT4), (300, 512, INT8), (200, 512, INT4)]
-    _no_pooling_case(ops, oracle, rng, specs, 2500, 80, np.int64, 16, FP16, "300 K positions of 512 columns")
+    _no_pooling_case(ops, oracle, rng, specs, 2500, 80, np.int64, row_alignment, FP16, "300 K positions of 512 columns")
 
 
-def test_no_pooling_with_more_tables_than_the_kernel_keeps_in_lds(ops, oracle):
-    """1100 small tables (some without any index): the table boundaries no longer fit the
-    workgroup's LDS and the bisection reads them from memory."""
+@pytest.mark.parametrize("row_alignment", [4, 16])
+def test_no_pooling_with_more_tables_than_the_kernel_keeps_in_lds(ops, oracle, row_alignment):
+    """1100 small tables (some without any index). Off the 16-byte grid (sequence_lookup_kernel) the table boundaries no
+    longer fit the workgroup's LDS and the bisection reads them from memory; on it (sequence_stream_kernel) a wave finds
+    its table in two steps of 64."""
     rng = np.random.default_rng(990)
     D, T, B = 32, 1100, 2
     tys = [INT4, INT8, FP16]
     specs = [(int(rng.integers(3, 12)), D, tys[t % 3]) for t in range(T)]
-    weights, wo, _ = build_weights(rng, specs, 16)
+    weights, wo, _ = build_weights(rng, specs, row_alignment)
     lens = rng.integers(0, 4, size=T * B)
     lens[5 * B:9 * B] = 0
     off = np.concatenate([[0], np.cumsum(lens)]).astype(np.int64)
@@ -442,8 +446,8 @@ def test_no_pooling_with_more_tables_than_the_kernel_keeps_in_lds(ops, oracle):
     D_offsets = (np.arange(T + 1) * D).astype(np.int32)
     got = ops.int_nbit_split_embedding_codegen_lookup_function(
         cu(weights), torch.zeros(0, dtype=torch.uint8, device="cuda"), cu(np.zeros(T, np.int32)), cu(wo), cu(wt),
-        cu(D_offsets), T * D, 0, D, D, D, 0, cu(idx), cu(off), ops.POOL_NONE, None, FP32, row_alignment=16)
-    ok, want = oracle.tbe_forward_nobag(weights, wo, wt, [s[0] for s in specs], D, idx, off, FP32, 16)
+        cu(D_offsets), T * D, 0, D, D, D, 0, cu(idx), cu(off), ops.POOL_NONE, None, FP32, row_alignment=row_alignment)
+    ok, want = oracle.tbe_forward_nobag(weights, wo, wt, [s[0] for s in specs], D, idx, off, FP32, row_alignment)
     assert ok
     H.assert_same_bits(got.cpu().numpy(), want, "no pooling, 1100 tables")
 
