@@ -104,24 +104,31 @@ def test_forward_replays_from_a_graph(oracle):
     H.assert_same_bits(again.cpu().view(torch.int16).numpy().view(np.uint16), want, "eager after trim")
 
 
-def test_forward_with_both_kernels_replays_from_a_graph(oracle):
+@pytest.mark.parametrize("route,dims,B,L", [("one launch", (128, 64), 16384, 33), ("side stream", (256, 256), 28000, 19),
+                                            ("narrow lanes", (128, 64), 4096, 130)])
+def test_forward_with_both_kernels_replays_from_a_graph(oracle, route, dims, B, L):
     """A forward large enough to order its bags, over tables for both lookup kernels (4-bit rows of a
-    lean shape, and 2-bit / odd-width rows): the general kernel runs on the plan's side stream beside
-    the lean one (event fork and join). Captured, that is a graph with two branches; every replay is
-    checked against the oracle, with eager forwards of the same plan in between."""
+    lean shape, and 2-bit / odd-width rows): one launch of both. Where all lean tables have wide 4-bit
+    rows in bags too short to be laid end to end, the general kernel runs on the plan's side stream
+    beside the lean one (event fork and join), which captured is a graph with two branches. With few
+    bags all tables take the general kernel's 4-byte lanes. Every replay is checked against the oracle,
+    with eager forwards of the same plan in between."""
     assert torch.cuda.is_available()
     from fbgemm_amd import ops
     from helpers import INT2
     from test_tbe_gpu import build_weights
     rng = np.random.default_rng(77)
-    specs = [(3000, 128, INT4), (500, 32, INT2), (2000, 64, INT4), (700, 40, INT4)]
-    T, B, L = len(specs), 4096, 130  # 2.13 M lookups: the scheduler runs, and with it the side stream
+    odd = INT2 if route == "side stream" else INT4  # 40 columns of 4 bits are the lean kernel's, and not wide
+    specs = [(3000, dims[0], INT4), (500, 32, INT2), (2000, dims[1], INT4), (700, 40, odd)]
+    T = len(specs)  # 2.1 M lookups: the scheduler runs
     weights, wo, _ = build_weights(rng, specs, 16)
     tys = np.array([s[2] for s in specs], np.uint8)
     D_offsets = np.concatenate([[0], np.cumsum([s[1] for s in specs])]).astype(np.int32)
     total_D = int(D_offsets[-1])
-    lens = rng.integers(L - 30, L + 31, size=T * B)
-    lens[-1] += T * B * L - int(lens.sum())
+    spread = L // 4
+    lens = rng.integers(L - spread, L + spread + 1, size=T * B)
+    short = max((1 << 21) - int(lens.sum()), 0)
+    lens[:short] += 1
     off = np.concatenate([[0], np.cumsum(lens)]).astype(np.int64)
     n = int(off[-1])
     assert n >= 1 << 21
@@ -134,7 +141,7 @@ def test_forward_with_both_kernels_replays_from_a_graph(oracle):
     meta = (cu(weights), torch.zeros(0, dtype=torch.uint8, device="cuda"), cu(np.zeros(T, np.int32)), cu(wo), cu(tys), cu(D_offsets))
     st = ops.Status()
     call = lambda: ops.int_nbit_split_embedding_codegen_lookup_function(
-        *meta, total_D, 32, 128, 0, 0, 0, d_idx, d_off, 0, None, FP16, row_alignment=16, status=st)
+        *meta, total_D, 40 if odd == INT2 else 32, dims[0], 0, 0, 0, d_idx, d_off, 0, None, FP16, row_alignment=16, status=st)
 
     def expect(idx):
         rc, want = oracle.tbe_forward(weights, wo, tys, D_offsets, total_D, idx, off, 0, None, FP16, 16)
