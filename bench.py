@@ -93,12 +93,12 @@ def parse():
 
 
 # the lookup kernels of a forward as the summaries name them (the last one is the general kernel)
-LOOKUP_KERNELS = ("lookup_lean_kernel", "lookup_lean_wide4_kernel", "lookup_lean_wide4_redo_kernel", "lookup_kernel")
+LOOKUP_KERNELS = ("lookup_lean_kernel", "lookup_lean_wide4_kernel", "lookup_lean_wide4_redo_kernel", "lookup_both_kernel", "lookup_kernel")
 
 
 def traffic_from_profile(config_id):
     """HBM bytes the lookup kernels of one forward move (lookup_lean_kernel, and lookup_kernel for
-    the tables the lean kernel does not take), from the committed hardware-counter
+    the tables the lean kernel does not take; or both as lookup_both_kernel), from the committed hardware-counter
     summary of this configuration (profiles/lookup_kernel_config<N>.txt): FETCH_SIZE
     and WRITE_SIZE (KiB per dispatch), each scaled by what the same counter read
     for the plain copy of known size that ran in the same process. None when the
@@ -138,13 +138,13 @@ def profile_kernel_us(config_id):
     calls = {k: int(c) for k, c, _ in rows}
     total = {k: int(c) * float(v) for k, c, v in rows}
     # every forward launches one of the two lean kernels (the trace holds both while the plan is still
-    # choosing between them); the redo kernel goes with the four-wave instance
-    forwards = calls.get("lookup_lean_kernel", 0) + calls.get("lookup_lean_wide4_kernel", 0)
+    # choosing between them) or the launch of both kernels; the redo kernel goes with the four-wave instance
+    forwards = sum(calls.get(k, 0) for k in ("lookup_lean_kernel", "lookup_lean_wide4_kernel", "lookup_both_kernel"))
     lean = sum(total.get(k, 0.0) for k in LOOKUP_KERNELS[:-1]) / forwards if forwards else 0.0
     general = total.get("lookup_kernel", 0.0) / calls["lookup_kernel"] if calls.get("lookup_kernel") else 0.0
     if not lean and not general:
         return None
-    # with kernels of both kinds the general one runs beside the lean one (side stream): the longer of the two
+    # a general kernel of its own runs beside the lean one (side stream): the longer of the two
     return round(max(lean, general) / 1e3, 2)
 
 
@@ -691,7 +691,7 @@ def side_op(a):
         st = ops.Status()
         launch = lambda: ops.int_nbit_split_embedding_codegen_lookup_function(*args, row_alignment=16, status=st)
         alg_bytes, units = n * (D // 2 + 4 + D * 2 + 8), n
-        kernel, workload = "sequence_lookup_kernel", f"PoolingMode.NONE, {T} int4 tables x {E} rows x {D}, {n} int64 indices -> fp16 rows (output allocated per call)"
+        kernel, workload = "sequence_stream_kernel", f"PoolingMode.NONE, {T} int4 tables x {E} rows x {D}, {n} int64 indices -> fp16 rows (output allocated per call)"
     else:
         T, B = 32, max(1, int(4096 * a.scale))
         E = max(1000, int(2_000_000 * a.scale))
@@ -873,7 +873,7 @@ def time_tbe(p, a, torch, np, steps, warmup, graph, accumulate):
         bits, pos = st.read()
         assert bits == 0, f"the lookup rejected its inputs: status {bits:#x} at {pos}"
         kernel_ms = k0.elapsed_time(k1) / steps
-        kernel_name = "lookup_lean_kernel or lookup_lean_wide4_kernel (+ lookup_kernel for tables of other shapes, beside it), back to back"
+        kernel_name = "lookup_lean_kernel or lookup_lean_wide4_kernel (+ lookup_kernel for tables of other shapes, beside it or as lookup_both_kernel), back to back"
     return {"ms_per_step": ms_per_step, "forward_ms": forward_ms, "kernel_ms": kernel_ms, "kernel": kernel_name,
             "checked": checked}
 
