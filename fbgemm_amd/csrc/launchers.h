@@ -18,6 +18,7 @@ hipError_t launch_lengths_to_offsets(const void* lengths, bool is64, int64_t n, 
 hipError_t launch_status_report(Status* st, int32_t bits, hipStream_t stream);
 hipError_t launch_status_clear(Status* st, int32_t mark, hipStream_t stream); // mark: what `pad` becomes
 hipError_t launch_status_done(int32_t* word, int32_t number, hipStream_t stream); // pinned host word := number, behind the stream's work
+hipError_t launch_status_counted(FlaggedStatus* st, int64_t* warning, hipStream_t stream); // *warning := st->counted := 0
 hipError_t launch_bag_order(const void* offsets, bool off64, int32_t B, int32_t T, BagEntry* order, hipStream_t stream);
 hipError_t launch_sequence_lookup(const TableDesc* tables, const uint8_t* w0, const uint8_t* w1, const void* indices,
                                   bool idx64, const void* offsets, int32_t B, int32_t T, int64_t total_L, int32_t D,

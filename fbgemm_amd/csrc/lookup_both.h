@@ -11,8 +11,8 @@
 
 namespace fbgemm_amd {
 
-// One instance per index type and arithmetic. `a` carries the general tables' list, `lean` the other one.
-template <typename index_t, bool EXACT>
+// One instance per index type and arithmetic, and those of checked forwards. `a` carries the general tables' list, `lean` the other one.
+template <typename index_t, bool EXACT, bool CHECKED>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(FBGEMM_AMD_MIN_WAVES, 8))) void lookup_both_kernel(const LookupArgs a, const WorkRun lean,
                                                                                                                      unsigned general_blocks) {
   constexpr int ROW_WORDS = MAX_GROUPS * MAX_ROUND * (int)sizeof(StageRow) / 4, MUL_WORDS = MAX_GROUPS * MAX_ROUND * (int)sizeof(StageMul) / 4;
@@ -31,15 +31,15 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(FBGEMM_AMD_M
   if (general) {
     StageRow* stage_row = reinterpret_cast<StageRow*>(lds);
     StageMul* stage_mul = reinterpret_cast<StageMul*>(lds + ROW_WORDS);
-    run_table<index_t, false>(a, d, ww.table, ww.first_bag, lane, stage_row, stage_mul);
+    run_table<index_t, false, CHECKED>(a, d, ww.table, ww.first_bag, lane, stage_row, stage_mul);
   } else {
-    lean_dispatch<index_t, EXACT, false>(a, d, ww.table, ww.first_bag, lane, lds);
+    lean_dispatch<index_t, EXACT, false, CHECKED>(a, d, ww.table, ww.first_bag, lane, lds);
   }
 }
 
-#define FBGEMM_AMD_DEFINE_LOOKUP_BOTH_LAUNCH(FN, INDEX_T, EXACT)                                                                  \
+#define FBGEMM_AMD_DEFINE_LOOKUP_BOTH_LAUNCH(FN, INDEX_T, EXACT, CHECKED)                                                         \
   hipError_t FN(const LookupArgs& a, const WorkRun& lean, unsigned general_blocks, unsigned blocks, hipStream_t stream) {         \
-    hipLaunchKernelGGL((lookup_both_kernel<INDEX_T, EXACT>), dim3(blocks), dim3(64), 0, stream, a, lean, general_blocks);         \
+    hipLaunchKernelGGL((lookup_both_kernel<INDEX_T, EXACT, CHECKED>), dim3(blocks), dim3(64), 0, stream, a, lean, general_blocks); \
     return hipGetLastError();                                                                                                     \
   }
 

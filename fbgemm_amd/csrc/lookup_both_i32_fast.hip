@@ -2,5 +2,5 @@
 #include "lookup_both.h"
 
 namespace fbgemm_amd {
-FBGEMM_AMD_DEFINE_LOOKUP_BOTH_LAUNCH(launch_lookup_both_i32_fast, int32_t, false)
+FBGEMM_AMD_DEFINE_LOOKUP_BOTH_LAUNCH(launch_lookup_both_i32_fast, int32_t, false, false)
 } // namespace fbgemm_amd

@@ -2,5 +2,5 @@
 #include "lookup_both.h"
 
 namespace fbgemm_amd {
-FBGEMM_AMD_DEFINE_LOOKUP_BOTH_LAUNCH(launch_lookup_both_i64_exact, int64_t, true)
+FBGEMM_AMD_DEFINE_LOOKUP_BOTH_LAUNCH(launch_lookup_both_i64_exact, int64_t, true, false)
 } // namespace fbgemm_amd

@@ -178,7 +178,8 @@ __device__ __forceinline__ void burst_store(const LookupArgs& a, const float (&a
 }
 
 // blockIdx: (bag, table, window of columns)
-template <typename index_t, int WAVES>
+// CHECKED: a checked forward's launch (LookupArgs::check_rows); the other instance keeps its registers and its time.
+template <typename index_t, int WAVES, bool CHECKED>
 __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(WAVES == 1 ? 5 : 4, 8))) void lookup_burst_kernel(const LookupArgs a, int lds_bytes) {
   constexpr int THREADS = 64 * WAVES;
   constexpr int K = BURST_COLS / THREADS; // columns per lane
@@ -211,7 +212,11 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(WAVE
     len = 0;
   }
   if (a.check_total && bag == a.B - 1 && o1 - base != a.index_size && tid == 0) report(a.status, ERR_LENGTH_MISMATCH);
+  if (CHECKED && table == a.T - 1 && bag == a.B - 1 && tid == 0) check_end(a, o1);
   const int n = (int)len;
+  const int64_t row_bound = index_bound<CHECKED>(a, d, table, tid == 0);
+  const int64_t logical = CHECKED && a.remap ? a.logical_rows[table] : 0;
+  int counted = 0; // a checked forward: this thread's indices outside the table
 
   int64_t remap_base = 0, remap_cap = 0, rank_base = -1;
   bool remapped = false;
@@ -272,9 +277,10 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(WAVE
       if (tid < left) {
         const int64_t pos = pos0 + r0 + tid;
         bool ok = true;
+        if (CHECKED && a.remap) row = logical_index(row, logical);
         if (remapped) {
           if (row < 0 || row >= remap_cap) {
-            report_index(a.status, pos);
+            if (!CHECKED) report_index(a.status, pos);
             ok = false;
           } else {
             if (rank_base >= 0) {
@@ -290,9 +296,14 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(WAVE
         } else if (d.skip_minus_one && row == -1) {
           ok = false;
         }
-        if (ok && (row < 0 || row >= d.num_rows)) {
-          report_index(a.status, pos);
-          ok = false;
+        if (ok && (row < 0 || row >= row_bound)) {
+          if (CHECKED) {
+            ++counted;
+            row = 0;
+          } else {
+            report_index(a.status, pos);
+            ok = false;
+          }
         }
         if (ok) off = row * d.row_stride;
       }
@@ -332,6 +343,7 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(WAVE
     }
     if (r0 + cap < n) __syncthreads(); // the staged rows are free again
   }
+  if (CHECKED && counted && a.warning && blockIdx.z == 0) status_count(a.status, counted);
   if (a.normalize && n > 0) {
     const float inv = 1.0f / (float)n;
 #pragma unroll
@@ -345,8 +357,14 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(WAVE
 #define FBGEMM_AMD_DEFINE_LOOKUP_BURST_LAUNCH(FN, INDEX_T)                                                  \
   hipError_t FN(const LookupArgs& a, dim3 grid, bool four_waves, int lds_bytes, hipStream_t stream) {       \
     const unsigned lds = (unsigned)((four_waves ? 256 : 64) * (sizeof(StageRow) + sizeof(StageMul)) + lds_bytes + 16); \
-    if (four_waves) hipLaunchKernelGGL((lookup_burst_kernel<INDEX_T, 4>), grid, dim3(256), lds, stream, a, lds_bytes); \
-    else hipLaunchKernelGGL((lookup_burst_kernel<INDEX_T, 1>), grid, dim3(64), lds, stream, a, lds_bytes);  \
+    if (a.check_rows) {                                                                                     \
+      if (four_waves) hipLaunchKernelGGL((lookup_burst_kernel<INDEX_T, 4, true>), grid, dim3(256), lds, stream, a, lds_bytes); \
+      else hipLaunchKernelGGL((lookup_burst_kernel<INDEX_T, 1, true>), grid, dim3(64), lds, stream, a, lds_bytes); \
+    } else if (four_waves) {                                                                                \
+      hipLaunchKernelGGL((lookup_burst_kernel<INDEX_T, 4, false>), grid, dim3(256), lds, stream, a, lds_bytes); \
+    } else {                                                                                                \
+      hipLaunchKernelGGL((lookup_burst_kernel<INDEX_T, 1, false>), grid, dim3(64), lds, stream, a, lds_bytes); \
+    }                                                                                                       \
     return hipGetLastError();                                                                               \
   }
 

@@ -38,10 +38,14 @@ struct Status {
 // says that a pinned host word follows, which every report sets besides. The host then reads that
 // word after its wait, and neither clears the block before the call nor copies it back after it
 // unless something was reported: two operations on the stream less per call.
+// `counted` is where a checked forward adds up the indices it has repaired; the word STATUS_COUNTED
+// words behind the flag says that it is not zero.
 constexpr int32_t STATUS_FLAGGED = 0x464c4147;
+constexpr int STATUS_COUNTED = 4;
 struct FlaggedStatus {
   Status st;
   int32_t* flag;
+  unsigned long long counted;
 };
 
 #if defined(__HIPCC__)
@@ -53,6 +57,12 @@ __device__ __forceinline__ void status_or(Status* st, int32_t bits) {
 __device__ __forceinline__ void status_index(Status* st, int64_t pos) {
   atomicMin(&st->first_bad_pos, (unsigned long long)pos);
   status_or(st, ERR_INDEX_OUT_OF_RANGE);
+}
+// Checked forwards only, whose block is a FlaggedStatus.
+__device__ __forceinline__ void status_count(Status* st, int n) {
+  FlaggedStatus* fs = reinterpret_cast<FlaggedStatus*>(st);
+  atomicAdd(&fs->counted, (unsigned long long)n);
+  __hip_atomic_store(fs->flag + STATUS_COUNTED, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 #endif
 
@@ -194,6 +204,11 @@ struct LookupArgs {
   WaveWork* redo;
   int32_t* redo_count;
   Status* status;
+  // A checked forward (fbgemm_amd_tbe_forward_checked): an index outside its table reads row 0 and is counted instead of
+  // reported; offsets that are not in order from 0 to index_size are reported.
+  const int64_t* check_rows;   // T row counts, or nullptr: not checked
+  const int64_t* logical_rows; // T row counts before pruning, with `remap` only
+  int64_t* warning;            // set to zero by the launch; nullptr: nothing is counted
 };
 
 // The burst kernel's windows of columns, the bytes of a staged row of the widest window of a launch,

@@ -385,6 +385,26 @@ struct __attribute__((aligned(8))) StageMul {
   float bias;  // w * row bias
 };
 
+// The rows an index of `table` may name; in a checked forward the table's own count, which the caller holds and which may
+// be less than what the weights buffer has room for. A count that cannot be right makes the caller look at it.
+template <bool CHECKED = true>
+__device__ __forceinline__ int64_t index_bound(const LookupArgs& a, const TableDesc& d, int table, bool reporter) {
+  if (!CHECKED || !a.check_rows) return d.num_rows;
+  const int64_t rows = a.check_rows[table];
+  if (rows > 0 && rows <= d.num_rows) return rows;
+  if (reporter) report(a.status, ERR_INDEX_OUT_OF_RANGE);
+  return d.num_rows;
+}
+// One thread of a checked forward, at the last bag of all, which ends at `end`.
+__device__ __forceinline__ void check_end(const LookupArgs& a, int64_t end) {
+  if (end != a.index_size) report(a.status, ERR_LENGTH_MISMATCH);
+  if (a.warning) *a.warning = 0;
+}
+// What the check of a pruned table does to an index before the mapping: outside the rows before pruning it is row 0.
+__device__ __forceinline__ int64_t logical_index(int64_t row, int64_t logical_rows) {
+  return row != -1 && (row < 0 || row >= logical_rows) ? 0 : row;
+}
+
 constexpr int MAX_GROUPS = 32; // bags per wave at most; lanes per bag >= 2
 constexpr int MAX_ROUND = 8;
 constexpr int64_t NO_ENTRY = INT64_MIN;

@@ -44,7 +44,7 @@ namespace fbgemm_amd {
 // permute. `lanes` then need not divide 64; the lanes left over shadow the last
 // bag of the wave (same addresses, nothing written), and so do chunk slots past
 // the end of the row.
-template <typename index_t, bool GENERAL, int TY, int VB, int C, int ROUND, bool PRESCALE, bool INHDR = false>
+template <typename index_t, bool GENERAL, bool CHECKED, int TY, int VB, int C, int ROUND, bool PRESCALE, bool INHDR = false>
 __device__ __forceinline__ bool pool_bags(const LookupArgs& a, const TableDesc& d, int table, int first_slot,
                                           int lane, StageRow* stage_row, StageMul* stage_mul) {
   constexpr int BITS = type_bits(TY);
@@ -124,6 +124,7 @@ __device__ __forceinline__ bool pool_bags(const LookupArgs& a, const TableDesc& 
     }
     if (GENERAL && a.check_total && bag == a.B - 1 && o1 - base != a.index_size && reporter)
       report(a.status, ERR_LENGTH_MISMATCH);
+    if (CHECKED && table == a.T - 1 && bag == a.B - 1 && reporter) check_end(a, o1);
   }
   const int n = (int)len; // same for every lane of the bag
 
@@ -140,6 +141,9 @@ __device__ __forceinline__ bool pool_bags(const LookupArgs& a, const TableDesc& 
       if (a.rank_records) rank_base = a.rank_offsets[table];
     }
   }
+
+  const int64_t row_bound = index_bound<CHECKED>(a, d, table, lane == 0);
+  int counted = 0; // a checked forward: this lane's indices outside the table
 
   const index_t* idx = reinterpret_cast<const index_t*>(a.indices);
   const uint8_t* wbase = (d.placement ? a.weights[1] : a.weights[0]) + d.weights_offset;
@@ -215,16 +219,18 @@ __device__ __forceinline__ bool pool_bags(const LookupArgs& a, const TableDesc& 
                                 : (int64_t) reinterpret_cast<const int32_t*>(a.remap)[remap_base + row];
               }
               ok = row != -1;
-              if (ok && (row < 0 || row >= d.num_rows)) {
-                if (pass == 0) report_index(a.status, pos);
-                ok = false;
-              }
             }
           } else if (d.skip_minus_one && row == -1) {
             ok = false;
-          } else if (row < 0 || row >= d.num_rows) {
-            if (pass == 0) report_index(a.status, pos);
-            ok = false;
+          }
+          if (ok && (row < 0 || row >= row_bound)) {
+            if (CHECKED) {
+              counted += pass == 0 ? 1 : 0;
+              row = 0;
+            } else {
+              if (pass == 0) report_index(a.status, pos);
+              ok = false;
+            }
           }
           if (ok) off = row * d.row_stride;
         }
@@ -401,17 +407,18 @@ __device__ __forceinline__ bool pool_bags(const LookupArgs& a, const TableDesc& 
       }
     }
   }
+  if (CHECKED && counted && a.warning) status_count(a.status, counted); // here: a wave that gives up starts over
   return true;
 }
 
-template <typename index_t, bool GENERAL, int TY, int VB, int C, int ROUND, bool INHDR = false>
+template <typename index_t, bool GENERAL, bool CHECKED, int TY, int VB, int C, int ROUND, bool INHDR = false>
 __device__ __forceinline__ void run_bags(const LookupArgs& a, const TableDesc& d, int table, int first_slot, int lane,
                                          StageRow* stage_row, StageMul* stage_mul) {
   if constexpr (Accum<TY, VB>::kPrescaled) {
-    if (!pool_bags<index_t, GENERAL, TY, VB, C, ROUND, true, INHDR>(a, d, table, first_slot, lane, stage_row, stage_mul))
-      pool_bags<index_t, GENERAL, TY, VB, C, ROUND, false, INHDR>(a, d, table, first_slot, lane, stage_row, stage_mul);
+    if (!pool_bags<index_t, GENERAL, CHECKED, TY, VB, C, ROUND, true, INHDR>(a, d, table, first_slot, lane, stage_row, stage_mul))
+      pool_bags<index_t, GENERAL, CHECKED, TY, VB, C, ROUND, false, INHDR>(a, d, table, first_slot, lane, stage_row, stage_mul);
   } else {
-    pool_bags<index_t, GENERAL, TY, VB, C, ROUND, true, INHDR>(a, d, table, first_slot, lane, stage_row, stage_mul);
+    pool_bags<index_t, GENERAL, CHECKED, TY, VB, C, ROUND, true, INHDR>(a, d, table, first_slot, lane, stage_row, stage_mul);
   }
 }
 
@@ -419,7 +426,7 @@ __device__ __forceinline__ void run_bags(const LookupArgs& a, const TableDesc& d
 // TableDesc::chunks): 16-byte chunks with up to 4 (fp16 / bf16 / fp32), 2
 // (int8) or 1 (int4) chunks per lane so that a lane holds at most 32
 // accumulators; 8-byte ones for 2-bit rows; 4-byte and element-sized chunks for everything else.
-template <typename index_t, bool GENERAL, int TY>
+template <typename index_t, bool GENERAL, bool CHECKED, int TY>
 __device__ __forceinline__ void pool_dispatch_vb(const LookupArgs& a, const TableDesc& d, int table, int first_slot,
                                                  int lane, StageRow* stage_row, StageMul* stage_mul) {
   constexpr int BITS = type_bits(TY);
@@ -428,8 +435,8 @@ __device__ __forceinline__ void pool_dispatch_vb(const LookupArgs& a, const Tabl
   // rows in flight per lane: ROUND * chunks = 8 loads of 16 bytes
   if constexpr (TY == ST_INT4 || TY == ST_INT8) {
     if (d.inline_hdr) {
-      if (d.chunks == 2 && MAXC >= 2) run_bags<index_t, GENERAL, TY, 16, (MAXC >= 2 ? 2 : 1), 4, true>(a, d, table, first_slot, lane, stage_row, stage_mul);
-      else run_bags<index_t, GENERAL, TY, 16, 1, 8, true>(a, d, table, first_slot, lane, stage_row, stage_mul);
+      if (d.chunks == 2 && MAXC >= 2) run_bags<index_t, GENERAL, CHECKED, TY, 16, (MAXC >= 2 ? 2 : 1), 4, true>(a, d, table, first_slot, lane, stage_row, stage_mul);
+      else run_bags<index_t, GENERAL, CHECKED, TY, 16, 1, 8, true>(a, d, table, first_slot, lane, stage_row, stage_mul);
       return;
     }
   }
@@ -437,16 +444,16 @@ __device__ __forceinline__ void pool_dispatch_vb(const LookupArgs& a, const Tabl
     if constexpr (TY == ST_INT2) {
       // not selected by the host
     } else {
-      if (d.chunks == 4 && MAXC >= 4) run_bags<index_t, GENERAL, TY, 16, (MAXC >= 4 ? 4 : 1), 2>(a, d, table, first_slot, lane, stage_row, stage_mul);
-      else if (d.chunks == 2 && MAXC >= 2) run_bags<index_t, GENERAL, TY, 16, (MAXC >= 2 ? 2 : 1), 4>(a, d, table, first_slot, lane, stage_row, stage_mul);
-      else run_bags<index_t, GENERAL, TY, 16, 1, 8>(a, d, table, first_slot, lane, stage_row, stage_mul);
+      if (d.chunks == 4 && MAXC >= 4) run_bags<index_t, GENERAL, CHECKED, TY, 16, (MAXC >= 4 ? 4 : 1), 2>(a, d, table, first_slot, lane, stage_row, stage_mul);
+      else if (d.chunks == 2 && MAXC >= 2) run_bags<index_t, GENERAL, CHECKED, TY, 16, (MAXC >= 2 ? 2 : 1), 4>(a, d, table, first_slot, lane, stage_row, stage_mul);
+      else run_bags<index_t, GENERAL, CHECKED, TY, 16, 1, 8>(a, d, table, first_slot, lane, stage_row, stage_mul);
     }
   } else if (TY == ST_INT2 && d.vb == 8) {
-    if constexpr (TY == ST_INT2) run_bags<index_t, GENERAL, TY, 8, 1, 8>(a, d, table, first_slot, lane, stage_row, stage_mul);
+    if constexpr (TY == ST_INT2) run_bags<index_t, GENERAL, CHECKED, TY, 8, 1, 8>(a, d, table, first_slot, lane, stage_row, stage_mul);
   } else if (d.vb == 4) {
-    run_bags<index_t, GENERAL, TY, 4, 1, 8>(a, d, table, first_slot, lane, stage_row, stage_mul);
+    run_bags<index_t, GENERAL, CHECKED, TY, 4, 1, 8>(a, d, table, first_slot, lane, stage_row, stage_mul);
   } else {
-    run_bags<index_t, GENERAL, TY, MINVB, 1, 8>(a, d, table, first_slot, lane, stage_row, stage_mul);
+    run_bags<index_t, GENERAL, CHECKED, TY, MINVB, 1, 8>(a, d, table, first_slot, lane, stage_row, stage_mul);
   }
 }
 
@@ -455,24 +462,24 @@ __device__ __forceinline__ void pool_dispatch_vb(const LookupArgs& a, const Tabl
 #endif
 
 // The bags of table `table` from position `first_slot` of its order on, as many as a wave takes.
-template <typename index_t, bool GENERAL>
+template <typename index_t, bool GENERAL, bool CHECKED>
 __device__ __forceinline__ void run_table(const LookupArgs& a, const TableDesc& d, int table, int first_slot, int lane, StageRow* stage_row,
                                           StageMul* stage_mul) {
   switch (d.ty) {
-    case ST_INT4: pool_dispatch_vb<index_t, GENERAL, ST_INT4>(a, d, table, first_slot, lane, stage_row, stage_mul); break;
-    case ST_INT8: pool_dispatch_vb<index_t, GENERAL, ST_INT8>(a, d, table, first_slot, lane, stage_row, stage_mul); break;
-    case ST_FP16: pool_dispatch_vb<index_t, GENERAL, ST_FP16>(a, d, table, first_slot, lane, stage_row, stage_mul); break;
-    case ST_INT2: pool_dispatch_vb<index_t, GENERAL, ST_INT2>(a, d, table, first_slot, lane, stage_row, stage_mul); break;
-    case ST_FP32: pool_dispatch_vb<index_t, GENERAL, ST_FP32>(a, d, table, first_slot, lane, stage_row, stage_mul); break;
-    case ST_BF16: pool_dispatch_vb<index_t, GENERAL, ST_BF16>(a, d, table, first_slot, lane, stage_row, stage_mul); break;
-    case ST_FP8: pool_dispatch_vb<index_t, GENERAL, ST_FP8>(a, d, table, first_slot, lane, stage_row, stage_mul); break;
+    case ST_INT4: pool_dispatch_vb<index_t, GENERAL, CHECKED, ST_INT4>(a, d, table, first_slot, lane, stage_row, stage_mul); break;
+    case ST_INT8: pool_dispatch_vb<index_t, GENERAL, CHECKED, ST_INT8>(a, d, table, first_slot, lane, stage_row, stage_mul); break;
+    case ST_FP16: pool_dispatch_vb<index_t, GENERAL, CHECKED, ST_FP16>(a, d, table, first_slot, lane, stage_row, stage_mul); break;
+    case ST_INT2: pool_dispatch_vb<index_t, GENERAL, CHECKED, ST_INT2>(a, d, table, first_slot, lane, stage_row, stage_mul); break;
+    case ST_FP32: pool_dispatch_vb<index_t, GENERAL, CHECKED, ST_FP32>(a, d, table, first_slot, lane, stage_row, stage_mul); break;
+    case ST_BF16: pool_dispatch_vb<index_t, GENERAL, CHECKED, ST_BF16>(a, d, table, first_slot, lane, stage_row, stage_mul); break;
+    case ST_FP8: pool_dispatch_vb<index_t, GENERAL, CHECKED, ST_FP8>(a, d, table, first_slot, lane, stage_row, stage_mul); break;
     default: break;
   }
 }
 
 // One item of the work list: `wave` is the position in the list (or the wave's
 // number for a single-table call).
-template <typename index_t, bool GENERAL>
+template <typename index_t, bool GENERAL, bool CHECKED>
 __device__ __forceinline__ void run_item(const LookupArgs& a, int64_t wave, int lane, StageRow* stage_row, StageMul* stage_mul) {
   int table = 0, first_slot;
   if (a.work) {
@@ -483,7 +490,7 @@ __device__ __forceinline__ void run_item(const LookupArgs& a, int64_t wave, int 
     first_slot = (int)(wave * a.single.bags);
   }
   const TableDesc d = a.tables ? a.tables[table] : a.single;
-  run_table<index_t, GENERAL>(a, d, table, first_slot, lane, stage_row, stage_mul);
+  run_table<index_t, GENERAL, CHECKED>(a, d, table, first_slot, lane, stage_row, stage_mul);
 }
 
 
@@ -491,12 +498,14 @@ __device__ __forceinline__ void run_item(const LookupArgs& a, int64_t wave, int 
 // needs no more than its own 4 KB of LDS.
 // GENERAL = false is the table-batched operator's subset (no logical->physical
 // remap, no positional weights, offsets indexing one shared index array).
+// CHECKED: a checked forward's launch (LookupArgs::check_rows), of that subset (in
+// the GENERAL instances, whose registers are all in use, it made spills).
 //
 // The work list of a table-batched call is 8 runs, one per XCD: whole tables
 // (or slices of them) are pinned to one XCD's L2 instead of spreading their hot
 // rows over all eight. Workgroup i takes item i >> 3 of run i & 7 (workgroups
 // are handed to the XCDs round-robin).
-template <typename index_t, bool GENERAL>
+template <typename index_t, bool GENERAL, bool CHECKED>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(FBGEMM_AMD_MIN_WAVES, 8))) void lookup_kernel(const LookupArgs a) {
   __shared__ StageRow stage_row[MAX_GROUPS * MAX_ROUND];
   __shared__ StageMul stage_mul[MAX_GROUPS * MAX_ROUND];
@@ -512,14 +521,14 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(FBGEMM_AMD_M
     wave = (int64_t)blockIdx.x;
     if (wave >= a.num_waves) return;
   }
-  run_item<index_t, GENERAL>(a, wave, lane, stage_row, stage_mul);
+  run_item<index_t, GENERAL, CHECKED>(a, wave, lane, stage_row, stage_mul);
 }
 
 
 // Defines the launcher of one instance of lookup_kernel.
-#define FBGEMM_AMD_DEFINE_LOOKUP_LAUNCH(FN, INDEX_T, GENERAL)                                             \
+#define FBGEMM_AMD_DEFINE_LOOKUP_LAUNCH(FN, INDEX_T, GENERAL, CHECKED)                                    \
   hipError_t FN(const LookupArgs& a, unsigned blocks, hipStream_t stream) {                              \
-    hipLaunchKernelGGL((lookup_kernel<INDEX_T, GENERAL>), dim3(blocks), dim3(64), 0, stream, a);         \
+    hipLaunchKernelGGL((lookup_kernel<INDEX_T, GENERAL, CHECKED>), dim3(blocks), dim3(64), 0, stream, a);         \
     return hipGetLastError();                                                                            \
   }
 

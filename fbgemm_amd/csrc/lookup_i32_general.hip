@@ -2,5 +2,5 @@
 #include "lookup_general.h"
 
 namespace fbgemm_amd {
-FBGEMM_AMD_DEFINE_LOOKUP_LAUNCH(launch_lookup_i32_general, int32_t, true)
+FBGEMM_AMD_DEFINE_LOOKUP_LAUNCH(launch_lookup_i32_general, int32_t, true, false)
 } // namespace fbgemm_amd

@@ -7,5 +7,5 @@
 #include "lookup_general.h"
 
 namespace fbgemm_amd {
-FBGEMM_AMD_DEFINE_LOOKUP_LAUNCH(launch_lookup_i64, int64_t, false)
+FBGEMM_AMD_DEFINE_LOOKUP_LAUNCH(launch_lookup_i64, int64_t, false, false)
 } // namespace fbgemm_amd

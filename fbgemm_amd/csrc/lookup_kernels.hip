@@ -158,6 +158,11 @@ __global__ void status_done_kernel(int32_t* word, int32_t number) {
   __hip_atomic_store(word, number, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
+__global__ void status_counted_kernel(FlaggedStatus* st, int64_t* warning) {
+  if (warning) *warning = (int64_t)st->counted;
+  st->counted = 0;
+}
+
 // dense[i] = remap[remap_offsets[t] + idx[i]] for tables with a mapping, a copy
 // otherwise (…/embedding_forward_quantized_cpu_template.cpp:605-659).
 template <typename index_t, typename remap_t>
@@ -182,6 +187,8 @@ hipError_t launch_lookup_i64(const LookupArgs& a, unsigned blocks, hipStream_t s
 hipError_t launch_lookup_i32(const LookupArgs& a, unsigned blocks, hipStream_t stream);
 hipError_t launch_lookup_i64_general(const LookupArgs& a, unsigned blocks, hipStream_t stream);
 hipError_t launch_lookup_i32_general(const LookupArgs& a, unsigned blocks, hipStream_t stream);
+hipError_t launch_lookup_i64_checked(const LookupArgs& a, unsigned blocks, hipStream_t stream);
+hipError_t launch_lookup_i32_checked(const LookupArgs& a, unsigned blocks, hipStream_t stream);
 
 hipError_t launch_lookup_lean_i64_exact(const LookupArgs& a, unsigned blocks, hipStream_t stream);
 hipError_t launch_lookup_lean_i32_exact(const LookupArgs& a, unsigned blocks, hipStream_t stream);
@@ -191,6 +198,10 @@ hipError_t launch_lookup_lean_i64_exact_w4(const LookupArgs& a, unsigned blocks,
 hipError_t launch_lookup_lean_i32_exact_w4(const LookupArgs& a, unsigned blocks, hipStream_t stream);
 hipError_t launch_lookup_lean_i64_fast_w4(const LookupArgs& a, unsigned blocks, hipStream_t stream);
 hipError_t launch_lookup_lean_i32_fast_w4(const LookupArgs& a, unsigned blocks, hipStream_t stream);
+hipError_t launch_lookup_lean_i64_checked(const LookupArgs& a, unsigned blocks, hipStream_t stream);
+hipError_t launch_lookup_lean_i32_checked(const LookupArgs& a, unsigned blocks, hipStream_t stream);
+hipError_t launch_lookup_lean_i64_checked_w4(const LookupArgs& a, unsigned blocks, hipStream_t stream);
+hipError_t launch_lookup_lean_i32_checked_w4(const LookupArgs& a, unsigned blocks, hipStream_t stream);
 hipError_t launch_lookup_lean_i64_exact_q8(const LookupArgs& a, unsigned blocks, hipStream_t stream);
 hipError_t launch_lookup_lean_i32_exact_q8(const LookupArgs& a, unsigned blocks, hipStream_t stream);
 hipError_t launch_lookup_lean_i64_fast_q8(const LookupArgs& a, unsigned blocks, hipStream_t stream);
@@ -203,6 +214,12 @@ hipError_t launch_lookup_lean(const LookupArgs& a, bool idx64, bool exact, bool 
   if (a.num_waves <= 0) return hipSuccess;
   const int64_t blocks = a.xcd_start ? 8 * a.num_waves : a.num_waves;
   if (blocks > 0x7fffffffLL || a.positional) return hipErrorInvalidValue;
+  if (a.check_rows) {
+    if (!exact || a.out_ty == ST_INT8 || !a.tables) return hipErrorInvalidValue;
+    if (wide4 && (!a.redo || !a.redo_count)) return hipErrorInvalidValue;
+    if (wide4) return idx64 ? launch_lookup_lean_i64_checked_w4(a, (unsigned)blocks, stream) : launch_lookup_lean_i32_checked_w4(a, (unsigned)blocks, stream);
+    return idx64 ? launch_lookup_lean_i64_checked(a, (unsigned)blocks, stream) : launch_lookup_lean_i32_checked(a, (unsigned)blocks, stream);
+  }
   if (a.out_ty == ST_INT8) { // the instances whose output stage quantizes the pooled vectors (lean_store_q8)
     if (exact) return idx64 ? launch_lookup_lean_i64_exact_q8(a, (unsigned)blocks, stream) : launch_lookup_lean_i32_exact_q8(a, (unsigned)blocks, stream);
     return idx64 ? launch_lookup_lean_i64_fast_q8(a, (unsigned)blocks, stream) : launch_lookup_lean_i32_fast_q8(a, (unsigned)blocks, stream);
@@ -221,6 +238,10 @@ hipError_t launch_lookup(const LookupArgs& a, bool idx64, hipStream_t stream) {
   const int64_t blocks = a.xcd_start ? 8 * a.num_waves : a.num_waves;
   if (blocks > 0x7fffffffLL) return hipErrorInvalidValue;
   const bool general = a.remap || a.positional || a.check_total;
+  if (a.check_rows) {
+    if (general || !a.tables) return hipErrorInvalidValue;
+    return idx64 ? launch_lookup_i64_checked(a, (unsigned)blocks, stream) : launch_lookup_i32_checked(a, (unsigned)blocks, stream);
+  }
   if (general) return idx64 ? launch_lookup_i64_general(a, (unsigned)blocks, stream) : launch_lookup_i32_general(a, (unsigned)blocks, stream);
   return idx64 ? launch_lookup_i64(a, (unsigned)blocks, stream) : launch_lookup_i32(a, (unsigned)blocks, stream);
 }
@@ -229,14 +250,17 @@ hipError_t launch_lookup_both_i64_exact(const LookupArgs& a, const WorkRun& lean
 hipError_t launch_lookup_both_i64_fast(const LookupArgs& a, const WorkRun& lean, unsigned general_blocks, unsigned blocks, hipStream_t stream);
 hipError_t launch_lookup_both_i32_exact(const LookupArgs& a, const WorkRun& lean, unsigned general_blocks, unsigned blocks, hipStream_t stream);
 hipError_t launch_lookup_both_i32_fast(const LookupArgs& a, const WorkRun& lean, unsigned general_blocks, unsigned blocks, hipStream_t stream);
+hipError_t launch_lookup_both_i64_checked(const LookupArgs& a, const WorkRun& lean, unsigned general_blocks, unsigned blocks, hipStream_t stream);
+hipError_t launch_lookup_both_i32_checked(const LookupArgs& a, const WorkRun& lean, unsigned general_blocks, unsigned blocks, hipStream_t stream);
 
 // Both kernels in one launch (lookup_both.h): `a` with the general tables' list, `lean` the lean tables'.
 hipError_t launch_lookup_both(const LookupArgs& a, const WorkRun& lean, bool idx64, bool exact, hipStream_t stream) {
   const int64_t general = 8 * a.num_waves, blocks = general + 8 * lean.num_waves;
   if (blocks <= 0) return hipSuccess;
   if (!lookup_both_fits(a.num_waves, lean.num_waves) || !a.tables || !a.work || !a.xcd_start || !lean.work || !lean.xcd_start || a.remap || a.positional || a.check_total ||
-      a.out_ty == ST_INT8)
+      a.out_ty == ST_INT8 || (a.check_rows && !exact))
     return hipErrorInvalidValue;
+  if (a.check_rows) return idx64 ? launch_lookup_both_i64_checked(a, lean, (unsigned)general, (unsigned)blocks, stream) : launch_lookup_both_i32_checked(a, lean, (unsigned)general, (unsigned)blocks, stream);
   if (exact) return idx64 ? launch_lookup_both_i64_exact(a, lean, (unsigned)general, (unsigned)blocks, stream) : launch_lookup_both_i32_exact(a, lean, (unsigned)general, (unsigned)blocks, stream);
   return idx64 ? launch_lookup_both_i64_fast(a, lean, (unsigned)general, (unsigned)blocks, stream) : launch_lookup_both_i32_fast(a, lean, (unsigned)general, (unsigned)blocks, stream);
 }
@@ -288,6 +312,11 @@ hipError_t launch_status_clear(Status* st, int32_t mark, hipStream_t stream) {
 
 hipError_t launch_status_done(int32_t* word, int32_t number, hipStream_t stream) {
   hipLaunchKernelGGL(status_done_kernel, dim3(1), dim3(1), 0, stream, word, number);
+  return hipGetLastError();
+}
+
+hipError_t launch_status_counted(FlaggedStatus* st, int64_t* warning, hipStream_t stream) {
+  hipLaunchKernelGGL(status_counted_kernel, dim3(1), dim3(1), 0, stream, st, warning);
   return hipGetLastError();
 }
 

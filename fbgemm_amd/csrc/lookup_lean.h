@@ -34,6 +34,9 @@
 //    row-at-a-time loop that converts integers to float before the fma. Both
 //    round identically; the slow one only has to be correct.
 //  * what is staged per entry is the row number (32 bits), not its byte offset.
+//  * CHECKED instances (exact, float output) are those of a checked forward (LookupArgs::check_rows): 157 registers. With the
+//    check as a branch the one kernel took 167 and 0.7 % longer on 64 mixed tables of 2048 bags, and the tolerance-grade
+//    instances spilled.
 // Three kinds of kernel are made from this file: lookup_lean_kernel (every shape,
 // float output), its Q8 instances (the 8-bit pooled output quantized in the
 // output stage, lean_store_q8) and lookup_lean_wide4_kernel with its redo kernel
@@ -124,9 +127,11 @@ struct LeanLane {
   int64_t remap_base, remap_cap; // pruned table: its slice of the remap array
   int64_t rank_base;             // >= 0: the table's first rank record (its mapping is order-preserving)
   bool remapped;
+  int64_t rows;                  // index_bound
+  int64_t logical;               // checked forward with a mapping: the table's rows before pruning
 };
 
-template <typename index_t>
+template <typename index_t, bool CHECKED>
 __device__ __forceinline__ LeanLane lean_lane(const LookupArgs& a, const TableDesc& d, int table, int first_slot, int lane) {
   LeanLane L;
   const int S = d.lanes;
@@ -183,8 +188,11 @@ __device__ __forceinline__ LeanLane lean_lane(const LookupArgs& a, const TableDe
       len = 0;
     }
     if (a.check_total && L.bag == a.B - 1 && o1 - base != a.index_size && reporter) report(a.status, ERR_LENGTH_MISMATCH);
+    if (CHECKED && table == a.T - 1 && L.bag == a.B - 1 && reporter) check_end(a, o1);
   }
   L.n = (int)len;
+  L.rows = index_bound<CHECKED>(a, d, table, lane == 0);
+  L.logical = CHECKED && a.remap ? a.logical_rows[table] : 0;
   L.remap_base = 0;
   L.remap_cap = 0;
   L.rank_base = -1;
@@ -221,19 +229,27 @@ constexpr int LEAN_SKIP = -1;             // an entry that adds nothing (a prune
 // leaves its position in `bad_pos` (the smallest wins); the caller reports it once its loop is
 // over (lean_report_bad): an atomic inside the loop would count as a store in flight, and with
 // loads and stores in flight together every wait of the loop becomes a wait for everything.
+// (A checked forward rejects none: they read row 0, and `bad_pos` counts them, downwards.)
 constexpr int64_t LEAN_NO_BAD_POS = INT64_MAX;
-__device__ __forceinline__ int lean_row(const TableDesc& d, const LeanLane& L, int64_t row, int64_t pos, int64_t& bad_pos) {
+template <bool CHECKED>
+__device__ __forceinline__ int lean_row(const LookupArgs& a, const TableDesc& d, const LeanLane& L, int64_t row, int64_t pos, int64_t& bad_pos) {
   if (!L.remapped && d.skip_minus_one && row == -1) return LEAN_SKIP;
-  if (row < 0 || row >= d.num_rows) {
+  if (row < 0 || row >= L.rows) {
+    if (CHECKED) {
+      --bad_pos;
+      return 0;
+    }
     bad_pos = pos < bad_pos ? pos : bad_pos;
     return LEAN_SKIP;
   }
   return (int)row;
 }
 constexpr int64_t LEAN_PRUNED = INT64_MIN; // what lean_remap returns for an entry that adds nothing
+template <bool CHECKED>
 __device__ __forceinline__ int64_t lean_remap(const LookupArgs& a, const LeanLane& L, int64_t logical, int64_t pos, int64_t& bad_pos) {
+  if (CHECKED) logical = logical_index(logical, L.logical);
   if (logical < 0 || logical >= L.remap_cap) {
-    bad_pos = pos < bad_pos ? pos : bad_pos;
+    if (!CHECKED) bad_pos = pos < bad_pos ? pos : bad_pos;
     return LEAN_PRUNED;
   }
   if (L.rank_base >= 0) { // order-preserving mapping: the physical row is the rank among the kept rows
@@ -246,8 +262,11 @@ __device__ __forceinline__ int64_t lean_remap(const LookupArgs& a, const LeanLan
                               : (int64_t) reinterpret_cast<const int32_t*>(a.remap)[L.remap_base + logical];
   return m == -1 ? LEAN_PRUNED : m;
 }
+template <bool CHECKED>
 __device__ __forceinline__ void lean_report_bad(const LookupArgs& a, int64_t bad_pos) {
-  if (bad_pos != LEAN_NO_BAD_POS) report_index(a.status, bad_pos);
+  if (bad_pos == LEAN_NO_BAD_POS) return;
+  if (!CHECKED) report_index(a.status, bad_pos);
+  else if (a.warning) status_count(a.status, (int)(LEAN_NO_BAD_POS - bad_pos));
 }
 
 // The output of a wave through LDS, so that every store instruction writes runs
@@ -568,7 +587,7 @@ __device__ __forceinline__ void lean_write(const LookupArgs& a, const TableDesc&
 // valid row its units are not loaded at all.)
 // Returns false (wave-uniform, nothing written) when a scale is too large for
 // the pre-scaled arithmetic.
-template <typename index_t, bool EXACT, int TY, int C, bool INHDR, int R, bool Q8, int UL_CAP = 4, bool HDR_EARLY = false>
+template <typename index_t, bool EXACT, int TY, int C, bool INHDR, int R, bool Q8, bool CHECKED, int UL_CAP = 4, bool HDR_EARLY = false>
 __device__ __forceinline__ bool pool_lean(const LookupArgs& a, const TableDesc& d, int table, int first_slot, int lane,
                                           uint32_t* lds) {
   constexpr bool QUANT = TY == ST_INT8 || TY == ST_INT4;
@@ -590,7 +609,7 @@ __device__ __forceinline__ bool pool_lean(const LookupArgs& a, const TableDesc& 
   int* stage_row = reinterpret_cast<int*>(lds);                               // [2][MAX_GROUPS][LEAN_BLOCK]
   LeanMul* stage_mul = reinterpret_cast<LeanMul*>(lds + 2 * ROWS_BUF);        // [MAX_GROUPS][LEAN_BLOCK]
 
-  const LeanLane L = lean_lane<index_t>(a, d, table, first_slot, lane);
+  const LeanLane L = lean_lane<index_t, CHECKED>(a, d, table, first_slot, lane);
   const int S = d.lanes;
   const int sub = L.sub;
   const int n = L.n;
@@ -664,10 +683,14 @@ __device__ __forceinline__ bool pool_lean(const LookupArgs& a, const TableDesc& 
   };
   // indices that have arrived -> row numbers (negative: nothing to add), weights
   auto take_idx = [&](int blk) {
+    if (CHECKED && a.remap && !L.remapped) { // a table that is not pruned among pruned ones
+#pragma unroll
+      for (int j = 0; j < R; ++j) nrow[j] = logical_index(nrow[j], L.logical);
+    }
     if (L.remapped) {
 #pragma unroll
       for (int j = 0; j < R; ++j)
-        if (have[j]) nrow[j] = lean_remap(a, L, nrow[j], L.pos0 + blk * LEAN_BLOCK + sub + j * SL, bad_pos);
+        if (have[j]) nrow[j] = lean_remap<CHECKED>(a, L, nrow[j], L.pos0 + blk * LEAN_BLOCK + sub + j * SL, bad_pos);
     }
 #pragma unroll
     for (int j = 0; j < R; ++j) {
@@ -676,7 +699,7 @@ __device__ __forceinline__ bool pool_lean(const LookupArgs& a, const TableDesc& 
       // loaded, loads the next block's weight elsewhere and moves both at the end of the loop,
       // which waits for that load and for everything issued before it
       asm volatile("v_mov_b32 %0, %1" : "=v"(cw[j]) : "v"(nw[j]));
-      if (have[j]) crow[j] = nrow[j] == LEAN_PRUNED ? LEAN_SKIP : lean_row(d, L, nrow[j], L.pos0 + blk * LEAN_BLOCK + sub + j * SL, bad_pos);
+      if (have[j]) crow[j] = nrow[j] == LEAN_PRUNED ? LEAN_SKIP : lean_row<CHECKED>(a, d, L, nrow[j], L.pos0 + blk * LEAN_BLOCK + sub + j * SL, bad_pos);
     }
   };
   // The (scale, bias) headers of the rows staged last, asked for right in front of the first unit
@@ -895,7 +918,7 @@ __device__ __forceinline__ bool pool_lean(const LookupArgs& a, const TableDesc& 
   if constexpr (QUANT) {
     if (__builtin_amdgcn_ballot_w64(big) != 0ull) return false; // wave-uniform
   }
-  lean_report_bad(a, bad_pos);
+  lean_report_bad<CHECKED>(a, bad_pos);
   lean_write<EXACT, TY, C, INHDR, true, Q8>(a, d, L, table, acc, bsum, lds);
   return true;
 }
@@ -903,10 +926,10 @@ __device__ __forceinline__ bool pool_lean(const LookupArgs& a, const TableDesc& 
 // The same bags, one row at a time, integers converted to float before the fma:
 // for waves that met a scale the pre-scaled arithmetic cannot take. Every lane
 // walks its bag's entries itself; nothing is staged.
-template <typename index_t, bool EXACT, int TY, int C, bool INHDR, bool Q8>
+template <typename index_t, bool EXACT, int TY, int C, bool INHDR, bool Q8, bool CHECKED>
 __device__ __forceinline__ void pool_lean_slow(const LookupArgs& a, const TableDesc& d, int table, int first_slot, int lane, uint32_t* lds) {
   constexpr int E = TY == ST_INT4 ? 32 : 16;
-  const LeanLane L = lean_lane<index_t>(a, d, table, first_slot, lane);
+  const LeanLane L = lean_lane<index_t, CHECKED>(a, d, table, first_slot, lane);
   const int S = d.lanes;
   const index_t* idx = reinterpret_cast<const index_t*>(a.indices) + L.pos0;
   const uint8_t* wbase = (d.placement ? a.weights[1] : a.weights[0]) + d.weights_offset;
@@ -919,8 +942,9 @@ __device__ __forceinline__ void pool_lean_slow(const LookupArgs& a, const TableD
   for (int i = 0; i < L.n; ++i) {
     int64_t row = (int64_t)idx[i];
     const float w = a.sample_weights ? a.sample_weights[L.pos0 + i] : 1.0f;
-    if (L.remapped) row = lean_remap(a, L, row, L.pos0 + i, bad_pos);
-    const int r = row == LEAN_PRUNED ? LEAN_SKIP : lean_row(d, L, row, L.pos0 + i, bad_pos);
+    if (CHECKED && a.remap && !L.remapped) row = logical_index(row, L.logical);
+    if (L.remapped) row = lean_remap<CHECKED>(a, L, row, L.pos0 + i, bad_pos);
+    const int r = row == LEAN_PRUNED ? LEAN_SKIP : lean_row<CHECKED>(a, d, L, row, L.pos0 + i, bad_pos);
     if (r < 0) continue;
     const uint8_t* prow = wbase + (uint64_t)(uint32_t)r * (uint32_t)d.row_stride;
     float rs, rb;
@@ -939,34 +963,34 @@ __device__ __forceinline__ void pool_lean_slow(const LookupArgs& a, const TableD
       lean_chunk<TY, EXACT, true, C * E>(acc, c * E, raw, m);
     }
   }
-  lean_report_bad(a, bad_pos);
+  lean_report_bad<CHECKED>(a, bad_pos);
   lean_write<EXACT, TY, C, INHDR, false, Q8>(a, d, L, table, acc, bsum, lds);
 }
 
-template <typename index_t, bool EXACT, int TY, int C, bool INHDR, bool Q8>
+template <typename index_t, bool EXACT, int TY, int C, bool INHDR, bool Q8, bool CHECKED>
 __device__ __forceinline__ void run_lean(const LookupArgs& a, const TableDesc& d, int table, int first_slot, int lane,
                                          uint32_t* lds) {
   bool done;
-  if (d.lanes >= 8) done = pool_lean<index_t, EXACT, TY, C, INHDR, 1, Q8>(a, d, table, first_slot, lane, lds);
-  else if (d.lanes >= 4) done = pool_lean<index_t, EXACT, TY, C, INHDR, 2, Q8>(a, d, table, first_slot, lane, lds);
-  else done = pool_lean<index_t, EXACT, TY, C, INHDR, 4, Q8>(a, d, table, first_slot, lane, lds);
+  if (d.lanes >= 8) done = pool_lean<index_t, EXACT, TY, C, INHDR, 1, Q8, CHECKED>(a, d, table, first_slot, lane, lds);
+  else if (d.lanes >= 4) done = pool_lean<index_t, EXACT, TY, C, INHDR, 2, Q8, CHECKED>(a, d, table, first_slot, lane, lds);
+  else done = pool_lean<index_t, EXACT, TY, C, INHDR, 4, Q8, CHECKED>(a, d, table, first_slot, lane, lds);
   if constexpr (TY == ST_INT4 || TY == ST_INT8) {
-    if (!done) pool_lean_slow<index_t, EXACT, TY, C, INHDR, Q8>(a, d, table, first_slot, lane, lds);
+    if (!done) pool_lean_slow<index_t, EXACT, TY, C, INHDR, Q8, CHECKED>(a, d, table, first_slot, lane, lds);
   }
 }
 
 // Row types and the chunks per lane the host picks for lean shapes: 1 (4-bit), 2 (8-bit), 4 (fp16).
-template <typename index_t, bool EXACT, bool Q8>
+template <typename index_t, bool EXACT, bool Q8, bool CHECKED>
 __device__ __forceinline__ void lean_dispatch(const LookupArgs& a, const TableDesc& d, int table, int first_slot, int lane,
                                               uint32_t* lds) {
   if (d.ty == ST_INT4) {
-    if (d.inline_hdr) run_lean<index_t, EXACT, ST_INT4, 1, true, Q8>(a, d, table, first_slot, lane, lds);
-    else run_lean<index_t, EXACT, ST_INT4, 1, false, Q8>(a, d, table, first_slot, lane, lds);
+    if (d.inline_hdr) run_lean<index_t, EXACT, ST_INT4, 1, true, Q8, CHECKED>(a, d, table, first_slot, lane, lds);
+    else run_lean<index_t, EXACT, ST_INT4, 1, false, Q8, CHECKED>(a, d, table, first_slot, lane, lds);
   } else if (d.ty == ST_INT8) {
-    if (d.inline_hdr) run_lean<index_t, EXACT, ST_INT8, 2, true, Q8>(a, d, table, first_slot, lane, lds);
-    else run_lean<index_t, EXACT, ST_INT8, 2, false, Q8>(a, d, table, first_slot, lane, lds);
+    if (d.inline_hdr) run_lean<index_t, EXACT, ST_INT8, 2, true, Q8, CHECKED>(a, d, table, first_slot, lane, lds);
+    else run_lean<index_t, EXACT, ST_INT8, 2, false, Q8, CHECKED>(a, d, table, first_slot, lane, lds);
   } else if (d.ty == ST_FP16) {
-    run_lean<index_t, EXACT, ST_FP16, 4, false, Q8>(a, d, table, first_slot, lane, lds);
+    run_lean<index_t, EXACT, ST_FP16, 4, false, Q8, CHECKED>(a, d, table, first_slot, lane, lds);
   }
 }
 
@@ -999,14 +1023,14 @@ __device__ __forceinline__ bool lean_work_item(const LookupArgs& a, int& table, 
   return true;
 }
 
-template <typename index_t, bool EXACT, bool Q8>
+template <typename index_t, bool EXACT, bool Q8, bool CHECKED>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(FBGEMM_AMD_LEAN_MIN_WAVES, 8))) void lookup_lean_kernel(const LookupArgs a) {
   // 8 KB: while a bag is pooled, two buffers of staged rows (2 KB) and the multipliers (4 KB); at the end, the wave's output
   __shared__ __attribute__((aligned(16))) uint32_t lds[LEAN_LDS_WORDS + MAX_GROUPS];
   int table, first_slot;
   if (!lean_work_item(a, table, first_slot)) return;
   const TableDesc d = a.tables ? a.tables[table] : a.single;
-  lean_dispatch<index_t, EXACT, Q8>(a, d, table, first_slot, (int)threadIdx.x, lds);
+  lean_dispatch<index_t, EXACT, Q8, CHECKED>(a, d, table, first_slot, (int)threadIdx.x, lds);
 }
 
 // The instance for table-batched launches in which every table has 4-bit rows in bags of 8 lanes
@@ -1024,14 +1048,14 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(FBGEMM_AMD_L
 // the kernel reserve scratch memory. A wave that meets such a scale writes nothing and queues its
 // work item; lookup_lean_wide4_redo_kernel, launched behind this kernel in every forward, pools
 // the queued items with pool_lean_slow (usually none: 256 workgroups that read a zero and leave).
-template <typename index_t, bool EXACT>
+template <typename index_t, bool EXACT, bool CHECKED>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 8))) void lookup_lean_wide4_kernel(const LookupArgs a) {
   __shared__ __attribute__((aligned(16))) uint32_t lds[LEAN_LDS_WORDS + MAX_GROUPS];
   int table, first_slot;
   if (!lean_work_item(a, table, first_slot)) return;
   const TableDesc d = a.tables[table]; // table-batched launches only
   const int lane = (int)threadIdx.x;
-  const bool done = pool_lean<index_t, EXACT, ST_INT4, 1, false, 1, false, EXACT ? 2 : 4, EXACT>(a, d, table, first_slot, lane, lds);
+  const bool done = pool_lean<index_t, EXACT, ST_INT4, 1, false, 1, false, CHECKED, EXACT ? 2 : 4, EXACT>(a, d, table, first_slot, lane, lds);
   if (!done && lane == 0) { // wave-uniform verdict; nothing has been written or reported
     const int k = atomicAdd(a.redo_count, 1);
     WaveWork ww;
@@ -1042,7 +1066,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 8))) void
 }
 
 constexpr int LEAN_REDO_WORKGROUPS = 256;
-template <typename index_t, bool EXACT>
+template <typename index_t, bool EXACT, bool CHECKED>
 __global__ __launch_bounds__(64) void lookup_lean_wide4_redo_kernel(const LookupArgs a) {
   __shared__ __attribute__((aligned(16))) uint32_t lds[LEAN_LDS_WORDS + MAX_GROUPS];
   const int lane = (int)threadIdx.x;
@@ -1055,7 +1079,7 @@ __global__ __launch_bounds__(64) void lookup_lean_wide4_redo_kernel(const Lookup
   for (int i = (int)blockIdx.x; i < count; i += (int)gridDim.x) {
     const WaveWork ww = a.redo[i];
     const TableDesc d = a.tables ? a.tables[ww.table] : a.single;
-    pool_lean_slow<index_t, EXACT, ST_INT4, 1, false, false>(a, d, ww.table, ww.first_bag, lane, lds);
+    pool_lean_slow<index_t, EXACT, ST_INT4, 1, false, false, CHECKED>(a, d, ww.table, ww.first_bag, lane, lds);
   }
   if (ticket == (int)gridDim.x - 1 && lane == 0) { // for the next forward
     a.redo_count[0] = 0;
@@ -1063,16 +1087,16 @@ __global__ __launch_bounds__(64) void lookup_lean_wide4_redo_kernel(const Lookup
   }
 }
 
-#define FBGEMM_AMD_DEFINE_LEAN_LAUNCH(FN, INDEX_T, EXACT, Q8)                                            \
+#define FBGEMM_AMD_DEFINE_LEAN_LAUNCH(FN, INDEX_T, EXACT, Q8, CHECKED)                                   \
   hipError_t FN(const LookupArgs& a, unsigned blocks, hipStream_t stream) {                              \
-    hipLaunchKernelGGL((lookup_lean_kernel<INDEX_T, EXACT, Q8>), dim3(blocks), dim3(64), 0, stream, a);  \
+    hipLaunchKernelGGL((lookup_lean_kernel<INDEX_T, EXACT, Q8, CHECKED>), dim3(blocks), dim3(64), 0, stream, a); \
     return hipGetLastError();                                                                            \
   }
 
-#define FBGEMM_AMD_DEFINE_LEAN_WIDE4_LAUNCH(FN, INDEX_T, EXACT)                                           \
+#define FBGEMM_AMD_DEFINE_LEAN_WIDE4_LAUNCH(FN, INDEX_T, EXACT, CHECKED)                                  \
   hipError_t FN(const LookupArgs& a, unsigned blocks, hipStream_t stream) {                              \
-    hipLaunchKernelGGL((lookup_lean_wide4_kernel<INDEX_T, EXACT>), dim3(blocks), dim3(64), 0, stream, a); \
-    hipLaunchKernelGGL((lookup_lean_wide4_redo_kernel<INDEX_T, EXACT>), dim3(LEAN_REDO_WORKGROUPS), dim3(64), 0, stream, a); \
+    hipLaunchKernelGGL((lookup_lean_wide4_kernel<INDEX_T, EXACT, CHECKED>), dim3(blocks), dim3(64), 0, stream, a); \
+    hipLaunchKernelGGL((lookup_lean_wide4_redo_kernel<INDEX_T, EXACT, CHECKED>), dim3(LEAN_REDO_WORKGROUPS), dim3(64), 0, stream, a); \
     return hipGetLastError();                                                                            \
   }
 

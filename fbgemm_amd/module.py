@@ -345,6 +345,10 @@ class IntNBitTableBatchedEmbeddingBagsCodegen(torch.nn.Module):
         one_pass = (check and not hashed and self.bounds_check_mode_int != BoundsCheckMode.FATAL.value
                     and offsets.numel() > T  # B > 0
                     and (not arrayed or (self.original_rows_per_table.numel() == T and self._feature_remap_offsets.numel() == T + 1)))
+        if one_pass and self.pooling_mode != PoolingMode.NONE:
+            out = self._checked_forward(indices, offsets, per_sample_weights, arrayed)
+            if out is not None:
+                return out
         if one_pass:
             # the check, or check, mapping and check, on copies: the caller's tensors stay as they are
             indices, offsets = ops.check_remap_indices(
@@ -361,6 +365,35 @@ class IntNBitTableBatchedEmbeddingBagsCodegen(torch.nn.Module):
             fp8_exponent_bits=self.fp8_exponent_bits, fp8_exponent_bias=self.fp8_exponent_bias,
             index_remappings=self._feature_remap_array if fuse_remap else None,
             index_remappings_offsets=self._feature_remap_offsets if fuse_remap else None)
+
+    # Only what it saves to try: forwards left whose check is a pass of its own because an earlier one's offsets had to be
+    # repaired, and the number of offsets of the last forward that the lookup's kernels would not check.
+    _apart_left = 0
+    _apart_for = -1
+
+    def _checked_forward(self, indices, offsets, per_sample_weights, arrayed):
+        """The check in the lookup's own kernels, or None where it has to be a pass of its own."""
+        if self._apart_left > 0:
+            self._apart_left -= 1
+            return None
+        if self._apart_for == offsets.numel():
+            return None
+        longs = [self.rows_per_table, self.bounds_check_warning]
+        if arrayed:
+            longs += [self.original_rows_per_table, self._feature_remap_offsets]
+        if (indices.dtype != offsets.dtype or not (indices.is_contiguous() and offsets.is_contiguous())
+                or (offsets.numel() - 1) % self.rows_per_table.numel() != 0 or self.output_dtype not in ops._OUT_TORCH
+                or any(t.dtype != torch.int64 or not t.is_cuda or not t.is_contiguous() for t in longs)
+                or (arrayed and not (self._feature_remap_array.is_cuda and self._feature_remap_array.is_contiguous()))):
+            return None
+        out, repair = ops.checked_lookup(
+            self.weights_dev, self.weights_uvm, self.weights_placements, self.weights_offsets, self.weights_tys, self.D_offsets,
+            self.total_D, indices, offsets, int(self.pooling_mode), per_sample_weights, self.output_dtype, self.row_alignment,
+            (self.max_float8_D, self.fp8_exponent_bits, self.fp8_exponent_bias), self.rows_per_table, self.bounds_check_mode_int,
+            self.bounds_check_warning, *((self.original_rows_per_table, self._feature_remap_array, self._feature_remap_offsets) if arrayed else ()))
+        if out is None:
+            self._apart_left, self._apart_for = (64, -1) if repair else (0, offsets.numel())
+        return out
 
     def _check_and_remap(self, indices, offsets, per_sample_weights, check, hashed, arrayed, fuse_remap):
         """The operators one after the other: FATAL mode, hash-based pruning, no check."""

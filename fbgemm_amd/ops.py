@@ -466,6 +466,33 @@ def int_nbit_split_embedding_codegen_lookup_function(
     return out
 
 
+def checked_lookup(dev_weights, uvm_weights, weights_placements, weights_offsets, weights_tys, D_offsets, total_D, indices, offsets,
+                   pooling_mode, indice_weights, output_dtype, row_alignment, fp8, rows_per_table, bounds_check_mode, warning,
+                   logical_rows_per_table=None, index_remappings=None, index_remappings_offsets=None):
+    """``check_remap_indices`` and the pooled forward over what it returns, in the forward's own kernels
+    (fbgemm_amd_tbe_forward_checked), for inputs in the form that call takes (contiguous, one dtype, T*B + 1 offsets; ``fp8``:
+    max_float8_D, exponent bits and bias). Returns the output, or None where the two calls have to be made, and whether that is
+    because the check has offsets to repair. Waits for the result."""
+    if indice_weights is not None:
+        if indice_weights.numel() == 0:
+            indice_weights = None
+        elif indice_weights.size(0) != indices.numel():
+            return None, False
+        else:
+            indice_weights = indice_weights.float().contiguous()
+    plan = _plan_for(dev_weights, uvm_weights, weights_placements, weights_offsets, weights_tys, D_offsets, row_alignment)
+    _set_fp8(plan, *fp8)
+    if total_D != plan.total_D:
+        return None, False
+    out = torch.empty(((offsets.numel() - 1) // plan.T, total_D), dtype=_OUT_TORCH[output_dtype], device=dev_weights.device)
+    rc = check(_lib.lib().fbgemm_amd_tbe_forward_checked(
+        plan.handle, _ptr(dev_weights), _ptr(uvm_weights), _ptr(indices), _ptr(offsets), _bits(indices), indices.numel(), offsets.numel(),
+        pooling_mode, _ptr(indice_weights), output_dtype, _ptr(out), _ptr(rows_per_table), int(bounds_check_mode), _ptr(warning),
+        _ptr(logical_rows_per_table), _ptr(index_remappings), 32 if index_remappings is None else _bits(index_remappings),
+        _ptr(index_remappings_offsets), 0 if index_remappings_offsets is None else index_remappings_offsets.numel(), _stream()))
+    return (out, False) if rc == 0 else (None, rc == 2)
+
+
 def _set_fp8(plan, max_float8_D, exponent_bits, exponent_bias):
     """FP8 tables need the operator's exponent bits and bias (check_fp8_params of the reference)."""
     if max_float8_D:

@@ -266,7 +266,24 @@ int fbgemm_amd_tbe_forward_pruned(
     const int64_t* d_index_remappings_offsets, int64_t index_remappings_offsets_numel,
     void* d_status, void* stream);
 
-/* A compact form of the mappings for the call above. No counterpart in the
+/* The forward above with the checks of fbgemm_amd_check_remap_indices in it, on inputs as the caller
+ * has them: the lookup kernels judge every index as they read it (rows_per_table; with a mapping the rows
+ * before pruning first), take row 0 for one outside its table and, in mode 1 (WARNING), leave the number of
+ * those in *d_warning. Waits for the result: returns 0 when the output is what the check and the forward one
+ * after the other make. Otherwise the caller makes the two calls: 1, and nothing was done, for the 8-bit output, a
+ * plan in the tolerance-grade mode, a mapping over tables of other widths than the kernels' regular ones (unless
+ * the forward is small), a stream that is being captured; 2, with an output and a *d_warning that mean nothing, for
+ * offsets that are not in order from at least 0 to indices_numel, which the check repairs, and row counts below 1. */
+int fbgemm_amd_tbe_forward_checked(
+    fbgemm_amd_tbe_plan* plan, const void* d_dev_weights, const void* d_uvm_weights,
+    const void* d_indices, const void* d_offsets, int32_t index_bits,
+    int64_t indices_numel, int64_t offsets_numel, int32_t pooling_mode,
+    const float* d_indice_weights, int32_t output_ty, void* d_output,
+    const int64_t* d_rows_per_table, int32_t bounds_check_mode, int64_t* d_warning,
+    const int64_t* d_logical_rows_per_table, const void* d_index_remappings, int32_t remap_bits,
+    const int64_t* d_index_remappings_offsets, int64_t index_remappings_offsets_numel, void* stream);
+
+/* A compact form of the mappings for the forward before it. No counterpart in the
  * reference. For every table whose mapping is order-preserving (its kept rows
  * are numbered 0, 1, 2, ... in logical order: what embedding_bag_rowwise_prune
  * and the inference converter produce) the plan builds, on the device, 2 bits per

@@ -248,6 +248,11 @@ hipError_t launch_status_done(int32_t* word, int32_t number, hipStream_t) {
   *word = number;
   return LAUNCHED();
 }
+hipError_t launch_status_counted(FlaggedStatus* st, int64_t* warning, hipStream_t) {
+  if (warning) *warning = (int64_t)st->counted;
+  st->counted = 0;
+  return LAUNCHED();
+}
 hipError_t launch_bag_order(const void*, bool, int32_t B, int32_t T, BagEntry* order, hipStream_t) {
   memset(order, 0, sizeof(BagEntry) * (size_t)B * (size_t)T);
   return LAUNCHED();
