@@ -473,23 +473,26 @@ def checked_lookup(dev_weights, uvm_weights, weights_placements, weights_offsets
     (fbgemm_amd_tbe_forward_checked), for inputs in the form that call takes (contiguous, one dtype, T*B + 1 offsets; ``fp8``:
     max_float8_D, exponent bits and bias). Returns the output, or None where the two calls have to be made, and whether that is
     because the check has offsets to repair. Waits for the result."""
-    if indice_weights is not None:
-        if indice_weights.numel() == 0:
-            indice_weights = None
-        elif indice_weights.size(0) != indices.numel():
+    n = indices.numel()
+    weights = None
+    if indice_weights is not None and indice_weights.numel() > 0:
+        if indice_weights.size(0) != n:
             return None, False
-        else:
-            indice_weights = indice_weights.float().contiguous()
+        indice_weights = indice_weights.float().contiguous()  # held until the call has returned
+        weights = indice_weights.data_ptr()
     plan = _plan_for(dev_weights, uvm_weights, weights_placements, weights_offsets, weights_tys, D_offsets, row_alignment)
-    _set_fp8(plan, *fp8)
+    if fp8[0]:
+        _set_fp8(plan, *fp8)
     if total_D != plan.total_D:
         return None, False
-    out = torch.empty(((offsets.numel() - 1) // plan.T, total_D), dtype=_OUT_TORCH[output_dtype], device=dev_weights.device)
+    offsets_numel = offsets.numel()
+    out = dev_weights.new_empty(((offsets_numel - 1) // plan.T, total_D), dtype=_OUT_TORCH[output_dtype])
+    maps = (None, None, 32, None, 0) if index_remappings is None else (
+        logical_rows_per_table.data_ptr(), index_remappings.data_ptr(), _bits(index_remappings), index_remappings_offsets.data_ptr(),
+        index_remappings_offsets.numel())
     rc = check(_lib.lib().fbgemm_amd_tbe_forward_checked(
-        plan.handle, _ptr(dev_weights), _ptr(uvm_weights), _ptr(indices), _ptr(offsets), _bits(indices), indices.numel(), offsets.numel(),
-        pooling_mode, _ptr(indice_weights), output_dtype, _ptr(out), _ptr(rows_per_table), int(bounds_check_mode), _ptr(warning),
-        _ptr(logical_rows_per_table), _ptr(index_remappings), 32 if index_remappings is None else _bits(index_remappings),
-        _ptr(index_remappings_offsets), 0 if index_remappings_offsets is None else index_remappings_offsets.numel(), _stream()))
+        plan.handle, dev_weights.data_ptr(), uvm_weights.data_ptr(), indices.data_ptr(), offsets.data_ptr(), _bits(indices), n, offsets_numel,
+        pooling_mode, weights, output_dtype, out.data_ptr(), rows_per_table.data_ptr(), bounds_check_mode, warning.data_ptr(), *maps, _stream()))
     return (out, False) if rc == 0 else (None, rc == 2)
 
 
