@@ -93,7 +93,7 @@ def parse():
 
 
 # the lookup kernels of a forward as the summaries name them (the last one is the general kernel)
-LOOKUP_KERNELS = ("lookup_lean_kernel", "lookup_lean_wide4_kernel", "lookup_lean_wide4_redo_kernel", "lookup_both_kernel", "lookup_kernel")
+LOOKUP_KERNELS = ("lookup_lean_kernel", "lookup_lean_wide4_kernel", "lookup_lean_wide4_redo_kernel", "lookup_matrix_kernel", "lookup_both_kernel", "lookup_kernel")
 
 
 def traffic_from_profile(config_id):
@@ -139,7 +139,7 @@ def profile_kernel_us(config_id):
     total = {k: int(c) * float(v) for k, c, v in rows}
     # every forward launches one of the two lean kernels (the trace holds both while the plan is still
     # choosing between them) or the launch of both kernels; the redo kernel goes with the four-wave instance
-    forwards = sum(calls.get(k, 0) for k in ("lookup_lean_kernel", "lookup_lean_wide4_kernel", "lookup_both_kernel"))
+    forwards = sum(calls.get(k, 0) for k in ("lookup_lean_kernel", "lookup_lean_wide4_kernel", "lookup_matrix_kernel", "lookup_both_kernel"))
     lean = sum(total.get(k, 0.0) for k in LOOKUP_KERNELS[:-1]) / forwards if forwards else 0.0
     general = total.get("lookup_kernel", 0.0) / calls["lookup_kernel"] if calls.get("lookup_kernel") else 0.0
     if not lean and not general:
@@ -873,7 +873,7 @@ def time_tbe(p, a, torch, np, steps, warmup, graph, accumulate):
         bits, pos = st.read()
         assert bits == 0, f"the lookup rejected its inputs: status {bits:#x} at {pos}"
         kernel_ms = k0.elapsed_time(k1) / steps
-        kernel_name = "lookup_lean_kernel or lookup_lean_wide4_kernel (+ lookup_kernel for tables of other shapes, beside it or as lookup_both_kernel), back to back"
+        kernel_name = "lookup_lean_kernel, lookup_lean_wide4_kernel or lookup_matrix_kernel (+ lookup_kernel for tables of other shapes, beside it or as lookup_both_kernel), back to back"
     return {"ms_per_step": ms_per_step, "forward_ms": forward_ms, "kernel_ms": kernel_ms, "kernel": kernel_name,
             "checked": checked}
 

@@ -247,6 +247,20 @@ bool lean_shape(const TableDesc& d) {
 bool lean_wide4_shape(const TableDesc& d) {
   return lean_shape(d) && d.ty == ST_INT4 && d.lanes >= 8 && !d.inline_hdr;
 }
+// What lookup_matrix.h pools: 4- and 8-bit rows of 64 or 128 bytes of elements behind a half-precision header, on dword
+// boundaries, in tables that 32-bit offsets reach, with whole 16-byte pieces of output.
+bool matrix_shape(const TableDesc& d, int64_t total_D) {
+  if ((d.ty != ST_INT4 && d.ty != ST_INT8) || d.sb_fp32 || (d.data_bytes != 64 && d.data_bytes != 128)) return false;
+  if (d.weights_offset % 4 || d.row_stride % 4 || d.sb_off % 4 || d.data_off % 4 || d.out_col % 8 || total_D % 8) return false;
+  return d.num_rows > 0 && d.num_rows <= MATRIX_TABLE_BYTES / d.row_stride;
+}
+// Bags a wave of it pools, eight at a time: with 16 the second eight's entries are on their way while the first eight are
+// added up, which pays where enough waves are left (12 tables of 256 4-bit columns: x 131072 bags x 15 593 -> 564 us, 570 with
+// 32; x 9000 x 45 176 -> 187). The device holds 4096 waves at a time.
+int matrix_wave_bags(int64_t bags) { return bags >= 16 * 16384 ? 16 : 8; }
+// 0: no forward takes it, -1: by the rule (tests and benchmarks: fbgemm_amd_set_matrix).
+int g_matrix_override = -1;
+
 // When forwards that could take that instance do: 0 never, 2 always, 1 (default) whichever of
 // the two kernels the first forwards of a work set measure as the faster one (FBGEMM_AMD_WIDE4 at
 // load time; fbgemm_amd_set_wide4 for tests and benchmarks).
@@ -984,6 +998,11 @@ int fbgemm_amd_set_wide4(int32_t mode) {
   return 0;
 }
 
+int fbgemm_amd_set_matrix(int32_t on) {
+  g_matrix_override = on < 0 ? -1 : on != 0;
+  return 0;
+}
+
 int fbgemm_amd_set_lean(int32_t on) {
   g_lean_override = on < 0 ? -1 : (on != 0);
   return 0;
@@ -1101,6 +1120,13 @@ struct fbgemm_amd_tbe_plan {
   };
   struct Work {
     WorkList lean, general;
+    // the lean list's tables where the matrix kernel takes them all (made by the first forward outside a capture that
+    // could use it; until then such forwards take the lists above)
+    WorkList matrix;
+    bool matrix_made = false;
+    bool matrix_int4 = false, matrix_wide = false;
+    int matrix_bags = 0; // bags a wave of it pools
+    bool rest_counts = false; // the general list is so much beside it that its bags are worth ordering
     BagEntry* d_order[ORDER_SLOTS] = {nullptr, nullptr, nullptr, nullptr}; // T*B bags each, rewritten by every forward
     hipStream_t order_stream[ORDER_SLOTS] = {nullptr, nullptr, nullptr, nullptr};
     bool order_claimed[ORDER_SLOTS] = {false, false, false, false};
@@ -1165,7 +1191,7 @@ struct fbgemm_amd_tbe_plan {
 namespace {
 
 void free_work(fbgemm_amd_tbe_plan::Work& w) {
-  for (fbgemm_amd_tbe_plan::WorkList* l : {&w.lean, &w.general}) {
+  for (fbgemm_amd_tbe_plan::WorkList* l : {&w.lean, &w.general, &w.matrix}) {
     if (l->d_work) (void)hipFree(l->d_work);
     if (l->d_xcd_start) (void)hipFree(l->d_xcd_start);
     *l = fbgemm_amd_tbe_plan::WorkList();
@@ -1244,7 +1270,7 @@ int build_work_list(const std::vector<TableDesc>& tables, const std::vector<int>
   // CUs at all times; taking few tables at a time keeps the working set of
   // the XCD's L2 small (hot rows of a table are reused while they are there).
   for (int x = 0; x < nx; ++x) {
-    std::vector<std::pair<double, WaveWork>> keyed;
+    const size_t run_first = list.size();
     std::map<std::pair<int, int>, std::vector<Slice>> shapes; // slices of a shape, largest first (per_x order)
     for (const Slice& sl : per_x[x]) {
       const TableDesc& d = tables[sl.t];
@@ -1252,22 +1278,21 @@ int build_work_list(const std::vector<TableDesc>& tables, const std::vector<int>
     }
     size_t depth = 0;
     for (auto& kv : shapes) depth = std::max(depth, kv.second.size());
-    int gidx = 0;
     for (size_t i = 0; i < depth; ++i) {
+      std::vector<std::pair<double, WaveWork>> keyed;
       for (auto& kv : shapes) {
         if (i >= kv.second.size()) continue;
         const Slice& sl = kv.second[i];
         const int G = bags_per_wave(tables[sl.t].lanes, tables[sl.t].packed);
         for (int k = 0; k < sl.count; ++k)
-          keyed.push_back({(double)gidx + (k + 0.5) / sl.count, WaveWork{sl.t, (sl.first + k * sl.step) * G}});
+          keyed.push_back({(k + 0.5) / sl.count, WaveWork{sl.t, (sl.first + k * sl.step) * G}});
       }
-      ++gidx;
+      const auto earlier = [](const std::pair<double, WaveWork>& p, const std::pair<double, WaveWork>& q) { return p.first < q.first; };
+      if (!std::is_sorted(keyed.begin(), keyed.end(), earlier)) std::stable_sort(keyed.begin(), keyed.end(), earlier); // one slice is in order
+      for (auto& kv : keyed) list.push_back(kv.second);
     }
-    std::stable_sort(keyed.begin(), keyed.end(),
-                     [](const std::pair<double, WaveWork>& p, const std::pair<double, WaveWork>& q) { return p.first < q.first; });
-    for (auto& kv : keyed) list.push_back(kv.second);
     xcd_start[x + 1] = (int64_t)list.size();
-    longest = std::max<int64_t>(longest, (int64_t)keyed.size());
+    longest = std::max<int64_t>(longest, (int64_t)(list.size() - run_first));
   }
   out->num_waves = longest;
   HIP_TRY(hipMalloc((void**)&out->d_work, sizeof(WaveWork) * list.size()));
@@ -1275,6 +1300,42 @@ int build_work_list(const std::vector<TableDesc>& tables, const std::vector<int>
   HIP_TRY(hipMalloc((void**)&out->d_xcd_start, sizeof(int64_t) * 9));
   HIP_TRY(hipMemcpy(out->d_xcd_start, xcd_start.data(), sizeof(int64_t) * 9, hipMemcpyHostToDevice));
   return 0;
+}
+
+// The matrix kernel's list of a work set, where it takes all tables of the lean kernel's (which all have rows of one type
+// and width then). Without the memory for it the set's forwards take the lean kernels.
+void make_matrix_list(const fbgemm_amd_tbe_plan* plan, const std::vector<TableDesc>& tables, int32_t B, fbgemm_amd_tbe_plan::Work* w) {
+  w->matrix_made = true;
+  std::vector<int> members;
+  int64_t bags = 0;
+  std::vector<TableDesc> by_wave = tables;
+  double cost = 0.0, rest_cost = 0.0;
+  for (int t = 0; t < plan->T; ++t) {
+    if (!lean_shape(tables[t])) {
+      rest_cost += row_cost(tables[t]);
+      continue;
+    }
+    if (!matrix_shape(tables[t], plan->total_D)) return;
+    if (!members.empty() && (tables[t].ty != tables[members[0]].ty || tables[t].data_bytes != tables[members[0]].data_bytes)) return;
+    cost += row_cost(tables[t]);
+    members.push_back(t);
+    bags += B;
+  }
+  if (members.empty()) return;
+  w->matrix_bags = matrix_wave_bags(bags);
+  for (int t : members) { // so many bags a wave (bags_per_wave)
+    by_wave[t].lanes = 64 / w->matrix_bags;
+    by_wave[t].packed = 0;
+  }
+  w->matrix_int4 = tables[members[0]].ty == ST_INT4;
+  w->matrix_wide = tables[members[0]].data_bytes == 128;
+  w->rest_counts = 4.0 * rest_cost > cost;
+  if (build_work_list(by_wave, members, B, &w->matrix) != 0) {
+    if (w->matrix.d_work) (void)hipFree(w->matrix.d_work);
+    if (w->matrix.d_xcd_start) (void)hipFree(w->matrix.d_xcd_start);
+    w->matrix = fbgemm_amd_tbe_plan::WorkList();
+    (void)hipGetLastError();
+  }
 }
 
 // Cached work lists beyond this many: the least recently used one that no graph can hold is dropped.
@@ -1632,6 +1693,8 @@ int tbe_forward_impl(
   const RankRecord* rank_records = nullptr;
   const int64_t* rank_offsets = nullptr;
   bool reuse_order = false;
+  const bool ordered = sort_bags_default() && indices_numel >= (int64_t)SORT_MIN_LOOKUPS;
+  bool use_matrix = false;
   bool use_w4 = false;  // the lean tables take the four-waves-per-SIMD instance
   int measure_w4 = -1;  // >= 0: this forward times its lean kernel (0 / 1: which one) for the work set's choice
   {
@@ -1711,6 +1774,16 @@ int tbe_forward_impl(
     }
     it->second.pinned = it->second.pinned || capturing;
     it->second.last_use = ++plan->use_clock;
+    // Unweighted forwards in the tolerance-grade mode whose lean tables the matrix kernel takes all: it is the faster one
+    // wherever the lean kernels would get the 16-byte lanes (of 88 forwards of one row type and width, 12 000 to 500 000 bags of
+    // 2 to 100 rows, .34 to 1.01 of their time, .74 on average). Tables for the general kernel run beside it on the side
+    // stream, in forwards of the size that has one; smaller ones stay with the launch of both kernels (41 tables x 363 x 16,
+    // three of them 2-bit: 20.6 us there, 29.6 one behind the other).
+    if (g_matrix_override != 0 && plan->accumulate == FBGEMM_AMD_ACC_FAST && !checked && !d_indice_weights && !d_index_remappings && !d_q8_out &&
+        !burst.waves && variant != 2 && (uintptr_t)d_output % 16 == 0 && it->second.lean.num_waves > 0 && (it->second.general.num_waves == 0 || ordered)) {
+      if (!it->second.matrix_made && !capturing) make_matrix_list(plan, tables, B, &it->second);
+      use_matrix = it->second.matrix.num_waves > 0;
+    }
     // this stream's bag-order buffer: the one it has, else one nobody has claimed, else (outside
     // a capture) a new one; with all of that exhausted the first buffer is shared, and forwards
     // of this plan on the streams that share it must not overlap
@@ -1739,8 +1812,9 @@ int tbe_forward_impl(
           }
     }
     // the slot's side stream (default priority, like every stream here) and its two events
-    if (!capturing && !W.side_stream[order_slot] && W.lean.num_waves > 0 && W.general.num_waves > 0 &&
-        (W.lean_wide4 || d_index_remappings || d_q8_out)) {
+    if (!capturing && !W.side_stream[order_slot] && W.lean.num_waves > 0 &&
+        ((W.general.num_waves > 0 && (W.lean_wide4 || d_index_remappings || d_q8_out)) ||
+         (use_matrix && W.general.num_waves > 0))) {
       hipStream_t s2 = nullptr;
       hipEvent_t e1 = nullptr, e2 = nullptr;
       if (hipStreamCreateWithFlags(&s2, hipStreamNonBlocking) == hipSuccess &&
@@ -1757,7 +1831,7 @@ int tbe_forward_impl(
       }
     }
     // the lean kernel of this forward, where there is a choice
-    if (W.lean_wide4 && !d_q8_out && !burst.waves && W.d_redo[order_slot] && W.d_redo_count[order_slot] && sort_bags_default() &&
+    if (W.lean_wide4 && !use_matrix && !d_q8_out && !burst.waves && W.d_redo[order_slot] && W.d_redo_count[order_slot] && sort_bags_default() &&
         indices_numel >= (int64_t)SORT_MIN_LOOKUPS) {
       const int mode = wide4_mode();
       if (mode == 2) {
@@ -1856,7 +1930,36 @@ int tbe_forward_impl(
     HIP_TRY(launch_lookup_burst(a, index_bits == 64, plan->max_D, plan->max_bits, burst.waves, burst.lds_bytes, stream));
     return 0;
   }
-  if (sort_bags_default() && indices_numel >= (int64_t)SORT_MIN_LOOKUPS) {
+  static const int side_enabled = env_int("FBGEMM_AMD_SIDE_STREAM", 1);
+  // The matrix kernel's bags need no order: the tables that it does not take are ordered and pooled beside it.
+  if (use_matrix) {
+    LookupArgs m = a;
+    m.tables = plan->d_tables;
+    m.work = w.matrix.d_work;
+    m.xcd_start = w.matrix.d_xcd_start;
+    m.num_waves = w.matrix.num_waves;
+    m.wave_bags = w.matrix_bags;
+    hipStream_t side = side_enabled && w.general.num_waves > 0 ? w.side_stream[order_slot] : nullptr;
+    if (w.general.num_waves > 0) {
+      if (ordered && (!side || w.rest_counts)) {
+        if (!reuse_order) HIP_TRY(launch_bag_order(d_offsets, offset_bits == 64, B, plan->T, w.d_order[order_slot], stream));
+        a.order = w.d_order[order_slot];
+      }
+      if (side) {
+        HIP_TRY(hipEventRecord(w.side_fork[order_slot], stream));
+        HIP_TRY(hipStreamWaitEvent(side, w.side_fork[order_slot], 0));
+      }
+      a.work = w.general.d_work;
+      a.xcd_start = w.general.d_xcd_start;
+      a.num_waves = w.general.num_waves;
+      HIP_TRY(launch_lookup(a, index_bits == 64, side ? side : stream));
+      if (side) HIP_TRY(hipEventRecord(w.side_join[order_slot], side));
+    }
+    HIP_TRY(launch_lookup_matrix(m, index_bits == 64, w.matrix_int4, w.matrix_wide, stream));
+    if (side) HIP_TRY(hipStreamWaitEvent(stream, w.side_join[order_slot], 0));
+    return 0;
+  }
+  if (ordered) {
     if (!reuse_order) HIP_TRY(launch_bag_order(d_offsets, offset_bits == 64, B, plan->T, w.d_order[order_slot], stream));
     a.order = w.d_order[order_slot];
   }
@@ -1879,7 +1982,6 @@ int tbe_forward_impl(
   // Otherwise, in a forward long enough not to notice two events (the size from which the bags are ordered), the
   // general kernel runs on the slot's side stream, beside the lean one, forked off behind the scheduler and joined
   // before the forward's stream goes on.
-  static const int side_enabled = env_int("FBGEMM_AMD_SIDE_STREAM", 1);
   hipStream_t side = (side_enabled && w.lean.num_waves > 0 && w.general.num_waves > 0 && a.order) ? w.side_stream[order_slot] : nullptr;
   if (w.general.num_waves > 0) {
     a.work = w.general.d_work;

@@ -10,6 +10,7 @@
 namespace fbgemm_amd {
 hipError_t launch_lookup(const LookupArgs& a, bool idx64, hipStream_t stream);
 hipError_t launch_lookup_lean(const LookupArgs& a, bool idx64, bool exact, bool wide4, hipStream_t stream);
+hipError_t launch_lookup_matrix(const LookupArgs& a, bool idx64, bool int4, bool wide, hipStream_t stream); // rows of 4 or 8 bits, of 128 or 64 bytes
 // A grid that holds both kernels' lists, of which each may be as long as a grid can be
 inline bool lookup_both_fits(int64_t general_waves, int64_t lean_waves) { return 8 * (general_waves + lean_waves) <= 0x7fffffffLL; }
 hipError_t launch_lookup_both(const LookupArgs& a, const WorkRun& lean, bool idx64, bool exact, hipStream_t stream);

@@ -203,6 +203,7 @@ struct LookupArgs {
   // last one sets both counters back to zero.
   WaveWork* redo;
   int32_t* redo_count;
+  int32_t wave_bags;         // lookup_matrix_kernel only: bags a wave pools, 8, 16 or 32
   Status* status;
   // A checked forward (fbgemm_amd_tbe_forward_checked): an index outside its table reads row 0 and is counted instead of
   // reported; offsets that are not in order from 0 to index_size are reported.
@@ -218,6 +219,9 @@ constexpr int64_t burst_pitch(int32_t max_D, int32_t max_bits) {
   return (((int64_t)(max_D < BURST_COLS ? max_D : BURST_COLS) * max_bits + 7) / 8 + 15) / 16 * 16;
 }
 constexpr bool burst_fits(int32_t max_D, int32_t max_bits, int64_t lds_bytes) { return max_D > 0 && max_bits > 0 && lds_bytes >= 8 * burst_pitch(max_D, max_bits); }
+
+// The matrix kernel's tables, at most; its offsets of entries that add nothing lie behind them, and a row's width short of 2^32.
+constexpr int64_t MATRIX_TABLE_BYTES = 0xffff0000LL;
 
 // The bounds check with the pruned-row mapping (check_remap_kernel).
 struct CheckRemapArgs {

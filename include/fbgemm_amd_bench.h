@@ -56,12 +56,15 @@ int fbgemm_amd_bench_gather(const void* d_table, int64_t rows, int64_t row_strid
  * gives every bag a workgroup: 0 = never, 1 / 4 = every launch it can take, with
  * that many waves per bag, -1 = by the rule on sizes (the default; off while
  * fbgemm_amd_set_narrow_below_waves is 0).
+ * fbgemm_amd_set_matrix: 0 = the matrix kernel takes no forward, -1 = by the rule
+ * (the default).
  * fbgemm_amd_set_wide4: which lean kernel large forwards take whose lean tables
  * all have 4-bit rows in bags of 8 lanes and more: 0 = the general-purpose one,
  * 2 = the four-waves-per-SIMD instance, 1 = whichever the first forwards of a
  * batch size measure as the faster (the default, FBGEMM_AMD_WIDE4 at load
  * time), -1 = back to the default. */
 int fbgemm_amd_set_burst(int32_t waves);
+int fbgemm_amd_set_matrix(int32_t on);
 int fbgemm_amd_set_lean(int32_t on);
 int fbgemm_amd_set_narrow_below_waves(int32_t waves);
 int fbgemm_amd_set_wide4(int32_t mode);

@@ -209,6 +209,7 @@ hipError_t launch_lookup(const LookupArgs& a, bool, hipStream_t) {
   if (a.rank_offsets) (void)*(volatile const int64_t*)&a.rank_offsets[0];
   return LAUNCHED();
 }
+hipError_t launch_lookup_matrix(const LookupArgs& a, bool idx64, bool, bool, hipStream_t s) { return launch_lookup(a, idx64, s); }
 hipError_t launch_lookup_lean(const LookupArgs& a, bool idx64, bool, bool wide4, hipStream_t s) {
   if (wide4) { // the redo queue of that instance must be there, and as long as the work list
     if (!a.redo || !a.redo_count) return hipErrorInvalidValue;
