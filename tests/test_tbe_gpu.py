@@ -920,3 +920,36 @@ def test_remap_offsets_must_cover_every_feature(ops):
     rc = _lib.lib().fbgemm_amd_tbe_forward_pruned(plan.handle, p(d[0]), None, p(d[1]), p(d[2]), 64, 24, 13, 0, None, 0, p(d[5]),
                                                   p(d[3]), 32, p(d[4]), 3, p(st.buf), None)
     assert rc == -1 and b"need 4" in _lib.lib().fbgemm_amd_last_error()
+
+
+@pytest.mark.parametrize("B", [1000, 1025, 2049, 4097, 8192, 8193])
+@pytest.mark.parametrize("spread", ["fixed", "mixed"])
+def test_ordered_bags_give_the_unordered_bits(B, spread):
+    """Batch sizes at the edges of the scheduler's bags per thread and of its windows; bags of one length, and of lengths
+    from 0 to beyond its bins. Half of the tables at a time is too little to be ordered: the same bits."""
+    from fbgemm_amd import ops
+    T, D, rows = 6, 32, 500
+    gen = torch.Generator(device="cuda").manual_seed(B)
+    weights = torch.randint(0, 256, (T * rows * 32,), dtype=torch.uint8, generator=gen, device="cuda")
+    head = weights.view(T * rows, 32)[:, :4]
+    head.copy_(torch.rand(T * rows, 2, generator=gen, device="cuda").half().view(torch.uint8))
+    avg = -(-(2 * (1 << 20) + 2 * B) // (T * B)) + 1
+    lens = torch.full((T * B,), avg, device="cuda")
+    if spread == "mixed":
+        lens = torch.randint(0, 2 * avg, (T * B,), generator=gen, device="cuda")
+        lens[::997] = 1500
+        lens[1] += max(0, (1 << 21) - int(lens.sum()))
+    off = torch.nn.functional.pad(lens.cumsum(0), (1, 0))
+    idx = torch.randint(0, rows, (int(off[-1]),), generator=gen, device="cuda")
+    assert idx.numel() >= 1 << 21
+
+    def forward(t0, t1):
+        n = t1 - t0
+        o = off[t0 * B:t1 * B + 1]
+        i = idx[int(o[0]):int(o[-1])].contiguous()
+        dev = lambda x, ty: torch.tensor(x, dtype=ty, device="cuda")
+        return ops.int_nbit_split_embedding_codegen_lookup_function(
+            weights, weights[:0], dev([0] * n, torch.int32), dev([rows * 32 * t for t in range(t0, t1)], torch.int64), dev([INT4] * n, torch.uint8),
+            dev([D * t for t in range(n + 1)], torch.int32), D * n, 0, D, 0, 0, 0, i, (o - o[0]).contiguous(), 0, None, FP32, row_alignment=16)
+    whole = forward(0, T)
+    assert torch.equal(whole, torch.cat([forward(0, 3), forward(3, T)], 1))
