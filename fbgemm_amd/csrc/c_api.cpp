@@ -315,6 +315,10 @@ int wide4_mode() {
 // LDS: large launches want many workgroups resident, so they stage in 4 KB what takes at most two
 // stagings there (8-bit, 100 wide, 8192 x 60: 35.6 -> 31.2), in 8 KB otherwise (fp16, 200 wide, 16384 x 25:
 // 47.5 against 49.2); small ones stage as much as they can.
+// Lengths instead of offsets: up to so many bags every workgroup adds up those in front of its own, a launch less (what they read
+// together grows with the square of the bags). us a call, 8-bit rows of 100 columns, lengths turned into offsets first -> added up:
+//   1 bag x 5 18.1 -> 14.4    300 x 40 19.7 -> 16.8    1024 x 5 19.1 -> 15.8    2048 x 40 22.0 -> 18.8    4096 x 5 20.4 -> 18.9
+constexpr int64_t BURST_MAX_LENGTHS = 4096;
 constexpr int BURST_FOUR_WAVES_LDS = 32768;
 struct Burst {
   int waves = 0; // 0: another kernel takes the launch
@@ -907,17 +911,20 @@ int spmdm_launch_impl(
   // Ordering the bags pays once several waves' worth of bags and enough lookups exist
   // (the scheduler launch costs 6-8 us and buys ~5 % of the lookup: it pays from a few million lookups on)
   const bool sort = K == 1 && !burst.waves && sort_bags_default() && output_size > 2 * G && index_size >= (int64_t)SORT_MIN_LOOKUPS;
-  if (cfg->use_offsets) {
+  const bool lengths_in_kernel = !cfg->use_offsets && K == 1 && burst.waves && output_size <= BURST_MAX_LENGTHS;
+  const bool to_offsets = !cfg->use_offsets && !lengths_in_kernel;
+  if (!to_offsets) {
     a.offsets = d_offsets_or_lengths;
     a.off64 = cfg->offset_bits == 64;
+    a.lengths = lengths_in_kernel;
   }
-  if ((!cfg->use_offsets || sort) && noalloc) {
+  if ((to_offsets || sort) && noalloc) {
     // the static array: offsets first, then the bag order. Both are written in
     // full (output_size + 1 offsets, output_size entries) before they are read,
     // so what an earlier call left there does not matter.
     unsigned char* base;
     if (int rc = noalloc_scratch_ptr(&base)) return rc;
-    if (!cfg->use_offsets) {
+    if (to_offsets) {
       int64_t* offs = reinterpret_cast<int64_t*>(base);
       HIP_TRY(launch_lengths_to_offsets(d_offsets_or_lengths, cfg->offset_bits == 64, output_size, offs, stream));
       a.offsets = offs;
@@ -928,12 +935,12 @@ int spmdm_launch_impl(
       HIP_TRY(launch_bag_order(a.offsets, a.off64, (int32_t)output_size, 1, order, stream));
       a.order = order;
     }
-  } else if (!cfg->use_offsets || sort) {
+  } else if (to_offsets || sort) {
     // library-owned scratch: calls that use it must be ordered on one stream
     std::lock_guard<std::mutex> lk(g_mu);
     DeviceScratch* s;
     if (int rc = get_scratch(&s)) return rc;
-    if (!cfg->use_offsets) {
+    if (to_offsets) {
       if (int rc = grow(&s->offsets, &s->offsets_cap, output_size + 1, stream)) return rc;
       HIP_TRY(launch_lengths_to_offsets(d_offsets_or_lengths, cfg->offset_bits == 64, output_size, s->offsets, stream));
       a.offsets = s->offsets;

@@ -177,9 +177,39 @@ __device__ __forceinline__ void burst_store(const LookupArgs& a, const float (&a
   }
 }
 
+// The sum of the first `bag` lengths, for the whole workgroup: 16 loads in flight per thread.
+template <int WAVES, typename T>
+__device__ __forceinline__ int64_t burst_lengths_before(const T* lengths, int bag, int tid, int64_t* lds) {
+  constexpr int THREADS = 64 * WAVES;
+  int64_t sum = 0;
+  for (int i0 = 0; i0 < bag; i0 += 16 * THREADS) {
+    int v[16];
+#pragma unroll
+    for (int u = 0; u < 16; ++u) { // those past the bag read a length that does not count
+      const int i = i0 + u * THREADS + tid;
+      v[u] = (int)lengths[i < bag ? i : 0];
+      v[u] = i < bag ? v[u] : 0;
+    }
+#pragma unroll
+    for (int u = 0; u < 16; ++u) sum += v[u];
+  }
+#pragma unroll
+  for (int step = 32; step > 0; step >>= 1) sum += __shfl_xor(sum, step, 64);
+  if constexpr (WAVES > 1) {
+    if ((tid & 63) == 0) lds[tid >> 6] = sum;
+    __syncthreads();
+    sum = 0;
+#pragma unroll
+    for (int w = 0; w < WAVES; ++w) sum += lds[w];
+    __syncthreads(); // the rows' places are staged where the sums were
+  }
+  return sum;
+}
+
 // blockIdx: (bag, table, window of columns)
 // CHECKED: a checked forward's launch (LookupArgs::check_rows); the other instance keeps its registers and its time.
-template <typename index_t, int WAVES, bool CHECKED>
+// LENGTHS: a single table's launch that is handed lengths (LookupArgs::lengths): a workgroup adds up those in front of its bag.
+template <typename index_t, int WAVES, bool CHECKED, bool LENGTHS>
 __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(WAVES == 1 ? 5 : 4, 8))) void lookup_burst_kernel(const LookupArgs a, int lds_bytes) {
   constexpr int THREADS = 64 * WAVES;
   constexpr int K = BURST_COLS / THREADS; // columns per lane
@@ -199,8 +229,16 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(WAVE
 
   // the bag, judged like the other lookup kernels judge it
   const int64_t ob = (int64_t)table * a.B;
-  const int64_t o0 = read_offset(a.offsets, a.off64, ob + bag), o1 = read_offset(a.offsets, a.off64, ob + bag + 1);
-  const int64_t base = a.check_total ? read_offset(a.offsets, a.off64, ob) : 0;
+  int64_t o0, o1, base = 0;
+  if constexpr (LENGTHS) {
+    o0 = a.off64 ? burst_lengths_before<WAVES>(reinterpret_cast<const int64_t*>(a.offsets), bag, tid, reinterpret_cast<int64_t*>(burst_lds))
+                 : burst_lengths_before<WAVES>(reinterpret_cast<const int32_t*>(a.offsets), bag, tid, reinterpret_cast<int64_t*>(burst_lds));
+    o1 = o0 + (int64_t)(int)read_offset(a.offsets, a.off64, bag);
+  } else {
+    o0 = read_offset(a.offsets, a.off64, ob + bag);
+    o1 = read_offset(a.offsets, a.off64, ob + bag + 1);
+    if (a.check_total) base = read_offset(a.offsets, a.off64, ob);
+  }
   const int64_t pos0 = o0 - base;
   int64_t len = o1 - o0;
   if (len < 0) {
@@ -358,12 +396,15 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(WAVE
   hipError_t FN(const LookupArgs& a, dim3 grid, bool four_waves, int lds_bytes, hipStream_t stream) {       \
     const unsigned lds = (unsigned)((four_waves ? 256 : 64) * (sizeof(StageRow) + sizeof(StageMul)) + lds_bytes + 16); \
     if (a.check_rows) {                                                                                     \
-      if (four_waves) hipLaunchKernelGGL((lookup_burst_kernel<INDEX_T, 4, true>), grid, dim3(256), lds, stream, a, lds_bytes); \
-      else hipLaunchKernelGGL((lookup_burst_kernel<INDEX_T, 1, true>), grid, dim3(64), lds, stream, a, lds_bytes); \
+      if (four_waves) hipLaunchKernelGGL((lookup_burst_kernel<INDEX_T, 4, true, false>), grid, dim3(256), lds, stream, a, lds_bytes); \
+      else hipLaunchKernelGGL((lookup_burst_kernel<INDEX_T, 1, true, false>), grid, dim3(64), lds, stream, a, lds_bytes); \
+    } else if (a.lengths) {                                                                                 \
+      if (four_waves) hipLaunchKernelGGL((lookup_burst_kernel<INDEX_T, 4, false, true>), grid, dim3(256), lds, stream, a, lds_bytes); \
+      else hipLaunchKernelGGL((lookup_burst_kernel<INDEX_T, 1, false, true>), grid, dim3(64), lds, stream, a, lds_bytes); \
     } else if (four_waves) {                                                                                \
-      hipLaunchKernelGGL((lookup_burst_kernel<INDEX_T, 4, false>), grid, dim3(256), lds, stream, a, lds_bytes); \
+      hipLaunchKernelGGL((lookup_burst_kernel<INDEX_T, 4, false, false>), grid, dim3(256), lds, stream, a, lds_bytes); \
     } else {                                                                                                \
-      hipLaunchKernelGGL((lookup_burst_kernel<INDEX_T, 1, false>), grid, dim3(64), lds, stream, a, lds_bytes); \
+      hipLaunchKernelGGL((lookup_burst_kernel<INDEX_T, 1, false, false>), grid, dim3(64), lds, stream, a, lds_bytes); \
     }                                                                                                       \
     return hipGetLastError();                                                                               \
   }
