@@ -9,11 +9,9 @@ CFG=${1:-3}; OUT=${2:-profile_summary.txt}; shift; shift
 export TMPDIR=/tmp
 RAW=$(mktemp -d /tmp/fbgemm_amd_prof.XXXXXX)
 mkdir -p "$(dirname "$OUT")"
-# The counter passes run a handful of forwards, too few for the library to settle which lean kernel a
-# forward of wide 4-bit bags takes (it times both first): they are told to take the one the kernel trace
-# above shows for the steady state (PMC_EXTRA, "--wide4 on" for config 5).
+# PMC_EXTRA: arguments for the counter passes alone. They run a handful of forwards, too few for the library to settle which
+# lean kernel an exact or weighted forward of wide 4-bit bags takes (it times both first): "--wide4 on" or "off" for those.
 PMC_EXTRA=${PMC_EXTRA:-}
-case "$CFG $*" in "5 "*|"5") [ -z "$PMC_EXTRA" ] && PMC_EXTRA="--wide4 on";; esac
 BENCH="python3 bench.py --config $CFG --no-cpu --no-also --one-mode --no-check --calibration-copy-mib 1024 $*"
 {
   echo "# rocprofv3 summary, bench.py --config $CFG $*"
