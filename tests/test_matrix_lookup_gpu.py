@@ -184,3 +184,39 @@ def test_matrix_lookup_of_many_bags(fwd, D, ty):
         n = dev(lens[t * B:(t + 1) * B]).double()[:, None]
         err = (got[:, t * D:(t + 1) * D] - want).abs()
         assert bool((err <= (2 * n + 3) * 2.0 ** -23 * size).all())
+
+
+@pytest.mark.parametrize("beside", [False, True])
+def test_matrix_lookup_replays_from_a_graph(fwd, beside):
+    """Captured on a stream the plan has not met, alone and with 2-bit tables on the side stream; every replay against the
+    eager forward, with eager work of the same plan between the replays."""
+    from fbgemm_amd import ops
+    rng = np.random.default_rng(9)
+    specs = [(500, 128, INT8)] * 3 + ([(300, 32, INT2)] if beside else [])
+    weights, offs, _ = tables(rng, specs)
+    T, B = len(specs), 700
+    L = -(-(1 << 21) // (T * B)) if beside else 20  # the side stream belongs to forwards that order their bags
+    dev = lambda a: torch.from_numpy(np.ascontiguousarray(a)).cuda()
+    D = np.concatenate([[0], np.cumsum([s[1] for s in specs])]).astype(np.int32)
+    meta = (dev(weights), torch.zeros(0, dtype=torch.uint8, device="cuda"), dev(np.zeros(T, np.int32)), dev(offs), dev(np.array([s[2] for s in specs], np.uint8)), dev(D))
+    off = dev((np.arange(T * B + 1) * L).astype(np.int64))
+    idx = torch.zeros(T * B * L, dtype=torch.int64, device="cuda")
+    st = ops.Status()
+    call = lambda: ops.int_nbit_split_embedding_codegen_lookup_function(
+        *meta, int(D[-1]), 512, 512, 512, 512, 512, idx, off, 0, None, BF16, row_alignment=ALIGN, status=st, accumulate=ops.ACC_FAST)
+    call()
+    torch.cuda.synchronize()
+    stream = torch.cuda.Stream()
+    with torch.cuda.stream(stream):
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=stream):
+            captured = call()
+    torch.cuda.synchronize()
+    for _ in range(4):
+        idx.copy_(dev(rng.integers(0, 300, size=idx.numel())))
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(call(), captured)
+        torch.cuda.synchronize()
+    assert st.read() == (0, -1)
