@@ -1783,7 +1783,7 @@ int tbe_forward_impl(
     it->second.last_use = ++plan->use_clock;
     // Unweighted forwards in the tolerance-grade mode whose lean tables the matrix kernel takes all: it is the faster one
     // wherever the lean kernels would get the 16-byte lanes (of 88 forwards of one row type and width, 12 000 to 500 000 bags of
-    // 2 to 100 rows, .34 to 1.01 of their time, .74 on average). Tables for the general kernel run beside it on the side
+    // 2 to 100 rows, .38 to 1.01 of their time, .77 on average; calls of 9 to 11 us, which their submission bounds, to 1.03). Tables for the general kernel run beside it on the side
     // stream, in forwards of the size that has one; smaller ones stay with the launch of both kernels (41 tables x 363 x 16,
     // three of them 2-bit: 20.6 us there, 29.6 one behind the other).
     if (g_matrix_override != 0 && plan->accumulate == FBGEMM_AMD_ACC_FAST && !checked && !d_indice_weights && !d_index_remappings && !d_q8_out &&

@@ -21,9 +21,9 @@
 // since a long one has 16 rows per step and none waits for it. us a forward, lean kernels (the better of the two, with the
 // scheduler where the bags are ordered) -> here:
 //   104 tables x 16384 x 15, 4-bit, 256 wide (8 of them 2-bit, beside it)   695 -> 545
-//   18 x 4571 x 26, fp32 output: 4-bit, 256 wide 79 -> 46, 128 wide 59 -> 30; 8-bit, 128 wide 60 -> 35, 64 wide 50 -> 25
-//   46 x 3787 x 2:               4-bit, 256 wide 41 -> 30, 128 wide 29 -> 21; 8-bit, 128 wide 32 -> 25, 64 wide 22 -> 18
-//   6 x 7081 x 45, uniform rows: 4-bit, 256 wide 87 -> 84, 128 wide 66 -> 60; 8-bit, 128 wide 85 -> 82, 64 wide 72 -> 60
+//   18 x 4571 x 26, fp32 output: 4-bit, 256 wide 73 -> 50, 128 wide 53 -> 32; 8-bit, 128 wide 55 -> 38, 64 wide 45 -> 27
+//   46 x 3787 x 2:               4-bit, 256 wide 40 -> 29, 128 wide 29 -> 21; 8-bit, 128 wide 32 -> 25, 64 wide 22 -> 18
+//   6 x 7081 x 45, uniform rows: 4-bit, 256 wide 88 -> 85, 128 wide 65 -> 61; 8-bit, 128 wide 84 -> 82, 64 wide 69 -> 60
 //
 // Rows are loaded with buffer instructions: an entry that adds nothing (past the end, rejected, skipped) has an offset
 // past the table, for which the load returns zeros without a request, so no load is under a condition and the waits
