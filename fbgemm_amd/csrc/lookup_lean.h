@@ -963,7 +963,7 @@ __device__ __forceinline__ void pool_lean_slow(const LookupArgs& a, const TableD
       lean_chunk<TY, EXACT, true, C * E>(acc, c * E, raw, m);
     }
   }
-  lean_report_bad<CHECKED>(a, bad_pos);
+  if (!CHECKED || L.sub == 0) lean_report_bad<CHECKED>(a, bad_pos); // every lane of the bag has met the same: one of them counts
   lean_write<EXACT, TY, C, INHDR, false, Q8>(a, d, L, table, acc, bsum, lds);
 }
 

@@ -95,6 +95,49 @@ def test_same_as_check_and_forward(case, pruned, dtype):
             assert [(out is None, repair) for out, repair in calls] == [(not (taken and in_order), taken and not in_order)] * 2, (what, mode)
 
 
+def in_the_kernels(m, *args):
+    """A forward that has to be made in the lookup's own kernels."""
+    from fbgemm_amd import ops
+    run, calls = ops.checked_lookup, []
+    try:
+        ops.checked_lookup = lambda *a: calls.append(run(*a)) or calls[-1]
+        out = m(*args)
+    finally:
+        ops.checked_lookup = run
+    assert [c[0] is out for c in calls] == [True]
+    return out
+
+
+@pytest.mark.parametrize("dtype", [torch.int32, torch.int64])
+@pytest.mark.parametrize("case,pruned", [(c, p) for c in ("lean", "lean ordered", "wide") for p in (False, True)] + [("both", False)])
+def test_waves_that_cannot_be_prescaled_count_once(case, pruned, dtype):
+    """Scales and weights that send a wave of the lean kernels to its row-at-a-time loop, which every lane of a bag walks,
+    with indices outside the tables among them: still the same bits and the same count."""
+    import fbgemm_amd
+    rng = np.random.default_rng(7)
+    m, idx, off = make(case, pruned, 1, rng)
+    for (_, rows, _, ty, _), (_, head) in zip(m.embedding_specs, m.split_embedding_weights()):
+        if not ty.is_float():  # a few rows whose scale (or bias) is no number
+            head[3], head[rows // 2] = (torch.tensor(h, dtype=torch.float16).view(torch.uint8).cuda() for h in ([np.inf, 1.0], [np.nan, np.inf]))
+    hit = rng.random(len(idx)) < 0.02
+    idx[hit] = rng.choice([-2, 1000, 1 << 30], size=int(hit.sum()))
+    huge = torch.rand(len(idx), device="cuda")
+    huge[::977] = 2.0 ** 120
+    huge[::1999] = float("inf")
+    idx, off = (torch.from_numpy(a).cuda().to(dtype) for a in (idx, off))
+    lib = fbgemm_amd.lib()
+    try:
+        for wide4 in (0, 2) if case == "wide" else (-1,):  # both lean kernels of wide 4-bit rows
+            lib.fbgemm_amd_set_wide4(wide4)
+            for psw in (None, huge):
+                want, count = apart(m, idx, off, psw)
+                m.bounds_check_warning.fill_(77)
+                assert torch.equal(in_the_kernels(m, idx, off, psw).view(torch.int32), want.view(torch.int32))
+                assert int(m.bounds_check_warning) == count > 0
+    finally:
+        lib.fbgemm_amd_set_wide4(-1)
+
+
 def test_counts_and_apart_forwards():
     """What a forward that had to be repaired leaves behind: some forwards in two calls, then one again, on any stream."""
     rng = np.random.default_rng(0)
