@@ -1093,6 +1093,7 @@ struct fbgemm_amd_tbe_plan {
   int32_t* d_D_offsets = nullptr; // the T + 1 output column offsets, for the 8-bit pooled output
   int32_t max_D = 0;
   int32_t max_bits = 0;           // of the row types
+  bool rowless = false;           // a table has no rows
   float* pooled_tmp = nullptr;    // fp32 [B, total_D] the 8-bit pooled output is quantized from
   int64_t pooled_tmp_cap = 0;
   int64_t* seg_offsets = nullptr; // split bags: where every segment starts (T*B*K + 1)
@@ -1397,6 +1398,7 @@ int fbgemm_amd_tbe_plan_create(
     const int64_t next = it != p.end() ? *it : (d.placement ? uvm_bytes : dev_bytes);
     d.num_rows = std::max<int64_t>(0, (next - d.weights_offset) / d.row_stride);
     d.skip_minus_one = 1;
+    plan->rowless = plan->rowless || d.num_rows == 0;
     plan->has_fp8 = plan->has_fp8 || d.ty == ST_FP8;
     plan->max_bits = std::max(plan->max_bits, type_bits(d.ty));
     const bool q = quantised(d.ty);
@@ -1623,6 +1625,7 @@ int tbe_forward_impl(
   };
   if (plan->has_fp8 && plan->fp8_shift == 0)
     return fail(FBGEMM_AMD_E_ARG, "the plan holds FP8 tables: set their exponent bits and bias first (fbgemm_amd_tbe_plan_set_fp8)");
+  if (checked && plan->rowless) return FORWARD_NOT_TAKEN; // the row 0 that the kernels take for an index outside its table has to be there
 
   // Few, long bags, and the plan accepts sums in another order: every bag is cut into K segments that
   // are pooled as bags of their own into fp32 partial sums, which a second launch adds up in order.

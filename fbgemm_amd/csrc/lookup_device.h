@@ -386,7 +386,8 @@ struct __attribute__((aligned(8))) StageMul {
 };
 
 // The rows an index of `table` may name; in a checked forward the table's own count, which the caller holds and which may
-// be less than what the weights buffer has room for. A count that cannot be right makes the caller look at it.
+// be less than what the weights buffer has room for. A count that cannot be right makes the caller look at it. (No table of a
+// checked forward is without rows: fbgemm_amd_tbe_forward_checked.)
 template <bool CHECKED = true>
 __device__ __forceinline__ int64_t index_bound(const LookupArgs& a, const TableDesc& d, int table, bool reporter) {
   if (!CHECKED || !a.check_rows) return d.num_rows;

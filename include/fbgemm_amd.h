@@ -272,7 +272,7 @@ int fbgemm_amd_tbe_forward_pruned(
  * those in *d_warning. Waits for the result: returns 0 when the output is what the check and the forward one
  * after the other make. Otherwise the caller makes the two calls: 1, and nothing was done, for the 8-bit output, a
  * plan in the tolerance-grade mode, a mapping over tables of other widths than the kernels' regular ones (unless
- * the forward is small), a stream that is being captured; 2, with an output and a *d_warning that mean nothing, for
+ * the forward is small), a table without rows, a stream that is being captured; 2, with an output and a *d_warning that mean nothing, for
  * offsets that are not in order from at least 0 to indices_numel, which the check repairs, and row counts below 1. */
 int fbgemm_amd_tbe_forward_checked(
     fbgemm_amd_tbe_plan* plan, const void* d_dev_weights, const void* d_uvm_weights,

@@ -526,6 +526,47 @@ void plan_of_wide_4bit_tables() {
   }
 }
 
+// What a checked forward checks against; the stand-in's launches read none of it
+struct Checked {
+  int32_t T;
+  int64_t *rows, *logical, *remap_off, *warning;
+  void* remap;
+  explicit Checked(int32_t tables) : T(tables) {
+    for (int64_t** p : {&rows, &logical, &remap_off, &warning}) CHECK(hipMalloc((void**)p, 8 * (T + 1)) == hipSuccess);
+    CHECK(hipMalloc(&remap, 64) == hipSuccess);
+  }
+  ~Checked() {
+    for (void* p : {(void*)rows, (void*)logical, (void*)remap_off, (void*)warning, remap}) hipFree(p);
+  }
+  int operator()(fbgemm_amd_tbe_plan* plan, Buffers& b, int64_t B, int64_t n, bool pruned, hipStream_t s) {
+    return fbgemm_amd_tbe_forward_checked(plan, b.weights, nullptr, b.indices, b.offsets, 64, n, T * B + 1, 0, nullptr, 1, b.out, rows, 1, warning,
+                                          pruned ? logical : nullptr, pruned ? remap : nullptr, 32, pruned ? remap_off : nullptr,
+                                          pruned ? T + 1 : 0, s);
+  }
+};
+
+// In a checked forward an index outside its table reads row 0: a plan with a table that has no rows
+// (the last one's row 0 would lie behind the weights) is not for the kernels, whatever the forward's size.
+void checked_forwards_need_rows_everywhere() {
+  const Problem whole = make_problem(4);
+  Checked call(whole.T);
+  Buffers b(whole, 3000, 16);
+  for (int rowless : {-1, 1, 3}) {
+    Problem p = whole;
+    if (rowless == 1) p.wo[1] = p.wo[2] - 16; // no room for a row
+    if (rowless == 3) p.bytes = p.wo[3];
+    fbgemm_amd_tbe_plan* plan = nullptr;
+    CHECK(fbgemm_amd_tbe_plan_create(&plan, p.T, p.wo.data(), p.tys.data(), p.D_offsets.data(), nullptr, p.bytes, 0, 16) == 0);
+    for (int t = 0; t < 4; ++t) CHECK((fbgemm_amd_tbe_plan_num_rows(plan, t) == 0) == (t == rowless));
+    for (int64_t B : {2, 3000}) {
+      const long before = hip_stub_launches();
+      CHECK(call(plan, b, B, 16, false, hip_stub_stream(0)) == (rowless >= 0 ? 1 : 0));
+      CHECK((hip_stub_launches() == before) == (rowless >= 0));
+    }
+    fbgemm_amd_tbe_plan_destroy(plan);
+  }
+}
+
 // Records of mappings, a plan's and a caller's, where an allocation fails: the call says so, leaves nothing behind, no
 // error for the next launch to find either, and works once memory is there
 void records_without_memory() {
@@ -579,6 +620,7 @@ int main() {
   burst_launches_fit();
   row_reads_stay_in_the_row();
   checks_share_no_scratch();
+  checked_forwards_need_rows_everywhere();
   allocation_failures_in_a_first_forward();
   printf("launches %ld, device allocations %ld\n", hip_stub_launches(), hip_stub_total_allocations());
   printf("PASSED\n");
