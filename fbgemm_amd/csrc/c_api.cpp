@@ -1784,12 +1784,17 @@ int tbe_forward_impl(
     }
     it->second.pinned = it->second.pinned || capturing;
     it->second.last_use = ++plan->use_clock;
+    exact = plan->accumulate != FBGEMM_AMD_ACC_FAST;
+    // the tolerance-grade instances of the lean kernel do not check, those of the general one do not where there is a mapping.
+    // Refused before the forward takes anything of the work set that only its end gives back (the turn to measure).
+    if (checked && !burst.waves && ((!exact && it->second.lean.num_waves > 0) || (d_index_remappings && it->second.general.num_waves > 0)))
+      return FORWARD_NOT_TAKEN;
     // Unweighted forwards in the tolerance-grade mode whose lean tables the matrix kernel takes all: it is the faster one
     // wherever the lean kernels would get the 16-byte lanes (of 88 forwards of one row type and width, 12 000 to 500 000 bags of
     // 2 to 100 rows, .38 to 1.01 of their time, .77 on average; calls of 9 to 11 us, which their submission bounds, to 1.03). Tables for the general kernel run beside it on the side
     // stream, in forwards of the size that has one; smaller ones stay with the launch of both kernels (41 tables x 363 x 16,
     // three of them 2-bit: 20.6 us there, 29.6 one behind the other).
-    if (g_matrix_override != 0 && plan->accumulate == FBGEMM_AMD_ACC_FAST && !checked && !d_indice_weights && !d_index_remappings && !d_q8_out &&
+    if (g_matrix_override != 0 && !exact && !checked && !d_indice_weights && !d_index_remappings && !d_q8_out &&
         !burst.waves && variant != 2 && (uintptr_t)d_output % 16 == 0 && it->second.lean.num_waves > 0 && (it->second.general.num_waves == 0 || ordered)) {
       if (!it->second.matrix_made && !capturing) make_matrix_list(plan, tables, B, &it->second);
       use_matrix = it->second.matrix.num_waves > 0;
@@ -1856,9 +1861,6 @@ int tbe_forward_impl(
       }
     }
     w = W;
-    exact = plan->accumulate != FBGEMM_AMD_ACC_FAST;
-    // the tolerance-grade instances of the lean kernel do not check, those of the general one do not where there is a mapping
-    if (checked && !burst.waves && ((!exact && W.lean.num_waves > 0) || (d_index_remappings && W.general.num_waves > 0))) return FORWARD_NOT_TAKEN;
     if (!checked && d_index_remappings && plan->ranks.records && plan->ranks.source == d_index_remappings && plan->ranks.bits == remap_bits) {
       rank_records = plan->ranks.records;
       rank_offsets = plan->ranks.offsets;

@@ -567,6 +567,36 @@ void checked_forwards_need_rows_everywhere() {
   }
 }
 
+// A checked forward that the kernels do not take keeps nothing of the work set: the plain forwards
+// behind it go on measuring the two lean kernels, and settle on the faster one.
+void refused_checked_forwards_keep_no_turn() {
+  Problem p;
+  p.T = 3; // two wide 4-bit tables and a 2-bit one
+  p.tys = {3, 3, 4};
+  p.D_offsets = {0, 256, 512, 544};
+  p.wo = {0, 16384, 32768};
+  p.bytes = 40960;
+  const int64_t big_n = 1 << 21, B = 36000;
+  Checked call(p.T);
+  Buffers b(p, B, big_n);
+  CHECK(fbgemm_amd_set_matrix(0) == 0);
+  hip_stub_set_elapsed_ms(1.0f, 0.5f);
+  for (int fast : {0, 1}) {
+    fbgemm_amd_tbe_plan* plan = nullptr;
+    CHECK(fbgemm_amd_tbe_plan_create(&plan, p.T, p.wo.data(), p.tys.data(), p.D_offsets.data(), nullptr, p.bytes, 0, 16) == 0);
+    CHECK(fbgemm_amd_tbe_plan_set_accumulate(plan, fast ? FBGEMM_AMD_ACC_FAST : FBGEMM_AMD_ACC_EXACT) == 0);
+    for (int i = 0; i < 20; ++i) { // refused: a mapping beside a general table, the tolerance-grade mode
+      CHECK(call(plan, b, B, big_n, !fast, hip_stub_stream(i % 2)) == 1);
+      CHECK(forward(plan, p, b, B, big_n, hip_stub_stream(i % 2)) == 0);
+    }
+    const long settled = hip_stub_wide4_launches();
+    for (int i = 0; i < 6; ++i) CHECK(forward(plan, p, b, B, big_n, hip_stub_stream(i % 2)) == 0);
+    CHECK(hip_stub_wide4_launches() - settled == 6);
+    fbgemm_amd_tbe_plan_destroy(plan);
+  }
+  CHECK(fbgemm_amd_set_matrix(-1) == 0);
+}
+
 // Records of mappings, a plan's and a caller's, where an allocation fails: the call says so, leaves nothing behind, no
 // error for the next launch to find either, and works once memory is there
 void records_without_memory() {
@@ -621,6 +651,7 @@ int main() {
   row_reads_stay_in_the_row();
   checks_share_no_scratch();
   checked_forwards_need_rows_everywhere();
+  refused_checked_forwards_keep_no_turn();
   allocation_failures_in_a_first_forward();
   printf("launches %ld, device allocations %ld\n", hip_stub_launches(), hip_stub_total_allocations());
   printf("PASSED\n");
