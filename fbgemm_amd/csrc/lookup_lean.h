@@ -244,7 +244,7 @@ __device__ __forceinline__ int lean_row(const LookupArgs& a, const TableDesc& d,
   }
   return (int)row;
 }
-constexpr int64_t LEAN_PRUNED = INT64_MIN; // what lean_remap returns for an entry that adds nothing
+constexpr int64_t LEAN_PRUNED = INT64_MIN; // what lean_remap returns for an entry that adds nothing (an index may have this value too)
 template <bool CHECKED>
 __device__ __forceinline__ int64_t lean_remap(const LookupArgs& a, const LeanLane& L, int64_t logical, int64_t pos, int64_t& bad_pos) {
   if (CHECKED) logical = logical_index(logical, L.logical);
@@ -260,7 +260,7 @@ __device__ __forceinline__ int64_t lean_remap(const LookupArgs& a, const LeanLan
   }
   const int64_t m = a.remap64 ? reinterpret_cast<const int64_t*>(a.remap)[L.remap_base + logical]
                               : (int64_t) reinterpret_cast<const int32_t*>(a.remap)[L.remap_base + logical];
-  return m == -1 ? LEAN_PRUNED : m;
+  return m == -1 ? LEAN_PRUNED : (m < -1 ? -2 : m);
 }
 template <bool CHECKED>
 __device__ __forceinline__ void lean_report_bad(const LookupArgs& a, int64_t bad_pos) {
@@ -699,7 +699,7 @@ __device__ __forceinline__ bool pool_lean(const LookupArgs& a, const TableDesc& 
       // loaded, loads the next block's weight elsewhere and moves both at the end of the loop,
       // which waits for that load and for everything issued before it
       asm volatile("v_mov_b32 %0, %1" : "=v"(cw[j]) : "v"(nw[j]));
-      if (have[j]) crow[j] = nrow[j] == LEAN_PRUNED ? LEAN_SKIP : lean_row<CHECKED>(a, d, L, nrow[j], L.pos0 + blk * LEAN_BLOCK + sub + j * SL, bad_pos);
+      if (have[j]) crow[j] = L.remapped && nrow[j] == LEAN_PRUNED ? LEAN_SKIP : lean_row<CHECKED>(a, d, L, nrow[j], L.pos0 + blk * LEAN_BLOCK + sub + j * SL, bad_pos);
     }
   };
   // The (scale, bias) headers of the rows staged last, asked for right in front of the first unit
@@ -944,7 +944,7 @@ __device__ __forceinline__ void pool_lean_slow(const LookupArgs& a, const TableD
     const float w = a.sample_weights ? a.sample_weights[L.pos0 + i] : 1.0f;
     if (CHECKED && a.remap && !L.remapped) row = logical_index(row, L.logical);
     if (L.remapped) row = lean_remap<CHECKED>(a, L, row, L.pos0 + i, bad_pos);
-    const int r = row == LEAN_PRUNED ? LEAN_SKIP : lean_row<CHECKED>(a, d, L, row, L.pos0 + i, bad_pos);
+    const int r = L.remapped && row == LEAN_PRUNED ? LEAN_SKIP : lean_row<CHECKED>(a, d, L, row, L.pos0 + i, bad_pos);
     if (r < 0) continue;
     const uint8_t* prow = wbase + (uint64_t)(uint32_t)r * (uint32_t)d.row_stride;
     float rs, rb;

@@ -22,17 +22,20 @@ SHAPES = {
 }
 
 
-def make(case, pruned, mode, rng):
+def make(case, pruned, mode, rng, indices_dtype=torch.int32, entries=()):
     from fbgemm_amd import module as M
     tables, B, avg = SHAPES[case]
     specs = [("", int(rng.integers(200, 900)), d, M.SparseType(ty), M.EmbeddingLocation.DEVICE) for ty, d in tables]
     m = M.IntNBitTableBatchedEmbeddingBagsCodegen(specs, bounds_check_mode=M.BoundsCheckMode(mode), output_dtype=M.SparseType.FP32,
-                                                  pooling_mode=M.PoolingMode.MEAN, fp8_exponent_bits=4, fp8_exponent_bias=7)
+                                                  pooling_mode=M.PoolingMode.MEAN, fp8_exponent_bits=4, fp8_exponent_bias=7,
+                                                  indices_dtype=indices_dtype)
     m.quantize_and_assign([torch.from_numpy(rng.normal(size=(n, d)).astype(np.float32)) for _, n, d, _, _ in specs])
     logical = [n for _, n, _, _, _ in specs]
     if pruned:  # not all tables, and entries beyond the physical rows and below -1 among the mappings'
         maps = [None if t % 3 == 2 else torch.from_numpy(rng.integers(-1, n + 2, size=2 * n) - 3 * (rng.random(2 * n) < 0.01))
                 for t, n in enumerate(logical)]
+        for k, entry in enumerate(entries):
+            maps[0][3 + k::17] = entry
         m.set_index_remappings([None if a is None else a.cuda() for a in maps])
         logical = [n if a is None else 2 * n for n, a in zip(logical, maps)]
     lens = rng.integers(0, 2 * avg + 1, size=len(tables) * B)
@@ -136,6 +139,39 @@ def test_waves_that_cannot_be_prescaled_count_once(case, pruned, dtype):
                 assert int(m.bounds_check_warning) == count > 0
     finally:
         lib.fbgemm_amd_set_wide4(-1)
+
+
+IN_KERNELS = [(c, p) for c in SHAPES for p in (False, True) if not p or c in ("burst", "burst windows", "lean", "lean ordered", "wide")]
+
+
+@pytest.mark.parametrize("case,pruned", IN_KERNELS)
+def test_lowest_value_of_an_index(case, pruned):
+    """No value of an index, or of a mapping's entry, is anything but an index: the lowest is outside its table like any other."""
+    rng = np.random.default_rng(11)
+    low = -(1 << 63)
+    m, idx, off = make(case, pruned, 1, rng, torch.int64, (low, low + 1))
+    hit = rng.random(len(idx)) < 0.02
+    idx[hit] = rng.choice([low, low + 1, -1], size=int(hit.sum()))
+    idx, off = torch.from_numpy(idx).cuda(), torch.from_numpy(off).cuda()
+    want, count = apart(m, idx, off, None)
+    assert torch.equal(in_the_kernels(m, idx, off).view(torch.int32), want.view(torch.int32))
+    assert int(m.bounds_check_warning) == count > 0
+
+
+@pytest.mark.parametrize("case", ["burst", "lean", "wide", "general", "both"])
+def test_lowest_value_of_an_index_is_reported(case):
+    """The same in a forward that does not check."""
+    from fbgemm_amd import ops
+    m, idx, off = make(case, False, 0, np.random.default_rng(12))
+    at = len(idx) // 3
+    idx[at] = -(1 << 63)
+    st = ops.Status()
+    ops.int_nbit_split_embedding_codegen_lookup_function(
+        m.weights_dev, m.weights_uvm, m.weights_placements, m.weights_offsets, m.weights_tys, m.D_offsets, m.total_D, m.max_int2_D,
+        m.max_int4_D, m.max_int8_D, m.max_float16_D, m.max_float32_D, torch.from_numpy(idx).cuda(), torch.from_numpy(off).cuda(), 0, None,
+        m.output_dtype, row_alignment=m.row_alignment,
+        max_float8_D=m.max_float8_D, fp8_exponent_bits=4, fp8_exponent_bias=7, status=st)
+    assert st.read() == (ops.ERR_INDEX_OUT_OF_RANGE, at)
 
 
 def test_counts_and_apart_forwards():
