@@ -328,6 +328,7 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(WAVE
             } else {
               row = a.remap64 ? reinterpret_cast<const int64_t*>(a.remap)[remap_base + row]
                               : (int64_t) reinterpret_cast<const int32_t*>(a.remap)[remap_base + row];
+              if (CHECKED) row = checked_entry<index_t>(row);
             }
             ok = row != -1;
           }

@@ -406,6 +406,12 @@ __device__ __forceinline__ int64_t logical_index(int64_t row, int64_t logical_ro
   return row != -1 && (row < 0 || row >= logical_rows) ? 0 : row;
 }
 
+// An entry of a mapping as the check of a pass of its own hands it on: in the indices' type.
+template <typename index_t>
+__device__ __forceinline__ int64_t checked_entry(int64_t m) {
+  return (int64_t)(index_t)m;
+}
+
 constexpr int MAX_GROUPS = 32; // bags per wave at most; lanes per bag >= 2
 constexpr int MAX_ROUND = 8;
 constexpr int64_t NO_ENTRY = INT64_MIN;

@@ -245,7 +245,7 @@ __device__ __forceinline__ int lean_row(const LookupArgs& a, const TableDesc& d,
   return (int)row;
 }
 constexpr int64_t LEAN_PRUNED = INT64_MIN; // what lean_remap returns for an entry that adds nothing (an index may have this value too)
-template <bool CHECKED>
+template <typename index_t, bool CHECKED>
 __device__ __forceinline__ int64_t lean_remap(const LookupArgs& a, const LeanLane& L, int64_t logical, int64_t pos, int64_t& bad_pos) {
   if (CHECKED) logical = logical_index(logical, L.logical);
   if (logical < 0 || logical >= L.remap_cap) {
@@ -258,8 +258,9 @@ __device__ __forceinline__ int64_t lean_remap(const LookupArgs& a, const LeanLan
     if (!((r.bits >> bit) & 1u)) return LEAN_PRUNED;
     return (int64_t)(r.before + (uint32_t)__builtin_popcount(r.bits & ((1u << bit) - 1u)));
   }
-  const int64_t m = a.remap64 ? reinterpret_cast<const int64_t*>(a.remap)[L.remap_base + logical]
-                              : (int64_t) reinterpret_cast<const int32_t*>(a.remap)[L.remap_base + logical];
+  int64_t m = a.remap64 ? reinterpret_cast<const int64_t*>(a.remap)[L.remap_base + logical]
+                        : (int64_t) reinterpret_cast<const int32_t*>(a.remap)[L.remap_base + logical];
+  if (CHECKED) m = checked_entry<index_t>(m);
   return m == -1 ? LEAN_PRUNED : (m < -1 ? -2 : m);
 }
 template <bool CHECKED>
@@ -690,7 +691,7 @@ __device__ __forceinline__ bool pool_lean(const LookupArgs& a, const TableDesc& 
     if (L.remapped) {
 #pragma unroll
       for (int j = 0; j < R; ++j)
-        if (have[j]) nrow[j] = lean_remap<CHECKED>(a, L, nrow[j], L.pos0 + blk * LEAN_BLOCK + sub + j * SL, bad_pos);
+        if (have[j]) nrow[j] = lean_remap<index_t, CHECKED>(a, L, nrow[j], L.pos0 + blk * LEAN_BLOCK + sub + j * SL, bad_pos);
     }
 #pragma unroll
     for (int j = 0; j < R; ++j) {
@@ -943,7 +944,7 @@ __device__ __forceinline__ void pool_lean_slow(const LookupArgs& a, const TableD
     int64_t row = (int64_t)idx[i];
     const float w = a.sample_weights ? a.sample_weights[L.pos0 + i] : 1.0f;
     if (CHECKED && a.remap && !L.remapped) row = logical_index(row, L.logical);
-    if (L.remapped) row = lean_remap<CHECKED>(a, L, row, L.pos0 + i, bad_pos);
+    if (L.remapped) row = lean_remap<index_t, CHECKED>(a, L, row, L.pos0 + i, bad_pos);
     const int r = L.remapped && row == LEAN_PRUNED ? LEAN_SKIP : lean_row<CHECKED>(a, d, L, row, L.pos0 + i, bad_pos);
     if (r < 0) continue;
     const uint8_t* prow = wbase + (uint64_t)(uint32_t)r * (uint32_t)d.row_stride;

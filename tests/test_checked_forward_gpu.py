@@ -158,6 +158,16 @@ def test_lowest_value_of_an_index(case, pruned):
     assert int(m.bounds_check_warning) == count > 0
 
 
+@pytest.mark.parametrize("case", [c for c, p in IN_KERNELS if p])
+def test_entries_wider_than_the_indices(case):
+    """A mapping of 64-bit entries under 32-bit indices: what does not fit them is cut, as the check of its own cuts it."""
+    m, idx, off = make(case, True, 1, np.random.default_rng(13), torch.int64, ((1 << 32) - 1, (1 << 32) + 3, 1 << 31, (1 << 40) + 10_000))
+    idx, off = torch.from_numpy(idx).cuda().int(), torch.from_numpy(off).cuda().int()
+    want, count = apart(m, idx, off, None)
+    assert torch.equal(in_the_kernels(m, idx, off).view(torch.int32), want.view(torch.int32))
+    assert int(m.bounds_check_warning) == count > 0
+
+
 @pytest.mark.parametrize("case", ["burst", "lean", "wide", "general", "both"])
 def test_lowest_value_of_an_index_is_reported(case):
     """The same in a forward that does not check."""
