@@ -379,9 +379,11 @@ class IntNBitTableBatchedEmbeddingBagsCodegen(torch.nn.Module):
             index_remappings_offsets=self._feature_remap_offsets if fuse_remap else None)
 
     # Only what it saves to try: forwards left whose check is a pass of its own because an earlier one's offsets had to be
-    # repaired, and the number of offsets of the last forward that the lookup's kernels would not check.
+    # repaired; and the sizes of the last forward that the lookup's kernels would not check, with how many more of them are
+    # not tried. (What decides besides the sizes, the plan's arithmetic for one, may change.)
     _apart_left = 0
     _apart_for = -1
+    _apart_times = 0
 
     def _checked_forward(self, buffers, indices, offsets, per_sample_weights, arrayed, T):
         """The check in the lookup's own kernels, or None where it has to be a pass of its own."""
@@ -389,8 +391,13 @@ class IntNBitTableBatchedEmbeddingBagsCodegen(torch.nn.Module):
             self._apart_left -= 1
             return None
         n = offsets.numel()
-        if self._apart_for == n:
-            return None
+        sizes = (n, indices.numel().bit_length(), arrayed)
+        if self._apart_for == sizes:
+            self._apart_times -= 1
+            if self._apart_times >= 0:
+                return None
+        if per_sample_weights is not None and per_sample_weights.numel() > 0 and per_sample_weights.size(0) != indices.numel():
+            return None  # the check's to refuse
         rows, warning = buffers["rows_per_table"], buffers["bounds_check_warning"]
         maps = ()
         if arrayed:
@@ -406,7 +413,10 @@ class IntNBitTableBatchedEmbeddingBagsCodegen(torch.nn.Module):
             self.row_alignment, (self.max_float8_D, self.fp8_exponent_bits, self.fp8_exponent_bias), rows, self.bounds_check_mode_int,
             warning, *maps)
         if out is None:
-            self._apart_left, self._apart_for = (64, -1) if repair else (0, n)
+            if repair:
+                self._apart_left, self._apart_for = 64, -1
+            elif not torch.cuda.is_current_stream_capturing():  # a capture is refused for itself
+                self._apart_for, self._apart_times = sizes, 64
         return out
 
     def _check_and_remap(self, indices, offsets, per_sample_weights, check, hashed, arrayed, fuse_remap):

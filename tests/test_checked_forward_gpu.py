@@ -218,3 +218,45 @@ def test_counts_and_apart_forwards():
             f()
         errors.append(str(e.value))
     assert errors[0] == errors[1]
+
+
+def test_refusals_are_not_for_ever():
+    """A forward that the kernels do not check says little about others of its batch size: not where it was captured or its
+    arguments were wrong, and where the mapping or the plan's arithmetic was why, not once that has changed."""
+    from fbgemm_amd import ops
+    rng = np.random.default_rng(5)
+    m, idx, off = make("lean", False, 1, rng)
+    idx, off = torch.from_numpy(idx).cuda(), torch.from_numpy(off).cuda()
+    want, _ = apart(m, idx, off, None)
+    assert torch.equal(in_the_kernels(m, idx, off), want)
+    stream = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    with torch.cuda.stream(stream):
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=stream):
+            assert m._checked_forward(m._buffers, idx, off, None, False, len(m.embedding_specs)) is None
+            torch.zeros(8, device="cuda")  # a graph of something
+    torch.cuda.synchronize()
+    assert torch.equal(in_the_kernels(m, idx, off), want)
+    with pytest.raises(RuntimeError):
+        m(idx, off, torch.ones(len(idx) - 1, device="cuda"))
+    assert torch.equal(in_the_kernels(m, idx, off), want)
+    plan = ops._plan_for(m.weights_dev, m.weights_uvm, m.weights_placements, m.weights_offsets, m.weights_tys, m.D_offsets, m.row_alignment)
+    tried, run = [], ops.checked_lookup
+    try:
+        ops.checked_lookup = lambda *a: tried.append(run(*a)) or tried[-1]
+        plan.set_accumulate(ops.ACC_FAST)
+        for _ in range(10):
+            m(idx, off)
+        assert len(tried) == 1 and tried[0][0] is None
+        plan.set_accumulate(ops.ACC_EXACT)
+        for _ in range(60):
+            assert torch.equal(m(idx, off), want)
+        assert len(tried) == 6 and all(c[0] is not None for c in tried[1:])
+    finally:
+        ops.checked_lookup = run
+    m, idx, off = make("both", True, 1, rng)
+    idx, off = torch.from_numpy(idx % 200).cuda(), torch.from_numpy(off).cuda()
+    m(idx, off)
+    m.set_index_remappings([None] * len(m.embedding_specs))
+    assert torch.equal(in_the_kernels(m, idx, off), apart(m, idx, off, None)[0])
