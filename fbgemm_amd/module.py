@@ -391,13 +391,10 @@ class IntNBitTableBatchedEmbeddingBagsCodegen(torch.nn.Module):
             self._apart_left -= 1
             return None
         n = offsets.numel()
-        sizes = (n, indices.numel().bit_length(), arrayed)
-        if self._apart_for == sizes:
+        if self._apart_for != -1 and self._apart_for == (n, indices.numel().bit_length(), arrayed):
             self._apart_times -= 1
             if self._apart_times >= 0:
                 return None
-        if per_sample_weights is not None and per_sample_weights.numel() > 0 and per_sample_weights.size(0) != indices.numel():
-            return None  # the check's to refuse
         rows, warning = buffers["rows_per_table"], buffers["bounds_check_warning"]
         maps = ()
         if arrayed:
@@ -415,8 +412,10 @@ class IntNBitTableBatchedEmbeddingBagsCodegen(torch.nn.Module):
         if out is None:
             if repair:
                 self._apart_left, self._apart_for = 64, -1
-            elif not torch.cuda.is_current_stream_capturing():  # a capture is refused for itself
-                self._apart_for, self._apart_times = sizes, 64
+            elif not (torch.cuda.is_current_stream_capturing() or (per_sample_weights is not None and per_sample_weights.numel() > 0
+                                                                   and per_sample_weights.size(0) != indices.numel())):
+                # (a capture, and weights that are the check's to refuse, say nothing about the next forward)
+                self._apart_for, self._apart_times = (n, indices.numel().bit_length(), arrayed), 64
         return out
 
     def _check_and_remap(self, indices, offsets, per_sample_weights, check, hashed, arrayed, fuse_remap):
