@@ -223,6 +223,9 @@ constexpr bool burst_fits(int32_t max_D, int32_t max_bits, int64_t lds_bytes) { 
 
 // The matrix kernel's tables, at most; its offsets of entries that add nothing lie behind them, and a row's width short of 2^32.
 constexpr int64_t MATRIX_TABLE_BYTES = 0xffff0000LL;
+// Its runs of entries, at most: positions of the two stages behind a run are counted in 31 bits. Forwards with more lookups, whose
+// bags could be that long, are the lean kernels'.
+constexpr int64_t MATRIX_MAX_RUN = 0x7fffff00LL;
 
 // The bounds check with the pruned-row mapping (check_remap_kernel).
 struct CheckRemapArgs {

@@ -40,7 +40,6 @@ typedef float matrix_f32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int MATRIX_STAGE = 64;               // entries whose row numbers and headers are staged at a time
 constexpr uint32_t MATRIX_NO_ROW = 0xffff8000u; // offset of an entry that adds nothing; past every table (MATRIX_TABLE_BYTES)
-constexpr int64_t MATRIX_MAX_RUN = 0x7fffff00LL; // entries of a run: positions of the two stages behind it are counted in 31 bits
 constexpr int MATRIX_OUT_WORDS = 1024;         // four bags' output
 constexpr int MATRIX_LDS_WORDS = 2 * MATRIX_STAGE + MATRIX_OUT_WORDS; // in front of it the row offsets of two stages
 

@@ -58,6 +58,7 @@ long hip_stub_live_allocations(void);
 long hip_stub_total_allocations(void);
 long hip_stub_launches(void);
 long hip_stub_wide4_launches(void); // launches of the lean kernel's four-waves-per-SIMD instance
+long hip_stub_matrix_launches(void); // launches of the matrix kernel
 // what hipEventElapsedTime reports from now on: `general_ms` for a measurement of a forward whose last lean launch was
 // the general-purpose kernel, `wide4_ms` for one of the four-wave instance
 void hip_stub_set_elapsed_ms(float general_ms, float wide4_ms);

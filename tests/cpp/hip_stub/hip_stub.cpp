@@ -16,7 +16,7 @@ namespace {
 std::mutex g_mu;
 std::set<void*> g_live;
 std::set<hipStream_t> g_capturing;
-std::atomic<long> g_total{0}, g_launches{0}, g_fail_after{-1}, g_wide4{0}, g_device_waits{0};
+std::atomic<long> g_total{0}, g_launches{0}, g_fail_after{-1}, g_wide4{0}, g_matrix{0}, g_device_waits{0};
 std::vector<fbgemm_amd::CheckRemapArgs> g_checks; // those with a counter that have not finished
 thread_local hipError_t t_last_error = hipSuccess; // of an allocation that was made to fail
 std::atomic<int> g_last_lean_wide4{0};
@@ -145,6 +145,7 @@ long hip_stub_live_allocations(void) {
 long hip_stub_total_allocations(void) { return g_total.load(); }
 long hip_stub_launches(void) { return g_launches.load(); }
 long hip_stub_wide4_launches(void) { return g_wide4.load(); }
+long hip_stub_matrix_launches(void) { return g_matrix.load(); }
 void hip_stub_set_elapsed_ms(float general_ms, float wide4_ms) {
   g_elapsed_general = general_ms;
   g_elapsed_wide4 = wide4_ms;
@@ -209,7 +210,10 @@ hipError_t launch_lookup(const LookupArgs& a, bool, hipStream_t) {
   if (a.rank_offsets) (void)*(volatile const int64_t*)&a.rank_offsets[0];
   return LAUNCHED();
 }
-hipError_t launch_lookup_matrix(const LookupArgs& a, bool idx64, bool, bool, hipStream_t s) { return launch_lookup(a, idx64, s); }
+hipError_t launch_lookup_matrix(const LookupArgs& a, bool idx64, bool, bool, hipStream_t s) {
+  ++g_matrix;
+  return launch_lookup(a, idx64, s);
+}
 hipError_t launch_lookup_lean(const LookupArgs& a, bool idx64, bool, bool wide4, hipStream_t s) {
   if (wide4) { // the redo queue of that instance must be there, and as long as the work list
     if (!a.redo || !a.redo_count) return hipErrorInvalidValue;

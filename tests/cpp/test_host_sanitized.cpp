@@ -597,6 +597,29 @@ void refused_checked_forwards_keep_no_turn() {
   CHECK(fbgemm_amd_set_matrix(-1) == 0);
 }
 
+// The matrix kernel counts the entries of a run in 31 bits: forwards whose bags could be longer are not its
+void forwards_beyond_the_matrix_kernels_runs() {
+  Problem p;
+  p.T = 2;
+  p.tys = {3, 3};
+  p.D_offsets = {0, 256, 512};
+  p.wo = {0, 16384};
+  p.bytes = 32768;
+  const int64_t B = 9000;
+  Buffers b(p, B, 16); // no kernel reads the indices here
+  fbgemm_amd_tbe_plan* plan = nullptr;
+  CHECK(fbgemm_amd_tbe_plan_create(&plan, p.T, p.wo.data(), p.tys.data(), p.D_offsets.data(), nullptr, p.bytes, 0, 16) == 0);
+  CHECK(fbgemm_amd_tbe_plan_set_accumulate(plan, FBGEMM_AMD_ACC_FAST) == 0);
+  long before = hip_stub_matrix_launches();
+  for (int64_t n : {int64_t(1) << 20, fbgemm_amd::MATRIX_MAX_RUN}) {
+    CHECK(forward(plan, p, b, B, n, hip_stub_stream(0)) == 0);
+    CHECK(hip_stub_matrix_launches() == ++before);
+  }
+  for (int64_t n : {fbgemm_amd::MATRIX_MAX_RUN + 1, int64_t(0x7fffffff), int64_t(1) << 33}) CHECK(forward(plan, p, b, B, n, hip_stub_stream(0)) == 0);
+  CHECK(hip_stub_matrix_launches() == before);
+  fbgemm_amd_tbe_plan_destroy(plan);
+}
+
 // Records of mappings, a plan's and a caller's, where an allocation fails: the call says so, leaves nothing behind, no
 // error for the next launch to find either, and works once memory is there
 void records_without_memory() {
@@ -638,6 +661,7 @@ void lists_that_one_grid_cannot_hold() {
 
 int main() {
   lists_that_one_grid_cannot_hold();
+  forwards_beyond_the_matrix_kernels_runs();
   records_without_memory();
   plan_of_wide_4bit_tables();
   plan_create_failures();
