@@ -1193,6 +1193,7 @@ struct fbgemm_amd_tbe_plan {
   int32_t fp8_shift = 0; // FP8 rows: set by fbgemm_amd_tbe_plan_set_fp8
   float fp8_mult = 0.0f;
   bool has_fp8 = false;
+  int64_t matrix_forwards = 0; // fbgemm_amd_tbe_plan_matrix_forwards
   bool reuse_order = false; // benchmarks: forwards skip the scheduler and take the last bag order of their stream
 };
 
@@ -1798,6 +1799,7 @@ int tbe_forward_impl(
         !burst.waves && variant != 2 && (uintptr_t)d_output % 16 == 0 && it->second.lean.num_waves > 0 && (it->second.general.num_waves == 0 || ordered)) {
       if (!it->second.matrix_made && !capturing) make_matrix_list(plan, tables, B, &it->second);
       use_matrix = it->second.matrix.num_waves > 0;
+      plan->matrix_forwards += use_matrix;
     }
     // this stream's bag-order buffer: the one it has, else one nobody has claimed, else (outside
     // a capture) a new one; with all of that exhausted the first buffer is shared, and forwards
@@ -2285,6 +2287,12 @@ int fbgemm_amd_tbe_plan_reuse_order(fbgemm_amd_tbe_plan* plan, int32_t on) {
   std::lock_guard<std::mutex> lk(plan->mu);
   plan->reuse_order = on != 0;
   return 0;
+}
+
+int64_t fbgemm_amd_tbe_plan_matrix_forwards(fbgemm_amd_tbe_plan* plan) {
+  if (!plan) return 0;
+  std::lock_guard<std::mutex> lk(plan->mu);
+  return plan->matrix_forwards;
 }
 
 namespace {

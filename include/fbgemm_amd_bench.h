@@ -44,7 +44,8 @@ int fbgemm_amd_bench_gather(const void* d_table, int64_t rows, int64_t row_strid
                             void* stream);
 
 /* ---- libfbgemm_amd.so: process-wide switches ----------------------------------- *
- * Results are bit-identical under every setting. Not synchronised: set them while
+ * Results are bit-identical under every setting, but for the sums of the matrix
+ * kernel (tolerance-grade forwards only). Not synchronised: set them while
  * no other thread is inside the library.
  * fbgemm_amd_set_lean: 1 = shapes the lean kernel takes go to it (the default,
  * also FBGEMM_AMD_LEAN in the environment at load time), 0 = everything goes
@@ -75,6 +76,10 @@ int fbgemm_amd_set_wide4(int32_t mode);
  * is the lookup kernels back to back and a pair of events around the run gives
  * their average duration. 0 switches it off. */
 int fbgemm_amd_tbe_plan_reuse_order(struct fbgemm_amd_tbe_plan* plan, int32_t on);
+
+/* How many forwards of the plan have gone to the matrix kernel, captured ones
+ * among them: what a test of that kernel asks before it believes its result. */
+int64_t fbgemm_amd_tbe_plan_matrix_forwards(struct fbgemm_amd_tbe_plan* plan);
 
 #ifdef __cplusplus
 }
