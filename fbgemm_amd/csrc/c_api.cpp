@@ -1790,11 +1790,11 @@ int tbe_forward_impl(
     // Refused before the forward takes anything of the work set that only its end gives back (the turn to measure).
     if (checked && !burst.waves && ((!exact && it->second.lean.num_waves > 0) || (d_index_remappings && it->second.general.num_waves > 0)))
       return FORWARD_NOT_TAKEN;
-    // Unweighted forwards in the tolerance-grade mode whose lean tables the matrix kernel takes all: it is the faster one
-    // wherever the lean kernels would get the 16-byte lanes (of 88 forwards of one row type and width, 12 000 to 500 000 bags of
-    // 2 to 100 rows, .38 to 1.01 of their time, .77 on average; calls of 9 to 11 us, which their submission bounds, to 1.03). Tables for the general kernel run beside it on the side
-    // stream, in forwards of the size that has one; smaller ones stay with the launch of both kernels (41 tables x 363 x 16,
-    // three of them 2-bit: 20.6 us there, 29.6 one behind the other).
+    // Unweighted forwards in the tolerance-grade mode whose lean tables the matrix kernel takes all. Where the lean kernels
+    // would get the 16-byte lanes it takes, of 88 forwards of one row type and width, 12 000 to 500 000 bags of 2 to 100 rows,
+    // .38 to 1.01 of their time, .77 on average; in calls of 9 to 11 us, which their submission bounds, up to 1.03. Tables for the
+    // general kernel run beside it on the side stream, in forwards of the size that has one; smaller ones stay with the launch
+    // of both kernels (41 tables x 363 x 16, three of them 2-bit: 20.6 us there, 29.6 one behind the other).
     if (g_matrix_override != 0 && !exact && !checked && !d_indice_weights && !d_index_remappings && !d_q8_out && indices_numel <= MATRIX_MAX_RUN &&
         !burst.waves && variant != 2 && (uintptr_t)d_output % 16 == 0 && it->second.lean.num_waves > 0 && (it->second.general.num_waves == 0 || ordered)) {
       if (!it->second.matrix_made && !capturing) make_matrix_list(plan, tables, B, &it->second);

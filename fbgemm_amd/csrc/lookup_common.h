@@ -204,7 +204,7 @@ struct LookupArgs {
   WaveWork* redo;
   int32_t* redo_count;
   int32_t lengths;           // burst kernel, single tables only: `offsets` holds B lengths
-  int32_t wave_bags;         // lookup_matrix_kernel only: bags a wave pools, 8, 16 or 32
+  int32_t wave_bags;         // lookup_matrix_kernel only: bags a wave pools, 8 or 16
   Status* status;
   // A checked forward (fbgemm_amd_tbe_forward_checked): an index outside its table reads row 0 and is counted instead of
   // reported; offsets that are not in order from 0 to index_size are reported.

@@ -255,11 +255,11 @@ hipError_t launch_lookup_lean(const LookupArgs& a, bool idx64, bool exact, bool 
 hipError_t launch_lookup_matrix_i64(const LookupArgs& a, bool int4, bool wide, unsigned blocks, hipStream_t stream);
 hipError_t launch_lookup_matrix_i32(const LookupArgs& a, bool int4, bool wide, unsigned blocks, hipStream_t stream);
 
-// The matrix kernel (lookup_matrix.h) over a work list of eight bags a wave whose tables it takes.
+// The matrix kernel (lookup_matrix.h) over a work list of `wave_bags` bags a wave whose tables it takes.
 hipError_t launch_lookup_matrix(const LookupArgs& a, bool idx64, bool int4, bool wide, hipStream_t stream) {
   if (a.num_waves <= 0) return hipSuccess;
   const int64_t blocks = 8 * a.num_waves;
-  if (blocks > 0x7fffffffLL || a.wave_bags < 8 || a.wave_bags > 64 || a.wave_bags % 8 || !a.tables || !a.work || !a.xcd_start || !a.out_aligned || a.sample_weights || a.remap || a.check_rows || a.check_total || a.index_size > MATRIX_MAX_RUN ||
+  if (blocks > 0x7fffffffLL || (a.wave_bags != 8 && a.wave_bags != 16) || !a.tables || !a.work || !a.xcd_start || !a.out_aligned || a.sample_weights || a.remap || a.check_rows || a.check_total || a.index_size > MATRIX_MAX_RUN ||
       a.out_ty == ST_INT8)
     return hipErrorInvalidValue;
   return idx64 ? launch_lookup_matrix_i64(a, int4, wide, (unsigned)blocks, stream) : launch_lookup_matrix_i32(a, int4, wide, (unsigned)blocks, stream);
